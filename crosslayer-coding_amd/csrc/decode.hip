@@ -197,7 +197,7 @@ template <typename T, int NF, int TAIL, bool SLICED> constexpr int decode_min_wa
 constexpr int SLICED_NTOK = 4;   // tokens per wavefront in the sliced kernel
 
 // One wavefront per (target, token): walks all sources s <= t, accumulates in registers,
-// writes the output row once.  Used for small batches.
+// writes the output row once.  Used for small batches.  only_above >= 0: runs only if the list has more entries than that.
 //
 // SLICED (large batches): one launch per source layer `src`; one wavefront per
 // (target >= src, token, feature slice).  The feature axis is cut into `ns` slices and block b
@@ -220,7 +220,8 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<T, NF, TAIL, SLICED>(), 8)))
     const T *__restrict__ fscale, const float *__restrict__ skip_add, void *__restrict__ out,
     int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end,
     uint64_t src_mask, int out_f32, const int32_t *__restrict__ sptr, float *__restrict__ partial, int ns,
-    int src, int64_t pitch) {
+    int src, int64_t pitch, int64_t only_above) {
+  if (!SLICED && only_above >= 0 && row_ptr[L * Tn] <= only_above) return;
   constexpr int V = WVec<T>::V;
   constexpr int HV = V / 2;                       // elements per 8 bytes
   constexpr int NACC = NF * V + (TAIL == 1 ? HV : TAIL == 2 ? V : 0);
@@ -875,7 +876,9 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_decode_generic(
     const int32_t *row_ptr, const int32_t *col, const T *val, const T *wp, const float *bias_sum,
     const T *foff, const T *fscale, const float *skip_add, void *out, int64_t Tn, int64_t d,
-    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch) {
+    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch,
+    int64_t only_above) {
+  if (only_above >= 0 && row_ptr[L * Tn] <= only_above) return;
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int64_t blocks_per_t = (Tn + nwv - 1) / nwv;
   const int64_t t = t_end - 1 - (int64_t)blockIdx.x / blocks_per_t;
@@ -1218,7 +1221,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
                          const float *bias_sum, const void *foff, const void *fscale, const float *skip_add,
                          void *out, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
                          int64_t t_end, uint64_t src_mask, int out_f32, void *workspace, size_t workspace_bytes,
-                         hipStream_t stream) {
+                         hipStream_t stream, int64_t only_above = -1) {
   constexpr int V = WVec<T>::V;
   const int nwv = 4;
   const int64_t pitch = clt_pitch(d, (int)sizeof(T));
@@ -1244,7 +1247,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
                             L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, stream);
 #define CLT_DEC_ARGS(FO, FS)                                                                                    \
   row_ptr, col, (const T *)val, (const T *)wp, bias_sum, FO, FS, skip_add, out, Tn, d, F, L, tying, tb,         \
-      t_end, src_mask, out_f32, sptr, partial, ns, src, pitch
+      t_end, src_mask, out_f32, sptr, partial, ns, src, pitch, only_above
 #define CLT_DEC(NFN, TL, UN)                                                                                    \
   do {                                                                                                          \
     if (affine && can_slice)                                                                                    \
@@ -1359,7 +1362,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
   } else {
     const int64_t tb = t_begin; const int src = 0; (void)tb; (void)src;
     k_decode_generic<T><<<(unsigned)nblk, 256, 0, stream>>>(row_ptr, col, (const T *)val, (const T *)wp, bias_sum,
-        (const T *)foff, (const T *)fscale, skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, pitch);
+        (const T *)foff, (const T *)fscale, skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, pitch, only_above);
   }
 #undef CLT_DEC_TAIL
 #undef CLT_DEC
@@ -1394,6 +1397,21 @@ extern "C" int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, con
   if (dtype == CLT_F16)
     return launch_decode<f16_t>(row_ptr, col, val, w_packed, bias_sum, feat_offset, feat_scale, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, workspace, workspace_bytes, s);
   return launch_decode<float>(row_ptr, col, val, w_packed, bias_sum, feat_offset, feat_scale, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, workspace, workspace_bytes, s);
+}
+
+extern "C" int clt_decode_sparse_if_over(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                                         const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d,
+                                         int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask,
+                                         int dtype, int out_f32, int64_t max_entries, void *stream) {
+  if (dtype != CLT_BF16 && dtype != CLT_F16) return CLT_ERR_DTYPE;
+  if (T < 0 || d <= 0 || F <= 0 || L <= 0 || L > 64 || max_entries < 0) return CLT_ERR_ARG;
+  if (t_begin < 0 || t_end > L || t_begin > t_end || tying < 0 || tying > 2) return CLT_ERR_ARG;
+  if (T == 0 || t_begin == t_end) return CLT_OK;
+  if (!row_ptr || !w_packed || !out) return CLT_ERR_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == CLT_BF16)
+    return launch_decode<bf16_t>(row_ptr, col, val, w_packed, bias_sum, nullptr, nullptr, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, s, max_entries);
+  return launch_decode<f16_t>(row_ptr, col, val, w_packed, bias_sum, nullptr, nullptr, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, s, max_entries);
 }
 
 extern "C" int clt_pack_decoder(const void *w_ref, void *w_packed, int64_t d, int64_t F, int64_t n_dec,

@@ -1,0 +1,510 @@
+// Sparse cross-layer decode on the matrix cores (reference clt/models/decoder.py:176-340): decoder rows are gathered
+// from LDS tiles instead of from the L2 (spmm.h says why).
+//
+//   k_rec_count / k_rec_streams / k_rec_fill
+//                   survivor list (CSR by token) -> one stream of batches per wavefront of k_decode_tiles, in the order
+//                   in which it consumes them: by source, tile of SP_ROWS features, group of 16 tokens
+//   k_decode_tiles  one workgroup per (target, 64 columns, part of the tokens): every tile of every source's decoder
+//                   passes through LDS once, the sums stay in registers over all sources and features
+#include "spmm.h"
+
+namespace {
+
+__device__ __forceinline__ int64_t sp_slot(int tying, int64_t s, int64_t t, int64_t L) {
+  return tying == CLT_TYING_PER_SOURCE ? s : s * L - (s * (s - 1)) / 2 + (t - s);
+}
+
+constexpr int DT_WAVES = 16;
+constexpr int DT_GPW = 4;                  // groups of 16 tokens per wavefront: 64 accumulators per lane
+
+// Groups part * groups_per_part + wave + 16 gi of a part of the tokens belong to wavefront `wave`; the batches of its
+// groups, ordered by (source, tile, gi), are its stream.
+struct TilePlan {
+  int tiles, groups, parts, groups_per_part, streams, stages;
+  __host__ __device__ __forceinline__ int group(int stream, int gi) const {        // -1: none
+    const int part = stream / DT_WAVES, r = stream % DT_WAVES + gi * DT_WAVES, g = part * groups_per_part + r;
+    return r < groups_per_part && g < groups ? g : -1;
+  }
+};
+
+// ---- records ----------------------------------------------------------------------------------------
+constexpr int REC_THREADS = 256;
+constexpr int REC_MAX_TILES = 512;
+constexpr int REC_WINDOW = 128;            // batches put together in LDS at a time
+
+struct RecArgs {
+  const int32_t *row_ptr, *col;
+  const void *val;
+  int64_t Tn, L, max_entries;
+  uint64_t src_mask;
+  TilePlan p;
+  int32_t *start;          // [L * groups][SP_GROUP][tiles + 1] list position where a token's entries of a tile begin
+  uint16_t *batches;       // [L * tiles][groups] batches of (source, tile, group)
+  uint16_t *counts;        // [streams][stages][DT_GPW] the same by stream
+  uint32_t *offset;        // [streams][stages] batches of the stream before the stage
+  uint32_t *total;         // [streams] batches of the stream
+  uint32_t *recs;
+};
+
+// One workgroup per (group of 16 tokens, source).  Rows are sorted by feature, so a token's entries of one tile are a
+// run, found by binary search.  A layer outside src_mask counts as empty.
+__global__ __launch_bounds__(REC_THREADS) void k_rec_count(RecArgs A) {
+  extern __shared__ int32_t run_lds[];
+  if (A.row_ptr[A.L * A.Tn] > A.max_entries) return;      // more entries than the workspace was sized for
+  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles;
+  const int64_t tok0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Tn + tok0;
+  const bool on = (A.src_mask >> s) & 1ull;
+  int32_t *out = A.start + ((int64_t)s * A.p.groups + g) * SP_GROUP * (tiles + 1);
+  for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) {
+    const int tk = i / (tiles + 1), c = i - tk * (tiles + 1);
+    int32_t lo = 0;
+    if (on && tok0 + tk < A.Tn) {
+      int32_t hi = A.row_ptr[r0 + tk + 1];
+      lo = A.row_ptr[r0 + tk];
+      const int32_t bound = c * SP_ROWS;
+      if (c == tiles) lo = hi;
+      while (lo < hi) {
+        const int32_t mid = lo + ((hi - lo) >> 1);
+        if (A.col[mid] < bound) lo = mid + 1; else hi = mid;
+      }
+    }
+    run_lds[i] = lo;
+    out[i] = lo;
+  }
+  __syncthreads();
+  for (int c = tid; c < tiles; c += REC_THREADS) {
+    int32_t n = 0;
+#pragma unroll
+    for (int tk = 0; tk < SP_GROUP; ++tk) n += run_lds[tk * (tiles + 1) + c + 1] - run_lds[tk * (tiles + 1) + c];
+    A.batches[((int64_t)s * tiles + c) * A.p.groups + g] = (uint16_t)((n + SP_BATCH - 1) / SP_BATCH);
+  }
+}
+
+// One wavefront per stream: its batch counts per stage and where each stage begins.
+__global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
+  if (A.row_ptr[A.L * A.Tn] > A.max_entries) return;
+  const int stream = blockIdx.x, lane = threadIdx.x;
+  uint32_t run = 0;
+  for (int st0 = 0; st0 < A.p.stages; st0 += 64) {
+    const int st = st0 + lane;
+    uint32_t n[DT_GPW], sum = 0;
+#pragma unroll
+    for (int gi = 0; gi < DT_GPW; ++gi) {
+      const int g = A.p.group(stream, gi);
+      n[gi] = st < A.p.stages && g >= 0 ? A.batches[(int64_t)st * A.p.groups + g] : 0u;
+      sum += n[gi];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(incl, o);
+      if (lane >= o) incl += up;
+    }
+    if (st < A.p.stages) {
+      A.offset[(int64_t)stream * A.p.stages + st] = run + incl - sum;
+      *reinterpret_cast<uint2 *>(A.counts + ((int64_t)stream * A.p.stages + st) * DT_GPW) =
+          make_uint2(n[0] | (n[1] << 16), n[2] | (n[3] << 16));
+    }
+    run += __shfl(incl, 63);
+  }
+  if (lane == 0) A.total[stream] = run;
+}
+
+// first batch of a stream: those of the streams before it (all lanes of a wavefront take part)
+__device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stream, int lane) {
+  uint32_t n = 0;
+  for (int i = lane; i < stream; i += 64) n += total[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  return n;
+}
+
+// One workgroup per (group, source) again: the runs of a tile laid end to end in token order - a fixed order of every
+// sum - put together in LDS, REC_WINDOW batches at a time, and written out lane by lane.
+template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(RecArgs A) {
+  extern __shared__ int32_t fill_lds[];
+  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
+  if (A.row_ptr[A.L * A.Tn] > A.max_entries || !((A.src_mask >> s) & 1ull)) return;
+  int32_t *start = fill_lds;                               // [SP_GROUP][tiles + 1]
+  int32_t *off = start + SP_GROUP * (tiles + 1);           // [SP_GROUP][tiles] entries of the tile before this token's
+  int32_t *first = off + SP_GROUP * tiles;                 // [tiles + 1] first batch of the tile, counted within the group
+  uint32_t *dest = (uint32_t *)(first + tiles + 1);        // [tiles] its place among all batches
+  uint32_t *where = dest + tiles;                          // [REC_WINDOW] the same per batch of the window
+  uint16_t *win = (uint16_t *)(where + REC_WINDOW);        // [REC_WINDOW][64] words
+  const int64_t tok0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Tn + tok0;
+  const int32_t *src = A.start + ((int64_t)s * A.p.groups + g) * SP_GROUP * (tiles + 1);
+  for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) start[i] = src[i];
+  __syncthreads();
+  const int part = g / A.p.groups_per_part, r = g - part * A.p.groups_per_part;
+  const int stream = part * DT_WAVES + r % DT_WAVES, gi = r / DT_WAVES;
+  const int stage0 = __popcll(A.src_mask & ((1ull << s) - 1ull)) * tiles;      // stages of a decode before this source's
+  for (int c = tid; c < tiles; c += REC_THREADS) {
+    int32_t n = 0;
+#pragma unroll
+    for (int tk = 0; tk < SP_GROUP; ++tk) {
+      off[tk * tiles + c] = n;
+      n += start[tk * (tiles + 1) + c + 1] - start[tk * (tiles + 1) + c];
+    }
+    first[c] = (n + SP_BATCH - 1) / SP_BATCH;              // batches for now
+    const int64_t at = (int64_t)stream * A.p.stages + (int64_t)s * tiles + c;
+    uint32_t d = A.offset[at];
+    for (int j = 0; j < gi; ++j) d += A.counts[at * DT_GPW + j];
+    dest[c] = d;
+  }
+  const uint32_t base = stream_first(A.total, stream, lane);
+  __syncthreads();
+  if (tid < 64) {
+    int32_t run = 0;
+    for (int c0 = 0; c0 < tiles; c0 += 64) {
+      const int c = c0 + lane;
+      const int32_t nb = c < tiles ? first[c] : 0;
+      int32_t incl = nb;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t up = __shfl_up(incl, o);
+        if (lane >= o) incl += up;
+      }
+      if (c < tiles) first[c] = run + incl - nb;
+      run += __shfl(incl, 63);
+    }
+    if (lane == 0) first[tiles] = run;
+  }
+  __syncthreads();
+  const int32_t nb_all = first[tiles];
+  for (int32_t w0 = 0; w0 < nb_all; w0 += REC_WINDOW) {
+    const int32_t wn = nb_all - w0 < REC_WINDOW ? nb_all - w0 : REC_WINDOW;
+    for (int i = tid; i < wn * 32; i += REC_THREADS) reinterpret_cast<uint2 *>(win)[i] = make_uint2(0u, 0u);
+    for (int c = tid; c < tiles; c += REC_THREADS)
+      for (int32_t b = first[c]; b < first[c + 1]; ++b)
+        if (b >= w0 && b < w0 + wn) where[b - w0] = base + dest[c] + (uint32_t)(b - first[c]);
+    __syncthreads();
+    for (int tk = tid >> 6; tk < SP_GROUP; tk += REC_THREADS / 64) {
+      if (tok0 + tk >= A.Tn) break;
+      const int32_t e = A.row_ptr[r0 + tk + 1];
+      for (int32_t j = A.row_ptr[r0 + tk] + lane; j < e; j += 64) {
+        const int32_t f = A.col[j], c = f / SP_ROWS;
+        const int32_t p = off[tk * tiles + c] + j - start[tk * (tiles + 1) + c];
+        const int32_t b = first[c] + p / SP_BATCH - w0, k = p % SP_BATCH;
+        if (b < 0 || b >= wn) continue;
+        uint16_t *rec = win + b * 128 + (k >> 3) * 32;      // 16 lanes of two halves each
+        const int x = (k & 7) >> 1, half = k & 1;
+        rec[(4 * x + 0) * 2 + half] = (uint16_t)Elem<T>::raw(((const T *)A.val)[j]);
+        rec[(4 * x + 1) * 2 + half] = (uint16_t)(1u << tk);
+        rec[(4 * (k & 3) + 3) * 2 + ((k >> 2) & 1)] =
+            (uint16_t)sp_half_place((uint32_t)(f - c * SP_ROWS), (uint32_t)(stage0 + c) & 1u);
+      }
+    }
+    __syncthreads();
+    for (int32_t b = tid >> 6; b < wn; b += REC_THREADS / 64) {
+      A.recs[(uint64_t)where[b] * 64 + lane] = reinterpret_cast<const uint32_t *>(win)[b * 64 + lane];
+    }
+    __syncthreads();
+  }
+}
+
+// ---- decode -----------------------------------------------------------------------------------------
+struct TileArgs {
+  TilePlan p;
+  const uint16_t *counts;
+  const uint32_t *total;
+  const uint32_t *recs;
+  const void *wp;
+  const float *bias_sum, *skip_add;
+  void *out;
+  const int32_t *list_total;               // survivors of the batch
+  int64_t max_entries, Tn, d, F, L, pitch;
+  uint64_t src_mask;
+  int tying, t_begin, t_end, out_f32, col_parts;
+};
+
+constexpr int DT_FILLS = SP_ROWS / 8 / DT_WAVES;           // direct-to-LDS loads of a tile per wavefront
+constexpr int DT_RING = 8;                                 // records a wavefront keeps in LDS or on their way
+constexpr int DT_LDS = 2 * SP_TILE_BYTES + DT_WAVES * DT_RING * 256;
+static_assert(DT_FILLS == 4 && DT_RING == 8, "the wait counts below are written out");
+
+// Direct-to-LDS loads, 16 or 4 bytes per lane (lane i lands at lds_at + 16 i / 4 i).  As asm statements, so that the
+// compiler does not wait for them in front of every LDS read; whoever reads the data waits by hand.
+__device__ __forceinline__ void fill16(const char *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+__device__ __forceinline__ void fill4(const uint32_t *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+
+// Two tiles of 512 features x 64 columns in LDS, one being multiplied while the other comes in.  Each wavefront owns four
+// groups of 16 tokens and consumes its stream of batches through a ring of eight records in LDS: the vector memory path
+// returns in order, so a record waits behind whatever tile lines were asked for before it, and eight batches (~2 us)
+// cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so a tile
+// comes from HBM once.
+//
+// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.16 ms (98.6 GB of gathered rows, 31
+// TB/s) and 0.14 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 16.3 against
+// 34.2 ms.  Bound by LDS: 19 ns per batch and CU are 2.2 ms, of which 0.5 for the entries that fill batches up; 0.25 ms
+// are wavefronts waiting for the slowest one of a stage, 0.3 ms records queueing behind tile lines that come from HBM.
+// Measured and dropped: a wavefront of its own for the fills (fifteen share 64 groups badly: 3.98 ms); fewer lines on
+// their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought into the L2 early
+// (3.46 ms: the early loads block the records just as well).
+template <typename T>
+__global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
+  extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  if (*A.list_total > A.max_entries) return;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int pair = (seq / A.p.parts) * 8 + xcd, part = seq % A.p.parts;
+  if (pair >= (A.t_end - A.t_begin) * A.col_parts) return;
+  const int t = A.t_end - 1 - pair / A.col_parts, cp = pair % A.col_parts;      // longest first
+  const uint64_t mask = A.src_mask & ((2ull << t) - 1ull);
+  const int n_stages = __popcll(mask) * A.p.tiles;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)tile_lds;
+  const int stream = part * DT_WAVES + wave;
+
+  // This wavefront's share of a tile: 32 rows, sixteen at a time and one half of the columns at a time, 16 bytes of row
+  // lane / 4 per lane; which 16 bytes a lane brings is what exchanges the pieces.  (Both halves of a line are asked for
+  // one after the other: the second hits the L1.)
+  const uint32_t pitch_b = (uint32_t)(A.pitch * (int64_t)sizeof(T));
+  const uint32_t col_b = (((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4);
+  const int row_a = wave * 32 + (lane >> 2);
+  const uint32_t off_a = (uint32_t)row_a * pitch_b + col_b;
+  auto fill = [&](const char *src, int rows, uint32_t lds_at) {
+    if (rows >= SP_ROWS) {
+#pragma unroll
+      for (int i = 0; i < DT_FILLS; ++i)
+        fill16(src + (i & 1) * 64, off_a + (uint32_t)(i >> 1) * 16 * pitch_b, lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+    } else {                                               // past the matrix: nobody refers to these rows
+#pragma unroll
+      for (int i = 0; i < DT_FILLS; ++i) {
+        const int r = row_a + (i >> 1) * 16;
+        fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
+               lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+      }
+    }
+  };
+
+  auto tile_at = [&](int s) {
+    return (const char *)A.wp + sp_slot(A.tying, s, t, A.L) * A.F * (int64_t)pitch_b + (int64_t)cp * 128;
+  };
+
+  f32x4v_t acc[DT_GPW][4];
+#pragma unroll
+  for (int gi = 0; gi < DT_GPW; ++gi)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[gi][n] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
+
+  if (n_stages > 0) {
+    const uint32_t row_bit = 0x00010001u << (lane & 15);
+    const uint32_t ring = lds0 + 2 * SP_TILE_BYTES + (uint32_t)wave * (DT_RING * 256);
+    const uint32_t *recs = A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(stream_first(A.total, stream, lane)) * SP_REC_WORDS;
+    uint32_t rec_off = (uint32_t)lane * 4;                 // of the next record to ask for, this lane's word
+    uint32_t slot = 0;                                     // of the batch that is consumed next, in bytes
+    auto ask = [&](uint32_t at) {                          // the next record of the stream into the ring
+      fill4(recs, rec_off, ring + at);
+      rec_off += SP_REC_WORDS * 4;
+    };
+    uint32_t word;                                         // of the record after the batch at hand
+    const uint32_t ring_lane = ring + (uint32_t)lane * 4;
+    auto look = [&](uint32_t at) { word = *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)(ring_lane + at); };
+    // the next tile to bring in: where it begins and how many rows of the matrix are left from there on
+    uint64_t m = mask;
+    int s = __ffsll((unsigned long long)m) - 1, c = 0, rows = (int)A.F;
+    const char *tile = tile_at(s);
+    const uint32_t tile_step = SP_ROWS * pitch_b, lds_share = lds0 + (uint32_t)wave * 2048;
+    fill(tile, rows, lds_share);
+#pragma unroll
+    for (int i = 0; i < DT_RING; ++i) ask((uint32_t)i * 256);
+    const auto counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages;
+    uint2 cnt = make_uint2(counts[s * A.p.tiles].x, counts[s * A.p.tiles].y);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    look(0);
+    const uint32_t col = lds0 + (uint32_t)(lane & 3) * 8;
+    SpBatch<T> bt;
+    // The next batch's record becomes addresses and values, its slot in the ring the place of the one eight batches on.
+    // `since`: records asked for since the last tile's lines.
+    auto prepare = [&](int since) {
+      bt.address(word, col);
+      bt.read();                                           // (in vain if its tile is still on its way: read again then)
+      bt.pick(word, row_bit);
+      asm volatile("" ::"v"(bt.picked), "v"(bt.a0), "v"(bt.a1));        // the slot has been read
+      ask(slot);
+      slot = (slot + 256) & (DT_RING * 256 - 1);
+      // the record after it: seven were asked for since, and perhaps the four loads of a tile
+      asm volatile("s_cmp_lt_i32 %0, 8\n\ts_cbranch_scc1 .Lnot_late%=\n\ts_waitcnt vmcnt(7)\n.Lnot_late%=:\n\ts_waitcnt vmcnt(11)" ::"s"(since)
+                   : "scc", "memory");
+      look(slot);
+    };
+    prepare(DT_RING);
+    for (int st = 0; st < n_stages; ++st) {
+      const bool more = st + 1 < n_stages;
+      if (more) {
+        tile += tile_step;
+        rows -= SP_ROWS;
+        if (++c == A.p.tiles) {
+          c = 0;
+          m &= m - 1;
+          s = __ffsll((unsigned long long)m) - 1;
+          tile = tile_at(s);
+          rows = (int)A.F;
+        }
+      }
+      const int at = s * A.p.tiles + c;
+      const uint2 cnt_next = make_uint2(counts[at].x, counts[at].y);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();                        // tile st is complete, and nobody reads the other one any more
+      asm volatile("" ::: "memory");
+      bt.read();
+      if (more) fill(tile, rows, lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES);
+      int since = more ? 0 : DT_RING;                      // records asked for after these lines
+#pragma unroll
+      for (int gi = 0; gi < DT_GPW; ++gi) {
+        const int n = (int)((gi & 2 ? cnt.y : cnt.x) >> (gi & 1 ? 16 : 0)) & 0xFFFF;
+        for (int i = n; i > 0; --i) {
+          bt.finish(acc[gi]);
+          prepare(++since);
+        }
+      }
+      cnt = cnt_next;
+      // the tile's lines are waited for, not the records asked for behind them
+      if (since >= DT_RING) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      else if (since >= DT_RING / 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may be on its way into LDS when the workgroup ends
+  }
+
+#pragma unroll
+  for (int gi = 0; gi < DT_GPW; ++gi) {
+    const int g = A.p.group(stream, gi);
+    const int64_t tok = (int64_t)g * SP_GROUP + (lane & 15);
+    if (g < 0 || tok >= A.Tn) continue;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int64_t o = (int64_t)cp * SP_COLS + n * 16 + (lane >> 4) * 4;
+      f32x4v_t a = acc[gi][n];
+      const int64_t at = ((int64_t)t * A.Tn + tok) * A.d + o;
+      if (A.bias_sum) a += *reinterpret_cast<const f32x4v_t *>(A.bias_sum + (int64_t)t * A.d + o);
+      if (A.skip_add) a += *reinterpret_cast<const f32x4v_t *>(A.skip_add + at);
+      if (A.out_f32) *reinterpret_cast<f32x4v_t *>((float *)A.out + at) = a;
+      else *reinterpret_cast<uint2 *>((uint16_t *)A.out + at) = make_uint2(pack_pair<T>(a[0], a[1]), pack_pair<T>(a[2], a[3]));
+    }
+  }
+}
+
+static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+struct TileLayout {
+  TilePlan p;
+  int col_parts;
+  int64_t n_batches;
+  size_t start, batches, counts, offset, total, recs, bytes;
+};
+
+static TileLayout tile_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {
+  TileLayout l;
+  TilePlan &p = l.p;
+  p.tiles = (int)clt_ceil_div(F, SP_ROWS);
+  p.groups = (int)clt_ceil_div(Tn, SP_GROUP);
+  p.stages = (int)(L * p.tiles);
+  l.col_parts = (int)(d / SP_COLS);
+  // as many tokens per workgroup as its registers hold, unless that leaves compute units idle
+  for (int gpw = DT_GPW; gpw > 0; --gpw) {
+    p.parts = (int)clt_ceil_div(p.groups, DT_WAVES * gpw);
+    if ((int64_t)p.parts * l.col_parts * targets >= 512) break;
+  }
+  p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
+  p.streams = p.parts * DT_WAVES;
+  // every (source, tile, group) may leave its last batch part empty; a stream reads DT_RING batches past its end
+  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + DT_RING;
+  size_t at = 0;
+  auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
+  l.start = take(sizeof(int32_t) * (size_t)L * p.groups * SP_GROUP * (p.tiles + 1));
+  l.batches = take(sizeof(uint16_t) * (size_t)p.stages * p.groups);
+  l.counts = take(sizeof(uint16_t) * (size_t)p.streams * p.stages * DT_GPW);
+  l.offset = take(sizeof(uint32_t) * (size_t)p.streams * p.stages);
+  l.total = take(sizeof(uint32_t) * (size_t)p.streams);
+  l.recs = take((size_t)l.n_batches * 256);
+  l.bytes = at;
+  return l;
+}
+
+// LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile; 16-bit batch counts
+static bool tile_shape_ok(const TileLayout &l, int64_t d) {
+  return l.p.tiles <= REC_MAX_TILES && l.n_batches <= 0x00FFFFFFll && clt_pitch(d, 2) * 2 * SP_ROWS <= 0x7FFFFFFFll &&
+         l.p.groups <= 0xFFFF && (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll;
+}
+
+template <typename T> static int launch_tiles(RecArgs ra, TileArgs ta, int col_parts, hipStream_t stream) {
+  const int tiles = ra.p.tiles;
+  const size_t count_lds = sizeof(int32_t) * (size_t)SP_GROUP * (tiles + 1);
+  const size_t fill_lds = sizeof(int32_t) * (size_t)(SP_GROUP * (tiles + 1) + SP_GROUP * tiles + 2 * tiles + 1 + REC_WINDOW) + REC_WINDOW * 256;
+  if (hipFuncSetAttribute((const void *)k_rec_fill<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds) != hipSuccess ||
+      hipFuncSetAttribute((const void *)k_decode_tiles<T>, hipFuncAttributeMaxDynamicSharedMemorySize, DT_LDS) != hipSuccess)
+    return CLT_ERR_LAUNCH;
+  const dim3 grid((unsigned)ra.p.groups, (unsigned)ra.L);
+  k_rec_count<<<grid, REC_THREADS, count_lds, stream>>>(ra);
+  k_rec_streams<<<(unsigned)ra.p.streams, 64, 0, stream>>>(ra);
+  k_rec_fill<T><<<grid, REC_THREADS, fill_lds, stream>>>(ra);
+  const int64_t pairs = clt_ceil_div((int64_t)(ta.t_end - ta.t_begin) * col_parts, 8) * 8;
+  k_decode_tiles<T><<<(unsigned)(pairs * ta.p.parts), DT_WAVES * 64, DT_LDS, stream>>>(ta);
+  return clt_check_launch();
+}
+
+}  // namespace
+
+// Both routes priced from what they measured (bf16; L 2 - 24, d 256 - 2048, F 4096 - 32768, T 256 - 8192, 17 - 216 survivors
+// per token): the gather moves its rows at 17 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage
+// of the tiles takes 1.0 us plus 20.5 ns per batch, but no less than the 2.24 us in which 64 KB come into LDS, and the
+// longest workgroup bounds a launch of few.  At the line the two differ by less than a fifth either way: e.g. L = 12,
+// d = 768, F = 24576: 200 survivors per token 6.25 / 3.31 ms at T = 4096, 2.03 / 1.57 at 1024, 1.23 / 1.25 at 512; 50 per
+// token 2.58 / 1.71 ms at 4096, 1.43 / 1.55 at 2048.
+extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
+                                       int dtype) {
+  if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return 0;
+  if (T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return 0;
+  const TileLayout l = tile_layout(T, d, F, L, targets, entries);
+  if (!tile_shape_ok(l, d)) return 0;
+  // (source, target) pairs of the last `targets` layers, and the survivors they gather
+  const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
+  const double sparse_us = rows * d * 2 / 17e6 + pairs * T * d * 16 / 3.2e6;
+  const double per_batch = (double)entries / ((double)l.p.stages * l.p.groups) / SP_BATCH + 0.5;
+  const double stage_us = 1.0 + l.p.groups_per_part * (per_batch > 1 ? per_batch : 1) * 0.0205;
+  const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
+  const double tiles_us = (stages > longest ? stages : longest) * (stage_us > 2.24 ? stage_us : 2.24) + 20 + entries * 1.25e-5;
+  return tiles_us < 0.95 * sparse_us;
+}
+
+extern "C" size_t clt_decode_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {
+  if (T <= 0 || d < SP_COLS || F <= 0 || L <= 0 || targets <= 0 || max_entries < 0) return 0;
+  return tile_layout(T, d, F, L, targets, max_entries).bytes;
+}
+
+extern "C" int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                                const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                                int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
+                                int64_t max_entries, void *workspace, size_t workspace_bytes, void *stream) {
+  if (dtype != CLT_BF16 && dtype != CLT_F16) return CLT_ERR_DTYPE;
+  if (T < 0 || d <= 0 || F <= 0 || L <= 0 || L > 64 || d % SP_COLS != 0 || max_entries < 0) return CLT_ERR_ARG;
+  if (t_begin < 0 || t_end > L || t_begin > t_end) return CLT_ERR_ARG;
+  if (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE) return CLT_ERR_ARG;
+  if (T == 0 || t_begin == t_end) return CLT_OK;
+  if (!row_ptr || !col || !val || !w_packed || !out || !workspace) return CLT_ERR_ARG;
+  if (!clt_aligned16(w_packed) || !clt_aligned16(out) || !clt_aligned16(workspace) || (bias_sum && !clt_aligned16(bias_sum)) ||
+      (skip_add && !clt_aligned16(skip_add)))
+    return CLT_ERR_ALIGN;
+  const int64_t pitch = clt_pitch(d, 2);
+  const TileLayout l = tile_layout(T, d, F, L, t_end - t_begin, max_entries);
+  if (!tile_shape_ok(l, d)) return CLT_ERR_RANGE;
+  if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
+  char *ws = (char *)workspace;
+  RecArgs ra;
+  ra.row_ptr = row_ptr; ra.col = col; ra.val = val; ra.Tn = T; ra.L = L; ra.max_entries = max_entries; ra.src_mask = src_mask;
+  ra.p = l.p;
+  ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint16_t *)(ws + l.counts);
+  ra.offset = (uint32_t *)(ws + l.offset); ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint32_t *)(ws + l.recs);
+  TileArgs ta;
+  ta.p = l.p; ta.counts = ra.counts; ta.total = ra.total; ta.recs = ra.recs;
+  ta.wp = w_packed; ta.bias_sum = bias_sum; ta.skip_add = skip_add; ta.out = out;
+  ta.list_total = row_ptr + L * T; ta.max_entries = max_entries;
+  ta.Tn = T; ta.d = d; ta.F = F; ta.L = L; ta.pitch = pitch; ta.src_mask = src_mask;
+  ta.tying = tying; ta.t_begin = (int)t_begin; ta.t_end = (int)t_end; ta.out_f32 = out_f32; ta.col_parts = l.col_parts;
+  if (dtype == CLT_BF16) return launch_tiles<bf16_t>(ra, ta, l.col_parts, (hipStream_t)stream);
+  return launch_tiles<f16_t>(ra, ta, l.col_parts, (hipStream_t)stream);
+}

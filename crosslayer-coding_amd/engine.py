@@ -850,7 +850,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
                   ws: Optional[Workspace] = None) -> torch.Tensor:
     """Reconstructions [L, T, d] for targets [t_begin, t_end) (decoder.py:176-340).
 
-    With a workspace and a batch large enough to fill the GPU the XCD-sliced kernel is used."""
+    With a workspace and a batch large enough to fill the GPU the matrix-core kernel (``clt_decode_tiles``) or one of the
+    XCD-sliced gathers is used, whichever ``clt_decode_tiles_wanted`` prices lower."""
     nat.require_device(w_packed, "decode_sparse")
     L, T, F = surv.L, surv.T, surv.F
     t_end = L if t_end is None else t_end
@@ -873,6 +874,24 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
     need = lib.clt_decoder_slab_elems(d, F, L, nat.TYING[tying], nat.dtype_code(surv.dtype))
     if need < 0 or w_packed.numel() < need:
         raise nat.CLTNativeError(f"decode_sparse: packed decoders hold {w_packed.numel()} elements, the kernels index {need}")
+    if ws is not None and feat_offset is None and feat_scale is None:
+        # the survivor total: exact, or (a threshold list, sized for any batch) the last one seen for this shape, or 1 %
+        # of the features before there is one
+        exact = surv.status is None
+        total = surv.capacity if exact else surv.nnz_hint
+        if total is None:
+            total = L * T * F // 100
+        if total and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
+            cap = total if exact else min(surv.capacity, 2 * total + 65536)
+            nbytes = lib.clt_decode_tiles_workspace_bytes(T, d, F, L, t_end - t_begin, cap)
+            wbuf = ws.get("decode_tiles", nbytes)
+            args = (nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum), nat.ptr(skip_add),
+                    nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin, t_end, src_mask & ((1 << 64) - 1),
+                    nat.dtype_code(surv.dtype), 1 if out_f32 else 0, cap)
+            nat.check(lib.clt_decode_tiles(*args, nat.ptr(wbuf), wbuf.numel(), _stream(w_packed)), "clt_decode_tiles")
+            if not exact:      # a batch that outgrew the estimate is decoded by the gather, decided on the device
+                nat.check(lib.clt_decode_sparse_if_over(*args, _stream(w_packed)), "clt_decode_sparse_if_over")
+            return out
     wbuf, wbytes = None, 0
     if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size()):
         wbytes = lib.clt_decode_workspace_bytes(T, d, F, L)

@@ -408,6 +408,26 @@ int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, const void *va
                       void *stream);
 
 /*
+ * The same sums (untied and per-source decoders, no feature offset / scale, bf16 and fp16, d a multiple of 64) on the
+ * matrix cores: the survivors are regrouped into batches by tiles of 512 features x 16 tokens and the decoder rows are
+ * gathered from LDS.  Deterministic, equal to clt_decode_sparse up to fp32 summation order.
+ *   clt_decode_tiles_wanted: whether it is the faster of the two for `entries` survivors over L layers and `targets`
+ *   target layers (0 also for what it does not take).
+ *   The workspace is sized for max_entries survivors.  A list that turns out longer on the device (row_ptr[L*T] >
+ *   max_entries) is left alone: clt_decode_sparse_if_over decodes such a list and does nothing otherwise.
+ */
+int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
+size_t clt_decode_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries);
+int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                     const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                     int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
+                     int64_t max_entries, void *workspace, size_t workspace_bytes, void *stream);
+int clt_decode_sparse_if_over(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                              const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                              int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype,
+                              int out_f32, int64_t max_entries, void *stream);
+
+/*
  * Which schedule clt_decode_sparse takes for these shapes when it is given a workspace of
  * `workspace_bytes` (16-byte aligned weights assumed): one of CLT_ROUTE_*, or a negative error code.
  * A query for callers and tests; it launches nothing.

@@ -1,0 +1,133 @@
+"""The matrix-core decode (clt_decode_tiles) against dense products in float64, at the edges of its tiles: 512 features,
+16 tokens per group, 16 wavefronts x 4 groups per workgroup, 32 entries per batch, 64 columns."""
+import pytest
+import torch
+
+import crosslayer_coding_amd as cca
+from crosslayer_coding_amd import _native as nat
+from crosslayer_coding_amd import engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _lists(L, T, F, per_token, dtype, seed, heavy):
+    g = torch.Generator().manual_seed(seed)
+    act = torch.zeros(L, T, F)
+    for s in range(L):
+        keep = torch.rand(T, F, generator=g) < per_token / F
+        if heavy:                      # one token with every feature, one source with next to none
+            keep[T // 2] = True
+            keep[:, F // 2:] &= s != 1
+        act[s] = torch.where(keep, torch.randn(T, F, generator=g), torch.zeros(()))
+    act = act.to(dtype)
+    nz = act.reshape(L * T, F) != 0
+    row_ptr = torch.zeros(L * T + 1, dtype=torch.int32)
+    row_ptr[1:] = torch.cumsum(nz.sum(1), 0)
+    col = nz.nonzero()[:, 1].int()
+    return act, row_ptr, col, act.reshape(L * T, F)[nz]
+
+
+def _slot(tying, s, t, L):
+    return s if tying == "per_source" else s * L - (s * (s - 1)) // 2 + (t - s)
+
+
+def _run(dev, act, row_ptr, col, val, w, tying, d, bias, skip, t0, t1, mask, f32, cap, guarded):
+    L, T, F = act.shape
+    lib = nat.load()
+    slab = engine.alloc_packed(w.shape[0], F, d, act.dtype, dev)
+    slab[:, :, :d] = w.to(dev)
+    rp, c, v = row_ptr.to(dev), torch.cat([col, col.new_zeros(1)]).to(dev), torch.cat([val, val.new_zeros(1)]).to(dev)
+    b, k = (None if x is None else x.to(dev) for x in (bias, skip))
+    out = torch.full((L, T, d), 7.0, dtype=torch.float32 if f32 else act.dtype, device=dev)
+    nbytes = lib.clt_decode_tiles_workspace_bytes(T, d, F, L, t1 - t0, cap)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    args = (nat.ptr(rp), nat.ptr(c), nat.ptr(v), nat.ptr(slab), nat.ptr(b), nat.ptr(k), nat.ptr(out), T, d, F, L, nat.TYING[tying],
+            t0, t1, mask, nat.dtype_code(act.dtype), 1 if f32 else 0, cap)
+    for _ in range(2):                 # the second pass meets a workspace in use
+        nat.check(lib.clt_decode_tiles(*args, nat.ptr(ws), ws.numel(), nat.current_stream(rp.device)), "clt_decode_tiles")
+        if guarded:
+            nat.check(lib.clt_decode_sparse_if_over(*args, nat.current_stream(rp.device)), "clt_decode_sparse_if_over")
+    return out.cpu()
+
+
+@pytest.mark.parametrize("L,T,F,d,per_token,dtype,tying,heavy", [
+    (1, 1, 8, 64, 3, torch.bfloat16, "none", False),             # less than one of everything
+    (2, 16, 512, 64, 32, torch.bfloat16, "none", False),         # exactly one group, one tile
+    (3, 17, 513, 128, 60, torch.float16, "none", False),         # one token and one feature over
+    (3, 15, 1024, 64, 200, torch.bfloat16, "per_source", True),
+    (2, 1025, 1300, 192, 20, torch.bfloat16, "none", False),     # a workgroup's tokens and one more
+    (4, 300, 4096, 64, 1, torch.float16, "none", True),          # most batches empty
+    (2, 2100, 640, 256, 40, torch.bfloat16, "per_source", False),
+    (3, 64, 2048, 320, 700, torch.bfloat16, "none", True),       # far denser than the kernel is meant for
+])
+def test_decode_tiles_against_dense_products(L, T, F, d, per_token, dtype, tying, heavy):
+    dev = torch.device("cuda:0")
+    act, row_ptr, col, val = _lists(L, T, F, per_token, dtype, seed=L * 1000 + T, heavy=heavy)
+    g = torch.Generator().manual_seed(5)
+    n_dec = L if tying == "per_source" else L * (L + 1) // 2
+    w = (torch.rand(n_dec, F, d, generator=g) - 0.5).to(dtype)
+    bias, skip = torch.randn(L, d, generator=g), torch.randn(L, T, d, generator=g)
+    full = (1 << L) - 1
+    cases = [(0, L, full, True, None, None), (0, L, full, False, bias, skip)]
+    if L > 2:
+        cases.append((1, L, full & ~2, True, bias, None))        # a layer left out although it has survivors
+    for t0, t1, mask, f32, b, k in cases:
+        got = _run(dev, act, row_ptr, col, val, w, tying, d, b, k, t0, t1, mask, f32, col.numel(), False)
+        for t in range(L):
+            if not t0 <= t < t1:
+                assert (got[t] == 7.0).all()
+                continue
+            ref, mag, n = torch.zeros(T, d, dtype=torch.float64), torch.zeros(T, d, dtype=torch.float64), torch.zeros(T, 1)
+            for s in range(t + 1):
+                if mask >> s & 1:
+                    a, m = act[s].double(), w[_slot(tying, s, t, L)].double()
+                    ref += a @ m
+                    mag += a.abs() @ m.abs()
+                    n += (act[s] != 0).sum(1, keepdim=True)
+            for extra in (None if b is None else b[t].double(), None if k is None else k[t].double()):
+                if extra is not None:
+                    ref, mag = ref + extra, mag + extra.abs()
+            # products of two 16-bit numbers are exact in fp32; each of the n + 2 additions is off by at most 2^-23 of what
+            # has been summed, and the result is rounded once to the output type
+            bound = (n.double() + 2) * 2.0 ** -23 * mag
+            if not f32:
+                bound = bound + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * (ref.abs() + bound) + 2.0 ** -24
+            assert (got[t].double() - ref).abs().le(bound).all(), (t, (got[t].double() - ref).abs().max())
+
+
+def test_decode_tiles_leaves_longer_lists_to_the_gather():
+    dev = torch.device("cuda:0")
+    L, T, F, d = 2, 100, 1000, 128
+    act, row_ptr, col, val = _lists(L, T, F, 30, torch.bfloat16, seed=3, heavy=False)
+    w = (torch.rand(3, F, d, generator=torch.Generator().manual_seed(1)) - 0.5).bfloat16()
+    n = col.numel()
+    exact = _run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, L, 3, True, n, True)
+    over = _run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, L, 3, True, n - 1, True)
+    left = _run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, L, 3, True, n - 1, False)
+    assert (left == 7.0).all()
+    assert torch.allclose(exact, over, rtol=0, atol=60 * 2.0 ** -23 * 60)      # 60 terms below 60 in sum, summed in another order
+
+
+def test_decode_tiles_keeps_tokens_apart():
+    """Values that are not finite stay with their token although sixteen tokens share every product."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 1, 32, 512, 64
+    act, row_ptr, col, val = _lists(L, T, F, 40, torch.bfloat16, seed=9, heavy=False)
+    w = (torch.rand(1, F, d, generator=torch.Generator().manual_seed(1)) + 0.5).bfloat16()
+    val = val.clone()
+    val[row_ptr[3]] = float("nan")
+    val[row_ptr[7]] = float("inf")
+    got = _run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, 1, 1, True, col.numel(), False)[0]
+    fine = torch.ones(T, dtype=torch.bool)
+    fine[[3, 7]] = False
+    assert got[3].isnan().all() and (got[7] == float("inf")).all() and got[fine].isfinite().all()
+
+
+def test_the_model_takes_the_tiles_when_they_are_priced_lower():
+    lib = nat.load()
+    want = lambda T, k, **kw: lib.clt_decode_tiles_wanted(T, 768, 24576, 12, 12, 12 * T * k, nat.TYING[kw.get("tying", "none")],  # noqa: E731
+                                                          nat.dtype_code(kw.get("dtype", torch.bfloat16)))
+    assert want(4096, 200) == 1 and want(4096, 200, tying="per_source") == 1 and want(4096, 200, dtype=torch.float16) == 1
+    assert want(64, 200) == 0 and want(4096, 2) == 0
+    assert want(4096, 200, dtype=torch.float32) == 0 and want(4096, 200, tying="per_target") == 0
+    assert cca is not None
