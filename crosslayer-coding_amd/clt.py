@@ -321,7 +321,7 @@ class CrossLayerTranscoder(BaseTranscoder):
                        else (None, None))
         # ``decoder_step`` (an optimiser whose ``fuses_decoder_step()`` holds): the decoder weights take their
         # step inside the weight-gradient kernel, after everything that reads the old decoders (below)
-        dw_dec = None if decoder_step is not None else engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc)
+        dw_dec = None if decoder_step is not None else engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
         _, x_slab, _, _ = self.encoder_module.prepare_slab(inputs)
         x_slab = x_slab.contiguous()
         dw_enc, db_enc = engine.encoder_weight_grad(lists, dval, x_slab, F)

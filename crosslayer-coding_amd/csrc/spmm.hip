@@ -6,6 +6,9 @@
 //                   in which it consumes them: by source, tile of SP_ROWS features, group of 16 tokens
 //   k_decode_tiles  one workgroup per (target, 64 columns, part of the tokens): every tile of every source's decoder
 //                   passes through LDS once, the sums stay in registers over all sources and features
+//   k_grad_tiles    the transposed product of the backward pass: decoder weight gradients from the same lists by feature,
+//                   with the Adam step of the weights taken on the spot
+#include "adam.h"
 #include "spmm.h"
 
 namespace {
@@ -15,14 +18,15 @@ __device__ __forceinline__ int64_t sp_slot(int tying, int64_t s, int64_t t, int6
 }
 
 constexpr int DT_WAVES = 16;
-constexpr int DT_GPW = 4;                  // groups of 16 tokens per wavefront: 64 accumulators per lane
+constexpr int DT_GPW = 4;                  // groups of 16 output rows per wavefront: 64 accumulators per lane
 
-// Groups part * groups_per_part + wave + 16 gi of a part of the tokens belong to wavefront `wave`; the batches of its
-// groups, ordered by (source, tile, gi), are its stream.
-struct TilePlan {
-  int tiles, groups, parts, groups_per_part, streams, stages;
+// How one layer's output rows (tokens of a decode, features of a weight gradient) are dealt out.  Groups
+// part * groups_per_part + wave + waves * gi of a part belong to wavefront `wave` of its workgroups; the batches of its
+// groups, ordered by (layer, tile, gi), are its stream.
+struct SpPlan {
+  int tiles, groups, parts, groups_per_part, waves, streams, stages;
   __host__ __device__ __forceinline__ int group(int stream, int gi) const {        // -1: none
-    const int part = stream / DT_WAVES, r = stream % DT_WAVES + gi * DT_WAVES, g = part * groups_per_part + r;
+    const int part = stream / waves, r = stream % waves + gi * waves, g = part * groups_per_part + r;
     return r < groups_per_part && g < groups ? g : -1;
   }
 };
@@ -30,35 +34,38 @@ struct TilePlan {
 // ---- records ----------------------------------------------------------------------------------------
 constexpr int REC_THREADS = 256;
 constexpr int REC_MAX_TILES = 512;
-constexpr int REC_WINDOW = 128;            // batches put together in LDS at a time
 
+// The lists that are regrouped: rows r = layer * Rn + row, columns ascending within a row.
 struct RecArgs {
   const int32_t *row_ptr, *col;
+  const int32_t *src;      // the entry's value is val[src[j]]; null: val[j]
   const void *val;
-  int64_t Tn, L, max_entries;
-  uint64_t src_mask;
-  TilePlan p;
-  int32_t *start;          // [L * groups][SP_GROUP][tiles + 1] list position where a token's entries of a tile begin
-  uint16_t *batches;       // [L * tiles][groups] batches of (source, tile, group)
+  int64_t Rn, L, max_entries;
+  uint64_t layer_mask;
+  SpPlan p;
+  int window;              // batches put together in LDS at a time
+  int alternate;           // 1: stages of all layers follow each other, in two buffers in turn; 0: one buffer
+  int32_t *start;          // [L * groups][SP_GROUP][tiles + 1] list position where a row's entries of a tile begin
+  uint16_t *batches;       // [L * tiles][groups] batches of (layer, tile, group)
   uint16_t *counts;        // [streams][stages][DT_GPW] the same by stream
   uint32_t *offset;        // [streams][stages] batches of the stream before the stage
   uint32_t *total;         // [streams] batches of the stream
   uint32_t *recs;
 };
 
-// One workgroup per (group of 16 tokens, source).  Rows are sorted by feature, so a token's entries of one tile are a
-// run, found by binary search.  A layer outside src_mask counts as empty.
+// One workgroup per (group of 16 rows, layer).  Rows are sorted by column, so a row's entries of one tile are a run, found
+// by binary search.  A layer outside layer_mask counts as empty.
 __global__ __launch_bounds__(REC_THREADS) void k_rec_count(RecArgs A) {
   extern __shared__ int32_t run_lds[];
-  if (A.row_ptr[A.L * A.Tn] > A.max_entries) return;      // more entries than the workspace was sized for
+  if (A.row_ptr[A.L * A.Rn] > A.max_entries) return;      // more entries than the workspace was sized for
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles;
-  const int64_t tok0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Tn + tok0;
-  const bool on = (A.src_mask >> s) & 1ull;
+  const int64_t row0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Rn + row0;
+  const bool on = (A.layer_mask >> s) & 1ull;
   int32_t *out = A.start + ((int64_t)s * A.p.groups + g) * SP_GROUP * (tiles + 1);
   for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) {
     const int tk = i / (tiles + 1), c = i - tk * (tiles + 1);
     int32_t lo = 0;
-    if (on && tok0 + tk < A.Tn) {
+    if (on && row0 + tk < A.Rn) {
       int32_t hi = A.row_ptr[r0 + tk + 1];
       lo = A.row_ptr[r0 + tk];
       const int32_t bound = c * SP_ROWS;
@@ -82,7 +89,7 @@ __global__ __launch_bounds__(REC_THREADS) void k_rec_count(RecArgs A) {
 
 // One wavefront per stream: its batch counts per stage and where each stage begins.
 __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
-  if (A.row_ptr[A.L * A.Tn] > A.max_entries) return;
+  if (A.row_ptr[A.L * A.Rn] > A.max_entries) return;
   const int stream = blockIdx.x, lane = threadIdx.x;
   uint32_t run = 0;
   for (int st0 = 0; st0 < A.p.stages; st0 += 64) {
@@ -119,25 +126,26 @@ __device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stre
   return n;
 }
 
-// One workgroup per (group, source) again: the runs of a tile laid end to end in token order - a fixed order of every
-// sum - put together in LDS, REC_WINDOW batches at a time, and written out lane by lane.
+// One workgroup per (group, layer) again: the runs of a tile laid end to end in row order - a fixed order of every sum -
+// put together in LDS, `window` batches at a time, and written out lane by lane.
 template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(RecArgs A) {
   extern __shared__ int32_t fill_lds[];
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
-  if (A.row_ptr[A.L * A.Tn] > A.max_entries || !((A.src_mask >> s) & 1ull)) return;
+  if (A.row_ptr[A.L * A.Rn] > A.max_entries || !((A.layer_mask >> s) & 1ull)) return;
   int32_t *start = fill_lds;                               // [SP_GROUP][tiles + 1]
-  int32_t *off = start + SP_GROUP * (tiles + 1);           // [SP_GROUP][tiles] entries of the tile before this token's
+  int32_t *off = start + SP_GROUP * (tiles + 1);           // [SP_GROUP][tiles] entries of the tile before this row's
   int32_t *first = off + SP_GROUP * tiles;                 // [tiles + 1] first batch of the tile, counted within the group
   uint32_t *dest = (uint32_t *)(first + tiles + 1);        // [tiles] its place among all batches
-  uint32_t *where = dest + tiles;                          // [REC_WINDOW] the same per batch of the window
-  uint16_t *win = (uint16_t *)(where + REC_WINDOW);        // [REC_WINDOW][64] words
-  const int64_t tok0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Tn + tok0;
+  uint32_t *where = dest + tiles;                          // [window] the same per batch of the window
+  uint16_t *win = (uint16_t *)(where + A.window);          // [window][64] words
+  const int64_t row0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Rn + row0;
   const int32_t *src = A.start + ((int64_t)s * A.p.groups + g) * SP_GROUP * (tiles + 1);
   for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) start[i] = src[i];
   __syncthreads();
   const int part = g / A.p.groups_per_part, r = g - part * A.p.groups_per_part;
-  const int stream = part * DT_WAVES + r % DT_WAVES, gi = r / DT_WAVES;
-  const int stage0 = __popcll(A.src_mask & ((1ull << s) - 1ull)) * tiles;      // stages of a decode before this source's
+  const int stream = part * A.p.waves + r % A.p.waves, gi = r / A.p.waves;
+  const uint32_t stage0 = A.alternate ? (uint32_t)(__popcll(A.layer_mask & ((1ull << s) - 1ull)) * tiles) : 0u;
+  const uint32_t buffers = A.alternate ? 1u : 0u;
   for (int c = tid; c < tiles; c += REC_THREADS) {
     int32_t n = 0;
 #pragma unroll
@@ -171,15 +179,15 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
   }
   __syncthreads();
   const int32_t nb_all = first[tiles];
-  for (int32_t w0 = 0; w0 < nb_all; w0 += REC_WINDOW) {
-    const int32_t wn = nb_all - w0 < REC_WINDOW ? nb_all - w0 : REC_WINDOW;
-    for (int i = tid; i < wn * 32; i += REC_THREADS) reinterpret_cast<uint2 *>(win)[i] = make_uint2(0u, 0u);
+  for (int32_t w0 = 0; w0 < nb_all; w0 += A.window) {
+    const int32_t wn = nb_all - w0 < A.window ? nb_all - w0 : A.window;
+    for (int i = tid; i < wn * SP_REC_WORDS; i += REC_THREADS) reinterpret_cast<uint32_t *>(win)[i] = 0u;
     for (int c = tid; c < tiles; c += REC_THREADS)
       for (int32_t b = first[c]; b < first[c + 1]; ++b)
         if (b >= w0 && b < w0 + wn) where[b - w0] = base + dest[c] + (uint32_t)(b - first[c]);
     __syncthreads();
     for (int tk = tid >> 6; tk < SP_GROUP; tk += REC_THREADS / 64) {
-      if (tok0 + tk >= A.Tn) break;
+      if (row0 + tk >= A.Rn) break;
       const int32_t e = A.row_ptr[r0 + tk + 1];
       for (int32_t j = A.row_ptr[r0 + tk] + lane; j < e; j += 64) {
         const int32_t f = A.col[j], c = f / SP_ROWS;
@@ -188,10 +196,10 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
         if (b < 0 || b >= wn) continue;
         uint16_t *rec = win + b * 128 + (k >> 3) * 32;      // 16 lanes of two halves each
         const int x = (k & 7) >> 1, half = k & 1;
-        rec[(4 * x + 0) * 2 + half] = (uint16_t)Elem<T>::raw(((const T *)A.val)[j]);
+        rec[(4 * x + 0) * 2 + half] = (uint16_t)Elem<T>::raw(((const T *)A.val)[A.src ? A.src[j] : j]);
         rec[(4 * x + 1) * 2 + half] = (uint16_t)(1u << tk);
         rec[(4 * (k & 3) + 3) * 2 + ((k >> 2) & 1)] =
-            (uint16_t)sp_half_place((uint32_t)(f - c * SP_ROWS), (uint32_t)(stage0 + c) & 1u);
+            (uint16_t)sp_half_place((uint32_t)(f - c * SP_ROWS), (stage0 + c) & buffers);
       }
     }
     __syncthreads();
@@ -204,7 +212,7 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
 
 // ---- decode -----------------------------------------------------------------------------------------
 struct TileArgs {
-  TilePlan p;
+  SpPlan p;
   const uint16_t *counts;
   const uint32_t *total;
   const uint32_t *recs;
@@ -388,31 +396,202 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
   }
 }
 
+// ---- decoder weight gradient (and Adam) ---------------------------------------------------------------
+// dW[s->t][f][:] = sum over the tokens of feature f of value * g[t][token][:]: the same product with features in the
+// place of tokens - 16 features per group, tiles of 512 tokens x 64 columns of g[t].
+constexpr int GT_WAVES = 8;
+constexpr int GT_FILLS = SP_ROWS / 8 / GT_WAVES;
+constexpr int GT_LDS = SP_TILE_BYTES + GT_WAVES * DT_RING * 256;
+constexpr int GT_PITCH = SP_COLS + 4;      // fp32 row pitch of a group's gradient on its way through LDS
+static_assert(GT_LDS * 2 <= 160 * 1024 && SP_GROUP * GT_PITCH * 4 * GT_WAVES <= SP_TILE_BYTES, "two workgroups per CU");
+
+struct GradArgs {
+  SpPlan p;
+  const uint16_t *counts;
+  const uint32_t *offset, *total, *recs;
+  const void *g;             // [L][T][d]
+  void *w;                   // packed decoders, or null: the gradient goes to `out`
+  float *m, *v, *out;        // moments; [n_dec][F][d]
+  int64_t Tn, d, F, L, pitch, max_entries;
+  int64_t m_row, m_cols, m_dec;   // moments: elements between rows, between column parts of 64 and between decoders
+  const int32_t *list_total;
+  int col_parts, items;      // items of one (source, target) pair per XCD
+  AdamCoef adam;
+};
+
+// One workgroup per (source, target, 64 columns, part of the features): eight wavefronts, four groups of 16 features each.
+// The weights and moments stream through once (20 bytes per weight, nothing else from HBM), which bounds the kernel; so
+// two workgroups share a CU (80 KB of LDS each, one tile buffer) and one's products run under the other's streaming.
+// A group's sums go through LDS so that 16 lanes read and write 256 contiguous bytes of the moments.  An XCD takes one
+// eighth of the features of a pair with all its column parts: the batches' records are read from its L2 by all of them.
+template <typename T, bool ADAM>
+__global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
+  extern __shared__ __attribute__((aligned(128))) char grad_lds[];
+  if (*A.list_total > A.max_entries) return;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int slot = seq / A.items, item = xcd * A.items + seq % A.items;
+  if (item >= A.p.parts * A.col_parts) return;
+  const int part = item / A.col_parts, cp = item % A.col_parts;
+  // decoder `slot` of "0->0", "0->1", ..: source s, target t
+  int s = 0, t = slot;
+  while (t >= (int)A.L - s) { t -= (int)A.L - s; ++s; }
+  t += s;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)grad_lds;
+  const int stream = part * GT_WAVES + wave;
+
+  const uint32_t pitch_b = (uint32_t)(A.d * (int64_t)sizeof(T));
+  const uint32_t col_b = (((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4);
+  const int row_a = wave * 64 + (lane >> 2);
+  auto fill = [&](const char *src, int rows) {
+#pragma unroll
+    for (int i = 0; i < GT_FILLS; ++i) {
+      const int r = row_a + (i >> 1) * 16;
+      fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
+             lds0 + (uint32_t)(wave * 4096 + (i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+    }
+  };
+
+  f32x4v_t acc[DT_GPW][4];
+#pragma unroll
+  for (int gi = 0; gi < DT_GPW; ++gi)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[gi][n] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
+  {
+    const uint32_t row_bit = 0x00010001u << (lane & 15);
+    const uint32_t ring = lds0 + SP_TILE_BYTES + (uint32_t)wave * (DT_RING * 256);
+    const int stage0 = s * A.p.tiles;
+    const uint32_t *recs = A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(
+        stream_first(A.total, stream, lane) + A.offset[(int64_t)stream * A.p.stages + stage0]) * SP_REC_WORDS;
+    uint32_t rec_off = (uint32_t)lane * 4, at = 0, word;
+    const uint32_t ring_lane = ring + (uint32_t)lane * 4, col = lds0 + (uint32_t)(lane & 3) * 8;
+    const auto counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages + stage0;
+    const char *tile = (const char *)A.g + (int64_t)t * A.Tn * (int64_t)pitch_b + (int64_t)cp * 128;
+    fill(tile, (int)A.Tn);
+#pragma unroll
+    for (int i = 0; i < DT_RING; ++i) { fill4(recs, rec_off, ring + (uint32_t)i * 256); rec_off += SP_REC_WORDS * 4; }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto look = [&]() { word = *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)(ring_lane + at); };
+    look();
+    SpBatch<T> bt;
+    auto prepare = [&]() {                                 // as in k_decode_tiles; no tile line is ever behind a record
+      bt.address(word, col);
+      bt.read();
+      bt.pick(word, row_bit);
+      asm volatile("" ::"v"(bt.picked), "v"(bt.a0), "v"(bt.a1));
+      fill4(recs, rec_off, ring + at);
+      rec_off += SP_REC_WORDS * 4;
+      at = (at + 256) & (DT_RING * 256 - 1);
+      asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
+      look();
+    };
+    prepare();
+    int rows = (int)A.Tn;
+    for (int st = 0; st < A.p.tiles; ++st) {
+      const uint2 cnt = make_uint2(counts[st].x, counts[st].y);
+      if (st > 0) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();                      // nobody reads the last tile any more
+        asm volatile("" ::: "memory");
+        tile += SP_ROWS * pitch_b;
+        rows -= SP_ROWS;
+        fill(tile, rows);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      bt.read();
+#pragma unroll
+      for (int gi = 0; gi < DT_GPW; ++gi) {
+        const int n = (int)((gi & 2 ? cnt.y : cnt.x) >> (gi & 1 ? 16 : 0)) & 0xFFFF;
+        for (int i = n; i > 0; --i) { bt.finish(acc[gi]); prepare(); }
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                          // the tile's LDS is free
+    asm volatile("" ::: "memory");
+  }
+
+  float *const mine = (float *)(grad_lds + wave * (SP_GROUP * GT_PITCH * 4));
+#pragma unroll
+  for (int gi = 0; gi < DT_GPW; ++gi) {
+    const int g = A.p.group(stream, gi);
+    if (g < 0) break;
+    // rows of 64 columns: lane 16 r + c takes columns 4 c .. 4 c + 3 of rows r, r + 4, r + 8, r + 12
+    const int c4 = (lane & 15) * 4;
+    const int64_t f0 = (int64_t)g * SP_GROUP + (lane >> 4);
+    float *const m_at = A.m + slot * A.m_dec + (int64_t)cp * A.m_cols + f0 * A.m_row + c4;
+    float *const v_at = A.v + slot * A.m_dec + (int64_t)cp * A.m_cols + f0 * A.m_row + c4;
+    uint16_t *const w_at = (uint16_t *)A.w + ((int64_t)slot * A.F + f0) * A.pitch + (int64_t)cp * SP_COLS + c4;
+    f32x4v_t mm[4], vv[4];
+    uint2 ww[4];
+    if constexpr (ADAM) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t o = f0 + 4 * i < A.F ? 4 * i : -(f0 - (f0 < A.F ? f0 : 0));      // past the last feature: a row that exists
+        mm[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4v_t *>(m_at + o * A.m_row));
+        vv[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4v_t *>(v_at + o * A.m_row));
+        ww[i] = *reinterpret_cast<const uint2 *>(w_at + o * A.pitch);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      *reinterpret_cast<f32x4v_t *>(mine + (lane & 15) * GT_PITCH + n * 16 + (lane >> 4) * 4) = acc[gi][n];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4v_t gr = *reinterpret_cast<const f32x4v_t *>(mine + ((lane >> 4) + 4 * i) * GT_PITCH + c4);
+      if (f0 + 4 * i >= A.F) continue;
+      if constexpr (ADAM) {
+        float p[4];
+        unpack_pair<T>(ww[i].x, p[0], p[1]);
+        unpack_pair<T>(ww[i].y, p[2], p[3]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float m1 = mm[i][k], v1 = vv[i][k];
+          p[k] = adam_update(p[k], gr[k], m1, v1, A.adam);
+          mm[i][k] = m1;
+          vv[i][k] = v1;
+        }
+        __builtin_nontemporal_store(mm[i], reinterpret_cast<f32x4v_t *>(m_at + 4 * i * A.m_row));
+        __builtin_nontemporal_store(vv[i], reinterpret_cast<f32x4v_t *>(v_at + 4 * i * A.m_row));
+        *reinterpret_cast<uint2 *>(w_at + 4 * i * A.pitch) = make_uint2(pack_pair<T>(p[0], p[1]), pack_pair<T>(p[2], p[3]));
+      } else {
+        __builtin_nontemporal_store(gr, reinterpret_cast<f32x4v_t *>(A.out + ((int64_t)slot * A.F + f0 + 4 * i) * A.d + (int64_t)cp * SP_COLS + c4));
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");    // read before the next group's sums are written
+  }
+}
+
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-struct TileLayout {
-  TilePlan p;
+struct SpLayout {
+  SpPlan p;
   int col_parts;
   int64_t n_batches;
   size_t start, batches, counts, offset, total, recs, bytes;
 };
 
-static TileLayout tile_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {
-  TileLayout l;
-  TilePlan &p = l.p;
-  p.tiles = (int)clt_ceil_div(F, SP_ROWS);
-  p.groups = (int)clt_ceil_div(Tn, SP_GROUP);
+// `rows` output rows and `cols` tile rows per layer; `per_group` workgroups for every part of the rows
+static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int waves, int64_t per_part, int64_t max_entries) {
+  SpLayout l;
+  SpPlan &p = l.p;
+  p.tiles = (int)clt_ceil_div(cols, SP_ROWS);
+  p.groups = (int)clt_ceil_div(rows, SP_GROUP);
   p.stages = (int)(L * p.tiles);
+  p.waves = waves;
   l.col_parts = (int)(d / SP_COLS);
-  // as many tokens per workgroup as its registers hold, unless that leaves compute units idle
+  // as many rows per workgroup as its registers hold, unless that leaves compute units idle
   for (int gpw = DT_GPW; gpw > 0; --gpw) {
-    p.parts = (int)clt_ceil_div(p.groups, DT_WAVES * gpw);
-    if ((int64_t)p.parts * l.col_parts * targets >= 512) break;
+    p.parts = (int)clt_ceil_div(p.groups, waves * gpw);
+    if ((int64_t)p.parts * l.col_parts * per_part >= 512) break;
   }
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
-  p.streams = p.parts * DT_WAVES;
-  // every (source, tile, group) may leave its last batch part empty; a stream reads DT_RING batches past its end
-  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + DT_RING;
+  p.streams = p.parts * waves;
+  // every (layer, tile, group) may leave its last batch part empty; a stream reads a ring of batches past its end
+  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + 8;
   size_t at = 0;
   auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
   l.start = take(sizeof(int32_t) * (size_t)L * p.groups * SP_GROUP * (p.tiles + 1));
@@ -420,30 +599,79 @@ static TileLayout tile_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64
   l.counts = take(sizeof(uint16_t) * (size_t)p.streams * p.stages * DT_GPW);
   l.offset = take(sizeof(uint32_t) * (size_t)p.streams * p.stages);
   l.total = take(sizeof(uint32_t) * (size_t)p.streams);
-  l.recs = take((size_t)l.n_batches * 256);
+  l.recs = take((size_t)l.n_batches * SP_REC_WORDS * 4);
   l.bytes = at;
   return l;
 }
 
 // LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile; 16-bit batch counts
-static bool tile_shape_ok(const TileLayout &l, int64_t d) {
-  return l.p.tiles <= REC_MAX_TILES && l.n_batches <= 0x00FFFFFFll && clt_pitch(d, 2) * 2 * SP_ROWS <= 0x7FFFFFFFll &&
-         l.p.groups <= 0xFFFF && (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll;
+static bool sp_shape_ok(const SpLayout &l, int64_t row_bytes) {
+  return l.p.tiles <= REC_MAX_TILES && l.n_batches <= 0x00FFFFFFll && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
+         (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll;
 }
 
-template <typename T> static int launch_tiles(RecArgs ra, TileArgs ta, int col_parts, hipStream_t stream) {
+static void sp_place_workspace(RecArgs &ra, const SpLayout &l, char *ws) {
+  ra.p = l.p;
+  ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint16_t *)(ws + l.counts);
+  ra.offset = (uint32_t *)(ws + l.offset); ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint32_t *)(ws + l.recs);
+}
+
+template <typename T> static int launch_records(RecArgs ra, hipStream_t stream) {
   const int tiles = ra.p.tiles;
+  // a group's batches are put together at once where they are as many as usual
+  ra.window = tiles <= 16 ? 32 : 128;
   const size_t count_lds = sizeof(int32_t) * (size_t)SP_GROUP * (tiles + 1);
-  const size_t fill_lds = sizeof(int32_t) * (size_t)(SP_GROUP * (tiles + 1) + SP_GROUP * tiles + 2 * tiles + 1 + REC_WINDOW) + REC_WINDOW * 256;
-  if (hipFuncSetAttribute((const void *)k_rec_fill<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds) != hipSuccess ||
-      hipFuncSetAttribute((const void *)k_decode_tiles<T>, hipFuncAttributeMaxDynamicSharedMemorySize, DT_LDS) != hipSuccess)
+  const size_t fill_lds = sizeof(int32_t) * (size_t)(SP_GROUP * (tiles + 1) + SP_GROUP * tiles + 2 * tiles + 1 + ra.window) +
+                          (size_t)ra.window * SP_REC_WORDS * 4 + 8;
+  if (hipFuncSetAttribute((const void *)k_rec_fill<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds) != hipSuccess)
     return CLT_ERR_LAUNCH;
   const dim3 grid((unsigned)ra.p.groups, (unsigned)ra.L);
   k_rec_count<<<grid, REC_THREADS, count_lds, stream>>>(ra);
   k_rec_streams<<<(unsigned)ra.p.streams, 64, 0, stream>>>(ra);
   k_rec_fill<T><<<grid, REC_THREADS, fill_lds, stream>>>(ra);
+  return CLT_OK;
+}
+
+static SpLayout tile_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {
+  return sp_layout(Tn, F, d, L, DT_WAVES, targets, max_entries);
+}
+
+template <typename T> static int launch_tiles(RecArgs ra, TileArgs ta, int col_parts, hipStream_t stream) {
+  const int code = launch_records<T>(ra, stream);
+  if (code != CLT_OK) return code;
+  if (hipFuncSetAttribute((const void *)k_decode_tiles<T>, hipFuncAttributeMaxDynamicSharedMemorySize, DT_LDS) != hipSuccess)
+    return CLT_ERR_LAUNCH;
   const int64_t pairs = clt_ceil_div((int64_t)(ta.t_end - ta.t_begin) * col_parts, 8) * 8;
   k_decode_tiles<T><<<(unsigned)(pairs * ta.p.parts), DT_WAVES * 64, DT_LDS, stream>>>(ta);
+  return clt_check_launch();
+}
+
+static SpLayout grad_layout(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  // (a launch has a workgroup per pair, column part and part of the features: plenty, so the parts are as large as they get)
+  return sp_layout(F, T, d, L, GT_WAVES, 1 << 20, entries);
+}
+
+static int launch_grad(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val, GradArgs a,
+                       void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  const SpLayout l = grad_layout(a.Tn, a.d, a.F, a.L, a.max_entries);
+  if (!sp_shape_ok(l, a.d * 2)) return CLT_ERR_RANGE;
+  if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
+  RecArgs ra;
+  ra.row_ptr = list_ptr; ra.col = list_tok; ra.src = list_src; ra.val = val; ra.Rn = a.F; ra.L = a.L; ra.max_entries = a.max_entries;
+  ra.layer_mask = ~0ull; ra.alternate = 0;
+  sp_place_workspace(ra, l, (char *)workspace);
+  const int code = launch_records<bf16_t>(ra, stream);
+  if (code != CLT_OK) return code;
+  a.p = l.p; a.counts = ra.counts; a.offset = ra.offset; a.total = ra.total; a.recs = ra.recs;
+  a.list_total = list_ptr + a.L * a.F;
+  a.col_parts = l.col_parts;
+  a.items = (int)clt_ceil_div((int64_t)l.p.parts * l.col_parts, 8);
+  const int64_t blocks = 8 * (int64_t)a.items * (a.L * (a.L + 1) / 2);
+  if (blocks > 0x7FFFFFFFll) return CLT_ERR_RANGE;
+  const void *k = a.w ? (const void *)k_grad_tiles<bf16_t, true> : (const void *)k_grad_tiles<bf16_t, false>;
+  if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS) != hipSuccess) return CLT_ERR_LAUNCH;
+  if (a.w) k_grad_tiles<bf16_t, true><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
+  else k_grad_tiles<bf16_t, false><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
   return clt_check_launch();
 }
 
@@ -459,8 +687,8 @@ extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t 
                                        int dtype) {
   if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return 0;
   if (T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return 0;
-  const TileLayout l = tile_layout(T, d, F, L, targets, entries);
-  if (!tile_shape_ok(l, d)) return 0;
+  const SpLayout l = tile_layout(T, d, F, L, targets, entries);
+  if (!sp_shape_ok(l, clt_pitch(d, 2) * 2)) return 0;
   // (source, target) pairs of the last `targets` layers, and the survivors they gather
   const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
   const double sparse_us = rows * d * 2 / 17e6 + pairs * T * d * 16 / 3.2e6;
@@ -490,15 +718,13 @@ extern "C" int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, cons
       (skip_add && !clt_aligned16(skip_add)))
     return CLT_ERR_ALIGN;
   const int64_t pitch = clt_pitch(d, 2);
-  const TileLayout l = tile_layout(T, d, F, L, t_end - t_begin, max_entries);
-  if (!tile_shape_ok(l, d)) return CLT_ERR_RANGE;
+  const SpLayout l = tile_layout(T, d, F, L, t_end - t_begin, max_entries);
+  if (!sp_shape_ok(l, pitch * 2)) return CLT_ERR_RANGE;
   if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
-  char *ws = (char *)workspace;
   RecArgs ra;
-  ra.row_ptr = row_ptr; ra.col = col; ra.val = val; ra.Tn = T; ra.L = L; ra.max_entries = max_entries; ra.src_mask = src_mask;
-  ra.p = l.p;
-  ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint16_t *)(ws + l.counts);
-  ra.offset = (uint32_t *)(ws + l.offset); ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint32_t *)(ws + l.recs);
+  ra.row_ptr = row_ptr; ra.col = col; ra.src = nullptr; ra.val = val; ra.Rn = T; ra.L = L; ra.max_entries = max_entries;
+  ra.layer_mask = src_mask; ra.alternate = 1;
+  sp_place_workspace(ra, l, (char *)workspace);
   TileArgs ta;
   ta.p = l.p; ta.counts = ra.counts; ta.total = ra.total; ta.recs = ra.recs;
   ta.wp = w_packed; ta.bias_sum = bias_sum; ta.skip_add = skip_add; ta.out = out;
@@ -507,4 +733,48 @@ extern "C" int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, cons
   ta.tying = tying; ta.t_begin = (int)t_begin; ta.t_end = (int)t_end; ta.out_f32 = out_f32; ta.col_parts = l.col_parts;
   if (dtype == CLT_BF16) return launch_tiles<bf16_t>(ra, ta, l.col_parts, (hipStream_t)stream);
   return launch_tiles<f16_t>(ra, ta, l.col_parts, (hipStream_t)stream);
+}
+
+extern "C" int clt_grad_tiles_supported(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype) {
+  if (dtype != CLT_BF16 || T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || entries < 0) return 0;
+  const SpLayout l = grad_layout(T, d, F, L, entries);
+  return sp_shape_ok(l, d * 2) && 8 * clt_ceil_div((int64_t)l.p.parts * l.col_parts, 8) * (L * (L + 1) / 2) <= 0x7FFFFFFFll;
+}
+
+extern "C" size_t clt_grad_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  if (T <= 0 || d < SP_COLS || F <= 0 || L <= 0 || entries < 0) return 0;
+  return grad_layout(T, d, F, L, entries).bytes;
+}
+
+extern "C" int clt_decoder_grad_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
+                                      const void *g_model, float *out, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
+                                      int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  if (dtype != CLT_BF16) return CLT_ERR_DTYPE;
+  if (!clt_grad_tiles_supported(T, d, F, L, entries, dtype)) return CLT_ERR_ARG;
+  if (!list_ptr || !list_tok || !list_src || !val || !g_model || !out || !workspace) return CLT_ERR_ARG;
+  if (!clt_aligned16(g_model) || !clt_aligned16(out) || !clt_aligned16(workspace)) return CLT_ERR_ALIGN;
+  GradArgs a{};
+  a.g = g_model; a.out = out;
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.max_entries = entries;
+  return launch_grad(list_ptr, list_tok, list_src, val, a, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
+                                           const void *g_model, void *w_packed, float *m, float *v, int moments_by_tile, int64_t T,
+                                           int64_t d, int64_t F, int64_t L, int64_t entries, double lr, double beta1, double beta2,
+                                           double eps, int64_t step, int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  if (dtype != CLT_BF16) return CLT_ERR_DTYPE;
+  if (!clt_grad_tiles_supported(T, d, F, L, entries, dtype)) return CLT_ERR_ARG;
+  if (step < 1 || !(beta1 >= 0 && beta1 < 1) || !(beta2 >= 0 && beta2 < 1)) return CLT_ERR_ARG;
+  if (!list_ptr || !list_tok || !list_src || !val || !g_model || !w_packed || !m || !v || !workspace) return CLT_ERR_ARG;
+  if (!clt_aligned16(g_model) || !clt_aligned16(w_packed) || !clt_aligned16(m) || !clt_aligned16(v) || !clt_aligned16(workspace))
+    return CLT_ERR_ALIGN;
+  GradArgs a{};
+  a.g = g_model; a.w = w_packed; a.m = m; a.v = v;
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = clt_pitch(d, 2); a.max_entries = entries;
+  a.m_dec = F * d;
+  a.m_row = moments_by_tile ? SP_COLS : d;
+  a.m_cols = moments_by_tile ? F * SP_COLS : SP_COLS;
+  a.adam = adam_coef(lr, beta1, beta2, eps, step);
+  return launch_grad(list_ptr, list_tok, list_src, val, a, workspace, workspace_bytes, (hipStream_t)stream);
 }

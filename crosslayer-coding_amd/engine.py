@@ -636,8 +636,14 @@ def feature_lists(surv: SurvivorList, ws: Optional[Workspace] = None):
     return ptr, tok, src
 
 
+def grad_tiles_supported(T: int, d: int, F: int, L: int, entries: int, dtype: torch.dtype) -> bool:
+    """Whether the matrix-core weight-gradient kernels (``clt_decoder_grad_tiles``, untied decoders) take these shapes."""
+    return dtype == torch.bfloat16 and bool(nat.load().clt_grad_tiles_supported(T, d, F, L, entries, nat.dtype_code(dtype)))
+
+
 def decoder_weight_grad(lists, surv: SurvivorList, g: torch.Tensor, tying: str,
-                        feat_offset: Optional[torch.Tensor] = None, feat_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+                        feat_offset: Optional[torch.Tensor] = None, feat_scale: Optional[torch.Tensor] = None,
+                        ws: Optional[Workspace] = None) -> torch.Tensor:
     """fp32 [n_dec, F, d] gradient of the packed (feature-major) decoder weights (one matrix per
     (source, target) pair, per source or per target, as ``tying`` says); ``g`` is d loss / d rec in
     the model dtype; ``feat_offset`` / ``feat_scale`` [L, F]: the per-target affine terms the forward applied."""
@@ -647,6 +653,14 @@ def decoder_weight_grad(lists, surv: SurvivorList, g: torch.Tensor, tying: str,
     d = g.shape[2]
     n_dec = L * (L + 1) // 2 if tying == "none" else L
     out = torch.empty((n_dec, F, d), dtype=torch.float32, device=g.device)
+    n = surv.capacity
+    if tying == "none" and feat_offset is None and feat_scale is None and grad_tiles_supported(T, d, F, L, n, surv.dtype):
+        lib = nat.load()
+        wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_tiles_workspace_bytes(T, d, F, L, n))
+        code = lib.clt_decoder_grad_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(out), T, d,
+                                          F, L, n, nat.dtype_code(surv.dtype), nat.ptr(wbuf), wbuf.numel(), _stream(g))
+        nat.check(code, "clt_decoder_grad_tiles")
+        return out
     code = nat.load().clt_decoder_weight_grad(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g),
                                               nat.ptr(feat_offset), nat.ptr(feat_scale), nat.ptr(out), T, d, F, L,
                                               nat.TYING[tying], nat.dtype_code(surv.dtype), _stream(g))
@@ -672,6 +686,27 @@ def decoder_weight_grad_adam(lists, surv: SurvivorList, g: torch.Tensor, w_packe
                                                    nat.ptr(w_packed), nat.ptr(m), nat.ptr(v), T, d, F, L, lr, betas[0],
                                                    betas[1], eps, step, nat.dtype_code(surv.dtype), _stream(g))
     nat.check(code, "clt_decoder_weight_grad_adam")
+
+
+def decoder_grad_adam_tiles(lists, surv: SurvivorList, g: torch.Tensor, w_packed: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
+                            lr: float, betas, eps: float, step: int, ws: Optional[Workspace] = None) -> None:
+    """``decoder_weight_grad_adam`` on the matrix cores (bf16): moments as [n_dec, F, d] or as [n_dec, d // 64, F, 64]."""
+    assert g.dtype == surv.dtype and g.is_contiguous() and w_packed.dtype == surv.dtype and w_packed.is_contiguous()
+    ptr, tok, src = lists
+    L, T, F = surv.L, surv.T, surv.F
+    d = g.shape[2]
+    n_dec = L * (L + 1) // 2
+    by_tile = m.dim() == 4
+    assert tuple(w_packed.shape) == (n_dec, F, decoder_pitch(d, surv.dtype))
+    assert tuple(m.shape) == ((n_dec, d // 64, F, 64) if by_tile else (n_dec, F, d)) and v.shape == m.shape
+    assert m.dtype == torch.float32 and v.dtype == torch.float32 and m.is_contiguous() and v.is_contiguous()
+    lib = nat.load()
+    n = surv.capacity
+    wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_tiles_workspace_bytes(T, d, F, L, n))
+    code = lib.clt_decoder_grad_adam_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(w_packed),
+                                           nat.ptr(m), nat.ptr(v), 1 if by_tile else 0, T, d, F, L, n, lr, betas[0], betas[1], eps, step,
+                                           nat.dtype_code(surv.dtype), nat.ptr(wbuf), wbuf.numel(), _stream(g))
+    nat.check(code, "clt_decoder_grad_adam_tiles")
 
 
 def unpack_decoders(w_packed: torch.Tensor, w_refs_dev: torch.Tensor, w_refs_host, d: int, F: int) -> None:

@@ -29,6 +29,7 @@ class CLTAdam:
         # when something reads them (Decoder.sync_parameters).  False: rewrite them in every step
         self.defer_parameter_sync = True
         self._dec_layout = "rows"        # layout of state["dec_w"]: "rows" [n_dec, F, d] or "tiles" [n_dec, d // CS, F, CS]
+        self._dec_cols = 0               # CS of "tiles": 64 (matrix-core kernel) or 32 bytes of the model dtype
         self._w_tiles = None             # tiled copy of the decoder weights, valid while _w_tiles_gen matches the slab
         self._w_tiles_gen = None
         cfg = model.config
@@ -76,24 +77,24 @@ class CLTAdam:
         return (self.fuse_decoder_step and self.model.config.decoder_tying == "none"
                 and dec.feature_offset is None and dec.feature_scale is None)
 
-    def _decoder_moments_to(self, layout: str) -> None:
-        """Regroup both decoder moments: "rows" [n_dec, F, d] <-> "tiles" [n_dec, d // CS, F, CS] (CS = 32 bytes of
-        the model dtype).  Happens when the route of the decoder step changes, normally once."""
-        if layout == self._dec_layout:
+    def _decoder_moments_to(self, layout: str, cols: int = 0) -> None:
+        """Regroup both decoder moments: "rows" [n_dec, F, d] <-> "tiles" [n_dec, d // cols, F, cols].  Happens when the
+        route of the decoder step changes, normally once."""
+        if layout == self._dec_layout and cols == self._dec_cols:
             return
         cfg = self.model.config
         F, d = cfg.num_features, cfg.d_model
-        cs = 32 // self.model.decoder_module._ordered()[0].weight.element_size()
         out = []
         for t in self.state["dec_w"]:
             n_dec = t.shape[0]
+            if self._dec_layout == "tiles":
+                t = t.permute(0, 2, 1, 3).contiguous().view(n_dec, F, d)
             if layout == "tiles":
-                out.append(t.view(n_dec, F, d // cs, cs).permute(0, 2, 1, 3).contiguous())
-            else:
-                out.append(t.permute(0, 2, 1, 3).contiguous().view(n_dec, F, d))
+                t = t.view(n_dec, F, d // cols, cols).permute(0, 2, 1, 3).contiguous()
+            out.append(t)
             del t
         self.state["dec_w"] = tuple(out)
-        self._dec_layout = layout
+        self._dec_layout, self._dec_cols = layout, cols
 
     def decoder_moments(self):
         """(m, v) of the decoder weights as [n_dec, F, d] whatever layout the optimiser keeps them in."""
@@ -108,10 +109,11 @@ class CLTAdam:
         """The decoder weights' part of the NEXT ``step`` (which must follow with ``raw["dec_w"] = None``), taken
         straight from the survivor lists: gradient rows go from registers into the update of the moments and
         of the working copy of the weights; the checkpoint-layout parameters are then rewritten from that copy.
-        Two routes: over column tiles (tiled moments and a tiled weight copy, the gather of d loss /
-        d reconstruction served from LDS) when ``engine.decoder_tile_width`` takes the shape, else row by row on
-        the feature-major slab.  The row route is bit-identical to gradient-then-Adam; the tile route sums the
-        lists it cuts between lanes in another fixed association (equal to fp32 rounding, repeatable)."""
+        Three routes: bf16 on the matrix cores over tiles of 64 columns (``engine.grad_tiles_supported``; updates the
+        feature-major slab itself, whatever the moments' layout); float32, and widths that are not whole tiles, over
+        tiles of 32 bytes (tiled moments and a tiled weight copy) when ``engine.decoder_tile_width`` takes the shape; else
+        row by row on the feature-major slab.  The first and the last are bit-identical to gradient-then-Adam; the
+        32-byte tiles sum the lists they cut between lanes in another fixed association (equal to fp32 rounding)."""
         from . import engine
         dec = self.model.decoder_module
         packed = dec.packed()
@@ -120,8 +122,18 @@ class CLTAdam:
         d, F = ws[0].shape
         w_dev, w_host = self._pointer_table("w", ws)
         cs = engine.decoder_tile_width(surv.T, d, F, ws[0].dtype) if self.tile_decoder_step else 0
+        if engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype):
+            if cs:
+                self._decoder_moments_to("tiles", 64)
+            else:
+                self._decoder_moments_to("rows")
+            self._w_tiles_gen = None      # the slab changes under the tiled copy
+            engine.decoder_grad_adam_tiles(lists, surv, g_model, packed, *self.state["dec_w"], self.lr, self.betas, self.eps,
+                                           self.step_count + 1, ws=self.model._workspace())
+            self._after_slab_step(packed, w_dev, w_host, d, F)
+            return
         if cs and all(w.data_ptr() % 16 == 0 for w in ws):
-            self._decoder_moments_to("tiles")
+            self._decoder_moments_to("tiles", cs)
             dec._derived_copies = True      # the packed copy tells when the device may have repacked it
             if self._w_tiles is None or self._w_tiles_gen != dec.packed_generation():
                 self._w_tiles = engine.tile_decoders(packed, d, out=self._w_tiles)
@@ -141,6 +153,12 @@ class CLTAdam:
         m_w, v_w = self.state["dec_w"]
         engine.decoder_weight_grad_adam(lists, surv, g_model, packed, m_w, v_w, self.lr, self.betas, self.eps,
                                         self.step_count + 1)
+        self._after_slab_step(packed, w_dev, w_host, d, F)
+
+    def _after_slab_step(self, packed, w_dev, w_host, d: int, F: int) -> None:
+        """The feature-major slab has taken a step: the checkpoint-layout parameters follow, now or when they are read."""
+        from . import engine
+        dec = self.model.decoder_module
         if self.defer_parameter_sync:
             dec.mark_parameters_behind()
         else:
