@@ -30,10 +30,11 @@ namespace {
 
 constexpr int NBINS = 2048;
 constexpr uint32_t FINE16 = 1984;  // 16-bit keys: bins [0,FINE16) are one key wide
-constexpr int SAMPLE_N = 16384;
+constexpr int SAMPLE_MIN = 16384;        // keys sampled from the finished matrix per problem: at least, at most
+constexpr int SAMPLE_MAX = 262144;
+constexpr double SAMPLE_HITS = 32.0;     // of them expected above the threshold (between the two limits)
 constexpr int SAMPLE_WAVES = 64;         // sample taken before the pre-activations exist: wavefronts per layer,
 constexpr int SAMPLE_PRE_N = SAMPLE_WAVES * 1024;   // each 32 hashed tokens x 32 hashed features
-constexpr int SAMPLE_BLOCKS = 16;        // blocks per problem that gather the sample
 constexpr int SCAN_THREADS = 1024;
 constexpr int WBUF = 512;                // candidate entries buffered in LDS per wavefront
 constexpr int PASS_NV = 4;               // 16-byte loads in flight per lane in the pass
@@ -189,14 +190,13 @@ __device__ __forceinline__ uint64_t hash_index(uint64_t i, uint64_t n) {
   return __umul64hi(x, n);
 }
 
-// SAMPLE_BLOCKS blocks per problem: ranking keys of a hashed sample.
+// Ranking keys of a hashed sample, 1024 per block.
 template <typename T, bool GLOBAL>
 __global__ __launch_bounds__(256) void k_sample_keys(
     const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t lstride, const float *mean,
-    const float *denom, unsigned long long N, uint32_t *sample) {
-  constexpr int KB = Elem<T>::KEYBITS;
+    const float *denom, unsigned long long N, int sample_n, uint32_t *sample) {
   const int p = blockIdx.y;
-  const unsigned long long ns = N < (unsigned long long)SAMPLE_N ? N : (unsigned long long)SAMPLE_N;
+  const unsigned long long ns = N < (unsigned long long)sample_n ? N : (unsigned long long)sample_n;
   for (unsigned long long si = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; si < ns;
        si += (unsigned long long)gridDim.x * blockDim.x) {
     unsigned long long idx = (ns == N) ? si : hash_index(si, N);
@@ -205,38 +205,72 @@ __global__ __launch_bounds__(256) void k_sample_keys(
     else { l = p; t = idx / F; f = idx - t * F; }
     float x = Elem<T>::to_f32(pre[l * lstride + t * F + f]);
     typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
-    sample[(int64_t)p * SAMPLE_N + si] = rank_key_of<T>(rk(x, f));
+    sample[(int64_t)p * sample_n + si] = rank_key_of<T>(rk(x, f));
   }
 }
 
 // One block per problem: the cut key = the r-th largest sample key, r chosen so that the
 // expected number of elements above the cut is about 1.25 K plus six standard deviations.
 // Also resets the problem's histogram, pool counter and state.
+//
+// A sample of up to 65536 keys stays in registers (8 us for 16384 bf16 keys, 18 us for 65536, mostly the colliding
+// atomics of keys near zero).  A larger one (SN == 0) is read again from L2 for every radix level and counts only keys
+// that can matter: the r-th largest of the threads' own largest keys, taken down to its first radix digit, is a lower
+// bound of the answer.  At smaller sizes the extra sweep and level cost more than they save (16384 keys: 13 us).
 template <typename T, int SN>
 __global__ __launch_bounds__(SCAN_THREADS) void k_sample_cut(
-    const uint32_t *sample, unsigned long long N, unsigned long long K, SelState *st, uint32_t *hist,
+    const uint32_t *sample, int sample_n, unsigned long long N, unsigned long long K, SelState *st, uint32_t *hist,
     uint32_t *pool_count, uint32_t *aux_count, uint32_t path) {
   constexpr int KB = Elem<T>::KEYBITS;
-  constexpr int PER = SN / SCAN_THREADS;
+  constexpr int PER = SN ? SN / SCAN_THREADS : 1;
   __shared__ uint32_t lh[NBINS];
   const int p = blockIdx.x, tid = threadIdx.x;
-  const unsigned long long ns = N < (unsigned long long)SN ? N : (unsigned long long)SN;
+  const unsigned long long ns = N < (unsigned long long)sample_n ? N : (unsigned long long)sample_n;
   for (int i = tid; i < NBINS; i += SCAN_THREADS) hist[(int64_t)p * NBINS + i] = 0;
   if (tid == 0) { pool_count[p] = 0; if (aux_count) aux_count[p] = 0; }
+  const uint32_t *mine = sample + (int64_t)p * sample_n;
   uint32_t keys[PER];
   bool valid[PER];
+  if (SN) {
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    unsigned long long si = (unsigned long long)tid + (unsigned long long)i * SCAN_THREADS;
-    valid[i] = si < ns;
-    keys[i] = valid[i] ? sample[(int64_t)p * SN + si] : 0u;
+    for (int i = 0; i < PER; ++i) {
+      unsigned long long si = (unsigned long long)tid + (unsigned long long)i * SCAN_THREADS;
+      valid[i] = si < ns;
+      keys[i] = valid[i] ? mine[si] : 0u;
+    }
   }
+  uint32_t bound = 0, top = 0;
+  auto each = [&](auto f) {
+    if (SN) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (valid[i]) f(keys[i]);
+    } else {
+      // the slots of a problem are a multiple of four: reading a whole vector at the end stays inside them
+      for (unsigned i = 4u * tid; i < ns; i += 16u * SCAN_THREADS) {
+        uint4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const unsigned j = i + 4u * SCAN_THREADS * q;
+          v[q] = j < ns ? *reinterpret_cast<const uint4 *>(mine + j) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const unsigned j = i + 4u * SCAN_THREADS * q;
+          if (j < ns && v[q].x >= bound) f(v[q].x);
+          if (j + 1 < ns && v[q].y >= bound) f(v[q].y);
+          if (j + 2 < ns && v[q].z >= bound) f(v[q].z);
+          if (j + 3 < ns && v[q].w >= bound) f(v[q].w);
+        }
+      }
+    }
+  };
   unsigned long long r;
   if (ns == N && path != PATH_TILES) r = K;   // the sample is the whole problem
   else {
     double e = (double)K / (double)N * (double)ns;
-    // the sample taken ahead of the projection (PATH_TILES) is four times larger and made of 32 x 32
-    // blocks of tokens x features: a smaller relative margin, the same six standard deviations
+    // the sample taken ahead of the projection (PATH_TILES) is made of 32 x 32 blocks of tokens x features
+    // and is four times the smallest of the others: a smaller relative margin, the same six standard deviations
     r = path == PATH_TILES ? (unsigned long long)(1.2 * e + 6.0 * sqrt(e) + 16.0) + 1
                            : (unsigned long long)(1.25 * e + 6.0 * sqrt(e) + 16.0) + 1;
   }
@@ -245,20 +279,22 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_sample_cut(
     constexpr int NLEV = KB == 32 ? 3 : 2;
     const int shifts[3] = {KB == 32 ? 21 : 5, KB == 32 ? 10 : 0, 0};
     const int widths[3] = {11, KB == 32 ? 11 : 5, 10};
+    const bool narrow = SN == 0 && r <= SCAN_THREADS && ns >= 4ull * SCAN_THREADS;   // every thread has a key
+    if (narrow) each([&](uint32_t key) { top = key > top ? key : top; });
     uint32_t prefix = 0, prefix_mask = 0;  // decided high bits
     unsigned long long k_rem = r;
-    for (int lev = 0; lev < NLEV; ++lev) {
+    for (int lev = narrow ? -1 : 0; lev < NLEV; ++lev) {
       for (int i = tid; i < NBINS; i += SCAN_THREADS) lh[i] = 0;
       __syncthreads();
-      const int sh = shifts[lev];
-      const uint32_t dm = (1u << widths[lev]) - 1u;
-#pragma unroll
-      for (int i = 0; i < PER; ++i)
-        if (valid[i] && (keys[i] & prefix_mask) == prefix) atomicAdd(&lh[(keys[i] >> sh) & dm], 1u);
+      const int sh = lev < 0 ? shifts[0] : shifts[lev];
+      const uint32_t dm = (1u << (lev < 0 ? widths[0] : widths[lev])) - 1u;
+      if (lev < 0) atomicAdd(&lh[(top >> sh) & dm], 1u);
+      else each([&](uint32_t key) { if ((key & prefix_mask) == prefix) atomicAdd(&lh[(key >> sh) & dm], 1u); });
       __syncthreads();
       int bin; unsigned long long above, total;
       block_find_from_top(lh, (int)dm + 1, k_rem, bin, above, total);
       if (bin < 0) bin = 0;  // cannot happen (r <= ns); keep the cut low if it does
+      if (lev < 0) { bound = (uint32_t)bin << sh; continue; }
       k_rem -= above;
       prefix |= (uint32_t)bin << sh;
       prefix_mask |= dm << sh;
@@ -1308,7 +1344,7 @@ static int run_tokentopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
 struct SelLayout {
   size_t off_state, off_hist, off_poolcnt, off_sample, off_first, off_gt, off_eq, off_allot, off_keep, off_xcut, off_pool, total;
   unsigned long long pool_cap;  // entries per problem
-  int nprob;
+  int nprob, sample_n;          // problems; keys of the sample gathered from the matrix, per problem
 };
 
 static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode) {
@@ -1325,12 +1361,20 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   if (cap > hard) cap = hard;
   if (cap > 0xFFF00000ull) cap = 0xFFF00000ull;
   lo.pool_cap = cap;
+  // A sample with e keys above the threshold gives a cut with up to (1.25 + 6 / sqrt(e) + 17 / e) K candidates:
+  // 2.8 K at SAMPLE_HITS.  K elements are one in 1500 when 12 layers of 24576 features are ranked together and 200
+  // kept per token: the smallest sample then has 11 hits and a cut with 4.6 K, which is more than the pool holds -
+  // the rows left without pool space are read again from the matrix by every later stage (3000 tokens: 2.9 ms of 4.0).
+  // Ranked per layer the smallest sample has over 100 hits.
+  double ns = K ? SAMPLE_HITS * (double)N / (double)K : 0.0;
+  lo.sample_n = SAMPLE_MIN;
+  while (lo.sample_n < SAMPLE_MAX && (double)lo.sample_n < ns) lo.sample_n *= 4;
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
   lo.off_state = take(sizeof(SelState) * (size_t)lo.nprob);
   lo.off_hist = take(sizeof(uint32_t) * NBINS * (size_t)lo.nprob);
   lo.off_poolcnt = take(4 * (size_t)lo.nprob);
-  lo.off_sample = take(4 * (size_t)(SAMPLE_PRE_N > SAMPLE_N ? SAMPLE_PRE_N : SAMPLE_N) * (size_t)lo.nprob);
+  lo.off_sample = take(4 * (size_t)(SAMPLE_PRE_N > lo.sample_n ? SAMPLE_PRE_N : lo.sample_n) * (size_t)lo.nprob);
   lo.off_first = take(4 * R);
   lo.off_gt = take(4 * R);
   lo.off_eq = take(4 * R);
@@ -1361,8 +1405,14 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
   unsigned long long K = (unsigned long long)k * (unsigned long long)Tn;
   if (K > N) K = N;
   const int nprob = lo.nprob;
-  k_sample_keys<T, GLOBAL><<<dim3(SAMPLE_BLOCKS, nprob), 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, N, sample);
-  k_sample_cut<T, SAMPLE_N><<<nprob, SCAN_THREADS, 0, stream>>>(sample, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
+  k_sample_keys<T, GLOBAL><<<dim3(lo.sample_n / 1024, nprob), 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, N,
+                                                                              lo.sample_n, sample);
+  if (lo.sample_n == SAMPLE_MIN)
+    k_sample_cut<T, SAMPLE_MIN><<<nprob, SCAN_THREADS, 0, stream>>>(sample, lo.sample_n, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
+  else if (lo.sample_n <= SAMPLE_PRE_N)
+    k_sample_cut<T, SAMPLE_PRE_N><<<nprob, SCAN_THREADS, 0, stream>>>(sample, lo.sample_n, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
+  else
+    k_sample_cut<T, 0><<<nprob, SCAN_THREADS, 0, stream>>>(sample, lo.sample_n, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
   // two rows per wavefront: many more blocks than fit at once, so rows of very different
   // candidate counts balance out over the CUs
   int gx = (int)clt_ceil_div(Tn, 8);
@@ -1497,7 +1547,7 @@ static int run_encode_collect(const void *x, const void *w, const void *b, void 
   if (K > N) K = N;
   k_sample_mfma<T><<<dim3(SAMPLE_WAVES / 4, (unsigned)L), 256, 0, stream>>>((const T *)x, (const T *)w, (const T *)b, Tn, d,
                                                                           F, xs, wstr, bs, sample);
-  k_sample_cut<T, SAMPLE_PRE_N><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(sample, N, K, st, hist, poolcnt,
+  k_sample_cut<T, SAMPLE_PRE_N><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(sample, SAMPLE_PRE_N, N, K, st, hist, poolcnt,
                                                               (uint32_t *)(ws + tl.off_tcount), PATH_TILES);
   uint2 *tpool = (uint2 *)(ws + tl.off_tpool);
   CollectArgs ca;
