@@ -788,6 +788,130 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   __builtin_amdgcn_s_waitcnt(0);   // no direct-to-LDS load may be in flight when the block retires
 }
 
+// ---- short batches ------------------------------------------------------------------------------------
+// Fewer than BM tokens: the weights' one pass through the chip is the work, and a 256-token tile would multiply padding
+// and leave most CUs idle on a small model (12 tiles at L = 3, F = 1024).  A block takes 32 NF features x 32 MT tokens;
+// a stage is 128 bytes of K as above, and its four wavefronts split each stage's K between them - 32 K bytes each, so
+// that even one block has four matrix cores at work - and add their sums through LDS at the end, in a fixed order.
+// Three stages in LDS, two on their way: 30 - 72 KB in flight per CU, which is what HBM needs.
+//
+// Bound by the weights' HBM stream at few tokens (453 MB at L = 12, d = 768, F = 24576, bf16: 76 us for one token), by the
+// blocks' repeated reads of x towards 128, and by the chain of K stages on a small model.  Against the 256-token tiles on
+// a padded batch, us, at 1 / 32 / 77 / 128 / 255 tokens:
+//   L 12, d 768, F 24576, bf16      76 / 94 / 141 / 176 / 303  against  178 / 186 / 189 / 200 / 228
+//   L 16, d 2048, F 16384, bf16    197 / 206 / 266 / 309 / 549  against  334 / 335 / 337 / 346 / 382
+//   L 12, d 768, F 6144, float32    46 / 44 / 108 / 143 / 251  against  385 / 380 / 385 / 388 / 402
+//   L 3, d 768, F 1024, float32     13 / 12 / 14 / 18 / 18  against  184 / 185 / 187 / 188 / 189
+// Hence the rule of encode_short_ok: up to 128 tokens (one block along them, W is read once), and up to 255 in float32,
+// whose matrix products are what bounds, or where the large tiles would not fill the chip once.
+constexpr int SK_STAGES = 3;
+
+// 16 bytes per lane into LDS (lane i lands at lds_at + 16 i), as a statement the compiler does not count: it would wait
+// for the stages in flight before every fragment read.  The waits are written out by hand.
+__device__ __forceinline__ void sk_fill16(const void *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+
+template <typename T, int NF, int MT>
+__global__ __launch_bounds__(256, 2) void k_encode_short(const T *__restrict__ x, const T *__restrict__ w, const T *__restrict__ bias,
+                                                         T *__restrict__ pre, int M, int K, int N, int64_t xs, int64_t wstr,
+                                                         int64_t bs, int64_t ps) {
+  constexpr int WR = 32 * NF, XR = 32 * MT, BYTES = (WR + XR) * ROWB, LOADS = NF + MT;   // loads of a stage per wavefront
+  constexpr int RP = WR + 4;                                // fp32 row pitch of the partial sums
+  constexpr int RED = 4 * 32 * RP * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[SK_STAGES * BYTES > RED ? SK_STAGES * BYTES : RED];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * WR, m0 = blockIdx.y * XR, layer = blockIdx.z;
+  const int nk = K * (int)sizeof(T) / ROWB;
+  const char *wt = (const char *)(w + layer * wstr + (int64_t)n0 * K), *xt = (const char *)(x + layer * xs + (int64_t)m0 * K);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
+
+  // wavefront `wave` brings in the 8-row groups wave, wave + 4, ..: first those of W, then those of x.  Rows past the end
+  // repeat the last one; nothing is stored for them.
+  uint32_t off[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = (wave + 4 * (i < NF ? i : i - NF)) * 8 + (lane >> 3);
+    const int left = i < NF ? N - n0 : M - m0;
+    off[i] = (uint32_t)(r < left ? r : left - 1) * (uint32_t)K * (uint32_t)sizeof(T) + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) << 4);
+  }
+  auto issue = [&](int kt, uint32_t buf) {
+    const uint32_t at = lds0 + buf * BYTES + (uint32_t)wave * 1024;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      sk_fill16((i < NF ? wt : xt) + (int64_t)kt * ROWB, off[i], at + (uint32_t)((i < NF ? i : i - NF) * 4096 + (i < NF ? 0 : WR * ROWB)));
+  };
+
+  f32x16_t acc[NF][MT];
+#pragma unroll
+  for (int j = 0; j < NF; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[j][i][q] = 0.0f;
+  const int l31 = lane & 31, lh = lane >> 5;
+  const int frag = l31 * ROWB + (((wave * 2 + lh) ^ ((l31 >> 1) & 7)) << 4);      // this wavefront's quarter of a stage's K
+
+  issue(0, 0);
+  if (nk > 1) issue(1, 1);
+  uint32_t buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // stage kt has landed (only the next one's loads may be under way), and this wavefront's reads of the stage before are over
+    if (kt + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0070 | LOADS);      // vmcnt(LOADS) lgkmcnt(0)
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + 2 < nk) issue(kt + 2, buf == 0 ? 2 : buf - 1);
+    const unsigned char *st = lds + buf * BYTES + frag;
+    uint4 fw[NF], fx[MT];
+#pragma unroll
+    for (int j = 0; j < NF; ++j) fw[j] = *reinterpret_cast<const uint4 *>(st + j * 32 * ROWB);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) fx[i] = *reinterpret_cast<const uint4 *>(st + (WR + i * 32) * ROWB);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NF; ++j) Mma<T>::run(acc[j][i], fw[j], fx[i]);
+    buf = buf == SK_STAGES - 1 ? 0 : buf + 1;
+  }
+
+  float *red = reinterpret_cast<float *>(lds);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    __syncthreads();                                        // the stages, or the tokens before these, have been read
+#pragma unroll
+    for (int j = 0; j < NF; ++j)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+        *reinterpret_cast<float4 *>(red + (wave * 32 + l31) * RP + j * 32 + rg * 8 + lh * 4) =
+            make_float4(acc[j][i][rg * 4], acc[j][i][rg * 4 + 1], acc[j][i][rg * 4 + 2], acc[j][i][rg * 4 + 3]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NF; ++u) {
+      const int e = threadIdx.x + u * 256, tok = e / (WR / 4), c = e % (WR / 4) * 4;
+      const int m = m0 + i * 32 + tok, n = n0 + c;
+      if (m >= M || n >= N) continue;
+      const float *p = red + tok * RP + c;
+      float y[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float b = bias && n + q < N ? Elem<T>::to_f32(bias[layer * bs + n + q]) : 0.0f;
+        y[q] = b + ((p[q] + p[32 * RP + q]) + (p[64 * RP + q] + p[96 * RP + q]));
+      }
+      T *o = pre + layer * ps + (int64_t)m * N + n;
+      if ((N & 3) == 0) {                                   // whole quads, 8 or 16 bytes aligned (short_ok)
+        if constexpr (sizeof(T) == 4) *reinterpret_cast<float4 *>(o) = make_float4(y[0], y[1], y[2], y[3]);
+        else *reinterpret_cast<uint2 *>(o) = make_uint2(pack16x2<T>(y[0], y[1]), pack16x2<T>(y[2], y[3]));
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (n + q < N) o[q] = Elem<T>::from_f32(y[q]);
+      }
+    }
+  }
+}
+
 // Any shape: one thread per output, fp32 accumulation.
 template <typename T>
 __global__ void k_encode_generic(const T *x, const T *w, const T *bias, T *pre, int64_t M, int64_t K, int64_t N,
@@ -813,6 +937,36 @@ static bool encode_fast_ok(const void *x, const void *w, const void *b, const vo
          F < (1 << 30) && d < (1 << 30) && (!b || (((uintptr_t)b) % 16 == 0 && bs % 8 == 0));
 }
 
+// What k_encode_short takes: a batch shorter than one tile (where it is the faster one, see there), whole 128-byte stages,
+// aligned rows and output quads.
+template <typename T>
+static bool encode_short_ok(const void *x, const void *w, const void *pre, int64_t T_, int64_t d, int64_t F, int64_t L, int64_t xs,
+                            int64_t wstr, int64_t ps) {
+  constexpr int CE = 16 / (int)sizeof(T);
+  const bool faster = T_ <= 128 || (T_ < BM && (sizeof(T) == 4 || clt_ceil_div(F, BN) * L <= 256));
+  return faster && d % (ROWB / (int)sizeof(T)) == 0 && d < (1 << 22) && F < (1 << 30) && L <= 65535 && clt_aligned16(x) &&
+         clt_aligned16(w) && clt_aligned16(pre) && xs % CE == 0 && wstr % CE == 0 && (F % 4 != 0 || ps % 4 == 0);
+}
+
+template <typename T>
+static int launch_encode_short(const void *x, const void *w, const void *b, void *pre, int64_t T_, int64_t d, int64_t F, int64_t L,
+                               int64_t xs, int64_t wstr, int64_t bs, int64_t ps, hipStream_t stream) {
+  const int groups = (int)clt_ceil_div(T_, 32), ny = (int)clt_ceil_div(groups, 4), mt = (int)clt_ceil_div(groups, ny);
+  // 64 features per block, which halves what is read of x, unless that leaves compute units idle
+  const bool wide = clt_ceil_div(F, 64) * ny * L >= 256;
+  const dim3 grid((unsigned)clt_ceil_div(F, wide ? 64 : 32), (unsigned)ny, (unsigned)L);
+#define CLT_SHORT(NF, MT)                                                                                                  \
+  k_encode_short<T, NF, MT><<<grid, 256, 0, stream>>>((const T *)x, (const T *)w, (const T *)b, (T *)pre, (int)T_, (int)d, \
+                                                      (int)F, xs, wstr, bs, ps)
+#define CLT_SHORT_MT(NF)                                                                                                   \
+  switch (mt) { case 1: CLT_SHORT(NF, 1); break; case 2: CLT_SHORT(NF, 2); break; case 3: CLT_SHORT(NF, 3); break;         \
+                default: CLT_SHORT(NF, 4); break; }
+  if (wide) CLT_SHORT_MT(2) else CLT_SHORT_MT(1)
+#undef CLT_SHORT_MT
+#undef CLT_SHORT
+  return clt_check_launch();
+}
+
 // One persistent workgroup per CU (a whole number of rounds over the 8 XCDs, so that block b stays on XCD
 // b % 8 for all of its tiles), or one per tile when there are fewer tiles; 0 when the device cannot be asked.
 static int64_t persistent_grid(int64_t tiles) {
@@ -830,6 +984,8 @@ static int launch_encode(const void *x, const void *w, const void *b, void *pre,
                          const SelState *gate, const CollectArgs *ca, hipStream_t stream) {
   const bool fast = encode_fast_ok<T>(x, w, b, collect ? nullptr : pre, T_, d, F, xs, wstr, bs, collect ? 16 : ps);
   if (collect && !fast) return CLT_ERR_ARG;
+  if (!collect && encode_short_ok<T>(x, w, pre, T_, d, F, L, xs, wstr, ps))
+    return launch_encode_short<T>(x, w, b, pre, T_, d, F, L, xs, wstr, bs, ps, stream);
   if (fast) {
     const int64_t tm = clt_ceil_div(T_, BM), tn = clt_ceil_div(F, BN);
     const int64_t nblk = tm * tn * L;
@@ -931,6 +1087,9 @@ extern "C" int clt_encode_fast_path(const void *x, const void *w, const void *b,
                                     int64_t b_layer_stride, int64_t pre_layer_stride, int dtype) {
   if (!clt_model_dtype(dtype) || T <= 0 || d <= 0 || F <= 0 || L <= 0 || !x || !w || !pre) return 0;
   if (clt_ceil_div(T, BM) * clt_ceil_div(F, BN) * L > 2147483647LL) return 0;
+  if (dtype != CLT_F32 ? encode_short_ok<bf16_t>(x, w, pre, T, d, F, L, x_layer_stride, w_layer_stride, pre_layer_stride)
+                       : encode_short_ok<float>(x, w, pre, T, d, F, L, x_layer_stride, w_layer_stride, pre_layer_stride))
+    return 1;
   const bool fast = dtype != CLT_F32
                         ? encode_fast_ok<bf16_t>(x, w, b, pre, T, d, F, x_layer_stride, w_layer_stride, b_layer_stride, pre_layer_stride)
                         : encode_fast_ok<float>(x, w, b, pre, T, d, F, x_layer_stride, w_layer_stride, b_layer_stride, pre_layer_stride);

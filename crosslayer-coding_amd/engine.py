@@ -118,7 +118,8 @@ def _wants_sliced_decode(rows: int, slab_bytes: int) -> bool:
     return rows >= SLICED_DECODE_MIN_ROWS or slab_bytes >= SLICED_DECODE_MIN_SLAB_BYTES
 
 
-# token rows of one tile of the matrix-core encoder: shorter batches are padded to it (see ``encode``)
+# token rows of one tile of the matrix-core encoder: shorter batches are padded to it where the kernel for short ones
+# does not take them (see ``encode``)
 ENCODE_MIN_TOKENS = 256
 # widest d_model the gradient kernels that walk survivor lists take (a row is held by one wavefront, up to eight
 # 16-byte pieces per lane in bf16); wider models get their gradients from the dense formulation

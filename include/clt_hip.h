@@ -92,7 +92,8 @@ int clt_encode(const void *x, const void *w, const void *b, void *pre,
  * 1 when clt_encode runs these operands on the matrix cores: T >= 256, F >= 256, F % 4 == 0,
  * d a whole number of 128-byte stages (64 elements of 16 bits, 32 of fp32), 16-byte aligned
  * pointers, layer strides that keep every layer 16-byte aligned (the bias stride a multiple
- * of 8 elements).  0: the call is served by a generic kernel with one thread per output,
+ * of 8 elements); or a short batch, for which F and the bias may be anything: T <= 128, and
+ * T < 256 in fp32 and for models of at most 256 tiles of 256 features (L * ceil(F / 256)).  0: the call is served by a generic kernel with one thread per output,
  * two to three orders of magnitude slower on large shapes; a caller with such a shape does
  * better to hand over zero-padded copies (the host mirror does, crosslayer_coding_amd.engine.encode).
  * No counterpart in the reference (its F.linear takes any shape at one speed).
