@@ -1113,6 +1113,39 @@ __global__ void k_densify_scatter(const int32_t *row_ptr, const int32_t *col, co
   }
 }
 
+// Dense rows from their lists in one pass: a workgroup puts a piece of a row together in LDS - zeros, then the row's
+// survivors - and writes it out 16 bytes per lane.  Bound by the stream of stores.  Element-wise zeros in front of a scatter
+// (k_zero_rows, k_densify_scatter; still what rows that are not whole 16-byte pieces take) write at 2 TB/s and touch the
+// scattered lines twice.  L = 12, F = 24576, 1000 tokens, bf16 (590 MB): 0.36 -> 0.114 ms.
+constexpr int DENSIFY_BYTES = 32 * 1024;   // of LDS: five workgroups per CU
+
+template <typename T, typename OT>
+__global__ __launch_bounds__(256) void k_densify_rows(const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
+                                                      const T *__restrict__ val, OT *__restrict__ out, int64_t Tn, int64_t F, int pieces,
+                                                      int64_t out_layer_stride) {
+  constexpr int N = DENSIFY_BYTES / (int)sizeof(OT);
+  __shared__ __attribute__((aligned(16))) OT piece[N];
+  const int64_t r = blockIdx.x / pieces, c0 = (int64_t)(blockIdx.x % pieces) * N;
+  const int n = (int)(F - c0 < N ? F - c0 : N), quads = n * (int)sizeof(OT) / 16;
+  const int32_t b = row_ptr[r], e = row_ptr[r + 1];
+  for (int i = threadIdx.x; i < quads; i += 256) reinterpret_cast<uint4 *>(piece)[i] = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  for (int32_t j = b + (int32_t)threadIdx.x; j < e; j += 256) {
+    const int64_t c = col[j] - c0;
+    if (c < 0 || c >= n) continue;
+    if constexpr (std::is_same<T, OT>::value) piece[c] = val[j];
+    else piece[c] = (OT)Elem<T>::to_f32(val[j]);
+  }
+  __syncthreads();
+  uint4 *o = reinterpret_cast<uint4 *>(out + r / Tn * out_layer_stride + r % Tn * F + c0);
+  for (int i = threadIdx.x; i < quads; i += 256) o[i] = reinterpret_cast<const uint4 *>(piece)[i];
+}
+
+// zeros over whole 16-byte pieces
+__global__ __launch_bounds__(256) void k_zero_quads(uint4 *out, int64_t n) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 template <typename OT>
 __global__ void k_zero_rows(OT *out, int64_t Tn, int64_t F, int64_t L, int64_t out_layer_stride) {
   const int64_t per_layer = Tn * F;
@@ -1499,6 +1532,18 @@ extern "C" int clt_densify(const int32_t *row_ptr, const int32_t *col, const voi
   if (T == 0 || F == 0) return CLT_OK;
   if (!row_ptr || !out) return CLT_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
+  const int64_t oe = dtype == CLT_F32 || out_f32 ? 4 : 2, pieces = clt_ceil_div(F * oe, DENSIFY_BYTES);
+  if (F * oe % 16 == 0 && out_layer_stride * oe % 16 == 0 && clt_aligned16(out) && L * T * pieces <= 0x7FFFFFFFll) {
+    const unsigned blocks = (unsigned)(L * T * pieces);
+#define CLT_DENSIFY(TT, OT) \
+  k_densify_rows<TT, OT><<<blocks, 256, 0, s>>>(row_ptr, col, (const TT *)val, (OT *)out, T, F, (int)pieces, out_layer_stride)
+    if (dtype == CLT_F32) CLT_DENSIFY(float, float);
+    else if (out_f32 && dtype == CLT_F16) CLT_DENSIFY(f16_t, float);
+    else if (out_f32) CLT_DENSIFY(bf16_t, float);
+    else CLT_DENSIFY(bf16_t, bf16_t);
+#undef CLT_DENSIFY
+    return clt_check_launch();
+  }
   const int nb = 256 * 8;
   if (dtype == CLT_F32 || out_f32) k_zero_rows<float><<<nb, 256, 0, s>>>((float *)out, T, F, L, out_layer_stride);
   else k_zero_rows<bf16_t><<<nb, 256, 0, s>>>((bf16_t *)out, T, F, L, out_layer_stride);
@@ -1551,7 +1596,9 @@ extern "C" int clt_accumulate_dense(const int32_t *row_ptr, const int32_t *col, 
   hipStream_t s = (hipStream_t)stream;
   const unsigned nb = (unsigned)(clt_ceil_div(T, 4) < 8192 ? clt_ceil_div(T, 4) : 8192);
   if (init) {
-    if (dtype != CLT_F32) k_zero_rows<bf16_t><<<2048, 256, 0, s>>>((bf16_t *)acc, T, F, 1, T * F);
+    const int64_t bytes = T * F * (dtype != CLT_F32 ? 2 : 4);
+    if (bytes % 16 == 0 && clt_aligned16(acc)) k_zero_quads<<<2048, 256, 0, s>>>((uint4 *)acc, bytes / 16);
+    else if (dtype != CLT_F32) k_zero_rows<bf16_t><<<2048, 256, 0, s>>>((bf16_t *)acc, T, F, 1, T * F);
     else k_zero_rows<float><<<2048, 256, 0, s>>>((float *)acc, T, F, 1, T * F);
   }
   if (layer < 0) return clt_check_launch();   // clear only
