@@ -461,6 +461,33 @@ __device__ __forceinline__ UnitWork unit_work(const UnitPlan &up, int64_t Tn) {
   return w;
 }
 
+// ---- one launch per source, or one for all --------------------------------------------------------------
+// With a launch per source layer the partial rows [slice][target][token] collect their sources over the launches.  A short
+// batch leaves most of the chip idle in every one of them; it gets a single launch over all (source, target) pairs with a
+// partial row for each [slice][pair][token], and k_decode_reduce adds a target's sources in the same order: same bits.
+// L = 12, d = 768, F = 24576, bf16, 200 per token, us per decode, launch per source / one launch: 1 token 82 / 27,
+// 32 tokens 260 / 158, 77 tokens 380 / 310 (780 / 240 on activations whose fullest token has many times the mean: no launch
+// waits for it), 256 tokens 730 / 668, 512 tokens 1188 / 1167.
+struct PairAt { int src; int64_t t, row; bool first; };      // row: of the partial rows, in units of Tn rows
+__device__ __forceinline__ PairAt pair_at(int64_t target, int src, int slice, int64_t L, int64_t t_begin, int64_t t_end,
+                                          uint64_t src_mask) {
+  PairAt p;
+  if (src >= 0) {
+    p.src = src; p.t = t_begin + target; p.row = (int64_t)slice * L + p.t;
+    p.first = (src_mask & ((1ull << src) - 1ull)) == 0;      // the first source initialises the partial rows
+    return p;
+  }
+  p.src = 0; p.first = true;
+  for (;; ++p.src) {
+    if (!((src_mask >> p.src) & 1ull)) continue;
+    const int64_t from = p.src > t_begin ? p.src : t_begin;
+    if (target < t_end - from) { p.t = from + target; break; }
+    target -= t_end - from;
+  }
+  p.row = (int64_t)slice * (L * (L + 1) / 2) + decoder_slot(CLT_TYING_NONE, p.src, p.t, L);
+  return p;
+}
+
 // ---- quarter-row schedule -------------------------------------------------------------------------
 // Large batches, untied or per-source decoders, d a multiple of 256: the feature axis is cut into 2
 // slices and the columns into 4 quarters; workgroup b works on part b % 8 = (slice, quarter), so an XCD
@@ -543,7 +570,7 @@ template <typename T, int HQ, int HTAIL, int UU, bool AFFINE, bool PACK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(quarter_min_waves<T, HQ, HTAIL>(), 8))) void k_decode_quarter(
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp, const T *__restrict__ foff,
     const T *__restrict__ fscale, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin, uint64_t src_mask,
-    const int32_t *__restrict__ sptr, float *__restrict__ partial, int src, int64_t pitch, UnitPlan up) {
+    const int32_t *__restrict__ sptr, float *__restrict__ partial, int src_arg, int64_t pitch, UnitPlan up, int64_t t_end) {
   constexpr int V = WVec<T>::V;
   constexpr int NACC = HQ * V + (HTAIL ? V / 2 : 0);      // columns per lane: d / 64
   constexpr int NCP = QUARTER_PARTS;
@@ -553,12 +580,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(quarter_min
   const bool hi = grp != 0;                    // only the first lane group touches the partial row
   const UnitWork uw = unit_work(up, Tn);
   const int slice = uw.slice, cpart = uw.cpart;
-  const int64_t t = t_begin + uw.target;
+  const PairAt at = pair_at(uw.target, src_arg, slice, L, t_begin, t_end, src_mask);
+  const int src = at.src;
+  const int64_t t = at.t;
+  const bool first = at.first;
   const int64_t tok_end = uw.tok_end;
   const int64_t tok0 = uw.tok_begin + ((int64_t)uw.tb * nwv + wv) * QUARTER_NTOK;
   if (tok0 >= tok_end) return;
-  const uint64_t below = src_mask & ((1ull << src) - 1ull);
-  const bool first = below == 0;   // the first source initialises the partial rows
   int32_t mb = 0, me = 0;
   if (lane < QUARTER_NTOK && tok0 + lane < tok_end) {
     const int64_t r = (int64_t)src * Tn + tok0 + lane;
@@ -581,7 +609,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(quarter_min
     if (tok0 + i >= tok_end) break;
     if (b == e && !first) continue;
     // this lane's columns of the partial row (the first lane group writes it): pieces of V, then the tail
-    float *prow = partial + (((int64_t)slice * L + t) * Tn + tok0 + i) * d + (int64_t)cpart * (d / NCP);
+    float *prow = partial + (at.row * Tn + tok0 + i) * d + (int64_t)cpart * (d / NCP);
     float old[NACC], acc[NACC];
 #pragma unroll
     for (int j = 0; j < NACC; ++j) { old[j] = 0.0f; acc[j] = 0.0f; }
@@ -721,7 +749,7 @@ template <typename T, bool AFFINE, bool PACK, int NTOK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_decode_line(
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp, const T *__restrict__ foff,
     const T *__restrict__ fscale, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin, uint64_t src_mask,
-    const int32_t *__restrict__ sptr, float *__restrict__ partial, int src, UnitPlan lp, int64_t pitch) {
+    const int32_t *__restrict__ sptr, float *__restrict__ partial, int src_arg, UnitPlan lp, int64_t pitch, int64_t t_end) {
   constexpr int V = WVec<T>::V;                     // elements per lane: 16 bytes
   constexpr int LW = 8 * V;                         // columns per part: one 128-byte line
   constexpr int LINE_NTOK = NTOK;
@@ -729,13 +757,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
   const int ll = lane & 7, grp = lane >> 3;
   const int ns = lp.ns;
   const UnitWork uw = unit_work(lp, Tn);
-  const int64_t t = t_begin + uw.target;
   const int cpart = uw.cpart, slice = uw.slice;
+  const PairAt at = pair_at(uw.target, src_arg, slice, L, t_begin, t_end, src_mask);
+  const int src = at.src;
+  const int64_t t = at.t;
+  const bool first = at.first;
   const int64_t part_end = uw.tok_end;
   const int64_t tok0 = uw.tok_begin + ((int64_t)uw.tb * nwv + wv) * LINE_NTOK;
   if (tok0 >= part_end) return;
-  const uint64_t below = src_mask & ((1ull << src) - 1ull);
-  const bool first = below == 0;   // the first source initialises the partial rows
   int32_t mb = 0, me = 0;
   if (lane < LINE_NTOK && tok0 + lane < part_end) {
     const int64_t r = (int64_t)src * Tn + tok0 + lane;
@@ -817,7 +846,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
       csel = ll * 4 + ((grp >> 2) & 1) * 2 + ((grp >> 1) & 1);
       writer = (grp & 1) == 0;
     }
-    float *pp = partial + (((int64_t)slice * L + t) * Tn + tok0 + it) * d + (int64_t)cpart * LW + csel;
+    float *pp = partial + (at.row * Tn + tok0 + it) * d + (int64_t)cpart * LW + csel;
     if (writer) {
       const float old = first ? 0.0f : __builtin_nontemporal_load(pp);
       __builtin_nontemporal_store(old + r, pp);
@@ -845,13 +874,27 @@ __global__ void k_slice_ptr(const int32_t *row_ptr, const int32_t *col, int64_t 
 template <typename T>
 __global__ void k_decode_reduce(const float *__restrict__ partial, const float *__restrict__ bias_sum,
                                 const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d,
-                                int64_t L, int64_t t_begin, int64_t t_end, int ns, int out_f32, uint64_t src_mask) {
+                                int64_t L, int64_t t_begin, int64_t t_end, int ns, int out_f32, uint64_t src_mask,
+                                bool pairs = false) {
   const int64_t per_t = Tn * d, span = (t_end - t_begin) * per_t, slice_stride = L * per_t;
   for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < span; i += (int64_t)gridDim.x * blockDim.x * 4) {
     const int64_t g = t_begin * per_t + i;          // index into [L][T][d]
     const int64_t t = g / per_t, o = g % d;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (src_mask & ((2ull << t) - 1ull)) {            // some source <= t wrote partial rows
+    if (pairs) {                                      // a partial row per (source, target): sources first, then slices
+      const int64_t np = L * (L + 1) / 2, at = g - t * per_t;
+      for (int sl = 0; sl < ns; ++sl) {
+        float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+        for (int64_t s = 0; s <= t; ++s) {
+          if (!((src_mask >> s) & 1ull)) continue;
+          const float4 q = *reinterpret_cast<const float4 *>(partial + (sl * np + decoder_slot(CLT_TYING_NONE, s, t, L)) * per_t + at);
+          b.x += q.x; b.y += q.y; b.z += q.z; b.w += q.w;
+        }
+        if (sl == 0) a = b;
+        else { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; }
+      }
+    } else if (src_mask & ((2ull << t) - 1ull)) {     // some source <= t wrote partial rows
       a = *reinterpret_cast<const float4 *>(partial + g);
       for (int sl = 1; sl < ns; ++sl) {
         float4 b = *reinterpret_cast<const float4 *>(partial + sl * slice_stride + g);
@@ -1207,8 +1250,24 @@ __global__ __launch_bounds__(256) void k_accumulate_dense(const int32_t *__restr
 
 constexpr int DEC_SLICES = 8;  // one feature slice per XCD of an MI355X
 
+// Partial rows of a batch, in units of Tn rows of d: a target's feature slices, or for a short batch (whose rows then stay
+// below PAIR_BYTES) the pairs' of a launch over all sources with two slices.
+constexpr int64_t PAIR_BYTES = 256 << 20;
+static int64_t partial_rows(int64_t Tn, int64_t d, int64_t L) {
+  const int64_t by_target = DEC_SLICES * L, by_pair = L * (L + 1);
+  return by_pair > by_target && by_pair * Tn * d * 4 <= PAIR_BYTES ? by_pair : by_target;
+}
+static bool one_launch(int64_t Tn, int64_t d, int64_t L, int slices) {
+  const int64_t rows = slices * (L * (L + 1) / 2);
+  return rows <= partial_rows(Tn, d, L) && rows * Tn * d * 4 <= PAIR_BYTES;
+}
+
+static size_t partial_bytes(int64_t Tn, int64_t d, int64_t L) {
+  return ((size_t)partial_rows(Tn, d, L) * Tn * d * 4 + 255) & ~(size_t)255;
+}
+
 static size_t decode_ws_bytes(int64_t Tn, int64_t d, int64_t L) {
-  size_t part = ((size_t)DEC_SLICES * L * Tn * d * 4 + 255) & ~(size_t)255;
+  size_t part = partial_bytes(Tn, d, L);
   size_t sp = ((size_t)L * Tn * (DEC_SLICES + 1) * 4 + 255) & ~(size_t)255;
   return part + sp;
 }
@@ -1265,7 +1324,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
   int32_t *sptr = nullptr; float *partial = nullptr;
   if (can_slice) {
     partial = (float *)workspace;
-    sptr = (int32_t *)((char *)workspace + (((size_t)DEC_SLICES * L * Tn * d * 4 + 255) & ~(size_t)255));
+    sptr = (int32_t *)((char *)workspace + partial_bytes(Tn, d, L));
   }
   int64_t nblk = blocks_per_t * (t_end - t_begin);
   if (nblk <= 0) return CLT_OK;
@@ -1298,30 +1357,36 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
     else if (rem * 2 == chunk) CLT_DEC(NFN, 1, UN);        \
     else CLT_DEC(NFN, 2, UN);                              \
   } while (0)
+  // (source, target) pairs of a launch over all sources
+  int64_t n_pairs = 0;
+  for (int64_t s = 0; s < t_end; ++s)
+    if ((src_mask >> s) & 1ull) n_pairs += t_end - (s > t_begin ? s : t_begin);
   // quarter-row schedule: 2 feature slices x 4 column quarters (see k_decode_quarter)
   bool quartered = false; int quarter_ns = QUARTER_SLICES;
+  const bool quarter_pairs = one_launch(Tn, d, L, QUARTER_SLICES);
   if (route == CLT_ROUTE_LINE) {
     constexpr int ntok = 2;                               // tokens per wavefront
     const UnitPlan lp = make_unit_plan(line_slices(F), (int)(d * (int64_t)sizeof(T) / 128), Tn, nwv * ntok);
     // one 32-bit word per survivor and 32-bit row offsets: feature index below 2^16, matrix below 4 GiB
     const bool pack = sizeof(T) == 2 && F <= 65536 && F * pitch * (int64_t)sizeof(T) < (1ll << 32);
     k_slice_ptr<<<1024, 256, 0, stream>>>(row_ptr, col, L * Tn, F, lp.ns, sptr);
-    for (int src = 0; src < (int)t_end; ++src) {
-      if (!((src_mask >> src) & 1ull)) continue;
+    const bool pairs = one_launch(Tn, d, L, lp.ns);
+    for (int src = pairs ? -1 : 0; src < (pairs ? 0 : (int)t_end); ++src) {
+      if (!pairs && !((src_mask >> src) & 1ull)) continue;
       const int64_t tb = src > t_begin ? src : t_begin;
-      const int64_t lb = 8 * (int64_t)lp.bpx * (t_end - tb);
+      const int64_t lb = 8 * (int64_t)lp.bpx * (pairs ? n_pairs : t_end - tb);
       if (lb <= 0) continue;
       if (lb > 2147483647LL) return CLT_ERR_RANGE;
 #define CLT_DECL(AF, PK, NT)                                                                                          \
   k_decode_line<T, AF, PK, NT><<<(unsigned)lb, 256, 0, stream>>>(col, (const T *)val, (const T *)wp, (const T *)foff, \
-      (const T *)fscale, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, lp, pitch)
+      (const T *)fscale, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, lp, pitch, t_end)
 #define CLT_DECL2(AF, PK) CLT_DECL(AF, PK, ntok)
       if (affine) { if (pack) CLT_DECL2(true, true); else CLT_DECL2(true, false); }
       else { if (pack) CLT_DECL2(false, true); else CLT_DECL2(false, false); }
 #undef CLT_DECL2
 #undef CLT_DECL
     }
-    k_decode_reduce<T><<<2048, 256, 0, stream>>>(partial, bias_sum, skip_add, out, Tn, d, L, t_begin, t_end, lp.ns, out_f32, src_mask);
+    k_decode_reduce<T><<<2048, 256, 0, stream>>>(partial, bias_sum, skip_add, out, Tn, d, L, t_begin, t_end, lp.ns, out_f32, src_mask, pairs);
     return clt_check_launch();
   }
   if (route == CLT_ROUTE_QUARTER) {
@@ -1335,18 +1400,18 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
 #define CLT_DECQ(HQN, HTN, UN)                                                                                       \
   do {                                                                                                               \
     k_slice_ptr<<<1024, 256, 0, stream>>>(row_ptr, col, L * Tn, F, qs, sptr);                                        \
-    for (int src = 0; src < (int)t_end; ++src) {                                                                     \
-      if (!((src_mask >> src) & 1ull)) continue;                                                                     \
+    for (int src = quarter_pairs ? -1 : 0; src < (quarter_pairs ? 0 : (int)t_end); ++src) {                          \
+      if (!quarter_pairs && !((src_mask >> src) & 1ull)) continue;                                                   \
       const int64_t tb = src > t_begin ? src : t_begin;                                                              \
-      const int64_t qb = 8 * (int64_t)up.bpx * (t_end - tb);                                                         \
+      const int64_t qb = 8 * (int64_t)up.bpx * (quarter_pairs ? n_pairs : t_end - tb);                               \
       if (qb <= 0) continue;                                                                                         \
       if (qb > 2147483647LL) return CLT_ERR_RANGE;                                                                   \
       if (affine) k_decode_quarter<T, HQN, HTN, UN, true, false><<<(unsigned)qb, 256, 0, stream>>>(col, (const T *)val, (const T *)wp, \
-          (const T *)foff, (const T *)fscale, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up);      \
+          (const T *)foff, (const T *)fscale, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up, t_end);      \
       else if (qpack) k_decode_quarter<T, HQN, HTN, UN, false, sizeof(T) == 2><<<(unsigned)qb, 256, 0, stream>>>(col, (const T *)val, (const T *)wp, \
-          nullptr, nullptr, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up);                        \
+          nullptr, nullptr, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up, t_end);                        \
       else k_decode_quarter<T, HQN, HTN, UN, false, false><<<(unsigned)qb, 256, 0, stream>>>(col, (const T *)val, (const T *)wp, \
-          nullptr, nullptr, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up);                        \
+          nullptr, nullptr, Tn, d, F, L, tying, tb, src_mask, sptr, partial, src, pitch, up, t_end);                        \
     }                                                                                                                \
     quartered = true; quarter_ns = qs;                                                                               \
   } while (0)
@@ -1363,7 +1428,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
 #undef CLT_DECQ
   }
   if (quartered) {
-    k_decode_reduce<T><<<2048, 256, 0, stream>>>(partial, bias_sum, skip_add, out, Tn, d, L, t_begin, t_end, quarter_ns, out_f32, src_mask);
+    k_decode_reduce<T><<<2048, 256, 0, stream>>>(partial, bias_sum, skip_add, out, Tn, d, L, t_begin, t_end, quarter_ns, out_f32, src_mask, quarter_pairs);
     return clt_check_launch();
   }
   if (can_slice) k_slice_ptr<<<1024, 256, 0, stream>>>(row_ptr, col, L * Tn, F, ns, sptr);

@@ -396,7 +396,8 @@ int clt_pack_decoder(const void *w_ref, void *w_packed, int64_t d, int64_t F,
  * the decoders are not tied per target, 8 feature slices of whole rows otherwise - with one
  * launch per source layer, so that the eighth stays in one L2 while all tokens pass; partial
  * sums live as fp32 rows per (slice, target, token) in the workspace and are added in a fixed
- * order at the end.  All routes give the same result up to fp32 summation order.
+ * order at the end.  A short batch gets one launch for all sources, with partial rows per
+ * (slice, source, target, token) added in the same order.  All routes give the same result up to fp32 summation order.
  */
 size_t clt_decode_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L);
 int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, const void *val,
