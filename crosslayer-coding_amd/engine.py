@@ -114,8 +114,11 @@ SLICED_DECODE_MIN_ROWS = 8192
 SLICED_DECODE_MIN_SLAB_BYTES = 128 << 20
 
 
-def _wants_sliced_decode(rows: int, slab_bytes: int) -> bool:
-    return rows >= SLICED_DECODE_MIN_ROWS or slab_bytes >= SLICED_DECODE_MIN_SLAB_BYTES
+def _wants_sliced_decode(rows: int, slab_bytes: int, T: int, d: int, F: int, L: int, tying: str, dtype: torch.dtype) -> bool:
+    """... or rows too wide for a wavefront to hold (d > 1024 in fp32), which only the sliced schedules and the kernel for
+    any shape take: 1860 -> 23 us at L = 2, d = 2048, F = 4096, 77 tokens x 60."""
+    return (rows >= SLICED_DECODE_MIN_ROWS or slab_bytes >= SLICED_DECODE_MIN_SLAB_BYTES
+            or nat.load().clt_decode_route(T, d, F, L, nat.TYING[tying], nat.dtype_code(dtype), 0) == nat.ROUTE_GENERIC)
 
 
 # token rows of one tile of the matrix-core encoder: shorter batches are padded to it where the kernel for short ones
@@ -929,7 +932,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
                 nat.check(lib.clt_decode_sparse_if_over(*args, _stream(w_packed)), "clt_decode_sparse_if_over")
             return out
     wbuf, wbytes = None, 0
-    if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size()):
+    if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(), T, d, F, L, tying,
+                                               surv.dtype):
         wbytes = lib.clt_decode_workspace_bytes(T, d, F, L)
         wbuf = ws.get("decode", wbytes)
     code = lib.clt_decode_sparse(
@@ -948,7 +952,7 @@ def decode_route(T: int, d: int, F: int, L: int, tying: str, dtype: torch.dtype,
     rows = T * L if rows is None else rows
     n_dec = L * (L + 1) // 2 if tying == "none" else L
     slab_bytes = n_dec * F * decoder_pitch(d, dtype) * torch.empty((), dtype=dtype).element_size()
-    wbytes = lib.clt_decode_workspace_bytes(T, d, F, L) if _wants_sliced_decode(rows, slab_bytes) else 0
+    wbytes = lib.clt_decode_workspace_bytes(T, d, F, L) if _wants_sliced_decode(rows, slab_bytes, T, d, F, L, tying, dtype) else 0
     code = lib.clt_decode_route(T, d, F, L, nat.TYING[tying], nat.dtype_code(dtype), wbytes)
     if code < 0:
         nat.check(code, "clt_decode_route")
