@@ -1,0 +1,410 @@
+// Sparse cross-layer decode of float32 models (reference clt/models/decoder.py:176-340) from LDS tiles: the gather of
+// decode.hip is bound by the lines an L1 keeps outstanding, LDS hands rows out faster.
+//
+//   k_row_runs / k_row_streams / k_row_fill
+//                   survivor list (CSR by token) -> one stream of records per group of 16 tokens, in the order in which
+//                   k_decode_rows consumes them: by source, tile of SP_ROWS features, token
+//   k_decode_rows   one workgroup per (target, 32 columns, part of the tokens): every tile of every source's decoder passes
+//                   through LDS once, the sums stay in registers over all sources and features
+#include "spmm.h"
+
+namespace {
+
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+constexpr int DR_COLS = 32;                // columns of a tile: one 128-byte line
+constexpr int DR_TOK = SP_GROUP;           // tokens of a wavefront: four accumulators per lane each
+constexpr int DR_REC = 8;                  // entries of a record: a wavefront reads 8 rows x 16 bytes per lane
+constexpr int DR_WAVES = 16;
+constexpr int DR_RING = 8;                 // slots of four records that a wavefront keeps in LDS or on their way
+constexpr int DR_LDS = 2 * SP_TILE_BYTES + DR_WAVES * DR_RING * 256;
+constexpr int DR_THREADS = 256;
+constexpr int DR_MAX_TILES = 512;
+static_assert(DR_LDS <= 160 * 1024 && SP_ROWS / DR_REC <= 255, "record counts of a run are bytes");
+
+// An entry: where its tile row begins in LDS (tile buffer and row), and its value.  A run - one token's entries of one tile -
+// takes whole records; what is left of its last one repeats its last entry's place with value 0.
+struct RowPlan { int tiles, groups, parts, groups_per_part, stages; };
+
+struct RunArgs {
+  const int32_t *row_ptr, *col;
+  const float *val;
+  int64_t Tn, L;
+  uint64_t layer_mask;
+  RowPlan p;
+  int32_t *start;          // [L * groups][DR_TOK][tiles + 1] list position where a token's entries of a tile begin
+  uint4 *counts;           // [groups][stages] records per token, a byte each
+  uint32_t *offset;        // [groups][stages] records of the stage, then of the stream before it
+  uint32_t *total;         // [groups] records of the stream
+  uint2 *recs;
+};
+
+// One workgroup per (group of tokens, layer).  Rows are sorted by column, so a row's entries of one tile are a run, found by
+// binary search.  A layer outside layer_mask counts as empty.
+__global__ __launch_bounds__(DR_THREADS) void k_row_runs(RunArgs A) {
+  extern __shared__ int32_t run_lds[];
+  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles;
+  const int64_t tok0 = (int64_t)g * DR_TOK, r0 = (int64_t)s * A.Tn + tok0;
+  const bool on = (A.layer_mask >> s) & 1ull;
+  int32_t *out = A.start + ((int64_t)s * A.p.groups + g) * DR_TOK * (tiles + 1);
+  for (int i = tid; i < DR_TOK * (tiles + 1); i += DR_THREADS) {
+    const int tk = i / (tiles + 1), c = i - tk * (tiles + 1);
+    int32_t lo = 0;
+    if (on && tok0 + tk < A.Tn) {
+      int32_t hi = A.row_ptr[r0 + tk + 1];
+      lo = A.row_ptr[r0 + tk];
+      const int32_t bound = c * SP_ROWS;
+      if (c == tiles) lo = hi;
+      while (lo < hi) {
+        const int32_t mid = lo + ((hi - lo) >> 1);
+        if (A.col[mid] < bound) lo = mid + 1; else hi = mid;
+      }
+    }
+    run_lds[i] = lo;
+    out[i] = lo;
+  }
+  __syncthreads();
+  for (int c = tid; c < tiles; c += DR_THREADS) {
+    uint32_t w[4] = {0u, 0u, 0u, 0u}, sum = 0;
+#pragma unroll
+    for (int tk = 0; tk < DR_TOK; ++tk) {
+      const uint32_t n = (uint32_t)(run_lds[tk * (tiles + 1) + c + 1] - run_lds[tk * (tiles + 1) + c] + DR_REC - 1) / DR_REC;
+      w[tk >> 2] |= n << (8 * (tk & 3));
+      sum += n;
+    }
+    const int64_t at = (int64_t)g * A.p.stages + (int64_t)s * tiles + c;
+    A.counts[at] = make_uint4(w[0], w[1], w[2], w[3]);
+    A.offset[at] = sum;
+  }
+}
+
+// One wavefront per stream: where each of its stages begins.
+__global__ __launch_bounds__(64) void k_row_streams(RunArgs A) {
+  const int lane = threadIdx.x;
+  uint32_t *off = A.offset + (int64_t)blockIdx.x * A.p.stages;
+  uint32_t run = 0;
+  for (int st0 = 0; st0 < A.p.stages; st0 += 64) {
+    const int st = st0 + lane;
+    const uint32_t n = st < A.p.stages ? off[st] : 0u;
+    uint32_t incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(incl, o);
+      if (lane >= o) incl += up;
+    }
+    if (st < A.p.stages) off[st] = run + incl - n;
+    run += __shfl(incl, 63);
+  }
+  if (lane == 0) A.total[blockIdx.x] = run;
+}
+
+// One workgroup per (group, layer): every run into its records.
+__global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
+  extern __shared__ int32_t fill_lds[];
+  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
+  if (!((A.layer_mask >> s) & 1ull)) return;
+  int32_t *start = fill_lds;                               // [DR_TOK][tiles + 1]
+  uint32_t *dest = (uint32_t *)(start + DR_TOK * (tiles + 1));      // [DR_TOK][tiles] first record of the run
+  const int64_t tok0 = (int64_t)g * DR_TOK, r0 = (int64_t)s * A.Tn + tok0;
+  const int32_t *src = A.start + ((int64_t)s * A.p.groups + g) * DR_TOK * (tiles + 1);
+  for (int i = tid; i < DR_TOK * (tiles + 1); i += DR_THREADS) start[i] = src[i];
+  const uint32_t base = stream_first(A.total, g, lane);
+  const uint32_t stage0 = (uint32_t)(__popcll(A.layer_mask & ((1ull << s) - 1ull)) * tiles);
+  __syncthreads();
+  for (int c = tid; c < tiles; c += DR_THREADS) {
+    uint32_t d = base + A.offset[(int64_t)g * A.p.stages + (int64_t)s * tiles + c];
+    for (int tk = 0; tk < DR_TOK; ++tk) {
+      const int32_t b = start[tk * (tiles + 1) + c], n = start[tk * (tiles + 1) + c + 1] - b;
+      dest[tk * tiles + c] = d;
+      if (n % DR_REC != 0) {
+        const uint32_t row = (uint32_t)(A.col[b + n - 1] - c * SP_ROWS);
+        for (int i = n; i % DR_REC != 0; ++i) A.recs[(uint64_t)d * DR_REC + i] = make_uint2((((stage0 + c) & 1u) << 16) | (row << 7), 0u);
+      }
+      d += (uint32_t)(n + DR_REC - 1) / DR_REC;
+    }
+  }
+  __syncthreads();
+  for (int tk = tid >> 6; tk < DR_TOK; tk += DR_THREADS / 64) {
+    if (tok0 + tk >= A.Tn) break;
+    const int32_t e = A.row_ptr[r0 + tk + 1];
+    for (int32_t j = A.row_ptr[r0 + tk] + lane; j < e; j += 64) {
+      const int32_t f = A.col[j], c = f / SP_ROWS;
+      A.recs[(uint64_t)dest[tk * tiles + c] * DR_REC + (j - start[tk * (tiles + 1) + c])] =
+          make_uint2((((stage0 + c) & 1u) << 16) | ((uint32_t)(f - c * SP_ROWS) << 7), __float_as_uint(A.val[j]));
+    }
+  }
+}
+
+struct RowArgs {
+  RowPlan p;
+  const uint4 *counts;
+  const uint32_t *total;
+  const uint2 *recs;
+  const float *wp, *bias_sum, *skip_add;
+  float *out;
+  int64_t Tn, d, F, L, pitch;
+  uint64_t src_mask;
+  int tying, t_begin, t_end, col_parts;
+};
+
+// Two tiles of 512 features x 32 columns in LDS, one being read while the other comes in.  A wavefront owns 16 tokens; a
+// record is one 16-byte read per lane (8 lanes a row, 8 rows) and four multiply-adds, its eight partial sums per column meet
+// at the end.  The records come through a ring as in k_decode_tiles.  Workgroups that share a tile follow each other on one XCD.
+//
+// L = 12, d = 768, F = 6144, 1024 tokens, 200 survivors per token, untied: 1.80 ms (49 GB of gathered rows, 27 TB/s) against
+// 2.33 ms of the gather from the L2s; 2.05 against 2.67 ms where tokens differ in their survivors (a stage waits for its
+// fullest wavefront).  Bound by what LDS returns: 5.7 ns per record and CU for 1 KB of rows and half as much of record.
+// Measured and dropped: the rows of the next record asked for ahead of the barrier (6.8 ns: register moves); four records in
+// one word per lane, handed out by DPP operands (7.6 ns: bound by instruction issue).
+__global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
+  extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int pair = (seq / A.p.parts) * 8 + xcd, part = seq % A.p.parts;
+  if (pair >= (A.t_end - A.t_begin) * A.col_parts) return;
+  const int t = A.t_end - 1 - pair / A.col_parts, cp = pair % A.col_parts;      // longest first
+  const uint64_t mask = A.src_mask & ((2ull << t) - 1ull);
+  const int n_stages = __popcll(mask) * A.p.tiles;
+  const int g = part * A.p.groups_per_part + wave;
+  const bool mine = wave < A.p.groups_per_part && g < A.p.groups;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)tile_lds;
+
+  // this wavefront's share of a tile: 32 rows, eight at a time, 16 bytes per lane
+  const uint32_t pitch_b = (uint32_t)(A.pitch * 4);
+  const int row_a = wave * 32 + (lane >> 3);
+  const uint32_t col_b = (uint32_t)(lane & 7) * 16;
+  auto fill = [&](const char *src, int rows, uint32_t lds_at) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = row_a + 8 * i;                         // past the matrix: nobody refers to these rows
+      sp_fill16(src, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b, lds_at + (uint32_t)i * 1024);
+    }
+  };
+  auto tile_at = [&](int s) { return (const char *)A.wp + sp_slot(A.tying, s, t, A.L) * A.F * (int64_t)pitch_b + (int64_t)cp * 128; };
+
+  f32x4v_t acc[DR_TOK];
+#pragma unroll
+  for (int i = 0; i < DR_TOK; ++i) acc[i] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
+
+  if (n_stages > 0) {
+    const uint32_t ring = lds0 + 2 * SP_TILE_BYTES + (uint32_t)wave * (DR_RING * 256);
+    const uint32_t *recs = (const uint32_t *)(A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(stream_first(A.total, mine ? g : 0, lane)) * DR_REC);
+    uint32_t rec_off = (uint32_t)lane * 4;                 // of the next slot to ask for, this lane's word
+    auto ask = [&](uint32_t at) {
+      sp_fill4(recs, rec_off, ring + at);
+      rec_off += 256;
+    };
+    uint64_t m = mask;
+    int s = __ffsll((unsigned long long)m) - 1, c = 0, rows = (int)A.F;
+    const char *tile = tile_at(s);
+    const uint32_t lds_share = lds0 + (uint32_t)wave * 4096;
+    fill(tile, rows, lds_share);
+#pragma unroll
+    for (int i = 0; i < DR_RING; ++i) ask((uint32_t)i * 256);
+    const auto counts = (const __attribute__((address_space(4))) uint4 *)(uintptr_t)A.counts + (int64_t)(mine ? g : 0) * A.p.stages;
+    auto count_at = [&](int at) {
+      return mine ? make_uint4(counts[at].x, counts[at].y, counts[at].z, counts[at].w) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    uint4 cnt = count_at(s * A.p.tiles);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    uint32_t at = 0;                                       // of the next record to read, within the ring
+    int since = DR_RING;                                   // slots asked for since the last tile's lines
+    const uint32_t ring_lane = ring + (uint32_t)(lane >> 3) * 8, col_lane = lds0 + col_b;
+    auto next = [&](u32x2_t &r) {
+      r = *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)(ring_lane + at);
+      at = (at + 64) & (DR_RING * 256 - 1);
+      if ((at & 255) == 0) {
+        asm volatile("" ::"v"(r.x), "v"(r.y));             // the slot has been read
+        ask((at - 256) & (DR_RING * 256 - 1));
+        ++since;
+        // the slot after it: seven were asked for since, and perhaps the four loads of a tile
+        if (since < DR_RING) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
+      }
+    };
+    // (what lies behind the stream's end may hold anything: the place is kept inside the tiles)
+    auto read = [&](const u32x2_t &r) {
+      return *(__attribute__((address_space(3))) f32x4v_t *)(uintptr_t)((r.x & 0x1FF80u) + col_lane);
+    };
+    u32x2_t r0, r1;                                        // the next two records
+    next(r0);
+    next(r1);
+    for (int st = 0; st < n_stages; ++st) {
+      const bool more = st + 1 < n_stages;
+      if (more) {
+        tile += SP_ROWS * pitch_b;
+        rows -= SP_ROWS;
+        if (++c == A.p.tiles) {
+          c = 0;
+          m &= m - 1;
+          s = __ffsll((unsigned long long)m) - 1;
+          tile = tile_at(s);
+          rows = (int)A.F;
+        }
+      }
+      const uint4 cnt_next = count_at(s * A.p.tiles + c);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();                        // tile st is complete, and nobody reads the other one any more
+      asm volatile("" ::: "memory");
+      if (more) {
+        fill(tile, rows, lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES);
+        since = 0;
+      } else since = DR_RING;
+      const uint32_t words[4] = {cnt.x, cnt.y, cnt.z, cnt.w};
+#pragma unroll
+      for (int tk = 0; tk < DR_TOK; ++tk) {
+        int n = (int)(words[tk >> 2] >> (8 * (tk & 3))) & 0xFF;
+        for (; n >= 2; n -= 2) {
+          const f32x4v_t w0 = read(r0), w1 = read(r1);
+          const float v0 = __uint_as_float(r0.y), v1 = __uint_as_float(r1.y);
+          next(r0);
+          next(r1);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[tk][q] = fmaf(v1, w1[q], fmaf(v0, w0[q], acc[tk][q]));
+        }
+        if (n > 0) {
+          const f32x4v_t w0 = read(r0);
+          const float v0 = __uint_as_float(r0.y);
+          r0 = r1;
+          next(r1);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[tk][q] = fmaf(v0, w0[q], acc[tk][q]);
+        }
+      }
+      cnt = cnt_next;
+      // the tile's lines are waited for, not the slots asked for behind them; this wavefront's reads of the tile are over
+      if (since >= DR_RING) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+      else if (since >= DR_RING / 2) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may be on its way into LDS when the workgroup ends
+  }
+
+  // lane 8 j + i holds entries j of every record, columns 4 i .. 4 i + 3: the eight sums meet in every lane, row tk is written
+  // by lanes 8 (tk % 8) .. + 7
+#pragma unroll
+  for (int tk = 0; tk < DR_TOK; ++tk) {
+    f32x4v_t a = acc[tk];
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[q] += __shfl_xor(a[q], o);
+    const int64_t tok = (int64_t)g * DR_TOK + tk;
+    if (!mine || tok >= A.Tn || (lane >> 3) != (tk & 7)) continue;
+    const int64_t o = (int64_t)cp * DR_COLS + (lane & 7) * 4, at = ((int64_t)t * A.Tn + tok) * A.d + o;
+    if (A.bias_sum) a += *reinterpret_cast<const f32x4v_t *>(A.bias_sum + (int64_t)t * A.d + o);
+    if (A.skip_add) a += *reinterpret_cast<const f32x4v_t *>(A.skip_add + at);
+    *reinterpret_cast<f32x4v_t *>(A.out + at) = a;
+  }
+}
+
+static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+struct RowLayout {
+  RowPlan p;
+  int col_parts;
+  int64_t n_recs;
+  size_t start, counts, offset, total, recs, bytes;
+};
+
+static RowLayout row_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  RowLayout l;
+  RowPlan &p = l.p;
+  p.tiles = (int)clt_ceil_div(F, SP_ROWS);
+  p.groups = (int)clt_ceil_div(Tn, DR_TOK);
+  p.stages = (int)(L * p.tiles);
+  p.parts = (int)clt_ceil_div(p.groups, DR_WAVES);
+  p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
+  l.col_parts = (int)(d / DR_COLS);
+  // every run may leave its last record part empty, but no more runs than entries; a stream reads a ring past its end
+  const int64_t runs = (int64_t)p.stages * p.groups * DR_TOK;
+  l.n_recs = entries / DR_REC + (runs < entries ? runs : entries) + (DR_RING + 2) * 4;
+  size_t at = 0;
+  auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
+  l.start = take(sizeof(int32_t) * (size_t)L * p.groups * DR_TOK * (p.tiles + 1));
+  l.counts = take(sizeof(uint4) * (size_t)p.groups * p.stages);
+  l.offset = take(sizeof(uint32_t) * (size_t)p.groups * p.stages);
+  l.total = take(sizeof(uint32_t) * (size_t)p.groups);
+  l.recs = take((size_t)l.n_recs * DR_REC * sizeof(uint2));
+  l.bytes = at;
+  return l;
+}
+
+// LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile
+static bool row_shape_ok(const RowLayout &l, int64_t row_bytes) {
+  return l.p.tiles <= DR_MAX_TILES && l.n_recs <= 0x03FFFFFFll && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
+         (int64_t)l.p.stages * l.p.groups <= 0x07FFFFFFll;
+}
+
+}  // namespace
+
+// Both routes priced from what they measured (L 4 - 16, d 256 - 2048, F 2048 - 16384, T 64 - 3000, 20 - 200 survivors per token):
+// the gather moves its rows at 23 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage of the tiles takes
+// 1.4 us plus 5.7 ns per record, but no less than the 2.4 us in which 64 KB come into LDS, and the longest workgroup bounds a
+// launch of few.  us, gather / tiles: L = 12, d = 768, F = 6144, 1024 tokens: 667 / 941 with 20 per token, 1052 / 1045 with
+// 60, 2328 / 1798 with 200; L = 6, d = 1024, F = 16384, 3000 tokens x 200: 2599 / 2909; L = 16, d = 256, F = 2048, 1024 x 60:
+// 659 / 354.
+extern "C" int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
+                                      int dtype) {
+  if (dtype != CLT_F32 || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return 0;
+  if (T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return 0;
+  const RowLayout l = row_layout(T, d, F, L, entries);
+  if (!row_shape_ok(l, clt_pitch(d, 4) * 4)) return 0;
+  const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
+  const double sparse_us = rows * d * 4 / 23e6 + pairs * T * d * 16 / 3.6e6;
+  const double run = (double)entries / ((double)l.p.stages * T);
+  const double recs = l.p.groups_per_part * DR_TOK * (run < run / DR_REC + 0.5 ? run : run / DR_REC + 0.5);
+  const double stage_us = 1.4 + recs * 0.0057;
+  const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
+  const double rows_us = (stages > longest ? stages : longest) * (stage_us > 2.4 ? stage_us : 2.4) + 20 + entries * 2e-5;
+  return rows_us < 0.95 * sparse_us;
+}
+
+extern "C" size_t clt_decode_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  if (T <= 0 || d < DR_COLS || F <= 0 || L <= 0 || entries < 0) return 0;
+  return row_layout(T, d, F, L, entries).bytes;
+}
+
+extern "C" int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const float *val, const float *w_packed,
+                               const float *bias_sum, const float *skip_add, float *out, int64_t T, int64_t d, int64_t F, int64_t L,
+                               int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int64_t entries, void *workspace,
+                               size_t workspace_bytes, void *stream) {
+  if (T < 0 || d <= 0 || F <= 0 || L <= 0 || L > 64 || d % DR_COLS != 0 || entries < 0) return CLT_ERR_ARG;
+  if (t_begin < 0 || t_end > L || t_begin > t_end) return CLT_ERR_ARG;
+  if (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE) return CLT_ERR_ARG;
+  if (T == 0 || t_begin == t_end) return CLT_OK;
+  if (!row_ptr || !col || !val || !w_packed || !out || !workspace) return CLT_ERR_ARG;
+  if (!clt_aligned16(w_packed) || !clt_aligned16(out) || !clt_aligned16(workspace) || (bias_sum && !clt_aligned16(bias_sum)) ||
+      (skip_add && !clt_aligned16(skip_add)))
+    return CLT_ERR_ALIGN;
+  const int64_t pitch = clt_pitch(d, 4);
+  const RowLayout l = row_layout(T, d, F, L, entries);
+  if (!row_shape_ok(l, pitch * 4)) return CLT_ERR_RANGE;
+  if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  char *ws = (char *)workspace;
+  RunArgs ra;
+  ra.row_ptr = row_ptr; ra.col = col; ra.val = val; ra.Tn = T; ra.L = L; ra.layer_mask = src_mask; ra.p = l.p;
+  ra.start = (int32_t *)(ws + l.start); ra.counts = (uint4 *)(ws + l.counts); ra.offset = (uint32_t *)(ws + l.offset);
+  ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint2 *)(ws + l.recs);
+  RowArgs a;
+  a.p = l.p; a.counts = ra.counts; a.total = ra.total; a.recs = ra.recs;
+  a.wp = w_packed; a.bias_sum = bias_sum; a.skip_add = skip_add; a.out = out;
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = pitch; a.src_mask = src_mask;
+  a.tying = tying; a.t_begin = (int)t_begin; a.t_end = (int)t_end; a.col_parts = l.col_parts;
+  const int64_t pairs = clt_ceil_div((t_end - t_begin) * l.col_parts, 8) * 8;
+  if (pairs * l.p.parts > 0x7FFFFFFFll) return CLT_ERR_RANGE;
+  if (hipFuncSetAttribute((const void *)k_decode_rows, hipFuncAttributeMaxDynamicSharedMemorySize, DR_LDS) != hipSuccess)
+    return CLT_ERR_LAUNCH;
+  const size_t run_lds = sizeof(int32_t) * (size_t)DR_TOK * (l.p.tiles + 1);
+  const dim3 grid((unsigned)l.p.groups, (unsigned)L);
+  const size_t fill_bytes = run_lds + sizeof(uint32_t) * (size_t)DR_TOK * l.p.tiles;
+  if (hipFuncSetAttribute((const void *)k_row_fill, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_bytes) != hipSuccess)
+    return CLT_ERR_LAUNCH;
+  k_row_runs<<<grid, DR_THREADS, run_lds, s>>>(ra);
+  k_row_streams<<<(unsigned)l.p.groups, 64, 0, s>>>(ra);
+  k_row_fill<<<grid, DR_THREADS, fill_bytes, s>>>(ra);
+  k_decode_rows<<<(unsigned)(pairs * l.p.parts), DR_WAVES * 64, DR_LDS, s>>>(a);
+  return clt_check_launch();
+}

@@ -41,6 +41,29 @@ constexpr int SP_HALF_BYTES = SP_TILE_BYTES / 2;
 __host__ __device__ __forceinline__ uint32_t sp_swap(uint32_t r) { return (r >> 2) & 1u; }
 __device__ __forceinline__ uint32_t sp_half_place(uint32_t r, uint32_t buffer) { return (buffer << 15) | (r << 5) | (sp_swap(r) << 4); }
 
+// what the kernels over tiles share: a decoder's place in the slab, a stream's first record, loads into LDS
+__device__ __forceinline__ int64_t sp_slot(int tying, int64_t s, int64_t t, int64_t L) {
+  return tying == CLT_TYING_PER_SOURCE ? s : s * L - (s * (s - 1)) / 2 + (t - s);
+}
+
+// first batch (record) of a stream: those of the streams before it (all lanes of a wavefront take part)
+__device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stream, int lane) {
+  uint32_t n = 0;
+  for (int i = lane; i < stream; i += 64) n += total[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  return n;
+}
+
+// Direct-to-LDS loads, 16 or 4 bytes per lane (lane i lands at lds_at + 16 i / 4 i).  As asm statements, so that the
+// compiler does not wait for them in front of every LDS read; whoever reads the data waits by hand.
+__device__ __forceinline__ void sp_fill16(const char *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+__device__ __forceinline__ void sp_fill4(const uint32_t *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+}
+
 template <typename T> struct SpMma;
 template <> struct SpMma<bf16_t> {
   typedef __attribute__((ext_vector_type(8))) __bf16 frag_t;

@@ -13,10 +13,6 @@
 
 namespace {
 
-__device__ __forceinline__ int64_t sp_slot(int tying, int64_t s, int64_t t, int64_t L) {
-  return tying == CLT_TYING_PER_SOURCE ? s : s * L - (s * (s - 1)) / 2 + (t - s);
-}
-
 constexpr int DT_WAVES = 16;
 constexpr int DT_GPW = 4;                  // groups of 16 output rows per wavefront: 64 accumulators per lane
 
@@ -115,15 +111,6 @@ __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
     run += __shfl(incl, 63);
   }
   if (lane == 0) A.total[stream] = run;
-}
-
-// first batch of a stream: those of the streams before it (all lanes of a wavefront take part)
-__device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stream, int lane) {
-  uint32_t n = 0;
-  for (int i = lane; i < stream; i += 64) n += total[i];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-  return n;
 }
 
 // One workgroup per (group, layer) again: the runs of a tile laid end to end in row order - a fixed order of every sum -
@@ -230,15 +217,6 @@ constexpr int DT_RING = 8;                                 // records a wavefron
 constexpr int DT_LDS = 2 * SP_TILE_BYTES + DT_WAVES * DT_RING * 256;
 static_assert(DT_FILLS == 4 && DT_RING == 8, "the wait counts below are written out");
 
-// Direct-to-LDS loads, 16 or 4 bytes per lane (lane i lands at lds_at + 16 i / 4 i).  As asm statements, so that the
-// compiler does not wait for them in front of every LDS read; whoever reads the data waits by hand.
-__device__ __forceinline__ void fill16(const char *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
-}
-__device__ __forceinline__ void fill4(const uint32_t *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
-}
-
 // Two tiles of 512 features x 64 columns in LDS, one being multiplied while the other comes in.  Each wavefront owns four
 // groups of 16 tokens and consumes its stream of batches through a ring of eight records in LDS: the vector memory path
 // returns in order, so a record waits behind whatever tile lines were asked for before it, and eight batches (~2 us)
@@ -277,12 +255,12 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
     if (rows >= SP_ROWS) {
 #pragma unroll
       for (int i = 0; i < DT_FILLS; ++i)
-        fill16(src + (i & 1) * 64, off_a + (uint32_t)(i >> 1) * 16 * pitch_b, lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+        sp_fill16(src + (i & 1) * 64, off_a + (uint32_t)(i >> 1) * 16 * pitch_b, lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
     } else {                                               // past the matrix: nobody refers to these rows
 #pragma unroll
       for (int i = 0; i < DT_FILLS; ++i) {
         const int r = row_a + (i >> 1) * 16;
-        fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
+        sp_fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
                lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
       }
     }
@@ -305,7 +283,7 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
     uint32_t rec_off = (uint32_t)lane * 4;                 // of the next record to ask for, this lane's word
     uint32_t slot = 0;                                     // of the batch that is consumed next, in bytes
     auto ask = [&](uint32_t at) {                          // the next record of the stream into the ring
-      fill4(recs, rec_off, ring + at);
+      sp_fill4(recs, rec_off, ring + at);
       rec_off += SP_REC_WORDS * 4;
     };
     uint32_t word;                                         // of the record after the batch at hand
@@ -447,7 +425,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
 #pragma unroll
     for (int i = 0; i < GT_FILLS; ++i) {
       const int r = row_a + (i >> 1) * 16;
-      fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
+      sp_fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
              lds0 + (uint32_t)(wave * 4096 + (i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
     }
   };
@@ -469,7 +447,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
     const char *tile = (const char *)A.g + (int64_t)t * A.Tn * (int64_t)pitch_b + (int64_t)cp * 128;
     fill(tile, (int)A.Tn);
 #pragma unroll
-    for (int i = 0; i < DT_RING; ++i) { fill4(recs, rec_off, ring + (uint32_t)i * 256); rec_off += SP_REC_WORDS * 4; }
+    for (int i = 0; i < DT_RING; ++i) { sp_fill4(recs, rec_off, ring + (uint32_t)i * 256); rec_off += SP_REC_WORDS * 4; }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     auto look = [&]() { word = *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)(ring_lane + at); };
     look();
@@ -479,7 +457,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
       bt.read();
       bt.pick(word, row_bit);
       asm volatile("" ::"v"(bt.picked), "v"(bt.a0), "v"(bt.a1));
-      fill4(recs, rec_off, ring + at);
+      sp_fill4(recs, rec_off, ring + at);
       rec_off += SP_REC_WORDS * 4;
       at = (at + 256) & (DT_RING * 256 - 1);
       asm volatile("s_waitcnt vmcnt(7)" ::: "memory");

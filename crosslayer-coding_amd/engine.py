@@ -889,8 +889,9 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
                   ws: Optional[Workspace] = None) -> torch.Tensor:
     """Reconstructions [L, T, d] for targets [t_begin, t_end) (decoder.py:176-340).
 
-    With a workspace and a batch large enough to fill the GPU the matrix-core kernel (``clt_decode_tiles``) or one of the
-    XCD-sliced gathers is used, whichever ``clt_decode_tiles_wanted`` prices lower."""
+    With a workspace and a batch large enough to fill the GPU a gather from LDS tiles (16 bits: ``clt_decode_tiles`` on the
+    matrix cores; fp32: ``clt_decode_rows``) or one of the XCD-sliced gathers from the L2s is used, whichever
+    ``clt_decode_tiles_wanted`` / ``clt_decode_rows_wanted`` prices lower."""
     nat.require_device(w_packed, "decode_sparse")
     L, T, F = surv.L, surv.T, surv.F
     t_end = L if t_end is None else t_end
@@ -930,6 +931,13 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
             nat.check(lib.clt_decode_tiles(*args, nat.ptr(wbuf), wbuf.numel(), _stream(w_packed)), "clt_decode_tiles")
             if not exact:      # a batch that outgrew the estimate is decoded by the gather, decided on the device
                 nat.check(lib.clt_decode_sparse_if_over(*args, _stream(w_packed)), "clt_decode_sparse_if_over")
+            return out
+        if total and exact and lib.clt_decode_rows_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
+            wbuf = ws.get("decode_rows", lib.clt_decode_rows_workspace_bytes(T, d, F, L, total))
+            code = lib.clt_decode_rows(nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed),
+                                       nat.ptr(bias_sum), nat.ptr(skip_add), nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin,
+                                       t_end, src_mask & ((1 << 64) - 1), total, nat.ptr(wbuf), wbuf.numel(), _stream(w_packed))
+            nat.check(code, "clt_decode_rows")
             return out
     wbuf, wbytes = None, 0
     if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(), T, d, F, L, tying,

@@ -410,6 +410,21 @@ int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, const void *va
                       void *stream);
 
 /*
+ * The same sums (untied and per-source decoders, no feature offset / scale, fp32, d a multiple of 32) with the decoder rows
+ * gathered from LDS: the survivors of 16 tokens at a time are regrouped into records of eight by tiles of 512 features.
+ * Deterministic, equal to clt_decode_sparse up to fp32 summation order.
+ *   clt_decode_rows_wanted: whether it is the faster of the two for `entries` survivors over L layers and `targets` target
+ *   layers (0 also for what it does not take).
+ *   `entries` must be no less than the list's length: the workspace is sized for it.
+ */
+int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
+size_t clt_decode_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries);
+int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const float *val, const float *w_packed,
+                    const float *bias_sum, const float *skip_add, float *out, int64_t T, int64_t d, int64_t F, int64_t L,
+                    int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int64_t entries, void *workspace,
+                    size_t workspace_bytes, void *stream);
+
+/*
  * The same sums (untied and per-source decoders, no feature offset / scale, bf16 and fp16, d a multiple of 64) on the
  * matrix cores: the survivors are regrouped into batches by tiles of 512 features x 16 tokens and the decoder rows are
  * gathered from LDS.  Deterministic, equal to clt_decode_sparse up to fp32 summation order.
