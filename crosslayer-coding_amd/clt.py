@@ -83,7 +83,7 @@ class _ReconstructionsWithGraph(torch.autograd.Function):
         grads = []
         for name, p in zip(ctx.names, ctx.params):
             gp = named.get(name)
-            grads.append(None if gp is None or not p.requires_grad else gp.to(p.dtype).reshape(p.shape))
+            grads.append(None if gp is None or not p.requires_grad else engine.parameter_gradient(gp, p.dtype).reshape(p.shape))
         return (None, None, None, *grads)
 
 

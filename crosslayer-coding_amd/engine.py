@@ -833,6 +833,21 @@ def encoder_weight_grad(lists, dval: torch.Tensor, x: torch.Tensor, F: int):
     return dw, db
 
 
+def parameter_gradient(g: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """A raw fp32 gradient in the parameter's dtype and layout.  A transposed view (a decoder's [F, d] rows seen as [d, F]) is
+    written out in one pass: autograd would otherwise keep its strides in the cast and copy it once more, element by element."""
+    rows = g.t() if g.dim() == 2 else None
+    if (rows is not None and rows.is_cuda and rows.is_contiguous() and not g.is_contiguous() and rows.dtype == torch.float32
+            and dtype in (torch.float32, torch.bfloat16) and rows.shape[0] % 8 == 0 and rows.shape[1] % 4 == 0
+            and rows.data_ptr() % 16 == 0 and rows.numel() > 0):
+        F, d = rows.shape
+        out = torch.empty((d, F), dtype=dtype, device=g.device)
+        code = nat.load().clt_transpose_grad(nat.ptr(rows), nat.ptr(out), F, d, nat.dtype_code(dtype), _stream(rows))
+        nat.check(code, "clt_transpose_grad")
+        return out
+    return g.to(dtype)
+
+
 def scatter_survivor_values(surv: SurvivorList, src: torch.Tensor, layer: int, dense: torch.Tensor) -> None:
     """dense[tok, col] = src[j] for the survivors j of ``layer`` (decoder.py:228-285 with activations.py:183-220: the
     kept activations' share of d loss / d activation behind a per-target feature scale)."""

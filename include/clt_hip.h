@@ -288,6 +288,12 @@ int clt_survivors_fit(int32_t *row_ptr, int64_t R, int64_t capacity, int32_t *st
 int clt_poison_if(void *buf, int64_t bytes, const int32_t *flag, void *stream);
 
 /*
+ * out [d][F] (model dtype: fp32 or bf16, rounded once) = the transpose of g [F][d] fp32: a decoder's gradient in the layout of
+ * its parameter.  F % 8 == 0, d % 4 == 0, both 16-byte aligned.
+ */
+int clt_transpose_grad(const float *g, void *out, int64_t F, int64_t d, int dtype, void *stream);
+
+/*
  * clt_threshold_count for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * Same arguments and result as clt_threshold_count without the workspace: the per-row counters live
