@@ -4,6 +4,9 @@
 //   k_rec_count / k_rec_streams / k_rec_fill
 //                   survivor list (CSR by token) -> one stream of batches per wavefront of k_decode_tiles, in the order
 //                   in which it consumes them: by source, tile of SP_ROWS features, group of 16 tokens
+//   k_decode_repair / k_grad_repair
+//                   sums that are not finite once more, entry by entry: in the one-hot products an infinity or a NaN in a
+//                   tile row reaches all 16 output rows of a batch (0 * inf), here only the rows that refer to it
 //   k_decode_tiles  one workgroup per (target, 64 columns, part of the tokens): every tile of every source's decoder
 //                   passes through LDS once, the sums stay in registers over all sources and features
 //   k_grad_tiles    the transposed product of the backward pass: decoder weight gradients from the same lists by feature,
@@ -47,6 +50,7 @@ struct RecArgs {
   uint32_t *offset;        // [streams][stages] batches of the stream before the stage
   uint32_t *total;         // [streams] batches of the stream
   uint32_t *recs;
+  uint32_t *bad;           // number of groups whose sums are not finite, and which
 };
 
 // One workgroup per (group of 16 rows, layer).  Rows are sorted by column, so a row's entries of one tile are a run, found
@@ -111,6 +115,7 @@ __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
     run += __shfl(incl, 63);
   }
   if (lane == 0) A.total[stream] = run;
+  if (stream == 0 && lane == 0) *A.bad = 0u;
 }
 
 // One workgroup per (group, layer) again: the runs of a tile laid end to end in row order - a fixed order of every sum -
@@ -207,6 +212,9 @@ struct TileArgs {
   const float *bias_sum, *skip_add;
   void *out;
   const int32_t *list_total;               // survivors of the batch
+  const int32_t *row_ptr, *col;
+  const void *val;
+  uint32_t *bad;
   int64_t max_entries, Tn, d, F, L, pitch;
   uint64_t src_mask;
   int tying, t_begin, t_end, out_f32, col_parts;
@@ -216,6 +224,18 @@ constexpr int DT_FILLS = SP_ROWS / 8 / DT_WAVES;           // direct-to-LDS load
 constexpr int DT_RING = 8;                                 // records a wavefront keeps in LDS or on their way
 constexpr int DT_LDS = 2 * SP_TILE_BYTES + DT_WAVES * DT_RING * 256;
 static_assert(DT_FILLS == 4 && DT_RING == 8, "the wait counts below are written out");
+
+// Whether a wavefront's sums of a group (16 rows from row0 on, of n rows) are all finite; if not, the group goes on the list.
+__device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_on, uint32_t *bad, uint32_t item) {
+  float z = 0.0f;
+#pragma unroll
+  for (int n = 0; n < 4; ++n)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) z = fmaf(acc[n][q], 0.0f, z);
+  if (ballot64(row_on && z != z) == 0) return true;
+  if (lane_id() == 0) bad[1 + atomicAdd(bad, 1u)] = item;
+  return false;
+}
 
 // Two tiles of 512 features x 64 columns in LDS, one being multiplied while the other comes in.  Each wavefront owns four
 // groups of 16 tokens and consumes its stream of batches through a ring of eight records in LDS: the vector memory path
@@ -360,7 +380,8 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
   for (int gi = 0; gi < DT_GPW; ++gi) {
     const int g = A.p.group(stream, gi);
     const int64_t tok = (int64_t)g * SP_GROUP + (lane & 15);
-    if (g < 0 || tok >= A.Tn) continue;
+    if (g < 0) continue;
+    if (!sums_finite(acc[gi], tok < A.Tn, A.bad, (uint32_t)(((t - A.t_begin) * A.p.groups + g) * A.col_parts + cp)) || tok >= A.Tn) continue;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       const int64_t o = (int64_t)cp * SP_COLS + n * 16 + (lane >> 4) * 4;
@@ -371,6 +392,36 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
       if (A.out_f32) *reinterpret_cast<f32x4v_t *>((float *)A.out + at) = a;
       else *reinterpret_cast<uint2 *>((uint16_t *)A.out + at) = make_uint2(pack_pair<T>(a[0], a[1]), pack_pair<T>(a[2], a[3]));
     }
+  }
+}
+
+// The listed groups (16 tokens x 64 columns of a target): a thread sums 4 columns of a token over its survivors.
+template <typename T> __global__ __launch_bounds__(256) void k_decode_repair(TileArgs A) {
+  if (*A.list_total > A.max_entries) return;
+  const uint32_t n = *A.bad;
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const uint32_t item = A.bad[1 + i], cp = item % A.col_parts, g = item / A.col_parts % A.p.groups;
+    const int64_t t = A.t_begin + item / A.col_parts / A.p.groups, tok = (int64_t)g * SP_GROUP + (threadIdx.x >> 4);
+    if (tok >= A.Tn) continue;
+    const int64_t o = (int64_t)cp * SP_COLS + (threadIdx.x & 15) * 4, at = (t * A.Tn + tok) * A.d + o;
+    f32x4v_t a{0.f, 0.f, 0.f, 0.f};
+    for (int64_t s = 0; s <= t; ++s) {
+      if (!((A.src_mask >> s) & 1ull)) continue;
+      const T *w = (const T *)A.wp + sp_slot(A.tying, s, t, A.L) * A.F * A.pitch + o;
+      for (int32_t j = A.row_ptr[s * A.Tn + tok]; j < A.row_ptr[s * A.Tn + tok + 1]; ++j) {
+        const uint2 raw = *reinterpret_cast<const uint2 *>(w + (int64_t)A.col[j] * A.pitch);
+        const float v = Elem<T>::to_f32(((const T *)A.val)[j]);
+        float x[4];
+        unpack_pair<T>(raw.x, x[0], x[1]);
+        unpack_pair<T>(raw.y, x[2], x[3]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = fmaf(v, x[q], a[q]);
+      }
+    }
+    if (A.bias_sum) a += *reinterpret_cast<const f32x4v_t *>(A.bias_sum + t * A.d + o);
+    if (A.skip_add) a += *reinterpret_cast<const f32x4v_t *>(A.skip_add + at);
+    if (A.out_f32) *reinterpret_cast<f32x4v_t *>((float *)A.out + at) = a;
+    else *reinterpret_cast<uint2 *>((uint16_t *)A.out + at) = make_uint2(pack_pair<T>(a[0], a[1]), pack_pair<T>(a[2], a[3]));
   }
 }
 
@@ -392,7 +443,9 @@ struct GradArgs {
   float *m, *v, *out;        // moments; [n_dec][F][d]
   int64_t Tn, d, F, L, pitch, max_entries;
   int64_t m_row, m_cols, m_dec;   // moments: elements between rows, between column parts of 64 and between decoders
-  const int32_t *list_total;
+  const int32_t *list_total, *list_ptr, *list_tok, *list_src;
+  const void *val;
+  uint32_t *bad;
   int col_parts, items;      // items of one (source, target) pair per XCD
   AdamCoef adam;
 };
@@ -496,6 +549,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
   for (int gi = 0; gi < DT_GPW; ++gi) {
     const int g = A.p.group(stream, gi);
     if (g < 0) break;
+    if (!sums_finite(acc[gi], (int64_t)g * SP_GROUP + (lane & 15) < A.F, A.bad, (uint32_t)((slot * A.p.groups + g) * A.col_parts + cp))) continue;
     // rows of 64 columns: lane 16 r + c takes columns 4 c .. 4 c + 3 of rows r, r + 4, r + 8, r + 12
     const int c4 = (lane & 15) * 4;
     const int64_t f0 = (int64_t)g * SP_GROUP + (lane >> 4);
@@ -543,17 +597,54 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
   }
 }
 
+// The listed groups (16 features x 64 columns of a decoder): a thread sums 4 columns of a feature over its list and steps.
+template <typename T, bool ADAM> __global__ __launch_bounds__(256) void k_grad_repair(GradArgs A) {
+  if (*A.list_total > A.max_entries) return;
+  const uint32_t n = *A.bad;
+  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const uint32_t item = A.bad[1 + i], cp = item % A.col_parts, g = item / A.col_parts % A.p.groups;
+    const int64_t slot = item / A.col_parts / A.p.groups, f = (int64_t)g * SP_GROUP + (threadIdx.x >> 4);
+    if (f >= A.F) continue;
+    int64_t s = 0, t = slot;
+    while (t >= A.L - s) { t -= A.L - s; ++s; }
+    t += s;
+    const int c4 = (threadIdx.x & 15) * 4;
+    const T *g_at = (const T *)A.g + t * A.Tn * A.d + (int64_t)cp * SP_COLS + c4;
+    float gr[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int32_t j = A.list_ptr[s * A.F + f]; j < A.list_ptr[s * A.F + f + 1]; ++j) {
+      const uint2 raw = *reinterpret_cast<const uint2 *>(g_at + (int64_t)A.list_tok[j] * A.d);
+      const float v = Elem<T>::to_f32(((const T *)A.val)[A.list_src[j]]);
+      float x[4];
+      unpack_pair<T>(raw.x, x[0], x[1]);
+      unpack_pair<T>(raw.y, x[2], x[3]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) gr[q] = fmaf(v, x[q], gr[q]);
+    }
+    if constexpr (ADAM) {
+      const int64_t at = slot * A.m_dec + (int64_t)cp * A.m_cols + f * A.m_row + c4;
+      T *w = (T *)A.w + (slot * A.F + f) * A.pitch + (int64_t)cp * SP_COLS + c4;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) w[q] = Elem<T>::from_f32(adam_update(Elem<T>::to_f32(w[q]), gr[q], A.m[at + q], A.v[at + q], A.adam));
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) A.out[(slot * A.F + f) * A.d + (int64_t)cp * SP_COLS + c4 + q] = gr[q];
+    }
+  }
+}
+constexpr unsigned REPAIR_BLOCKS = 512;
+
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct SpLayout {
   SpPlan p;
   int col_parts;
-  int64_t n_batches;
-  size_t start, batches, counts, offset, total, recs, bytes;
+  int64_t n_batches, n_groups;
+  size_t bad, start, batches, counts, offset, total, recs, bytes;
 };
 
-// `rows` output rows and `cols` tile rows per layer; `per_group` workgroups for every part of the rows
-static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int waves, int64_t per_part, int64_t max_entries) {
+// `rows` output rows and `cols` tile rows per layer; `per_part` workgroups for every part of the rows; `outputs` times that
+// many rows come out
+static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int waves, int64_t per_part, int64_t outputs, int64_t max_entries) {
   SpLayout l;
   SpPlan &p = l.p;
   p.tiles = (int)clt_ceil_div(cols, SP_ROWS);
@@ -578,6 +669,8 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
   l.offset = take(sizeof(uint32_t) * (size_t)p.streams * p.stages);
   l.total = take(sizeof(uint32_t) * (size_t)p.streams);
   l.recs = take((size_t)l.n_batches * SP_REC_WORDS * 4);
+  l.n_groups = outputs * p.groups * l.col_parts;
+  l.bad = take(sizeof(uint32_t) * (size_t)(l.n_groups + 1));
   l.bytes = at;
   return l;
 }
@@ -585,13 +678,14 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
 // LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile; 16-bit batch counts
 static bool sp_shape_ok(const SpLayout &l, int64_t row_bytes) {
   return l.p.tiles <= REC_MAX_TILES && l.n_batches <= 0x00FFFFFFll && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
-         (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll;
+         (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll && l.n_groups <= 0x7FFFFFFFll;
 }
 
 static void sp_place_workspace(RecArgs &ra, const SpLayout &l, char *ws) {
   ra.p = l.p;
   ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint16_t *)(ws + l.counts);
   ra.offset = (uint32_t *)(ws + l.offset); ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint32_t *)(ws + l.recs);
+  ra.bad = (uint32_t *)(ws + l.bad);
 }
 
 template <typename T> static int launch_records(RecArgs ra, hipStream_t stream) {
@@ -611,7 +705,7 @@ template <typename T> static int launch_records(RecArgs ra, hipStream_t stream) 
 }
 
 static SpLayout tile_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {
-  return sp_layout(Tn, F, d, L, DT_WAVES, targets, max_entries);
+  return sp_layout(Tn, F, d, L, DT_WAVES, targets, targets, max_entries);
 }
 
 template <typename T> static int launch_tiles(RecArgs ra, TileArgs ta, int col_parts, hipStream_t stream) {
@@ -621,12 +715,13 @@ template <typename T> static int launch_tiles(RecArgs ra, TileArgs ta, int col_p
     return CLT_ERR_LAUNCH;
   const int64_t pairs = clt_ceil_div((int64_t)(ta.t_end - ta.t_begin) * col_parts, 8) * 8;
   k_decode_tiles<T><<<(unsigned)(pairs * ta.p.parts), DT_WAVES * 64, DT_LDS, stream>>>(ta);
+  k_decode_repair<T><<<REPAIR_BLOCKS, 256, 0, stream>>>(ta);
   return clt_check_launch();
 }
 
 static SpLayout grad_layout(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
   // (a launch has a workgroup per pair, column part and part of the features: plenty, so the parts are as large as they get)
-  return sp_layout(F, T, d, L, GT_WAVES, 1 << 20, entries);
+  return sp_layout(F, T, d, L, GT_WAVES, 1 << 20, L * (L + 1) / 2, entries);
 }
 
 static int launch_grad(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val, GradArgs a,
@@ -642,14 +737,20 @@ static int launch_grad(const int32_t *list_ptr, const int32_t *list_tok, const i
   if (code != CLT_OK) return code;
   a.p = l.p; a.counts = ra.counts; a.offset = ra.offset; a.total = ra.total; a.recs = ra.recs;
   a.list_total = list_ptr + a.L * a.F;
+  a.list_ptr = list_ptr; a.list_tok = list_tok; a.list_src = list_src; a.val = val; a.bad = ra.bad;
   a.col_parts = l.col_parts;
   a.items = (int)clt_ceil_div((int64_t)l.p.parts * l.col_parts, 8);
   const int64_t blocks = 8 * (int64_t)a.items * (a.L * (a.L + 1) / 2);
   if (blocks > 0x7FFFFFFFll) return CLT_ERR_RANGE;
   const void *k = a.w ? (const void *)k_grad_tiles<bf16_t, true> : (const void *)k_grad_tiles<bf16_t, false>;
   if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS) != hipSuccess) return CLT_ERR_LAUNCH;
-  if (a.w) k_grad_tiles<bf16_t, true><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
-  else k_grad_tiles<bf16_t, false><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
+  if (a.w) {
+    k_grad_tiles<bf16_t, true><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
+    k_grad_repair<bf16_t, true><<<REPAIR_BLOCKS, 256, 0, stream>>>(a);
+  } else {
+    k_grad_tiles<bf16_t, false><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
+    k_grad_repair<bf16_t, false><<<REPAIR_BLOCKS, 256, 0, stream>>>(a);
+  }
   return clt_check_launch();
 }
 
@@ -706,6 +807,7 @@ extern "C" int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, cons
   TileArgs ta;
   ta.p = l.p; ta.counts = ra.counts; ta.total = ra.total; ta.recs = ra.recs;
   ta.wp = w_packed; ta.bias_sum = bias_sum; ta.skip_add = skip_add; ta.out = out;
+  ta.row_ptr = row_ptr; ta.col = col; ta.val = val; ta.bad = ra.bad;
   ta.list_total = row_ptr + L * T; ta.max_entries = max_entries;
   ta.Tn = T; ta.d = d; ta.F = F; ta.L = L; ta.pitch = pitch; ta.src_mask = src_mask;
   ta.tying = tying; ta.t_begin = (int)t_begin; ta.t_end = (int)t_end; ta.out_f32 = out_f32; ta.col_parts = l.col_parts;
