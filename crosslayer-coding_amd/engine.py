@@ -114,11 +114,13 @@ SLICED_DECODE_MIN_ROWS = 8192
 SLICED_DECODE_MIN_SLAB_BYTES = 128 << 20
 
 
-def _wants_sliced_decode(rows: int, slab_bytes: int, T: int, d: int, F: int, L: int, tying: str, dtype: torch.dtype) -> bool:
-    """... or rows too wide for a wavefront to hold (d > 1024 in fp32), which only the sliced schedules and the kernel for
-    any shape take: 1860 -> 23 us at L = 2, d = 2048, F = 4096, 77 tokens x 60."""
-    return (rows >= SLICED_DECODE_MIN_ROWS or slab_bytes >= SLICED_DECODE_MIN_SLAB_BYTES
-            or nat.load().clt_decode_route(T, d, F, L, nat.TYING[tying], nat.dtype_code(dtype), 0) == nat.ROUTE_GENERIC)
+# bytes of a row from which on it does not fit a wavefront's registers (five pieces of 16 bytes a lane): only the sliced
+# schedules and the kernel for any shape take it, 1860 -> 23 us at L = 2, d = 2048, F = 4096, float32, 77 tokens x 60
+WAVEFRONT_ROW_BYTES = 5 * 1024
+
+
+def _wants_sliced_decode(rows: int, slab_bytes: int, row_bytes: int) -> bool:
+    return rows >= SLICED_DECODE_MIN_ROWS or slab_bytes >= SLICED_DECODE_MIN_SLAB_BYTES or row_bytes >= WAVEFRONT_ROW_BYTES
 
 
 # token rows of one tile of the matrix-core encoder: shorter batches are padded to it where the kernel for short ones
@@ -929,14 +931,15 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
     need = lib.clt_decoder_slab_elems(d, F, L, nat.TYING[tying], nat.dtype_code(surv.dtype))
     if need < 0 or w_packed.numel() < need:
         raise nat.CLTNativeError(f"decode_sparse: packed decoders hold {w_packed.numel()} elements, the kernels index {need}")
-    if ws is not None and feat_offset is None and feat_scale is None:
+    if ws is not None and tying != "per_target" and feat_offset is None and feat_scale is None:
         # the survivor total: exact, or (a threshold list, sized for any batch) the last one seen for this shape, or 1 %
         # of the features before there is one
         exact = surv.status is None
         total = surv.capacity if exact else surv.nnz_hint
         if total is None:
             total = L * T * F // 100
-        if total and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
+        wide = surv.dtype == torch.float32
+        if total and not wide and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
             cap = total if exact else min(surv.capacity, 2 * total + 65536)
             nbytes = lib.clt_decode_tiles_workspace_bytes(T, d, F, L, t_end - t_begin, cap)
             wbuf = ws.get("decode_tiles", nbytes)
@@ -947,7 +950,7 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
             if not exact:      # a batch that outgrew the estimate is decoded by the gather, decided on the device
                 nat.check(lib.clt_decode_sparse_if_over(*args, _stream(w_packed)), "clt_decode_sparse_if_over")
             return out
-        if total and exact and lib.clt_decode_rows_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
+        if total and wide and exact and lib.clt_decode_rows_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
             wbuf = ws.get("decode_rows", lib.clt_decode_rows_workspace_bytes(T, d, F, L, total))
             code = lib.clt_decode_rows(nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed),
                                        nat.ptr(bias_sum), nat.ptr(skip_add), nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin,
@@ -955,8 +958,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
             nat.check(code, "clt_decode_rows")
             return out
     wbuf, wbytes = None, 0
-    if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(), T, d, F, L, tying,
-                                               surv.dtype):
+    if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(),
+                                               d * w_packed.element_size()):
         wbytes = lib.clt_decode_workspace_bytes(T, d, F, L)
         wbuf = ws.get("decode", wbytes)
     code = lib.clt_decode_sparse(
@@ -974,8 +977,9 @@ def decode_route(T: int, d: int, F: int, L: int, tying: str, dtype: torch.dtype,
     lib = nat.load()
     rows = T * L if rows is None else rows
     n_dec = L * (L + 1) // 2 if tying == "none" else L
-    slab_bytes = n_dec * F * decoder_pitch(d, dtype) * torch.empty((), dtype=dtype).element_size()
-    wbytes = lib.clt_decode_workspace_bytes(T, d, F, L) if _wants_sliced_decode(rows, slab_bytes, T, d, F, L, tying, dtype) else 0
+    elem = torch.empty((), dtype=dtype).element_size()
+    slab_bytes = n_dec * F * decoder_pitch(d, dtype) * elem
+    wbytes = lib.clt_decode_workspace_bytes(T, d, F, L) if _wants_sliced_decode(rows, slab_bytes, d * elem) else 0
     code = lib.clt_decode_route(T, d, F, L, nat.TYING[tying], nat.dtype_code(dtype), wbytes)
     if code < 0:
         nat.check(code, "clt_decode_route")
