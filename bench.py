@@ -26,6 +26,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0       # MI355X HBM3E, GB/s
+LDS_PEAK_GBS = 256 * 128 * 2.4          # compute units x bytes per clock x GHz
 MFMA_BF16_PEAK_TF = 2500.0  # dense bf16, TFLOP/s
 MFMA_FP32_PEAK_TF = 157.3
 
@@ -212,6 +213,9 @@ def run_gpu(args):
     dense_first, dense_end = dec.last_route.get("dense_targets", (L, L))
     n_dense = dense_end - dense_first
     table, forwards = profiled_traffic(wl.name)
+    wanted = nat.load().clt_decode_rows_wanted if wl.dtype == "float32" else nat.load().clt_decode_tiles_wanted
+    tiled = ((surv.status is None or wl.dtype != "float32")
+             and wanted(T, d, F, L, L, nnz_total, nat.TYING[wl.decoder_tying], nat.dtype_code(model.dtype)))
     if n_dense > 0:
         # decoders tied per target: targets [dense_first, L) are dense products on the MFMA kernel
         flop = 2.0 * T * F * d * n_dense
@@ -226,6 +230,21 @@ def run_gpu(args):
         }
         decode_stage = {"ms": st["decode"], "bound": "mfma", "achieved": tf, "peak": mfma_peak, "unit": "TFLOP/s",
                         "frac": tf / mfma_peak}
+    elif tiled:
+        kname = "k_decode_rows" if wl.dtype == "float32" else "k_decode_tiles"
+        roofline = {
+            "kernel": f"{kname} (sparse cross-layer decode from LDS tiles; one launch per step, with the regrouping of the list before it)",
+            "bound": "lds", "achieved": dec_gbs, "peak": LDS_PEAK_GBS, "unit": "GB/s", "frac": dec_gbs / LDS_PEAK_GBS, "traffic": None,
+            "hbm_compulsory_frac": dec_c_gbs / HBM_PEAK_GBS,
+            "hbm": {"peak": HBM_PEAK_GBS, "compulsory_bytes_per_launch": work["decode_compulsory_bytes"], "compulsory_GBps": dec_c_gbs,
+                    "compulsory_frac": dec_c_gbs / HBM_PEAK_GBS},
+            "note": "achieved = decoder rows read from LDS (one per active (token, feature, source->target)) / the whole decode "
+                    "stage; peak = 256 compute units x 128 bytes per clock at 2.4 GHz.  Records, rows that fill a batch up and the "
+                    "tiles' way into LDS are LDS traffic too and not counted",
+            "algorithmic_bytes_per_launch": work["decode_gathered_bytes"], "avg_launch_ms": st["decode"], "launches_per_step": 1,
+        }
+        decode_stage = {"ms": st["decode"], "bound": "lds", "achieved": dec_gbs, "peak": LDS_PEAK_GBS, "unit": "GB/s",
+                        "frac": dec_gbs / LDS_PEAK_GBS, "compulsory_GBps": dec_c_gbs, "compulsory_frac": dec_c_gbs / HBM_PEAK_GBS}
     else:
         sliced = route in (nat.ROUTE_QUARTER, nat.ROUTE_LINE, nat.ROUTE_SLICED)
         n_dec_launch = L if sliced else 1
@@ -676,7 +695,15 @@ def run_backward(args):
     # copy read and written and the parameter rewritten from the copy
     hbm_bytes = pairs * F * d * ((16 + 4 * esz) if fused else 4) + L * wl.tokens * d * esz + surv.nnz * (8 + esz)
     tiled = fused and opt._dec_layout == "tiles"
-    if tiled:
+    matrix = fused and engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, surv.dtype)
+    if matrix:
+        # through the HBM interface go both moments and the weights, read and written, the loss gradient and the lists
+        hbm_bytes = pairs * F * d * (16 + 2 * esz) + L * wl.tokens * d * esz + surv.nnz * (8 + esz)
+        roofline = {"kernel": f"k_grad_tiles ({dw_name}, one launch per step, with the regrouping of the lists before it)",
+                    "bound": "hbm", "achieved": hbm_bytes / dw_sec / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": hbm_bytes / dw_sec / 1e9 / HBM_PEAK_GBS, "traffic": None, "lds_gather_GBps": gathered / dw_sec / 1e9,
+                    "note": "achieved = compulsory HBM bytes of the stage (moments, weights, loss gradient, lists) / the stage's time"}
+    elif tiled:
         # Column-tile route: the gather of the loss gradient is LDS traffic; through the HBM interface go both
         # moments (read and written: 16 bytes per decoder element), the tiled weight copy (read and written) and
         # the conversion that follows (tiles read, feature-major slab and checkpoint layout written): 5 elements.
@@ -708,7 +735,7 @@ def run_backward(args):
                             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": adam_bytes / adam_sec / 1e9 / HBM_PEAK_GBS}
     return {
         "stages_ms": stages, "roofline": roofline,
-        "decoder_step_route": (("column tiles" if tiled else "rows") if fused else "gradient then Adam") if opt is not None else None,
+        "decoder_step_route": (("matrix cores" if matrix else "column tiles" if tiled else "rows") if fused else "gradient then Adam") if opt is not None else None,
         "metric": ("CLT training step tokens/sec (forward, MSE loss, gradients, Adam lr 1e-4 with fp32 moments)"
                    if opt is not None else "CLT forward + MSE loss + gradients tokens/sec (no optimizer step)"),
         "value": wl.tokens * args.steps / wall, "unit": "tokens/s", "n_gpus": 1, "steps": args.steps,
