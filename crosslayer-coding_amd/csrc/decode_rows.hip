@@ -142,6 +142,8 @@ struct RowArgs {
   const uint2 *recs;
   const float *wp, *bias_sum, *skip_add;
   float *out;
+  const int32_t *row_ptr, *col;
+  const float *val;
   int64_t Tn, d, F, L, pitch;
   uint64_t src_mask;
   int tying, t_begin, t_end, col_parts;
@@ -283,19 +285,46 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
 
   // lane 8 j + i holds entries j of every record, columns 4 i .. 4 i + 3: the eight sums meet in every lane, row tk is written
   // by lanes 8 (tk % 8) .. + 7
-#pragma unroll
-  for (int tk = 0; tk < DR_TOK; ++tk) {
-    f32x4v_t a = acc[tk];
+  auto meet = [&](f32x4v_t a) {
 #pragma unroll
     for (int o = 8; o < 64; o <<= 1)
 #pragma unroll
       for (int q = 0; q < 4; ++q) a[q] += __shfl_xor(a[q], o);
+    return a;
+  };
+  const int64_t o = (int64_t)cp * DR_COLS + (lane & 7) * 4;
+  auto write = [&](int tk, f32x4v_t a) {
     const int64_t tok = (int64_t)g * DR_TOK + tk;
-    if (!mine || tok >= A.Tn || (lane >> 3) != (tk & 7)) continue;
-    const int64_t o = (int64_t)cp * DR_COLS + (lane & 7) * 4, at = ((int64_t)t * A.Tn + tok) * A.d + o;
+    if (!mine || tok >= A.Tn || (lane >> 3) != (tk & 7)) return;
+    const int64_t at = ((int64_t)t * A.Tn + tok) * A.d + o;
     if (A.bias_sum) a += *reinterpret_cast<const f32x4v_t *>(A.bias_sum + (int64_t)t * A.d + o);
     if (A.skip_add) a += *reinterpret_cast<const f32x4v_t *>(A.skip_add + at);
     *reinterpret_cast<f32x4v_t *>(A.out + at) = a;
+  };
+  uint32_t again = 0;                                      // tokens whose sums are not finite
+#pragma unroll
+  for (int tk = 0; tk < DR_TOK; ++tk) {
+    const f32x4v_t a = meet(acc[tk]);
+    const float z = fmaf(a[0], 0.0f, fmaf(a[1], 0.0f, fmaf(a[2], 0.0f, a[3] * 0.0f)));
+    if (ballot64(z != z) != 0) again |= 1u << tk;
+    else write(tk, a);
+  }
+  // Those once more without the places that fill records up: 0 * inf of such a place would turn an infinity into a NaN.
+  for (; again != 0; again &= again - 1) {
+    const int tk = __ffs(again) - 1;
+    f32x4v_t a{0.f, 0.f, 0.f, 0.f};
+    for (uint64_t m = mask; m != 0; m &= m - 1) {
+      const int s = __ffsll((unsigned long long)m) - 1;
+      const float *w = A.wp + sp_slot(A.tying, s, t, A.L) * A.F * A.pitch + o;
+      const int32_t *row = A.row_ptr + (int64_t)s * A.Tn + (int64_t)g * DR_TOK + tk;
+      for (int32_t j = row[0] + (lane >> 3); j < row[1]; j += DR_REC) {
+        const f32x4v_t x = *reinterpret_cast<const f32x4v_t *>(w + (int64_t)A.col[j] * A.pitch);
+        const float v = A.val[j];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = fmaf(v, x[q], a[q]);
+      }
+    }
+    write(tk, meet(a));
   }
 }
 
@@ -391,6 +420,7 @@ extern "C" int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const
   RowArgs a;
   a.p = l.p; a.counts = ra.counts; a.total = ra.total; a.recs = ra.recs;
   a.wp = w_packed; a.bias_sum = bias_sum; a.skip_add = skip_add; a.out = out;
+  a.row_ptr = row_ptr; a.col = col; a.val = val;
   a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = pitch; a.src_mask = src_mask;
   a.tying = tying; a.t_begin = (int)t_begin; a.t_end = (int)t_end; a.col_parts = l.col_parts;
   const int64_t pairs = clt_ceil_div((t_end - t_begin) * l.col_parts, 8) * 8;

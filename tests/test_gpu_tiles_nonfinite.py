@@ -1,4 +1,4 @@
-"""Infinities and NaNs in the operands of the one-hot matrix products (decode and weight gradient from LDS tiles) reach the
+"""Infinities and NaNs in the operands of the products from LDS tiles (decodes and weight gradient) reach the
 output rows whose lists refer to them and no others, although a batch's 16 rows are multiplied together."""
 import pytest
 import torch
@@ -81,3 +81,33 @@ def test_weight_gradient(adam):
                 mag[f] = act[s, r, f].double().abs() @ gm[t, r].double().abs()
             _check(got[slot], ref, mag)
             slot += 1
+
+
+def test_decode_rows(monkeypatch):
+    """The float32 decode multiplies the places that fill a record up (a run's last entry once more, value 0) with that entry's
+    decoder row: an infinity there stays an infinity."""
+    g, keep, act, surv = _lists(torch.float32)
+    monkeypatch.setattr(nat.load(), "clt_decode_rows_wanted", lambda *a: 1)
+    n_dec = L * (L + 1) // 2
+    w = engine.alloc_packed(n_dec, F, d, torch.float32, torch.device("cuda:0"))
+    wc = torch.randn(n_dec, F, d, generator=g)
+    for i, tok in enumerate((0, 17, 199)):        # the last features of a token's runs, which are shorter than a record
+        kept = keep[0, tok].nonzero()[:, 0]
+        for c in range(3):
+            wc[i, kept[kept < 512 * (c + 1)][-1], 5 + 40 * c] = float("inf") * (-1) ** c
+    wc[1, 512, 3], wc[4, 700, 64] = float("nan"), float("inf")
+    w[:, :, :d] = wc.cuda()
+    bias = torch.randn(L, d, generator=g)
+    got = engine.decode_sparse(surv, w, "none", d, bias_sum=bias.cuda(), ws=engine.Workspace(torch.device("cuda:0"))).cpu().double()
+    for t in range(L):
+        ref, mag = bias[t].double().expand(T, d).clone(), bias[t].double().abs().expand(T, d).clone()
+        for s in range(t + 1):
+            m = wc[s * L - s * (s - 1) // 2 + t - s].double()
+            for tok in range(T):
+                f = keep[s, tok]
+                ref[tok] += act[s, tok, f].double() @ m[f]
+                mag[tok] += act[s, tok, f].double().abs() @ m[f].abs()
+        assert torch.equal(got[t].isnan(), ref.isnan()) and torch.equal(got[t].isinf(), ref.isinf()) and bool(ref.isinf().any())
+        fin = ref.isfinite()
+        # at most K sources' entries and eight sums more, each addition off by at most 2^-24 of what has been summed
+        assert bool(((got[t] - ref).abs() <= (L * K + 16) * 2.0 ** -24 * mag)[fin].all())
