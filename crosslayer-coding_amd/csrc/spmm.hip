@@ -123,7 +123,11 @@ __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
 template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(RecArgs A) {
   extern __shared__ int32_t fill_lds[];
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
-  if (A.row_ptr[A.L * A.Rn] > A.max_entries || !((A.layer_mask >> s) & 1ull)) return;
+  if (A.row_ptr[A.L * A.Rn] > A.max_entries) return;
+  // A wavefront at the end of its stream takes the record that follows for addresses, of LDS reads that nobody multiplies: the
+  // next stream's first one, or this one behind the last stream, which refers to the first row of the first buffer.
+  if (g == 0 && s == 0 && tid < 64) A.recs[(uint64_t)stream_first(A.total, A.p.streams, lane) * SP_REC_WORDS + lane] = 0u;
+  if (!((A.layer_mask >> s) & 1ull)) return;
   int32_t *start = fill_lds;                               // [SP_GROUP][tiles + 1]
   int32_t *off = start + SP_GROUP * (tiles + 1);           // [SP_GROUP][tiles] entries of the tile before this row's
   int32_t *first = off + SP_GROUP * tiles;                 // [tiles + 1] first batch of the tile, counted within the group
@@ -659,8 +663,8 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
   }
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
   p.streams = p.parts * waves;
-  // every (layer, tile, group) may leave its last batch part empty; a stream reads a ring of batches past its end
-  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + 8;
+  // every (layer, tile, group) may leave its last batch part empty; a stream asks for a ring of batches and one more past its end
+  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + DT_RING + 1;
   size_t at = 0;
   auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
   l.start = take(sizeof(int32_t) * (size_t)L * p.groups * SP_GROUP * (p.tiles + 1));

@@ -40,7 +40,7 @@ def _run(dev, act, row_ptr, col, val, w, tying, d, bias, skip, t0, t1, mask, f32
     b, k = (None if x is None else x.to(dev) for x in (bias, skip))
     out = torch.full((L, T, d), 7.0, dtype=torch.float32 if f32 else act.dtype, device=dev)
     nbytes = lib.clt_decode_tiles_workspace_bytes(T, d, F, L, t1 - t0, cap)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev)      # what lies behind the records must not matter
     args = (nat.ptr(rp), nat.ptr(c), nat.ptr(v), nat.ptr(slab), nat.ptr(b), nat.ptr(k), nat.ptr(out), T, d, F, L, nat.TYING[tying],
             t0, t1, mask, nat.dtype_code(act.dtype), 1 if f32 else 0, cap)
     for _ in range(2):                 # the second pass meets a workspace in use
@@ -93,6 +93,18 @@ def test_decode_tiles_against_dense_products(L, T, F, d, per_token, dtype, tying
             if not f32:
                 bound = bound + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * (ref.abs() + bound) + 2.0 ** -24
             assert (got[t].double() - ref).abs().le(bound).all(), (t, (got[t].double() - ref).abs().max())
+
+
+def test_decode_tiles_of_empty_lists():
+    """No stream has a record: every wavefront meets the one behind the last stream."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 2, 40, 1100, 128
+    act, row_ptr, col, val = _lists(L, T, F, 0, torch.bfloat16, seed=3, heavy=False)
+    w = (torch.rand(3, F, d, generator=torch.Generator().manual_seed(1)) - 0.5).bfloat16()
+    bias = torch.randn(L, d, generator=torch.Generator().manual_seed(2))
+    for cap in (0, 1000):
+        got = _run(dev, act, row_ptr, col, val, w, "none", d, bias, None, 0, L, 3, True, cap, False)
+        assert torch.equal(got, bias.unsqueeze(1).expand(L, T, d))
 
 
 def test_decode_tiles_leaves_longer_lists_to_the_gather():

@@ -3,7 +3,7 @@ edges of their tiles: 512 tokens, 16 features per group, 8 wavefronts x 4 groups
 import pytest
 import torch
 
-from crosslayer_coding_amd import engine
+from crosslayer_coding_amd import _native as nat, engine
 
 pytestmark = pytest.mark.gpu
 
@@ -25,6 +25,7 @@ def test_grad_tiles_against_dense_products(L, T, F, d, per_token):
     assert engine.grad_tiles_supported(T, d, F, L, surv.capacity, torch.bfloat16)
     ws = engine.Workspace(dev)
     lists = engine.feature_lists(surv, ws)
+    ws.get("grad_tiles", nat.load().clt_grad_tiles_workspace_bytes(T, d, F, L, surv.capacity)).fill_(0xFF)      # must not matter
     got = engine.decoder_weight_grad(lists, surv, gm.to(dev), "none", ws=ws).cpu()
     assert torch.equal(got, engine.decoder_weight_grad(lists, surv, gm.to(dev), "none", ws=ws).cpu())
     slot = 0
