@@ -67,6 +67,7 @@ _SIGNATURES = {
     "clt_decode_rows_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "clt_decode_rows": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _i64, _vp, _sz, _vp]),
     "clt_decode_tiles_wanted": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _int, _int]),
+    "clt_decode_tiles_max_entries": (_i64, [_i64, _i64, _i64, _i64, _i64]),
     "clt_decode_tiles_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64]),
     "clt_decode_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int, _i64,
                                 _vp, _sz, _vp]),

@@ -680,8 +680,9 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
 }
 
 // LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile; 16-bit batch counts
+constexpr int64_t SP_MAX_BATCHES = 0x00FFFFFF;
 static bool sp_shape_ok(const SpLayout &l, int64_t row_bytes) {
-  return l.p.tiles <= REC_MAX_TILES && l.n_batches <= 0x00FFFFFFll && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
+  return l.p.tiles <= REC_MAX_TILES && l.n_batches <= SP_MAX_BATCHES && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
          (int64_t)l.p.stages * l.p.groups <= 0x7FFFFFFFll && l.n_groups <= 0x7FFFFFFFll;
 }
 
@@ -780,6 +781,12 @@ extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t 
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
   const double tiles_us = (stages > longest ? stages : longest) * (stage_us > 2.24 ? stage_us : 2.24) + 20 + entries * 1.25e-5;
   return tiles_us < 0.95 * sparse_us;
+}
+
+extern "C" int64_t clt_decode_tiles_max_entries(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets) {
+  if (T <= 0 || d < SP_COLS || F <= 0 || L <= 0 || targets <= 0) return 0;
+  const SpLayout l = tile_layout(T, d, F, L, targets, 0);
+  return sp_shape_ok(l, clt_pitch(d, 2) * 2) ? (SP_MAX_BATCHES - l.n_batches) * SP_BATCH + SP_BATCH - 1 : 0;
 }
 
 extern "C" size_t clt_decode_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries) {

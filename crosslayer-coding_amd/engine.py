@@ -940,7 +940,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
             total = L * T * F // 100
         wide = surv.dtype == torch.float32
         if total and not wide and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
-            cap = total if exact else min(surv.capacity, 2 * total + 65536)
+            # room for twice that many, or what the records can count where that is less
+            cap = total if exact else min(surv.capacity, 2 * total + 65536, lib.clt_decode_tiles_max_entries(T, d, F, L, t_end - t_begin))
             nbytes = lib.clt_decode_tiles_workspace_bytes(T, d, F, L, t_end - t_begin, cap)
             wbuf = ws.get("decode_tiles", nbytes)
             args = (nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum), nat.ptr(skip_add),

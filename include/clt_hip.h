@@ -436,10 +436,12 @@ int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const float *val
  * gathered from LDS.  Deterministic, equal to clt_decode_sparse up to fp32 summation order.
  *   clt_decode_tiles_wanted: whether it is the faster of the two for `entries` survivors over L layers and `targets`
  *   target layers (0 also for what it does not take).
- *   The workspace is sized for max_entries survivors.  A list that turns out longer on the device (row_ptr[L*T] >
- *   max_entries) is left alone: clt_decode_sparse_if_over decodes such a list and does nothing otherwise.
+ *   The workspace is sized for max_entries survivors, of which clt_decode_tiles_max_entries is the largest number that
+ *   the records of these shapes can count (more: CLT_ERR_RANGE).  A list that turns out longer on the device
+ *   (row_ptr[L*T] > max_entries) is left alone: clt_decode_sparse_if_over decodes such a list and does nothing otherwise.
  */
 int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
+int64_t clt_decode_tiles_max_entries(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets);
 size_t clt_decode_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t max_entries);
 int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
                      const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
