@@ -203,7 +203,7 @@ constexpr int SLICED_NTOK = 4;   // tokens per wavefront in the sliced kernel
 constexpr int DECODE_FEW = 1024, DECODE_FEW_U = 16;
 
 // One wavefront per (target, token): walks all sources s <= t, accumulates in registers,
-// writes the output row once.  Used for small batches.  only_above >= 0: runs only if the list has more entries than that.
+// writes the output row once.  Used for small batches.
 //
 // SLICED (large batches): one launch per source layer `src`; one wavefront per
 // (target >= src, token, feature slice).  The feature axis is cut into `ns` slices and block b
@@ -226,8 +226,7 @@ __attribute__((amdgpu_waves_per_eu(decode_min_waves<T, NF, TAIL, SLICED>(), 8)))
     const T *__restrict__ fscale, const float *__restrict__ skip_add, void *__restrict__ out,
     int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end,
     uint64_t src_mask, int out_f32, const int32_t *__restrict__ sptr, float *__restrict__ partial, int ns,
-    int src, int64_t pitch, int64_t only_above) {
-  if (!SLICED && only_above >= 0 && row_ptr[L * Tn] <= only_above) return;
+    int src, int64_t pitch) {
   constexpr int V = WVec<T>::V;
   constexpr int HV = V / 2;                       // elements per 8 bytes
   constexpr int NACC = NF * V + (TAIL == 1 ? HV : TAIL == 2 ? V : 0);
@@ -449,10 +448,10 @@ static UnitPlan make_unit_plan(int ns, int ncp, int64_t Tn, int tok_per_block) {
 
 // this block's work: target index (relative), unit -> (slice, column part), its token range and its token block
 struct UnitWork { int64_t target; int slice, cpart; int64_t tok_begin, tok_end; int tb; };
-__device__ __forceinline__ UnitWork unit_work(const UnitPlan &up, int64_t Tn) {
+__device__ __forceinline__ UnitWork unit_work(const UnitPlan &up, int64_t Tn, int64_t block) {
   UnitWork w;
-  const int xcd = (int)(blockIdx.x & 7);
-  const int64_t i = (int64_t)(blockIdx.x >> 3);
+  const int xcd = (int)(block & 7);
+  const int64_t i = block >> 3;
   w.target = i / up.bpx;
   const int j = (int)(i % up.bpx);
   int unit;
@@ -589,7 +588,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(quarter_min
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int ll = lane & (QLANES - 1), grp = lane / QLANES;
   const bool hi = grp != 0;                    // only the first lane group touches the partial row
-  const UnitWork uw = unit_work(up, Tn);
+  const UnitWork uw = unit_work(up, Tn, (int64_t)blockIdx.x);
   const int slice = uw.slice, cpart = uw.cpart;
   const PairAt at = pair_at(uw.target, src_arg, slice, L, t_begin, t_end, src_mask);
   const int src = at.src;
@@ -756,6 +755,42 @@ template <typename T, int UU, bool PACK> struct LineBatch {
   }
 };
 
+// the n <= 64 survivors that a wavefront holds one per lane, two batches of loads in flight
+template <typename T, bool PACK>
+__device__ __forceinline__ void line_chunk(float *acc, const T *wbase, int64_t pitch, int32_t my_col, float my_val, int n, int ll, int grp) {
+  // 16 bits: feature index (< 65536) and value travel to their lane group in one 32-bit word
+  const uint32_t my_pk = PACK ? ((uint32_t)my_col | (raw16_of<T>(my_val) << 16)) : 0u;
+  constexpr int R = 8 * LINE_UU;                 // survivors per batch
+  LineBatch<T, LINE_UU, PACK> ra, rb;
+  ra.load(wbase, pitch, my_pk, my_col, my_val, 0, n, ll, grp);
+  for (int i0 = 0; i0 < n; i0 += 2 * R) {
+    if (i0 + R < n) rb.load(wbase, pitch, my_pk, my_col, my_val, i0 + R, n, ll, grp);
+    ra.consume(acc);
+    if (i0 + R < n) {
+      if (i0 + 2 * R < n) ra.load(wbase, pitch, my_pk, my_col, my_val, i0 + 2 * R, n, ll, grp);
+      rb.consume(acc);
+    }
+  }
+}
+
+// Reduce-scatter of 8 sums over the eight lane groups (fixed order): every step hands half of the accumulators to the partner
+// group and adds the half that comes back, so a lane ends with the sum of ONE column, 8 * (lane % 8) + lane / 8.
+__device__ __forceinline__ float line_scatter8(const float *acc, int grp) {
+  float a4[4], a2[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float keep = (grp & 4) ? acc[j + 4] : acc[j], send = (grp & 4) ? acc[j] : acc[j + 4];
+    a4[j] = keep + __shfl_xor(send, 32);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float keep = (grp & 2) ? a4[j + 2] : a4[j], send = (grp & 2) ? a4[j] : a4[j + 2];
+    a2[j] = keep + __shfl_xor(send, 16);
+  }
+  const float keep = (grp & 1) ? a2[1] : a2[0], send = (grp & 1) ? a2[0] : a2[1];
+  return keep + __shfl_xor(send, 8);
+}
+
 template <typename T, bool AFFINE, bool PACK, int NTOK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_decode_line(
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp, const T *__restrict__ foff,
@@ -767,7 +802,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int ll = lane & 7, grp = lane >> 3;
   const int ns = lp.ns;
-  const UnitWork uw = unit_work(lp, Tn);
+  const UnitWork uw = unit_work(lp, Tn, (int64_t)blockIdx.x);
   const int cpart = uw.cpart, slice = uw.slice;
   const PairAt at = pair_at(uw.target, src_arg, slice, L, t_begin, t_end, src_mask);
   const int src = at.src;
@@ -800,7 +835,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     float acc[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] = 0.0f;
-    LineBatch<T, LINE_UU, PACK> ra, rb;
     for (int32_t j0 = b; j0 < e; j0 += 64) {
       const int n = (e - j0) < 64 ? (e - j0) : 64;
       int32_t my_col = cur_col; float my_val = Elem<T>::to_f32(cur_val);
@@ -812,36 +846,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
         if (foff) my_val = Elem<T>::round(my_val + Elem<T>::to_f32(foff[t * F + my_col]));
         if (fscale) my_val = Elem<T>::round(my_val * Elem<T>::to_f32(fscale[t * F + my_col]));
       }
-      // bf16: feature index (< 65536) and value travel to their lane group in one 32-bit word
-      const uint32_t my_pk = PACK ? ((uint32_t)my_col | (raw16_of<T>(my_val) << 16)) : 0u;
-      constexpr int R = 8 * LINE_UU;                 // survivors per batch
-      ra.load(wbase, pitch, my_pk, my_col, my_val, 0, n, ll, grp);
-      for (int i0 = 0; i0 < n; i0 += 2 * R) {
-        if (i0 + R < n) rb.load(wbase, pitch, my_pk, my_col, my_val, i0 + R, n, ll, grp);
-        ra.consume(acc);
-        if (i0 + R < n) {
-          if (i0 + 2 * R < n) ra.load(wbase, pitch, my_pk, my_col, my_val, i0 + 2 * R, n, ll, grp);
-          rb.consume(acc);
-        }
-      }
+      line_chunk<T, PACK>(acc, wbase, pitch, my_col, my_val, n, ll, grp);
     }
-    // reduce-scatter over the eight lane groups (fixed order): every step hands half of the accumulators to
-    // the partner group and adds the half that comes back, so a lane ends with the sum of ONE column
+    // reduce-scatter over the eight lane groups (fixed order): a lane ends with the sum of ONE column
     float r; int csel; bool writer = true;
     if constexpr (V == 8) {
-      float a4[4], a2[2];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float keep = (grp & 4) ? acc[j + 4] : acc[j], send = (grp & 4) ? acc[j] : acc[j + 4];
-        a4[j] = keep + __shfl_xor(send, 32);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float keep = (grp & 2) ? a4[j + 2] : a4[j], send = (grp & 2) ? a4[j] : a4[j + 2];
-        a2[j] = keep + __shfl_xor(send, 16);
-      }
-      const float keep = (grp & 1) ? a2[1] : a2[0], send = (grp & 1) ? a2[0] : a2[1];
-      r = keep + __shfl_xor(send, 8);
+      r = line_scatter8(acc, grp);
       csel = ll * 8 + grp;
     } else {
       float a2[2];
@@ -861,6 +871,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     if (writer) {
       const float old = first ? 0.0f : __builtin_nontemporal_load(pp);
       __builtin_nontemporal_store(old + r, pp);
+    }
+  }
+}
+
+// A list that is longer than `only_above`, in one launch and without a workspace; nothing happens to a shorter one.  For the
+// threshold list that outgrew what the tiles were given: the host does not know, so the launch is always made, and its
+// OVER_BLOCKS workgroups - as many as are resident, taking the plan's blocks in turn - leave at once in the ordinary case.
+//
+// Units of one cache line of columns as in the line schedule, with every source in the place of one: a workgroup keeps the sums
+// of up to OVER_TOKENS tokens in LDS and takes one source after the other over all of them, so that the workgroups of an XCD
+// gather from about one matrix at a time, which its L2 holds.  Bound by that gather, as the schedules with a launch per source
+// are, whose partial rows it does without.  Those / this, ms, bf16, untied, 200 survivors per token: L = 12, d = 768, F = 24576,
+// 4096 tokens 5.90 / 6.05, 512 tokens 1.15 / 1.07; L = 24, d = 1024, F = 32768 (a line of every row is more than an L2), 2048
+// tokens 17.2 / 20.4; 50 per token: L = 4, F = 8192, 512 tokens, d = 2560 0.159 / 0.161, d = 4096 0.245 / 0.245.  Hence
+// also how many tokens a workgroup takes: a 64th, so that the workgroups of an XCD share one unit (a 288-token share, with
+// four units of the XCD in flight: 10.2 ms in place of 6.05).
+// Measured and dropped: the sums of two tokens at a time in registers over all sources (13.2 ms: the wavefronts of an XCD
+// drift apart over the sources, and no L2 holds them all); one pass of k_decode (11.4 ms, 32.3, and 4.2 and 6.7 ms of the
+// last two, whose rows only k_decode_generic takes).
+constexpr int OVER_WAVES = 16, OVER_TOKENS = 288, OVER_BLOCKS = 2 * 256;
+template <typename T, bool PACK>
+__global__ __launch_bounds__(OVER_WAVES * 64) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_decode_over(
+    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
+    const float *__restrict__ bias_sum, const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d, int64_t F,
+    int64_t L, int tying, int t_end, uint64_t src_mask, int out_f32, UnitPlan lp, int ntok, int64_t pitch, int64_t blocks,
+    int64_t only_above) {
+  extern __shared__ float sums[];                            // [ntok][64]
+  if (row_ptr[L * Tn] <= only_above) return;
+  const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ll = lane & 7, grp = lane >> 3;
+  for (int64_t block = blockIdx.x; block < blocks; block += gridDim.x) {
+    const UnitWork uw = unit_work(lp, Tn, block);
+    const int t = t_end - 1 - (int)uw.target;                // longest first
+    const int64_t tok0 = uw.tok_begin + (int64_t)uw.tb * ntok + wv;      // this wavefront's: every OVER_WAVES-th from here
+    const int64_t left = (uw.tok_end < tok0 - wv + ntok ? uw.tok_end : tok0 - wv + ntok) - tok0;
+    const int n_mine = left > 0 ? (int)((left + OVER_WAVES - 1) / OVER_WAVES) : 0;
+    float *mine = sums + wv * 64;
+    for (int i = 0; i < n_mine; ++i) mine[i * (OVER_WAVES * 64) + lane] = 0.0f;
+    for (uint64_t m = src_mask & ((2ull << t) - 1ull); m != 0; m &= m - 1) {
+      const int s = __ffsll((unsigned long long)m) - 1;
+      __syncthreads();                                       // the workgroup stays together
+      const T *wbase = wp + decoder_slot(tying, s, t, L) * F * pitch + (int64_t)uw.cpart * 64;
+      int32_t mb = 0, me = 0;                                // the tokens' lists, a lane each
+      if (lane < n_mine) {
+        const int64_t r = (int64_t)s * Tn + tok0 + lane * OVER_WAVES;
+        mb = row_ptr[r]; me = row_ptr[r + 1];
+      }
+      int32_t nb = __builtin_amdgcn_readlane(mb, 0), ne = __builtin_amdgcn_readlane(me, 0), nxt_col = 0;
+      T nxt_val = Elem<T>::from_raw(0u);
+      if (lane < ne - nb) { nxt_col = col[nb + lane]; nxt_val = val[nb + lane]; }
+      for (int i = 0; i < n_mine; ++i) {
+        const int32_t b = nb, e = ne, cur_col = nxt_col;
+        const T cur_val = nxt_val;
+        if (i + 1 < n_mine) {
+          nb = __builtin_amdgcn_readlane(mb, i + 1); ne = __builtin_amdgcn_readlane(me, i + 1);
+          nxt_col = 0; nxt_val = Elem<T>::from_raw(0u);
+          if (lane < ne - nb) { nxt_col = col[nb + lane]; nxt_val = val[nb + lane]; }
+        }
+        if (b == e) continue;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int32_t j0 = b; j0 < e; j0 += 64) {
+          const int n = (e - j0) < 64 ? (e - j0) : 64;
+          int32_t my_col = cur_col; float my_val = Elem<T>::to_f32(cur_val);
+          if (j0 > b) {
+            my_col = 0; my_val = 0.0f;
+            if (lane < n) { my_col = col[j0 + lane]; my_val = Elem<T>::to_f32(val[j0 + lane]); }
+          }
+          line_chunk<T, PACK>(acc, wbase, pitch, my_col, my_val, n, ll, grp);
+        }
+        mine[i * (OVER_WAVES * 64) + ll * 8 + grp] += line_scatter8(acc, grp);
+      }
+    }
+    for (int i = 0; i < n_mine; ++i) {
+      const int64_t o = (int64_t)uw.cpart * 64 + ll * 8 + grp, at = ((int64_t)t * Tn + tok0 + i * OVER_WAVES) * d + o;
+      float y = mine[i * (OVER_WAVES * 64) + ll * 8 + grp];
+      if (bias_sum) y += bias_sum[(int64_t)t * d + o];
+      if (skip_add) y += skip_add[at];
+      if (out_f32) ((float *)out)[at] = y;
+      else ((T *)out)[at] = Elem<T>::from_f32(y);
     }
   }
 }
@@ -930,9 +1019,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_decode_generic(
     const int32_t *row_ptr, const int32_t *col, const T *val, const T *wp, const float *bias_sum,
     const T *foff, const T *fscale, const float *skip_add, void *out, int64_t Tn, int64_t d,
-    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch,
-    int64_t only_above) {
-  if (only_above >= 0 && row_ptr[L * Tn] <= only_above) return;
+    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch) {
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   const int64_t blocks_per_t = (Tn + nwv - 1) / nwv;
   const int64_t t = t_end - 1 - (int64_t)blockIdx.x / blocks_per_t;
@@ -1324,7 +1411,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
                          const float *bias_sum, const void *foff, const void *fscale, const float *skip_add,
                          void *out, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
                          int64_t t_end, uint64_t src_mask, int out_f32, void *workspace, size_t workspace_bytes,
-                         hipStream_t stream, int64_t only_above = -1) {
+                         hipStream_t stream) {
   constexpr int V = WVec<T>::V;
   const int nwv = 4;
   const int64_t pitch = clt_pitch(d, (int)sizeof(T));
@@ -1351,7 +1438,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
                             L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, stream);
 #define CLT_DEC_ARGS(FO, FS)                                                                                    \
   row_ptr, col, (const T *)val, (const T *)wp, bias_sum, FO, FS, skip_add, out, Tn, d, F, L, tying, tb,         \
-      t_end, src_mask, out_f32, sptr, partial, ns, src, pitch, only_above
+      t_end, src_mask, out_f32, sptr, partial, ns, src, pitch
 #define CLT_DEC(NFN, TL, UN)                                                                                    \
   do {                                                                                                          \
     if (affine && can_slice)                                                                                    \
@@ -1474,7 +1561,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
   } else {
     const int64_t tb = t_begin; const int src = 0; (void)tb; (void)src;
     k_decode_generic<T><<<(unsigned)nblk, 256, 0, stream>>>(row_ptr, col, (const T *)val, (const T *)wp, bias_sum,
-        (const T *)foff, (const T *)fscale, skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, pitch, only_above);
+        (const T *)foff, (const T *)fscale, skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, pitch);
   }
 #undef CLT_DEC_TAIL
 #undef CLT_DEC
@@ -1511,19 +1598,47 @@ extern "C" int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, con
   return launch_decode<float>(row_ptr, col, val, w_packed, bias_sum, feat_offset, feat_scale, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, workspace, workspace_bytes, s);
 }
 
+template <typename T>
+static int launch_decode_over(const int32_t *row_ptr, const int32_t *col, const void *val, const void *wp, const float *bias_sum,
+                              const float *skip_add, void *out, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
+                              int64_t t_end, uint64_t src_mask, int out_f32, int64_t only_above, hipStream_t stream) {
+  const int64_t pitch = clt_pitch(d, 2);
+  const int units = (int)(d / 64);
+  // tokens of a workgroup: the workgroups of an XCD share the tokens of one unit
+  const int64_t share = clt_ceil_div(Tn, OVER_BLOCKS / 8 * OVER_WAVES) * OVER_WAVES;
+  const int ntok = share < OVER_TOKENS ? (int)share : OVER_TOKENS;
+  const UnitPlan lp = make_unit_plan(1, units, Tn, ntok);
+  const int64_t blocks = 8 * (int64_t)lp.bpx * (t_end - t_begin);
+  const unsigned grid = (unsigned)(blocks < OVER_BLOCKS ? blocks : OVER_BLOCKS);
+  const int lds = ntok * 64 * (int)sizeof(float);
+  // one 32-bit word per survivor and 32-bit row offsets: feature index below 2^16, matrix below 4 GiB
+  const bool pack = F <= 65536 && F * pitch * 2 < (1ll << 32);
+  const void *k = pack ? (const void *)k_decode_over<T, true> : (const void *)k_decode_over<T, false>;
+  if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return CLT_ERR_LAUNCH;
+#define CLT_OVER(PK)                                                                                                             \
+  k_decode_over<T, PK><<<grid, OVER_WAVES * 64, lds, stream>>>(row_ptr, col, (const T *)val, (const T *)wp, bias_sum, skip_add,  \
+                                                               out, Tn, d, F, L, tying, (int)t_end, src_mask, out_f32, lp, ntok, \
+                                                               pitch, blocks, only_above)
+  if (pack) CLT_OVER(true); else CLT_OVER(false);
+#undef CLT_OVER
+  return clt_check_launch();
+}
+
 extern "C" int clt_decode_sparse_if_over(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
                                          const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d,
                                          int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask,
                                          int dtype, int out_f32, int64_t max_entries, void *stream) {
   if (dtype != CLT_BF16 && dtype != CLT_F16) return CLT_ERR_DTYPE;
-  if (T < 0 || d <= 0 || F <= 0 || L <= 0 || L > 64 || max_entries < 0) return CLT_ERR_ARG;
-  if (t_begin < 0 || t_end > L || t_begin > t_end || tying < 0 || tying > 2) return CLT_ERR_ARG;
+  if (T < 0 || d <= 0 || F <= 0 || L <= 0 || L > 64 || d % 64 != 0 || max_entries < 0) return CLT_ERR_ARG;
+  if (t_begin < 0 || t_end > L || t_begin > t_end) return CLT_ERR_ARG;
+  if (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE) return CLT_ERR_ARG;
   if (T == 0 || t_begin == t_end) return CLT_OK;
   if (!row_ptr || !w_packed || !out) return CLT_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == CLT_BF16)
-    return launch_decode<bf16_t>(row_ptr, col, val, w_packed, bias_sum, nullptr, nullptr, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, s, max_entries);
-  return launch_decode<f16_t>(row_ptr, col, val, w_packed, bias_sum, nullptr, nullptr, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, nullptr, 0, s, max_entries);
+  if (!clt_aligned16(w_packed)) return CLT_ERR_ALIGN;
+  if (T * (d / 64) > 0x7FFFFFFFll) return CLT_ERR_RANGE;       // blocks of a target
+  const auto run = dtype == CLT_BF16 ? launch_decode_over<bf16_t> : launch_decode_over<f16_t>;
+  return run(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, max_entries,
+             (hipStream_t)stream);
 }
 
 extern "C" int clt_pack_decoder(const void *w_ref, void *w_packed, int64_t d, int64_t F, int64_t n_dec,

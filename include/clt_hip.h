@@ -438,7 +438,8 @@ int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const float *val
  *   target layers (0 also for what it does not take).
  *   The workspace is sized for max_entries survivors, of which clt_decode_tiles_max_entries is the largest number that
  *   the records of these shapes can count (more: CLT_ERR_RANGE).  A list that turns out longer on the device
- *   (row_ptr[L*T] > max_entries) is left alone: clt_decode_sparse_if_over decodes such a list and does nothing otherwise.
+ *   (row_ptr[L*T] > max_entries) is left alone: clt_decode_sparse_if_over decodes such a list, in about the time of
+ *   clt_decode_sparse with its workspace, and does nothing otherwise.
  */
 int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
 int64_t clt_decode_tiles_max_entries(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets);

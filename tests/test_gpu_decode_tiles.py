@@ -120,6 +120,120 @@ def test_decode_tiles_leaves_longer_lists_to_the_gather():
     assert torch.allclose(exact, over, rtol=0, atol=60 * 2.0 ** -23 * 60)      # 60 terms below 60 in sum, summed in another order
 
 
+@pytest.mark.parametrize("L,T,F,d,per_token,dtype,tying,heavy", [
+    (1, 1, 8, 64, 3, torch.bfloat16, "none", False),
+    (3, 17, 513, 192, 60, torch.float16, "none", False),
+    (5, 130, 1100, 704, 90, torch.bfloat16, "per_source", True),           # units that are no whole rounds over the XCDs
+    (2, 40, 70000, 64, 900, torch.bfloat16, "none", False),                # indices of more than 16 bits
+    (3, 1900, 1024, 1024, 3, torch.float16, "none", False),                # more blocks than workgroups
+    (64, 3, 600, 64, 4, torch.bfloat16, "per_source", False),
+])
+def test_gather_of_longer_lists(L, T, F, d, per_token, dtype, tying, heavy):
+    """clt_decode_sparse_if_over in place of the tiles that leave such a list alone, against dense products."""
+    dev = torch.device("cuda:0")
+    act, row_ptr, col, val = _lists(L, T, F, per_token, dtype, seed=L + T, heavy=heavy)
+    g = torch.Generator().manual_seed(5)
+    n_dec = L if tying == "per_source" else L * (L + 1) // 2
+    w = (torch.rand(n_dec, F, d, generator=g) - 0.5).to(dtype)
+    bias, skip = torch.randn(L, d, generator=g), torch.randn(L, T, d, generator=g)
+    full, n = (1 << L) - 1, col.numel()
+    for t0, t1, mask, f32, b, k in [(0, L, full, True, None, None), (L // 2, L, full & ~2, False, bias, skip)]:
+        got = _run(dev, act, row_ptr, col, val, w, tying, d, b, k, t0, t1, mask, f32, n - 1, True)
+        for t in range(L):
+            if not t0 <= t < t1:
+                assert (got[t] == 7.0).all()
+                continue
+            ref, mag, cnt = torch.zeros(T, d, dtype=torch.float64), torch.zeros(T, d, dtype=torch.float64), torch.zeros(T, 1)
+            for s in range(t + 1):
+                if mask >> s & 1:
+                    a, m = act[s].double(), w[_slot(tying, s, t, L)].double()
+                    ref, mag, cnt = ref + a @ m, mag + a.abs() @ m.abs(), cnt + (act[s] != 0).sum(1, keepdim=True)
+            for extra in (None if b is None else b[t].double(), None if k is None else k[t].double()):
+                if extra is not None:
+                    ref, mag = ref + extra, mag + extra.abs()
+            # as above; the eight lane groups' sums meet in three more additions
+            bound = (cnt.double() + 6) * 2.0 ** -23 * mag
+            if not f32:
+                bound = bound + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * (ref.abs() + bound) + 2.0 ** -24
+            assert (got[t].double() - ref).abs().le(bound).all(), (t, (got[t].double() - ref).abs().max())
+
+
+def test_a_captured_decode_follows_a_threshold_list_that_outgrows_its_estimate(monkeypatch):
+    """The room is fixed when the graph is captured; replays on thin and dense lists, with eager work between them."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 3, 600, 4096, 128
+    monkeypatch.setattr(nat.load(), "clt_decode_tiles_wanted", lambda *a: 1)
+    lists = {k: _lists(L, T, F, k, torch.bfloat16, seed=k, heavy=False) for k in (10, 100)}
+    assert lists[10][2].numel() < 20000 < 2 * 20000 + 65536 < lists[100][2].numel()
+    cap = lists[100][2].numel() + 1000
+    surv = engine.SurvivorList(torch.zeros(L * T + 1, dtype=torch.int32, device=dev), torch.zeros(cap, dtype=torch.int32, device=dev),
+                               torch.zeros(cap, dtype=torch.bfloat16, device=dev), T, F, L, torch.bfloat16,
+                               torch.zeros(1, dtype=torch.int32, device=dev), 20000)
+    w = engine.alloc_packed(L * (L + 1) // 2, F, d, torch.bfloat16, dev)
+    w[:, :, :d] = torch.randn(L * (L + 1) // 2, F, d, generator=torch.Generator().manual_seed(1)).bfloat16().to(dev)
+    ws = engine.Workspace(dev)
+
+    def fill(k):
+        _, row_ptr, col, val = lists[k]
+        surv.row_ptr.copy_(row_ptr)
+        surv.col[: col.numel()].copy_(col)
+        surv.val[: val.numel()].copy_(val)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fill(10)
+        engine.decode_sparse(surv, w, "none", d, ws=ws)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = engine.decode_sparse(surv, w, "none", d, ws=ws)
+    for k in (100, 10, 100, 100, 10):
+        fill(k)
+        graph.replay()
+        got = out.float()
+        eager = engine.decode_sparse(surv, w, "none", d, ws=ws).float()
+        ref = engine.decode_sparse(surv, w, "none", d, ws=None).float()
+        torch.cuda.synchronize()
+        assert torch.equal(got, eager)
+        # the same sums in another order, rounded to bf16: a last place where that decides
+        assert bool(((got - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-3).all()) and float(ref.norm()) > 0
+
+
+def test_an_outgrown_threshold_list_costs_what_the_gather_costs():
+    """Rows of more than five registers' worth of pieces, for which a single pass over the sources has only the kernel for any
+    shape (28 times the gather's time here); the gather measured beside it, the best of five, allowed a factor of four."""
+    dev = torch.device("cuda:0")
+    L, T, F, d, k = 4, 512, 8192, 2560, 50
+    g = torch.Generator(device=dev).manual_seed(1)
+    rows, n = L * T, L * T * k
+    col = (torch.rand(rows, k, generator=g, device=dev) * (F // k)).int() + torch.arange(k, device=dev, dtype=torch.int32) * (F // k)
+    ptr = torch.arange(0, n + 1, k, dtype=torch.int32, device=dev)
+    val = torch.randn(n, generator=g, device=dev).bfloat16()
+    w = engine.alloc_packed(L * (L + 1) // 2, F, d, torch.bfloat16, dev)
+    w[:, :, :d] = torch.randn(F, d, generator=g, device=dev).bfloat16()
+    ws, lib, stream = engine.Workspace(dev), nat.load(), nat.current_stream(dev)
+    out, over = (torch.empty(L, T, d, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    wbuf = ws.get("decode", lib.clt_decode_workspace_bytes(T, d, F, L))
+    shape = (T, d, F, L, nat.TYING["none"], 0, L, (1 << L) - 1, nat.CLT_BF16, 0)
+    head = (nat.ptr(ptr), nat.ptr(col), nat.ptr(val), nat.ptr(w))
+    calls = {"gather": lambda: lib.clt_decode_sparse(*head, None, None, None, None, nat.ptr(out), *shape, nat.ptr(wbuf), wbuf.numel(), stream),
+             "over": lambda: lib.clt_decode_sparse_if_over(*head, None, None, nat.ptr(over), *shape, n - 1, stream)}
+    ms = {}
+    for name, call in calls.items():
+        best = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            assert call() == 0
+            b.record()
+            torch.cuda.synchronize()
+            best.append(a.elapsed_time(b))
+        ms[name] = min(best[1:])
+    assert float((out.float() - over.float()).norm() / out.float().norm()) < 1e-3      # bf16 results of sums in another order
+    assert ms["over"] <= 4 * ms["gather"], ms
+
+
 def test_decode_tiles_keeps_tokens_apart():
     """Values that are not finite stay with their token although sixteen tokens share every product."""
     dev = torch.device("cuda:0")
