@@ -199,8 +199,14 @@ constexpr int SLICED_NTOK = 4;   // tokens per wavefront in the sliced kernel
 // latency, so 16 survivors are asked for at once, and every row has a workgroup, and so an L1, to itself.
 // L = 3, d = 768, float32, 32 tokens x 16 survivors: 33.6 -> 19.9 us; a forward waited for 176 -> 165 us, L = 2, d = 512, 500
 // tokens 304 -> 291 us.  Above the line a SIMD has several rows to switch between, and 16 in flight cost wavefronts; rows of
-// more than four registers' worth of pieces (NF = 4) would need 320 registers for them.
+// more than four registers' worth of pieces (NF = 4) would need 320 registers for them.  In bf16 three pieces and a half one
+// (d = 1792) are kept to 8 in flight: at 16 they need 19 registers more than there are, and every survivor pays for moving
+// them.  L = 4, 32 tokens x 100, us, launch of many rows / this: d = 1536 bf16 70 / 46, fp16 88 / 45; d = 1792 bf16 75 / 58 (143
+// at 16), fp16 91 / 49; d = 2000 78 / 61; d = 896 float32 80 / 50.
 constexpr int DECODE_FEW = 1024, DECODE_FEW_U = 16;
+template <typename T, int NF, int TAIL> constexpr int decode_few_in_flight() {
+  return std::is_same<T, bf16_t>::value && NF == 3 && TAIL == 1 ? 8 : DECODE_FEW_U;
+}
 
 // One wavefront per (target, token): walks all sources s <= t, accumulates in registers,
 // writes the output row once.  Used for small batches.
@@ -1448,7 +1454,7 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
     else if (can_slice)                                                                                         \
       k_decode<T, NFN, TL, UN, false, true><<<(unsigned)nblk, 256, 0, stream>>>(CLT_DEC_ARGS(nullptr, nullptr)); \
     else if (few && NFN < 4)                                                                                    \
-      k_decode<T, NFN, TL, DECODE_FEW_U, false, false><<<(unsigned)(Tn * (t_end - t_begin)), 64, 0, stream>>>(CLT_DEC_ARGS(nullptr, nullptr)); \
+      k_decode<T, NFN, TL, decode_few_in_flight<T, NFN, TL>(), false, false><<<(unsigned)(Tn * (t_end - t_begin)), 64, 0, stream>>>(CLT_DEC_ARGS(nullptr, nullptr)); \
     else                                                                                                        \
       k_decode<T, NFN, TL, UN, false, false><<<(unsigned)nblk, 256, 0, stream>>>(CLT_DEC_ARGS(nullptr, nullptr)); \
   } while (0)
