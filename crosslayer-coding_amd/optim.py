@@ -24,7 +24,10 @@ class CLTAdam:
         self.lr, self.betas, self.eps = float(lr), (float(betas[0]), float(betas[1])), float(eps)
         self.step_count = 0
         self.fuse_decoder_step = True    # untied decoders: Adam inside the weight-gradient kernel (training_step)
-        self.tile_decoder_step = True    # ... over column tiles, when the shape allows (moments and a weight copy tiled)
+        # ... over column tiles, when the shape allows: float32 and widths that are not whole tiles of 64 take that kernel
+        # (moments and a weight copy tiled) or go row by row; for bf16 in whole tiles of 64 columns, which the matrix-core
+        # kernel takes either way, only what the moments are laid out as
+        self.tile_decoder_step = True
         # the in-kernel decoder step rewrites the feature-major slab only; the checkpoint-layout parameters follow
         # when something reads them (Decoder.sync_parameters).  False: rewrite them in every step
         self.defer_parameter_sync = True
@@ -123,10 +126,10 @@ class CLTAdam:
         w_dev, w_host = self._pointer_table("w", ws)
         cs = engine.decoder_tile_width(surv.T, d, F, ws[0].dtype) if self.tile_decoder_step else 0
         if engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype):
-            if cs:
-                self._decoder_moments_to("tiles", 64)
-            else:
-                self._decoder_moments_to("rows")
+            # (the kernel takes moments as rows and as tiles of 64 columns: once they are the latter they stay, whatever
+            # batch length comes next)
+            if self._dec_cols != 64:
+                self._decoder_moments_to(*(("tiles", 64) if cs else ("rows",)))
             self._w_tiles_gen = None      # the slab changes under the tiled copy
             engine.decoder_grad_adam_tiles(lists, surv, g_model, packed, *self.state["dec_w"], self.lr, self.betas, self.eps,
                                            self.step_count + 1, ws=self.model._workspace())

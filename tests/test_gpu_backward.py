@@ -348,6 +348,22 @@ def test_optimiser_moves_between_the_tiled_and_the_row_route(dev):
     _assert_same_training((None, runs[0][0], None, runs[0][1]), (None, runs[1][0], None, runs[1][1]), torch.bfloat16, 4)
 
 
+def test_batch_lengths_in_turn_leave_the_moments_where_they_are(dev):
+    # bf16 in whole tiles of 64 columns: the kernel is the same on either side of the batch length up to which the 32-byte
+    # tiles would fit LDS, so the moments (at full size several GB) are regrouped once and not at every change of length
+    import crosslayer_coding_amd as cca
+    wl = BASE.scaled("bw-lengths", num_layers=2, d_model=128, num_features=256, tokens=4500, dtype="bfloat16", k=10)
+    model, sd, x, targets = build(wl, dev)
+    opt = cca.CLTAdam(model, lr=1e-3)
+    assert engine.decoder_tile_width(4500, 128, 256, torch.bfloat16) == 0 < engine.decoder_tile_width(300, 128, 256, torch.bfloat16)
+    places = []
+    for T in (4500, 300, 4500, 300, 4500):
+        model.training_step({l: x[l][:T].to(dev) for l in range(2)}, {l: t[:T].to(dev) for l, t in targets.items()}, opt)
+        places.append(tuple(t.data_ptr() for t in opt.state["dec_w"]))
+    assert len(set(places[1:])) == 1
+    assert all(tuple(t.shape) == (3, 256, 128) for t in opt.decoder_moments())
+
+
 @pytest.mark.parametrize("tiled", [True, False], ids=["tile-route", "row-route"])
 def test_parameters_left_behind_by_the_decoder_step_are_current_whenever_they_are_read(dev, tiled):
     # The in-kernel decoder step rewrites the feature-major slab only; the checkpoint-layout parameters [d, F]
