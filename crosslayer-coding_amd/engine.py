@@ -138,6 +138,11 @@ def _stream(t: torch.Tensor) -> int:
     return nat.current_stream(t.device)
 
 
+def _aligned16(*tensors: Optional[torch.Tensor]) -> bool:
+    """What the kernels that work from LDS tiles ask of their operands; the gathers take any address."""
+    return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def encode(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor],
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """pre[l] = x[l] @ w[l].T + b[l] for stacked layers (parallel.py:286 per layer)."""
@@ -660,7 +665,8 @@ def decoder_weight_grad(lists, surv: SurvivorList, g: torch.Tensor, tying: str,
     n_dec = L * (L + 1) // 2 if tying == "none" else L
     out = torch.empty((n_dec, F, d), dtype=torch.float32, device=g.device)
     n = surv.capacity
-    if tying == "none" and feat_offset is None and feat_scale is None and grad_tiles_supported(T, d, F, L, n, surv.dtype):
+    if (tying == "none" and feat_offset is None and feat_scale is None and _aligned16(g)
+            and grad_tiles_supported(T, d, F, L, n, surv.dtype)):
         lib = nat.load()
         wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_tiles_workspace_bytes(T, d, F, L, n))
         code = lib.clt_decoder_grad_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(out), T, d,
@@ -931,7 +937,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
     need = lib.clt_decoder_slab_elems(d, F, L, nat.TYING[tying], nat.dtype_code(surv.dtype))
     if need < 0 or w_packed.numel() < need:
         raise nat.CLTNativeError(f"decode_sparse: packed decoders hold {w_packed.numel()} elements, the kernels index {need}")
-    if ws is not None and tying != "per_target" and feat_offset is None and feat_scale is None:
+    if (ws is not None and tying != "per_target" and feat_offset is None and feat_scale is None
+            and _aligned16(w_packed, bias_sum, skip_add, out)):
         # the survivor total: exact, or (a threshold list, sized for any batch) the last one seen for this shape, or 1 %
         # of the features before there is one
         exact = surv.status is None

@@ -125,7 +125,8 @@ class CLTAdam:
         d, F = ws[0].shape
         w_dev, w_host = self._pointer_table("w", ws)
         cs = engine.decoder_tile_width(surv.T, d, F, ws[0].dtype) if self.tile_decoder_step else 0
-        if engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype):
+        if (engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype)
+                and engine._aligned16(g_model, packed, *self.state["dec_w"])):
             # (the kernel takes moments as rows and as tiles of 64 columns: once they are the latter they stay, whatever
             # batch length comes next)
             if self._dec_cols != 64:
