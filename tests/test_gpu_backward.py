@@ -204,8 +204,9 @@ def _assert_same_training(a, b, dtype, steps):
     ("bfloat16", 128, "batchtopk", 1501)])  # two features fire on nearly every token: lists cut over many lanes
 def test_adam_inside_the_weight_gradient_kernel_equals_the_two_step_sequence(dev, dtype, d_model, fn, tokens):
     # untied decoders: training_step lets the decoder weights take their Adam step inside the weight-gradient
-    # kernel (no fp32 gradient in memory, parameters rewritten from the working copy), over column tiles where
-    # the shape allows and row by row otherwise; three steps must leave every parameter, the packed copy and
+    # kernel (no fp32 gradient in memory, parameters rewritten from the working copy): bf16 in whole tiles of 64 columns
+    # on the matrix cores (the two-step sequence takes its gradient from there too), the rest over tiles of 32 bytes
+    # where the shape allows and row by row otherwise; three steps must leave every parameter, the packed copy and
     # both moments bit-identical to gradient-then-Adam
     import crosslayer_coding_amd as cca
     wl = BASE.scaled("bw-fuse", num_layers=3, d_model=d_model, num_features=256, tokens=tokens, dtype=dtype,
@@ -324,12 +325,26 @@ def test_tiled_decoder_step_kernel_against_the_row_kernel(dev, dtype, T, F):
     assert float((y - w.float()).abs().max()) > 0          # and the step did move the weights
 
 
-def test_optimiser_moves_between_the_tiled_and_the_row_route(dev):
-    # one optimiser, steps taken in turn through the tiled kernel, the row kernel and gradient-then-Adam: the
-    # moments change layout under way and the tiled weight copy is rebuilt when the slab changed behind it;
-    # the result must be the one of three plain steps
+def _record_decoder_steps(monkeypatch):
+    """Which entry point every decoder step went to: "matrix", "tiles", "rows", or "gradient" for gradient-then-Adam."""
+    took = []
+    for name, what in (("decoder_grad_adam_tiles", "matrix"), ("decoder_weight_grad_adam_tiled", "tiles"),
+                       ("decoder_weight_grad_adam", "rows"), ("decoder_weight_grad", "gradient")):
+        def call(*a, _fn=getattr(engine, name), _what=what, **kw):
+            took.append(_what)
+            return _fn(*a, **kw)
+        monkeypatch.setattr(engine, name, call)
+    return took
+
+
+@pytest.mark.parametrize("dtype,d,route", [("bfloat16", 128, "matrix"), ("bfloat16", 80, "tiles"), ("float32", 64, "tiles")])
+def test_optimiser_moves_between_the_tiled_and_the_row_route(dev, monkeypatch, dtype, d, route):
+    # one optimiser, steps taken in turn through the tiled kernel, the row kernel and gradient-then-Adam (bf16 in whole tiles
+    # of 64 columns: the matrix-core kernel in the place of the first two): the moments change layout under way and the tiled
+    # weight copy is rebuilt when the slab changed behind it; the result must be the one of three plain steps
     import crosslayer_coding_amd as cca
-    wl = BASE.scaled("bw-mixed", num_layers=3, d_model=128, num_features=256, tokens=256, dtype="bfloat16", k=10)
+    wl = BASE.scaled("bw-mixed", num_layers=3, d_model=d, num_features=256, tokens=256, dtype=dtype, k=10)
+    took = _record_decoder_steps(monkeypatch)
     runs = []
     for mixed in (True, False):
         model, sd, x, targets = build(wl, dev)
@@ -345,7 +360,31 @@ def test_optimiser_moves_between_the_tiled_and_the_row_route(dev):
             model.training_step(inputs, tg, opt)
         runs.append(({k: v.detach().clone() for k, v in model.state_dict().items()},
                      [t.clone() for t in opt.decoder_moments()]))
-    _assert_same_training((None, runs[0][0], None, runs[0][1]), (None, runs[1][0], None, runs[1][1]), torch.bfloat16, 4)
+    assert took == [route, "matrix" if route == "matrix" else "rows", "gradient", route] + 4 * ["gradient"]
+    _assert_same_training((None, runs[0][0], None, runs[0][1]), (None, runs[1][0], None, runs[1][1]), getattr(torch, dtype), 4)
+
+
+def test_optimiser_moves_between_the_matrix_core_kernel_and_the_other_two(dev, monkeypatch):
+    # the same with one optimiser whose steps go to all three kernels: moments as tiles of 64 columns, as tiles of 32 bytes and
+    # as rows, and the tiled weight copy rebuilt after the matrix-core kernel has stepped the slab behind it
+    import crosslayer_coding_amd as cca
+    wl = BASE.scaled("bw-three", num_layers=3, d_model=128, num_features=256, tokens=256, dtype="bfloat16", k=10)
+    took, supported = _record_decoder_steps(monkeypatch), engine.grad_tiles_supported
+    plan, runs = ["tiles", "matrix", "tiles", "rows", "matrix", "gradient", "tiles"], []
+    for mixed in (True, False):
+        model, sd, x, targets = build(wl, dev)
+        opt = cca.CLTAdam(model, lr=1e-2)
+        inputs = {l: x[l].to(dev) for l in range(3)}
+        tg = {l: t.to(dev) for l, t in targets.items()}
+        for what in plan:
+            want = what if mixed else "gradient"
+            monkeypatch.setattr(engine, "grad_tiles_supported", supported if want in ("matrix", "gradient") else lambda *a: False)
+            opt.fuse_decoder_step, opt.tile_decoder_step = want != "gradient", want != "rows"
+            model.training_step(inputs, tg, opt)
+        runs.append(({k: v.detach().clone() for k, v in model.state_dict().items()},
+                     [t.clone() for t in opt.decoder_moments()]))
+    assert took == plan + ["gradient"] * len(plan)
+    _assert_same_training((None, runs[0][0], None, runs[0][1]), (None, runs[1][0], None, runs[1][1]), torch.bfloat16, len(plan))
 
 
 def test_batch_lengths_in_turn_leave_the_moments_where_they_are(dev):
@@ -364,14 +403,16 @@ def test_batch_lengths_in_turn_leave_the_moments_where_they_are(dev):
     assert all(tuple(t.shape) == (3, 256, 128) for t in opt.decoder_moments())
 
 
+@pytest.mark.parametrize("dtype,d", [("bfloat16", 128), ("bfloat16", 80), ("float32", 64)])
 @pytest.mark.parametrize("tiled", [True, False], ids=["tile-route", "row-route"])
-def test_parameters_left_behind_by_the_decoder_step_are_current_whenever_they_are_read(dev, tiled):
+def test_parameters_left_behind_by_the_decoder_step_are_current_whenever_they_are_read(dev, monkeypatch, tiled, dtype, d):
     # The in-kernel decoder step rewrites the feature-major slab only; the checkpoint-layout parameters [d, F]
     # follow when something reads them.  Against an optimiser that rewrites them in every step
     # (trainer.py:751-778: the reference's parameters are always current): state_dict(), named_parameters(),
     # decoders[key] and the forward must all see the same bits.
     import crosslayer_coding_amd as cca
-    wl = BASE.scaled("bw-lazy", num_layers=3, d_model=128, num_features=256, tokens=256, dtype="bfloat16", k=10)
+    wl = BASE.scaled("bw-lazy", num_layers=3, d_model=d, num_features=256, tokens=256, dtype=dtype, k=10)
+    took = _record_decoder_steps(monkeypatch)
     models, opts = [], []
     for defer in (True, False):
         model, sd, x, targets = build(wl, dev)
@@ -409,6 +450,7 @@ def test_parameters_left_behind_by_the_decoder_step_are_current_whenever_they_ar
     assert not lazy.decoder_module._params_behind
     a, b = lazy(inputs), eager(inputs)
     assert all(torch.equal(a[t], b[t]) for t in a)
+    assert set(took) == {"matrix" if (dtype, d) == ("bfloat16", 128) else "tiles" if tiled else "rows"}
 
 
 def test_tied_decoders_do_not_fuse_the_step(dev):
