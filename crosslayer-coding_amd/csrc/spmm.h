@@ -7,8 +7,8 @@
 // The gathered operand comes out of LDS through the transposing read, which takes an address per lane.
 //
 // Why: a gather through the vector memory path is bound by the L1's outstanding lines (15 TB/s at best on this part);
-// LDS hands out randomly chosen 32-byte pieces at 58 TB/s (2.26 ns per 512-byte transposing read and CU with random
-// rows, 2.04 ns without any bank conflict).  Fifteen sixteenths of the matrix instruction's products are with zeros,
+// LDS hands out randomly chosen 32-byte pieces at 59 TB/s (2.21 ns per 512-byte transposing read and CU with random
+// rows, 1.62 ns without any bank conflict; profiles/lds_read_probe.txt).  Fifteen sixteenths of the matrix instruction's products are with zeros,
 // which still leaves as many useful ones per cycle as the vector unit's dot products deliver, without their
 // unpacking; and lists of unequal length cost nothing, because a batch is filled from any of 16 output rows.
 #pragma once

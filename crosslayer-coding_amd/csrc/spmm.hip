@@ -244,13 +244,15 @@ __device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_o
 // Two tiles of 512 features x 64 columns in LDS, one being multiplied while the other comes in.  Each wavefront owns four
 // groups of 16 tokens and consumes its stream of batches through a ring of eight records in LDS: the vector memory path
 // returns in order, so a record waits behind whatever tile lines were asked for before it, and eight batches (~2 us)
-// cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so a tile
-// comes from HBM once.
+// cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so that one of
+// them brings it from HBM and the others find it in the L2.
 //
-// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.16 ms (98.6 GB of gathered rows, 31
-// TB/s) and 0.14 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 16.3 against
-// 34.2 ms.  Bound by LDS: 19 ns per batch and CU are 2.2 ms, of which 0.5 for the entries that fill batches up; 0.25 ms
-// are wavefronts waiting for the slowest one of a stage, 0.3 ms records queueing behind tile lines that come from HBM.
+// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.35 ms (98.6 GB of gathered rows, 29
+// TB/s) and 0.26 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.8 and 0.55
+// against 34.2 ms (profiles/forward_c1_kernel_trace.txt, forward_c2_kernel_trace.txt).  Bound by LDS, which is busy in 72 % of
+// the cycles: 21 ns per batch and CU are 2.4 ms, of which 19 % for the entries that fill batches up
+// (profiles/decode_tiles_c1_lds_counters.txt); in the rest wavefronts wait for the slowest one of a stage and records queue
+// behind tile lines that come from HBM (7.9 GB a launch, 2.9 of them weights).
 // Measured and dropped: a wavefront of its own for the fills (fifteen share 64 groups badly: 3.98 ms); fewer lines on
 // their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought into the L2 early
 // (3.46 ms: the early loads block the records just as well).

@@ -455,7 +455,10 @@ class Decoder(nn.Module):
         thresholds at the start of a training run, a very large k): every active (token, feature) of a source
         fetches a decoder row per target, k T rows of d elements, while the reference's dense product
         ``a[s] @ W[s->t].T`` (decoder.py:253-316) costs 2 T F d whatever the density.  With the measured rates of
-        ``route_rates`` the product wins above roughly 1.5 - 2 % of the features active per token."""
+        ``route_rates``, which are those of the gather from the L2s, the product is taken from roughly 2 - 3 % of the features
+        active per token on.  The decode from LDS tiles is not priced here: at L = 12, d = 768, F = 24576, 4096 tokens, bf16 a
+        forward on the lists takes 13.0 / 16.1 / 23.2 ms at 3 / 4 / 6 % and on the products 18.9 / 19.2 / 20.5, so between
+        there and 4.8 % the lists would be the faster route."""
         if self.config.num_layers > self.MAX_GATHER_LAYERS:
             return self.dense_pairs_wanted_for(0.0, surv.T, surv.dtype, skip_add, any_tying)
         if surv.nnz_hint is None and surv.status is not None:
