@@ -816,7 +816,7 @@ def main():
                     help="also run one 256 MiB elementwise copy (counter yardstick for profiled runs)")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py measures the one-GPU forward path; this build has no multi-GPU path "
+        print("bench.py measures the one-GPU forward path; this package has no multi-GPU path "
               f"(asked for --gpus {args.gpus})", file=sys.stderr)
         sys.exit(2)
     if not torch.cuda.is_available():

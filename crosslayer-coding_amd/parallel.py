@@ -45,7 +45,7 @@ def _world_size(process_group) -> int:
 def require_single_rank(process_group) -> None:
     if _world_size(process_group) != 1:
         raise NotImplementedError(
-            "this build implements the CLT forward path on one GPU (world_size 1); "
+            "this package implements the CLT forward path on one GPU (world_size 1); "
             "feature sharding over a process group is not part of it")
 
 

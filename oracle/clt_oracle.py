@@ -4,7 +4,7 @@ TEST INFRASTRUCTURE ONLY.  This module restates, with plain torch-CPU / numpy
 operations, the algorithm the reference runs on its forward path.  It exists so
 that the HIP kernels can be checked against it; nothing that ships (the package,
 its C-ABI library) may import or call it.  Only ``tests/``, the smoke check and
-the ``cpu_baseline`` leg of the benchmark use it, and there only as the checker
+the ``cpu_baseline`` leg of the benchmark use it, and there only to check against
 or as the timed CPU baseline.
 
 Every function cites the reference lines it follows (paths relative to the
@@ -132,7 +132,7 @@ def batchtopk_mask_topk(x: torch.Tensor, k_per_token: int,
                         x_for_ranking: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The same mask through the reference's own op sequence - torch.topk(sorted=False)
     then an index write (activations.py:21-32).  Ties fall wherever torch.topk puts them,
-    so this variant is used for the timed CPU baseline only, never as the parity checker."""
+    so this variant is used for the timed CPU baseline only, never for parity."""
     B = x.size(0)
     if k_per_token <= 0 or x.numel() == 0:
         return torch.zeros_like(x, dtype=torch.bool)
