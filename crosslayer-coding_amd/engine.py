@@ -14,7 +14,7 @@ Layouts
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Dict, Optional
+from typing import Dict, List, Optional
 
 import torch
 
@@ -79,31 +79,50 @@ def poison_if(buf: torch.Tensor, flag: torch.Tensor) -> None:
     nat.check(code, "clt_poison_if")
 
 
+def _capturing(device: torch.device) -> bool:
+    return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 class Workspace:
-    """Grow-only device buffers reused across calls on one stream."""
+    """Grow-only device buffers reused across calls on one stream.
+
+    A buffer handed out under a stream capture is written by every replay of that graph, whatever the eager calls
+    between them ask for: outgrown, it is put aside instead of freed (a batch denser than the captured one outgrows
+    the room of a threshold list at the same shape)."""
 
     def __init__(self, device: torch.device):
         self.device = device
         self._bufs: Dict[str, torch.Tensor] = {}
+        self._captured: set = set()             # names of buffers that a captured graph refers to
+        self._outgrown: List[torch.Tensor] = []
 
     def get(self, name: str, nbytes: int) -> torch.Tensor:
         buf = self._bufs.get(name)
         if buf is None or buf.numel() < nbytes:
-            self._bufs.pop(name, None)
+            old = self._bufs.pop(name, None)
+            if name in self._captured:
+                self._captured.discard(name)
+                self._outgrown.append(old)
+            del old
             buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=self.device)
             self._bufs[name] = buf
+        if _capturing(self.device):
+            self._captured.add(name)
         return buf
 
     def typed(self, name: str, shape, dtype: torch.dtype) -> torch.Tensor:
         n = 1
         for s in shape:
             n *= int(s)
-        item = torch.empty((), dtype=dtype).element_size()
-        buf = self.get(name, n * item)
-        return buf[: n * item].view(dtype).view(*shape)
+        nbytes = n * dtype.itemsize
+        buf = self.get(name, nbytes)
+        return buf[: nbytes].view(dtype).view(*shape)
 
     def release(self) -> None:
+        """Gives everything back; graphs captured with these buffers must not be replayed any more."""
         self._bufs.clear()
+        self._captured.clear()
+        self._outgrown.clear()
 
 
 # below this many (token, target) rows one wavefront per row already underfills the GPU

@@ -1,5 +1,7 @@
 """Which decode a survivor list is handed to, checked without a GPU: tensors without storage, native launches recorded in place
 of made."""
+import weakref
+
 import pytest
 import torch
 
@@ -75,3 +77,21 @@ def test_max_entries_is_the_largest_that_is_taken(recorder):
         assert recorder._lib.clt_decode_tiles(*args, n, 4096, 0, None) == -3            # CLT_ERR_WORKSPACE
         assert recorder._lib.clt_decode_tiles(*args, n + 1, 4096, 0, None) == -6        # CLT_ERR_RANGE
     assert recorder.clt_decode_tiles_max_entries(4096, 768, 513 * 512, 12, 12) == 0     # more tiles than the kernels take
+
+
+def test_a_buffer_that_a_captured_graph_writes_outlives_its_successor(monkeypatch):
+    """A denser batch of the captured shape outgrows the room of a threshold list; the graph's replays go on writing the old one."""
+    ws = engine.Workspace(torch.device("cpu"))
+    capturing = False
+    monkeypatch.setattr(engine, "_capturing", lambda device: capturing, raising=False)
+    alive = []
+    for grown_by, held in ((1, 0), (2, 1), (3, 1)):      # before a capture, right after one, once more
+        capturing = grown_by == 2
+        old = ws.get("list", 1000 * grown_by)
+        capturing = False
+        alive.append(weakref.ref(old))
+        del old
+        ws.get("list", 1000 * (grown_by + 1))
+        assert sum(r() is not None for r in alive) == held
+    ws.release()
+    assert all(r() is None for r in alive)

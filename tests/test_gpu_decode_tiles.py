@@ -200,6 +200,35 @@ def test_a_captured_decode_follows_a_threshold_list_that_outgrows_its_estimate(m
         assert bool(((got - ref).abs() <= 2.0 ** -7 * ref.abs() + 1e-3).all()) and float(ref.norm()) > 0
 
 
+def test_a_denser_eager_batch_leaves_the_captured_graph_its_room(monkeypatch):
+    """The room of a threshold list follows the last total seen, so an eager batch of the captured shape can outgrow the buffer
+    that the graph writes: memory allocated afterwards must not be that buffer's."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 3, 600, 4096, 128
+    monkeypatch.setattr(nat.load(), "clt_decode_tiles_wanted", lambda *a: 1)
+    _, row_ptr, col, val = _lists(L, T, F, 10, torch.bfloat16, seed=3, heavy=False)
+    surv = engine.SurvivorList(row_ptr.to(dev), col.to(dev), val.to(dev), T, F, L, torch.bfloat16,
+                               torch.zeros(1, dtype=torch.int32, device=dev), 20000)
+    w = engine.alloc_packed(L * (L + 1) // 2, F, d, torch.bfloat16, dev)
+    w[:, :, :d] = torch.randn(L * (L + 1) // 2, F, d, generator=torch.Generator().manual_seed(1)).bfloat16().to(dev)
+    ws = engine.Workspace(dev)
+    monkeypatch.setattr(engine.SurvivorList, "capacity", 1 << 30)      # arrays for any list the shape can produce
+    want = engine.decode_sparse(surv, w, "none", d, ws=ws)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = engine.decode_sparse(surv, w, "none", d, ws=ws)
+    room = ws.get("decode_tiles", 0).numel()
+    surv.nnz_hint = 200000
+    assert torch.equal(engine.decode_sparse(surv, w, "none", d, ws=ws), want)
+    assert ws.get("decode_tiles", 0).numel() > room
+    later = [torch.full((room,), 7, dtype=torch.uint8, device=dev) for _ in range(4)]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and all(bool((t == 7).all()) for t in later)
+
+
 def test_an_outgrown_threshold_list_costs_what_the_gather_costs():
     """Rows of more than five registers' worth of pieces, for which a single pass over the sources has only the kernel for any
     shape (28 times the gather's time here); the gather measured beside it, the best of five, allowed a factor of four."""
