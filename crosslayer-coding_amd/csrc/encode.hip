@@ -3,8 +3,8 @@
 // MFMA kernel for gfx950.  Both operands are K-contiguous (x is [T][d], W is [F][d]), so
 // one loader serves both.
 //
-//   block tile  256 tokens x 256 features, 4 wavefronts (2 x 2), wave tile 128 x 128:
-//               256 fp32 accumulators per lane, one wavefront per SIMD, one block per CU
+//   block tile  256 tokens x 256 features, 8 wavefronts (4 x 2), wave tile 64 x 128:
+//               128 fp32 accumulators per lane, two wavefronts per SIMD, one block per CU
 //   k step      128 bytes of K per LDS stage (64 bf16 / 32 fp32), two stages of 64 KB
 //   loads       global_load_lds_dwordx4: 16 bytes per lane straight into LDS, no staging
 //               registers.  LDS rows are 128 bytes; chunk c of row r lives at chunk position
@@ -16,8 +16,8 @@
 //   bias        the accumulators start from the bias, so it is added in fp32 before the one rounding
 //   epilogue    rounding, then the tile goes through LDS so that the stores are 16 bytes per lane
 //               and 256 contiguous bytes per token
-//   bf16        v_mfma_f32_32x32x16_bf16, fp32 accumulate, one rounding (v_cvt_pk_bf16_f32)
-//   fp32        v_mfma_f32_32x32x2_f32
+//   bf16        v_mfma_f32_16x16x32_bf16, fp32 accumulate, one rounding (v_cvt_pk_bf16_f32)
+//   fp32        v_mfma_f32_16x16x4_f32
 #include <type_traits>
 #include "select_state.h"
 
@@ -25,6 +25,7 @@ namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 constexpr int BM = 256;   // tokens per block
 constexpr int BN = 256;   // features per block
@@ -60,10 +61,46 @@ template <> struct Mma<float> {
   }
 };
 
-// 16 bytes per lane from global memory straight into LDS: lane i of the wavefront lands at
-// lds_base + 16 * i (lds_base must be wave-uniform).
-__device__ __forceinline__ void load16_to_lds(const void *gsrc, void *lds_base) {
-  __builtin_amdgcn_global_load_lds(gsrc, (__attribute__((address_space(3))) void *)lds_base, 16, 0, 0);
+// element j of a 16-byte slot as a float
+template <typename T> __device__ __forceinline__ float slot_elem(const uint4 &w, int j);
+template <> __device__ __forceinline__ float slot_elem<float>(const uint4 &w, int j) {
+  return __uint_as_float(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w);
+}
+
+// The same on 16 x 16 tiles, 64 bytes of K per row: what the 256 x 256 tiles are made of.  Under full load the part is held by
+// its power limit, and this shape moves its accumulators half as often per product: a loop of nothing but matrix
+// instructions on random bf16 operands runs at 2065 TFLOP/s with it and at 1795 with 32 x 32 x 16.
+template <typename T> struct Mma16;
+template <> struct Mma16<bf16_t> {
+  static constexpr int PARTS = 1;
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
+  }
+};
+template <> struct Mma16<f16_t> {
+  static constexpr int PARTS = 1;
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), acc, 0, 0, 0);
+  }
+};
+template <> struct Mma16<float> {
+  static constexpr int PARTS = 4;        // one instruction per element of the fragments
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int part) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(slot_elem<float>(a, part), slot_elem<float>(b, part), acc, 0, 0, 0);
+  }
+};
+
+// 16 or 4 bytes per lane from base + off (bytes) straight into LDS: lane i of the wavefront lands at lds_at + 16 i or 4 i
+// (lds_at wave-uniform).  As statements the compiler does not count: it cannot tell which of the loads on their way an
+// LDS read depends on and would wait for all of them in front of every fragment read.  The waits are written out by hand.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
+}
+__device__ __forceinline__ void fill16(const void *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"((const char *)base + off), "s"(lds_at) : "memory");
+}
+__device__ __forceinline__ void fill4(const void *base, uint32_t off, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"((const char *)base + off), "s"(lds_at) : "memory");
 }
 
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
@@ -77,11 +114,7 @@ template <typename T> __device__ __forceinline__ uint32_t pack16x2(float a, floa
   else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
-// element j of a 16-byte slot as a float / as raw bits
-template <typename T> __device__ __forceinline__ float slot_elem(const uint4 &w, int j);
-template <> __device__ __forceinline__ float slot_elem<float>(const uint4 &w, int j) {
-  return __uint_as_float(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w);
-}
+// the same of the 16-bit types
 template <> __device__ __forceinline__ float slot_elem<bf16_t>(const uint4 &w, int j) {
   const uint32_t u = (j >> 1) == 0 ? w.x : (j >> 1) == 1 ? w.y : (j >> 1) == 2 ? w.z : w.w;
   return __uint_as_float((j & 1) ? (u & 0xFFFF0000u) : (u << 16));
@@ -90,6 +123,7 @@ template <> __device__ __forceinline__ float slot_elem<f16_t>(const uint4 &w, in
   const uint32_t u = (j >> 1) == 0 ? w.x : (j >> 1) == 1 ? w.y : (j >> 1) == 2 ? w.z : w.w;
   return f16_bits_to_f32((j & 1) ? (u >> 16) : (u & 0xFFFFu));
 }
+// element j as raw bits
 template <typename T> __device__ __forceinline__ uint32_t slot_raw(const uint4 &w, int j);
 template <> __device__ __forceinline__ uint32_t slot_raw<float>(const uint4 &w, int j) {
   return j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w;
@@ -164,16 +198,22 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   // Persistent workgroups (the grid is one block per CU, block b takes the tiles b, b + gridDim.x, ...)
   // that overlap the start of the next tile with the end of this one: the epilogue parks only in the
   // second stage buffer, 32 tokens of a wave tile at a time, so the first stage of the next tile is asked
-  // for two stages before this tile's K loop ends and has landed when the epilogue is over.
-  // Two separate stage buffers (not one array with an offset): the compiler can then tell that
-  // a fragment read of one stage does not depend on the direct-to-LDS loads in flight into the
-  // other, and does not wait for them.
+  // for during the last two stages of this one.
+  //
+  // What bounds it: the power limit (1.7 - 1.9 GHz under load) and, at K of a few hundred, the epilogue and the turn of the
+  // tiles, which the matrix cores wait out.  Against 32 x 32 x 16 products with all loads of a stage asked for at one barrier
+  // (one stage to arrive) and a wait for the epilogue's stores at the turn, ms, bf16:
+  //   L 12, T 4096, d 768, F 24576   1.84 -> 1.66 (1117 TFLOP/s)      L 4, T 8192, d 2048, F 16384   1.82 -> 1.65 (1330)
+  //   T 8192, d 16384, F 2048        0.453 -> 0.388 (1420)            T = d = F = 8192               0.852 -> 0.768 (1430)
+  // The vendor library takes 0.377 and 0.67 ms for the d 16384 and the 8192 product.  float32 (L 12, T 1024, d 768, F 6144):
+  // 0.915 ms both.  Measured and dropped: the two wavefronts of a SIMD taking turns at multiplying and reading (1.95
+  // ms at the first shape: with 64 KB per stage also coming into LDS, the reads of a turn outlast the other's products).
   __shared__ __attribute__((aligned(16))) unsigned char stage0[STAGE];
   __shared__ __attribute__((aligned(16))) unsigned char stage1[STAGE];
   __shared__ uint16_t cand_list[COLLECT ? NWAVES : 1][COLLECT ? CAND_LIST : 1];   // per wavefront, see the emission
   __shared__ __attribute__((aligned(16))) T bias_lds[NWAVES][128];                // per wavefront: the bias of its features
-  __shared__ __attribute__((aligned(16))) T theta_lds[COLLECT == 2 ? NWAVES : 1][COLLECT == 2 ? 128 : 8];   // and their thresholds
-  __shared__ __attribute__((aligned(16))) uint32_t cut_lds[COLLECT == 1 ? NWAVES : 1][4];                   // the layer's cut key
+  __shared__ __attribute__((aligned(16))) T theta_lds[2][COLLECT == 2 ? NWAVES : 1][COLLECT == 2 ? 128 : 8];   // and their thresholds, this tile's and the next one's
+  __shared__ __attribute__((aligned(16))) uint32_t cut_lds[2][COLLECT == 1 ? NWAVES : 1][4];                // the layer's cut key, likewise
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -241,17 +281,19 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   while (bid < total_tiles && !wanted(bid)) bid += gridDim.x;
   if (bid >= total_tiles) return;
 
-  // ---- loader: wave `wave` brings in rows [32*wave, 32*wave+32) of both tiles, 8 rows (1 KB)
-  // per instruction.  Lane l lands at row l>>3, chunk position l&7 of its 8-row group and
-  // therefore fetches global chunk (l&7) ^ ((row >> 1) & 7).
+  // ---- loader.  Per stage a wavefront brings in four 8-row groups of the x tile (rows 32 * wave + 8 t) and one of each
+  // quarter j of the W tile (rows 128 * (wave / 4) + 32 j + 8 * (wave % 4)), 1 KB per instruction.  Lane l lands at row
+  // l>>3, chunk position l&7 of its group and therefore fetches global chunk (l&7) ^ ((row >> 1) & 7).
   const int lr = lane >> 3, lp = lane & 7;
   const int xrs = SEG ? sg.xrs : K, wrs = SEG ? sg.wrs : K;     // row strides
-  const int chE = (lp ^ (lane >> 4)) * CE;                      // 8-row groups starting at a multiple of 16
-  const int chO = (lp ^ ((lane >> 4) | 4)) * CE;                // ... at 8 mod 16
-  const int offE = lr * xrs + chE, offO = lr * xrs + chO;
-  const int woffE = SEG ? lr * wrs + chE : offE, woffO = SEG ? lr * wrs + chO : offO;
-  auto x_rows = [&](const TileAt &t) { return x + (int64_t)t.layer * xs + (int64_t)(t.m0 + wave * 32) * xrs; };
-  auto w_rows = [&](const TileAt &t) { return w + (int64_t)t.layer * wstr + (int64_t)(t.n0 + wave * 32) * wrs; };
+  const uint32_t chE = (uint32_t)(lp ^ (lane >> 4)) * 16u;          // 8-row groups starting at a multiple of 16
+  const uint32_t chO = (uint32_t)(lp ^ ((lane >> 4) | 4)) * 16u;    // ... at 8 mod 16
+  const uint32_t xoffE = (uint32_t)lr * (uint32_t)xrs * (uint32_t)sizeof(T) + chE, xoffO = xoffE - chE + chO;
+  const uint32_t woff = (uint32_t)lr * (uint32_t)wrs * (uint32_t)sizeof(T) + ((wave & 1) ? chO : chE);
+  auto x_rows = [&](const TileAt &t) { return (const char *)(x + (int64_t)t.layer * xs + (int64_t)(t.m0 + wave * 32) * xrs); };
+  auto w_rows = [&](const TileAt &t) {
+    return (const char *)(w + (int64_t)t.layer * wstr + (int64_t)(t.n0 + (wave >> 2) * 128 + (wave & 3) * 8) * wrs);
+  };
   // the stage walked kt-th by a tile (an index into K / BK)
   auto stage_k0 = [&](const TileAt &t, int kt) {
     int q = kt + t.rot;
@@ -259,9 +301,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
     if constexpr (ODD) return q < nk_real ? q : nk_real - 1;
     return q;
   };
-  auto issue_stage = [&](unsigned char *stage, const T *xt, const T *wt, int kst) {
-    unsigned char *xs_l = stage + wave * 32 * ROWB;
-    unsigned char *ws_l = xs_l + BM * ROWB;
+  // the i-th of a stage's eight loads: 8-row groups 0 - 3 of x, then W's quarters
+  auto issue = [&](unsigned char *stage, const char *xt, const char *wt, int kst, int i) {
     int64_t xk = (int64_t)kst * BK, wk = xk;
     if constexpr (SEG) {
       const int q = sg.sps == 1 ? kst : (int)__umulhi((uint32_t)kst, sg.magic);
@@ -269,40 +310,37 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
       xk = q * sg.xss + kin;
       wk = q * sg.wss + kin;
     }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      load16_to_lds(xt + (int64_t)t * 8 * xrs + xk + ((t & 1) ? offO : offE), xs_l + t * 8 * ROWB);
-      load16_to_lds(wt + (int64_t)t * 8 * wrs + wk + ((t & 1) ? woffO : woffE), ws_l + t * 8 * ROWB);
-    }
+    if (i < 4) fill16(xt + ((int64_t)(i * 8) * xrs + xk) * (int64_t)sizeof(T), (i & 1) ? xoffO : xoffE,
+                      lds_address(stage) + (wave * 32 + i * 8) * ROWB);
+    else fill16(wt + ((int64_t)((i - 4) * 32) * wrs + wk) * (int64_t)sizeof(T), woff,
+                lds_address(stage) + (BM + (wave >> 2) * 128 + (i - 4) * 32 + (wave & 3) * 8) * ROWB);
   };
 
-  // ---- fragment reader: row l31 of each 32-row group; chunk (kk*2 + lh) at its swizzled position
-  const int l31 = lane & 31, lh = lane >> 5;
-  const int xrow = (wm * 64 + l31) * ROWB;              // + i * 32 * ROWB
-  const int wrow = BM * ROWB + (wn * 128 + l31) * ROWB; // + j * 32 * ROWB
-  int koff[4];
+  // ---- fragment reader: row l15 of each 16-row group; chunk (ks*4 + lq) at its swizzled position
+  const int l15 = lane & 15, lq = lane >> 4;
+  const int xrow = (wm * 64 + l15) * ROWB;              // + i * 16 * ROWB
+  const int wrow = BM * ROWB + (wn * 128 + l15) * ROWB; // + j * 16 * ROWB
+  int koff[2];
 #pragma unroll
-  for (int kk = 0; kk < 4; ++kk) koff[kk] = ((kk * 2 + lh) ^ ((l31 >> 1) & 7)) << 4;
+  for (int ks = 0; ks < 2; ++ks) koff[ks] = ((ks * 4 + lq) ^ ((l15 >> 1) & 7)) << 4;
 
   // The accumulators start from the bias (the matrix core adds its products onto them in fp32), so
-  // the epilogue has no bias loads or adds: accumulator (j, rg*4+q) of a lane belongs to feature
-  // j*32 + rg*8 + (lane>>5)*4 + q of the wave tile, whatever the token group i.  Each wavefront brings
+  // the epilogue has no bias loads or adds: accumulator (j, q) of a lane belongs to feature
+  // j*16 + (lane>>4)*4 + q of the wave tile, whatever the token group i.  Each wavefront brings
   // the bias of its 128 features into LDS with one direct load ahead of the tile's stages - no register
   // holds it while the previous tile's epilogue runs - and reads it from there when the first stage has
   // landed.
-  f32x16_t acc[2][4];
+  f32x4_t acc[4][8];
   constexpr int BIAS_LANES = 128 * (int)sizeof(T) / 16;   // lanes of the one 16-byte-per-lane load
-  auto load_bias = [&](const TileAt &t) {
-    if (bias && lane < BIAS_LANES)
-      load16_to_lds(bias + (int64_t)t.layer * bs + t.n0 + wn * 128 + lane * CE, bias_lds[wave]);
+  auto load_bias = [&](const TileAt &t, int slot) {
+    if (bias && lane < BIAS_LANES) fill16(bias + (int64_t)t.layer * bs + t.n0 + wn * 128, lane * 16, lds_address(bias_lds[wave]));
     if constexpr (COLLECT == 2) {
       if (lane < BIAS_LANES)
-        load16_to_lds((const T *)ca.theta + (int64_t)t.layer * ca.theta_stride + t.n0 + wn * 128 + lane * CE, theta_lds[wave]);
+        fill16((const T *)ca.theta + (int64_t)t.layer * ca.theta_stride + t.n0 + wn * 128, lane * 16, lds_address(theta_lds[slot][wave]));
     }
     // the layer's cut travels the same way: four bytes into the wavefront's slot, read in the epilogue
     if constexpr (COLLECT == 1) {
-      if (lane == 0)
-        __builtin_amdgcn_global_load_lds(&ca.st[t.layer].cut_key, (__attribute__((address_space(3))) void *)cut_lds[wave], 4, 0, 0);
+      if (lane == 0) fill4(&ca.st[t.layer].cut_key, 0, lds_address(cut_lds[slot][wave]));
     }
   };
   if (!bias && lane < BIAS_LANES)   // no bias: the slot holds zeros for good
@@ -311,213 +349,201 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   // many of the outstanding direct loads are older than the one into the bias slot, would otherwise wait for
   // all of them (the stage just asked for included) before the first read.
   const uint32_t bias_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)
-                               reinterpret_cast<unsigned char *>(bias_lds[wave]) + (uint32_t)(lane >> 5) * 4u * (uint32_t)sizeof(T);
+                               reinterpret_cast<unsigned char *>(bias_lds[wave]) + (uint32_t)(lane >> 4) * 4u * (uint32_t)sizeof(T);
   auto init_acc = [&]() {
     typedef typename std::conditional<sizeof(T) == 4, uint4, uint2>::type braw_t;
-    braw_t raw[16];
-    // raw[4 j + rg] = the 4 values at feature j * 32 + rg * 8 of this lane's half.  All sixteen reads and their
+    braw_t raw[8];
+    // raw[j] = the 4 values at feature j * 16 of this lane's quarter.  All eight reads and their
     // wait are one statement, so no register is looked at before its value has arrived.
     if constexpr (sizeof(T) == 4) {
         asm volatile(
-                     "ds_read_b128 %0, %16\n\t"
-                     "ds_read_b128 %1, %16 offset:32\n\t"
-                     "ds_read_b128 %2, %16 offset:64\n\t"
-                     "ds_read_b128 %3, %16 offset:96\n\t"
-                     "ds_read_b128 %4, %16 offset:128\n\t"
-                     "ds_read_b128 %5, %16 offset:160\n\t"
-                     "ds_read_b128 %6, %16 offset:192\n\t"
-                     "ds_read_b128 %7, %16 offset:224\n\t"
-                     "ds_read_b128 %8, %16 offset:256\n\t"
-                     "ds_read_b128 %9, %16 offset:288\n\t"
-                     "ds_read_b128 %10, %16 offset:320\n\t"
-                     "ds_read_b128 %11, %16 offset:352\n\t"
-                     "ds_read_b128 %12, %16 offset:384\n\t"
-                     "ds_read_b128 %13, %16 offset:416\n\t"
-                     "ds_read_b128 %14, %16 offset:448\n\t"
-                     "ds_read_b128 %15, %16 offset:480\n\t"
+                     "ds_read_b128 %0, %8\n\t"
+                     "ds_read_b128 %1, %8 offset:64\n\t"
+                     "ds_read_b128 %2, %8 offset:128\n\t"
+                     "ds_read_b128 %3, %8 offset:192\n\t"
+                     "ds_read_b128 %4, %8 offset:256\n\t"
+                     "ds_read_b128 %5, %8 offset:320\n\t"
+                     "ds_read_b128 %6, %8 offset:384\n\t"
+                     "ds_read_b128 %7, %8 offset:448\n\t"
                      "s_waitcnt lgkmcnt(0)"
-                     : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(raw[2]), "=&v"(raw[3]), "=&v"(raw[4]), "=&v"(raw[5]), "=&v"(raw[6]), "=&v"(raw[7]), "=&v"(raw[8]), "=&v"(raw[9]), "=&v"(raw[10]), "=&v"(raw[11]), "=&v"(raw[12]), "=&v"(raw[13]), "=&v"(raw[14]), "=&v"(raw[15])
+                     : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(raw[2]), "=&v"(raw[3]), "=&v"(raw[4]), "=&v"(raw[5]), "=&v"(raw[6]), "=&v"(raw[7])
                      : "v"(bias_at));
     } else {
         asm volatile(
-                     "ds_read_b64 %0, %16\n\t"
-                     "ds_read_b64 %1, %16 offset:16\n\t"
-                     "ds_read_b64 %2, %16 offset:32\n\t"
-                     "ds_read_b64 %3, %16 offset:48\n\t"
-                     "ds_read_b64 %4, %16 offset:64\n\t"
-                     "ds_read_b64 %5, %16 offset:80\n\t"
-                     "ds_read_b64 %6, %16 offset:96\n\t"
-                     "ds_read_b64 %7, %16 offset:112\n\t"
-                     "ds_read_b64 %8, %16 offset:128\n\t"
-                     "ds_read_b64 %9, %16 offset:144\n\t"
-                     "ds_read_b64 %10, %16 offset:160\n\t"
-                     "ds_read_b64 %11, %16 offset:176\n\t"
-                     "ds_read_b64 %12, %16 offset:192\n\t"
-                     "ds_read_b64 %13, %16 offset:208\n\t"
-                     "ds_read_b64 %14, %16 offset:224\n\t"
-                     "ds_read_b64 %15, %16 offset:240\n\t"
+                     "ds_read_b64 %0, %8\n\t"
+                     "ds_read_b64 %1, %8 offset:32\n\t"
+                     "ds_read_b64 %2, %8 offset:64\n\t"
+                     "ds_read_b64 %3, %8 offset:96\n\t"
+                     "ds_read_b64 %4, %8 offset:128\n\t"
+                     "ds_read_b64 %5, %8 offset:160\n\t"
+                     "ds_read_b64 %6, %8 offset:192\n\t"
+                     "ds_read_b64 %7, %8 offset:224\n\t"
                      "s_waitcnt lgkmcnt(0)"
-                     : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(raw[2]), "=&v"(raw[3]), "=&v"(raw[4]), "=&v"(raw[5]), "=&v"(raw[6]), "=&v"(raw[7]), "=&v"(raw[8]), "=&v"(raw[9]), "=&v"(raw[10]), "=&v"(raw[11]), "=&v"(raw[12]), "=&v"(raw[13]), "=&v"(raw[14]), "=&v"(raw[15])
+                     : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(raw[2]), "=&v"(raw[3]), "=&v"(raw[4]), "=&v"(raw[5]), "=&v"(raw[6]), "=&v"(raw[7])
                      : "v"(bias_at));
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        float bv[4];
-        if constexpr (sizeof(T) == 4) {
-          const uint4 r = raw[j * 4 + rg];
-          bv[0] = __uint_as_float(r.x); bv[1] = __uint_as_float(r.y); bv[2] = __uint_as_float(r.z); bv[3] = __uint_as_float(r.w);
-        } else {
-          const uint2 r = raw[j * 4 + rg];
-          unpack_pair<T>(r.x, bv[0], bv[1]);
-          unpack_pair<T>(r.y, bv[2], bv[3]);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[i][j][rg * 4 + q] = bv[q];
+    for (int j = 0; j < 8; ++j) {
+      float bv[4];
+      if constexpr (sizeof(T) == 4) {
+        bv[0] = __uint_as_float(raw[j].x); bv[1] = __uint_as_float(raw[j].y); bv[2] = __uint_as_float(raw[j].z); bv[3] = __uint_as_float(raw[j].w);
+      } else {
+        unpack_pair<T>(raw[j].x, bv[0], bv[1]);
+        unpack_pair<T>(raw[j].y, bv[2], bv[3]);
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i][j] = f32x4_t{bv[0], bv[1], bv[2], bv[3]};
+    }
   };
 
-  // Software pipeline over the K stages.  Fragments are double-buffered in registers (fa/fb)
-  // and read one k-step ahead of the matrix ops that use them.  There is one barrier per
-  // stage, placed before the LAST k-step of a stage: at that point this wavefront's loads of
-  // the next stage have landed and its LDS reads of the current stage are complete, so after
-  // the barrier the next stage may be read (its first fragments are fetched under the last
-  // k-step's matrix ops) and the current one may be overwritten by the stage after next.
-  uint4 fa[6], fb[6];   // [0..1] x fragments, [2..5] W fragments
-  auto load_frags = [&](uint4 (&f)[6], const unsigned char *sb, int kk) {
-    // in the order the matrix ops of the next k-step want them: x0 and all of W first
-    f[0] = *reinterpret_cast<const uint4 *>(sb + xrow + koff[kk]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f[2 + j] = *reinterpret_cast<const uint4 *>(sb + wrow + j * 32 * ROWB + koff[kk]);
-    f[1] = *reinterpret_cast<const uint4 *>(sb + xrow + 32 * ROWB + koff[kk]);
+  // Software pipeline over the K stages.  A stage is four quarters of 16 matrix operations: quarter q multiplies all of the
+  // wavefront's tokens with 32 of its features (rows 32 q of the W half tile), over the stage's whole K.  The x fragments
+  // stay in registers for the stage, each being replaced by the next stage's behind its last use; the W fragments of the next
+  // quarter are read under this one's products.
+  // Two barriers per stage, before the second and before the last quarter.  At the first, x and the first half of W have been
+  // read by everybody, so six of the loads of the stage after next can be asked for, at the second the rest; and of the
+  // stage's own loads, what the next two quarters read has landed: all of it but the last eight loads, so that a load has
+  // a stage and a half to arrive.
+  uint4 fx[4][2], fw[2][2][2];           // [token group][k-step], [buffer][feature group][k-step]
+  auto read_x = [&](const unsigned char *st, int i, int ks) { fx[i][ks] = *reinterpret_cast<const uint4 *>(st + xrow + i * 16 * ROWB + koff[ks]); };
+  auto read_w = [&](const unsigned char *st, int q, int j, int ks) {
+    fw[q & 1][j][ks] = *reinterpret_cast<const uint4 *>(st + wrow + (q * 2 + j) * 16 * ROWB + koff[ks]);
   };
-  auto mma8 = [&](const uint4 (&f)[6]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Mma<T>::run(acc[i][j], f[2 + j], f[i]);
+  auto meet = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
   };
-  constexpr int MPI = sizeof(T) == 2 ? 1 : 4;   // matrix instructions per Mma::run
-  // interleave hint: the six LDS reads go out behind the first matrix ops of the k-step, one apiece
-  auto mix_ds = [&]() {
+  // `fresh`: the tile's first stage, all of which has landed before.
+  // `first` / `rest`: ask for the i-th of the six / two loads into `st`.  `last`: the tile's last stage.
+  // `m`: AND mask for the fragments of this stage (all ones, or zero for the appended stage, whose products must add nothing:
+  // both operands are cleared, so that an infinity in the repeated data cannot turn into a NaN).
+  auto body = [&](unsigned char *st, unsigned char *next, bool last, bool fresh, auto first, auto rest, uint32_t m) {
 #pragma unroll
-    for (int g = 0; g < 6; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, MPI, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 2 * MPI, 0);
-  };
-  // one stage except its last k-step, the barrier, then the last k-step overlapped with the loads that
-  // `refill` asks for (the stage after next, into `cur`) and, unless this is the tile's last stage,
-  // the first fragments of `nxt`
-  // `cm` / `nm`: AND masks for the fragments read from `cur` / `nxt` (all ones, or zero for the appended stage,
-  // whose products must add nothing: both operands are cleared, so that an infinity in the repeated data cannot
-  // turn into a NaN)
-  auto mask_frags = [&](uint4 (&f)[6], uint32_t m) {
+    for (int q = 0; q < 4; ++q) {
+      if (q == 1 || q == 3) {
+        if (q == 3 && last) __builtin_amdgcn_s_waitcnt(0xC07F);    // lgkmcnt(0)
+        else if (q == 1 && fresh) __builtin_amdgcn_s_waitcnt(0xC07F);
+        else __builtin_amdgcn_s_waitcnt(0x0078);                  // vmcnt(8) lgkmcnt(0)
+        meet();
+      }
 #pragma unroll
-    for (int i = 0; i < 6; ++i) { f[i].x &= m; f[i].y &= m; f[i].z &= m; f[i].w &= m; }
-  };
-  auto body = [&](unsigned char *cur, unsigned char *nxt, bool last, auto refill, uint32_t cm, uint32_t nm) {
-    load_frags(fb, cur, 1); mask_frags(fb, cm); mma8(fa); mix_ds();
-    load_frags(fa, cur, 2); mask_frags(fa, cm); mma8(fb); mix_ds();
-    load_frags(fb, cur, 3); mask_frags(fb, cm); mma8(fa); mix_ds();
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    refill();
-    if (!last) { load_frags(fa, nxt, 0); mask_frags(fa, nm); }
-    mma8(fb);
+      for (int g = 0; g < 8; ++g) {
+        const int ks = g >> 2, i = g & 3;
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, MPI, 0);
-      if (g < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        for (int part = 0; part < Mma16<T>::PARTS; ++part)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            uint4 xv = fx[i][ks], wv = fw[q & 1][j][ks];
+            if constexpr (ODD) {
+              xv.x &= m; xv.y &= m; xv.z &= m; xv.w &= m;
+              wv.x &= m; wv.y &= m; wv.z &= m; wv.w &= m;
+            }
+            Mma16<T>::run(acc[i][q * 2 + j], wv, xv, part);
+          }
+        if (q < 3 && g < 4) read_w(st, q + 1, g & 1, g >> 1);
+        if (q == 3 && !last) {
+          if (g < 4) read_w(next, 0, g & 1, g >> 1);
+          read_x(next, i, ks);
+        }
+        if (q == 0 && g == 1) rest(1);
+        if ((q == 1 || q == 2) && g < 6 && (g & 1) == 0) first((q - 1) * 3 + g / 2);
+        if (q == 3 && g == 1) rest(0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
 
   TileAt cur = locate(bid);
-  // both stage buffers are free at this point: the bias, then the first stage, then the second
-  load_bias(cur);
+  load_bias(cur, 0);
+  {
+    const int at = stage_k0(cur, 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) issue(stage0, x_rows(cur), w_rows(cur), at, i);
+  }
+  int slot = 0;
   __builtin_amdgcn_sched_barrier(0);
-  issue_stage(stage0, x_rows(cur), w_rows(cur), stage_k0(cur, 0));
-  issue_stage(stage1, x_rows(cur), w_rows(cur), stage_k0(cur, 1));
+  __builtin_amdgcn_s_waitcnt(0);
+  meet();
 
   for (;;) {
     int nbid = bid + (int)gridDim.x;
     while (nbid < total_tiles && !wanted(nbid)) nbid += gridDim.x;
     const bool has_next = nbid < total_tiles;
     const TileAt nxt_tile = locate(has_next ? nbid : bid);
-    const T *xt = x_rows(cur), *wt = w_rows(cur);
+    const char *xt = x_rows(cur), *wt = w_rows(cur), *xn = x_rows(nxt_tile), *wn_ = w_rows(nxt_tile);
     const int m0 = cur.m0, n0 = cur.n0, layer = cur.layer;
 
-    // only the first stage (this wavefront's 8 older loads, and the bias load before them) is waited for:
-    // at most the 8 loads of the second stage stay outstanding
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0x0F78);   // vmcnt(8)
-    // a bare barrier between two compiler-only fences: the fences of __syncthreads() would wait for the
-    // second stage too
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);    // nothing that reads the bias may move above the wait
-    init_acc();
-    load_frags(fa, stage0, 0);
-    // nk is even
-    for (int kt = 0; kt < nk - 2; kt += 2) {
-      body(stage0, stage1, false, [&]() { issue_stage(stage0, xt, wt, stage_k0(cur, kt + 2)); }, ~0u, ~0u);
-      body(stage1, stage0, false, [&]() { issue_stage(stage1, xt, wt, stage_k0(cur, kt + 3)); }, ~0u, ~0u);
+    // here the first stage and the bias have landed for every wavefront, and the second buffer is free
+    {
+      const int at = stage_k0(cur, 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) issue(stage1, xt, wt, at, i);
     }
-    // the last two stages: the first buffer is free after the first of them and takes the next tile's
-    // first stage; nothing may be in flight into the second one, which is parked in
-    constexpr uint32_t last_mask = odd ? 0u : ~0u;
-    body(stage0, stage1, false, [&]() {
-      if (has_next) issue_stage(stage0, x_rows(nxt_tile), w_rows(nxt_tile), stage_k0(nxt_tile, 0));
-    }, ~0u, last_mask);
-    body(stage1, stage0, true, [&]() {}, last_mask, ~0u);
+    init_acc();
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) read_w(stage0, 0, j, ks);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) read_x(stage0, i, ks);
+    int kt = 0;                           // nk is even
+    for (; kt < nk - 2; kt += 2) {
+      const int k1 = stage_k0(cur, kt + 1), k2 = stage_k0(cur, kt + 2), k3 = stage_k0(cur, kt + 3);
+      body(stage0, stage1, false, kt == 0, [&](int i) { issue(stage0, xt, wt, k2, i); },
+           [&](int i) { if (i == 0) issue(stage0, xt, wt, k2, 6); else if (kt > 0) issue(stage1, xt, wt, k1, 7); }, ~0u);
+      body(stage1, stage0, false, false, [&](int i) { issue(stage1, xt, wt, k3, i); },
+           [&](int i) { if (i == 0) issue(stage1, xt, wt, k3, 6); else issue(stage0, xt, wt, k2, 7); }, ~0u);
+    }
+    // the last two stages: the first buffer takes the next tile's first stage (at the end, one that nobody reads);
+    // nothing may be on its way into the second one, which is parked in
+    const int k1 = stage_k0(cur, kt + 1), k0 = stage_k0(nxt_tile, 0);
+    body(stage0, stage1, false, kt == 0, [&](int i) { issue(stage0, xn, wn_, k0, i); },
+         [&](int i) { if (i == 0) issue(stage0, xn, wn_, k0, 6); else if (kt > 0) issue(stage1, xt, wt, k1, 7); }, ~0u);
+    body(stage1, stage0, true, false, [&](int i) { if (i == 0) load_bias(nxt_tile, slot ^ 1); },
+         [&](int i) { if (i == 1) issue(stage0, xn, wn_, k0, 7); }, odd ? 0u : ~0u);
     // past the barrier of the last stage no wavefront reads either buffer any more
 
     // ---- epilogue.  The accumulator layout gives a lane 4 consecutive features of one token,
     // i.e. 8-byte pieces scattered over 32 rows per store - slow to write.  Each wavefront
     // therefore parks its tile in LDS, 32 tokens at a time (8 KB; two passes of 64 features for fp32) in its
     // eighth of the second stage buffer, and works on it row by row from there.
+    // The next tile's first stage and its bias, asked for a stage ago, are waited for here: the stores that follow may then stay
+    // under way into the next tile (loads and stores share a counter that runs in order).
     T *pl = pre + (int64_t)layer * ps;
     // The epilogue's addresses are rebuilt from the lane number for every tile.  Left visible as loop
     // invariants they would be computed once ahead of the tile loop and live across the K loop.
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    const int l31 = lane_e & 31, lh = lane_e >> 5;
+    const int l31 = lane_e & 31, lh = lane_e >> 5, l15e = lane_e & 15, lqe = lane_e >> 4;
     unsigned char *park = stage1 + wave * (STAGE / 8);
     constexpr int NPASS = sizeof(T) == 2 ? 1 : 2;           // feature halves per pass
-    constexpr int JP = 4 / NPASS;                            // 32-feature groups per pass
-    // token groups [i0, i0 + ni) of feature pass `pass` -> rows (i - i0) * 32 + l31 of 256 bytes
-    // (128 bf16 / 64 fp32), 16-byte slots XOR-swizzled with the row
-    auto park_rows = [&](int pass, int i0, int ni) {
+    constexpr int JP = 8 / NPASS;                            // 16-feature groups per pass
+    // the 32 tokens h of feature pass `pass` -> rows of 256 bytes (128 bf16 / 64 fp32), 16-byte slots XOR-swizzled with
+    // the row
+    auto park_rows = [&](int pass, int h) {
 #pragma unroll
       for (int jj = 0; jj < JP; ++jj) {
         const int j = pass * JP + jj;
+        const int nl = jj * 16 + lqe * 4;                    // feature inside this pass
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const int nl = jj * 32 + rg * 8 + lh * 4;          // feature inside this pass
-#pragma unroll
-          for (int ii = 0; ii < ni; ++ii) {
-            const int i = i0 + ii;
-            const int ml = ii * 32 + l31;                    // row inside the parked piece
-            float y[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) y[q] = acc[i][j][rg * 4 + q];
-            if (sizeof(T) == 4) {
-              const int slot = (nl >> 2) ^ (ml & 15);
-              *reinterpret_cast<float4 *>(park + ml * 256 + slot * 16) = make_float4(y[0], y[1], y[2], y[3]);
-            } else {
-              const int slot = (nl >> 3) ^ (ml & 15);
-              uint2 o;
-              o.x = pack16x2<T>(y[0], y[1]);
-              o.y = pack16x2<T>(y[2], y[3]);
-              *reinterpret_cast<uint2 *>(park + ml * 256 + slot * 16 + (nl & 4) * 2) = o;
-            }
+        for (int ii = 0; ii < 2; ++ii) {
+          const int ml = ii * 16 + l15e;                     // row inside the parked piece
+          const f32x4_t y = acc[h * 2 + ii][j];
+          if (sizeof(T) == 4) {
+            const int slot = (nl >> 2) ^ (ml & 15);
+            *reinterpret_cast<float4 *>(park + ml * 256 + slot * 16) = make_float4(y[0], y[1], y[2], y[3]);
+          } else {
+            const int slot = (nl >> 3) ^ (ml & 15);
+            uint2 o;
+            o.x = pack16x2<T>(y[0], y[1]);
+            o.y = pack16x2<T>(y[2], y[3]);
+            *reinterpret_cast<uint2 *>(park + ml * 256 + slot * 16 + (nl & 4) * 2) = o;
           }
         }
       }
@@ -528,7 +554,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
       if constexpr (COLLECT == 0) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-        park_rows(pass, h, 1);
+        park_rows(pass, h);
+        if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores: see below
         // the wavefront reads its own piece back: lane -> (row = it*4 + lane/16, slot = lane%16)
 #pragma unroll 4
         for (int it = 0; it < 8; ++it) {
@@ -559,7 +586,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
           // its own wait inside the statement: the compiler, which cannot tell the direct-to-LDS loads in flight
           // (the next tile's first stage) from the one into this slot, would wait for all of them first.
           uint32_t cut_key_v;
-          const uint32_t cut_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)cut_lds[wave];
+          const uint32_t cut_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)cut_lds[slot][wave];
           asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(cut_key_v) : "v"(cut_at) : "memory");
           cut_bits = key_value_bits<T>((uint32_t)__builtin_amdgcn_readfirstlane((int)cut_key_v));
         }
@@ -579,7 +606,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
             const uint4 v = *reinterpret_cast<const uint4 *>(myrow + ((sl ^ rsw) * 16));
             uint4 tv = make_uint4(0, 0, 0, 0);
             if constexpr (COLLECT == 2)
-              tv = *reinterpret_cast<const uint4 *>(theta_lds[wave] + pass * SEGW + sl * EPS);
+              tv = *reinterpret_cast<const uint4 *>(theta_lds[slot][wave] + pass * SEGW + sl * EPS);
             uint32_t m = 0;
 #pragma unroll
             for (int j = 0; j < EPS; ++j) {
@@ -607,7 +634,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
             fast_ok = cb >= 1u && cb <= Elem<T>::INF16;
             cm1 = (cb - 1u) | ((cb - 1u) << 16);
           } else {
-            theta_seg = theta_lds[wave] + pass * SEGW;
+            theta_seg = theta_lds[slot][wave] + pass * SEGW;
             bool bad = false;
             if (lane_e < 16) {   // every threshold of the segment must be a positive number
               const uint4 tv = *reinterpret_cast<const uint4 *>(theta_seg + lane_e * 8);
@@ -713,7 +740,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
         // atomic) and parks and emits both again.
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          park_rows(pass, h, 1);
+          park_rows(pass, h);
+          if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores: see below
           scan_piece(W[h]);
           // the first `shift` tokens of a shifted tile belong to its neighbour, which reports them, and so do the
           // features in front of on0 (bit b of word i of a lane = feature hs * SEGW / 2 + 32 i + b of the segment)
@@ -754,7 +782,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
           if (ok) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              park_rows(pass, h, 1);
+              park_rows(pass, h);
               emit_piece(W[h], incl[h] - cnt[h] - (hs ? 0u : part[h]), tot[h], mypool + off + (h ? tot[0] : 0u));
             }
           }
@@ -772,18 +800,12 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
     }
     if (!has_next) break;
-    // Every wavefront is done with its parked rows before the next tile's loads overwrite them.  The wait
-    // covers the epilogue's stores as well (and the next tile's first stage, long since landed): with only
-    // loads outstanding afterwards, the counted wait at the top of the tile is exact.
-    __builtin_amdgcn_s_waitcnt(0);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    // every wavefront is done with its parked rows before the next tile's loads overwrite them
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+    meet();
     bid = nbid;
     cur = nxt_tile;
-    load_bias(cur);
-    __builtin_amdgcn_sched_barrier(0);   // the bias stays ahead of the stage loads: the wait above counts on it
-    issue_stage(stage1, x_rows(cur), w_rows(cur), stage_k0(cur, 1));
+    slot ^= 1;
   }
   __builtin_amdgcn_s_waitcnt(0);   // no direct-to-LDS load may be in flight when the block retires
 }
@@ -806,8 +828,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
 // whose matrix products are what bounds, or where the large tiles would not fill the chip once.
 constexpr int SK_STAGES = 3;
 
-// 16 bytes per lane into LDS (lane i lands at lds_at + 16 i), as a statement the compiler does not count: it would wait
-// for the stages in flight before every fragment read.  The waits are written out by hand.
+// As fill16, from a scalar base.
 __device__ __forceinline__ void sk_fill16(const void *base, uint32_t off, uint32_t lds_at) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
 }
@@ -934,7 +955,7 @@ static bool encode_fast_ok(const void *x, const void *w, const void *b, const vo
   return (d % (ROWB / (int)sizeof(T)) == 0) && (F % 4 == 0) && T_ >= BM && F >= BN && clt_aligned16(x) &&
          clt_aligned16(w) && clt_aligned16(pre) && (xs % CE == 0) && (wstr % CE == 0) && (ps % 4 == 0) &&
          (ps * (int64_t)sizeof(T)) % 16 == 0 && (F * (int64_t)sizeof(T)) % 8 == 0 && T_ < (1 << 30) &&
-         F < (1 << 30) && d < (1 << 30) && (!b || (((uintptr_t)b) % 16 == 0 && bs % 8 == 0));
+         F < (1 << 30) && d < (1 << 27) && (!b || (((uintptr_t)b) % 16 == 0 && bs % 8 == 0));
 }
 
 // What k_encode_short takes: a batch shorter than one tile (where it is the faster one, see there), whole 128-byte stages,
