@@ -42,7 +42,6 @@ struct RecArgs {
   int64_t Rn, L, max_entries;
   uint64_t layer_mask;
   SpPlan p;
-  int window;              // batches put together in LDS at a time
   int alternate;           // 1: stages of all layers follow each other, in two buffers in turn; 0: one buffer
   int32_t *start;          // [L * groups][SP_GROUP][tiles + 1] list position where a row's entries of a tile begin
   uint16_t *batches;       // [L * tiles][groups] batches of (layer, tile, group)
@@ -118,38 +117,43 @@ __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
   if (stream == 0 && lane == 0) *A.bad = 0u;
 }
 
-// One workgroup per (group, layer) again: the runs of a tile laid end to end in row order - a fixed order of every sum -
-// put together in LDS, `window` batches at a time, and written out lane by lane.
+// The entries of a wavefront whose low three bits equal `mine`: `b0`, `b1`, `b2` are the ballots of the three bits.
+__device__ __forceinline__ uint64_t same_class(uint64_t valid, uint64_t b0, uint64_t b1, uint64_t b2, uint32_t mine) {
+  return valid & ~(b0 ^ (0ull - (uint64_t)(mine & 1u))) & ~(b1 ^ (0ull - (uint64_t)((mine >> 1) & 1u))) &
+         ~(b2 ^ (0ull - (uint64_t)((mine >> 2) & 1u)));
+}
+
+// One workgroup per (group, layer) again, a wavefront per tile: its entries become the tile's batches, put together in LDS and
+// written out lane by lane.
+//
+// Where an entry goes decides how fast LDS hands out its row.  The 64 lanes of a transposing read ask for sixteen 32-byte
+// pieces, eight rows by each half of the wavefront, and eight rows with different r % 8 cover all banks: 1.06 ns
+// per read and CU, against 2.19 with rows in random places (profiles/lds_read_probe.txt).  So the tile's entries are sorted by
+// r % 8 - within a class they keep their order by (row, column): the order of every sum is fixed - and dealt out in turn
+// to the 4 nb half reads of its nb batches: a half read then meets a class twice only if the class has more than 4 nb
+// entries.  A place that stays empty refers to the half read's first row, which costs no bank of its own.
+// (L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, bf16: this kernel 213 -> 158 us against entries in the
+// order of the lists, row by row through a window of 128 batches, k_decode_tiles 3.33 -> 3.17 ms; L = 24, d = 1024, F = 32768:
+// 433 -> 266 us, 15.77 -> 15.59 ms.  Bound by the chain of a tile's steps in each wavefront.)
+constexpr int REC_WINDOW = 8;                              // batches a wavefront puts together at a time
 template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(RecArgs A) {
   extern __shared__ int32_t fill_lds[];
-  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
+  const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63, wave = tid >> 6;
   if (A.row_ptr[A.L * A.Rn] > A.max_entries) return;
   // A wavefront at the end of its stream takes the record that follows for addresses, of LDS reads that nobody multiplies: the
   // next stream's first one, or this one behind the last stream, which refers to the first row of the first buffer.
   if (g == 0 && s == 0 && tid < 64) A.recs[(uint64_t)stream_first(A.total, A.p.streams, lane) * SP_REC_WORDS + lane] = 0u;
   if (!((A.layer_mask >> s) & 1ull)) return;
   int32_t *start = fill_lds;                               // [SP_GROUP][tiles + 1]
-  int32_t *off = start + SP_GROUP * (tiles + 1);           // [SP_GROUP][tiles] entries of the tile before this row's
-  int32_t *first = off + SP_GROUP * tiles;                 // [tiles + 1] first batch of the tile, counted within the group
-  uint32_t *dest = (uint32_t *)(first + tiles + 1);        // [tiles] its place among all batches
-  uint32_t *where = dest + tiles;                          // [window] the same per batch of the window
-  uint16_t *win = (uint16_t *)(where + A.window);          // [window][64] words
-  const int64_t row0 = (int64_t)g * SP_GROUP, r0 = (int64_t)s * A.Rn + row0;
+  uint32_t *dest = (uint32_t *)(start + SP_GROUP * (tiles + 1));       // [tiles] the tile's first batch among all of the stream
+  uint32_t *win = dest + tiles + wave * (REC_WINDOW * SP_REC_WORDS);   // this wavefront's batches
   const int32_t *src = A.start + ((int64_t)s * A.p.groups + g) * SP_GROUP * (tiles + 1);
   for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) start[i] = src[i];
-  __syncthreads();
   const int part = g / A.p.groups_per_part, r = g - part * A.p.groups_per_part;
   const int stream = part * A.p.waves + r % A.p.waves, gi = r / A.p.waves;
   const uint32_t stage0 = A.alternate ? (uint32_t)(__popcll(A.layer_mask & ((1ull << s) - 1ull)) * tiles) : 0u;
   const uint32_t buffers = A.alternate ? 1u : 0u;
   for (int c = tid; c < tiles; c += REC_THREADS) {
-    int32_t n = 0;
-#pragma unroll
-    for (int tk = 0; tk < SP_GROUP; ++tk) {
-      off[tk * tiles + c] = n;
-      n += start[tk * (tiles + 1) + c + 1] - start[tk * (tiles + 1) + c];
-    }
-    first[c] = (n + SP_BATCH - 1) / SP_BATCH;              // batches for now
     const int64_t at = (int64_t)stream * A.p.stages + (int64_t)s * tiles + c;
     uint32_t d = A.offset[at];
     for (int j = 0; j < gi; ++j) d += A.counts[at * DT_GPW + j];
@@ -157,52 +161,84 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
   }
   const uint32_t base = stream_first(A.total, stream, lane);
   __syncthreads();
-  if (tid < 64) {
-    int32_t run = 0;
-    for (int c0 = 0; c0 < tiles; c0 += 64) {
-      const int c = c0 + lane;
-      const int32_t nb = c < tiles ? first[c] : 0;
-      int32_t incl = nb;
+  for (int c = wave; c < tiles; c += REC_THREADS / 64) {
+    // row t's run: entries run_at + [run_off, ..) of the tile's, laid end to end
+    const int t16 = lane & 15;
+    const int32_t run_begin = start[t16 * (tiles + 1) + c];
+    int32_t run_off = start[t16 * (tiles + 1) + c + 1] - run_begin;
+    const int32_t len = run_off;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int32_t up = __shfl_up(incl, o);
-        if (lane >= o) incl += up;
+    for (int o = 1; o < 16; o <<= 1) {
+      const int32_t up = __shfl_up(run_off, o, 16);
+      if (t16 >= o) run_off += up;
+    }
+    const int32_t n = __builtin_amdgcn_readlane(run_off, 15);
+    if (n == 0) continue;
+    run_off -= len;
+    const int32_t run_at = run_begin - run_off;
+    const int32_t nb = (n + SP_BATCH - 1) / SP_BATCH, halves = 4 * nb;
+    const uint32_t magic = 0xFFFFFFFFu / (uint32_t)halves + 1u;          // p / halves = (p * magic) >> 32 for p, halves < 2^16
+    // the i-th entry: its row, place in the list and tile row
+    auto entry = [&](int32_t i, int &tk, int32_t &j) {
+      tk = 0;
+#pragma unroll
+      for (int t = 1; t < SP_GROUP; ++t) tk += i >= __builtin_amdgcn_readlane(run_off, t) ? 1 : 0;
+      j = __shfl(run_at, tk) + i;
+    };
+    uint32_t first = 0;                                    // lane l: entries of class l % 8, then where the class begins
+    for (int32_t i0 = 0; i0 < n; i0 += 64) {
+      int tk;
+      int32_t j;
+      const bool on = i0 + lane < n;
+      entry(on ? i0 + lane : n - 1, tk, j);
+      const uint32_t cls = (uint32_t)A.col[j];
+      const uint64_t v = __ballot(on), b0 = __ballot(cls & 1u), b1 = __ballot(cls & 2u), b2 = __ballot(cls & 4u);
+      first += (uint32_t)__popcll(same_class(v, b0, b1, b2, (uint32_t)lane));
+    }
+    {
+      const uint32_t mine = first;
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) {
+        const uint32_t up = __shfl_up(first, o, 8);
+        if ((lane & 7) >= o) first += up;
       }
-      if (c < tiles) first[c] = run + incl - nb;
-      run += __shfl(incl, 63);
+      first -= mine;
     }
-    if (lane == 0) first[tiles] = run;
-  }
-  __syncthreads();
-  const int32_t nb_all = first[tiles];
-  for (int32_t w0 = 0; w0 < nb_all; w0 += A.window) {
-    const int32_t wn = nb_all - w0 < A.window ? nb_all - w0 : A.window;
-    for (int i = tid; i < wn * SP_REC_WORDS; i += REC_THREADS) reinterpret_cast<uint32_t *>(win)[i] = 0u;
-    for (int c = tid; c < tiles; c += REC_THREADS)
-      for (int32_t b = first[c]; b < first[c + 1]; ++b)
-        if (b >= w0 && b < w0 + wn) where[b - w0] = base + dest[c] + (uint32_t)(b - first[c]);
-    __syncthreads();
-    for (int tk = tid >> 6; tk < SP_GROUP; tk += REC_THREADS / 64) {
-      if (row0 + tk >= A.Rn) break;
-      const int32_t e = A.row_ptr[r0 + tk + 1];
-      for (int32_t j = A.row_ptr[r0 + tk] + lane; j < e; j += 64) {
-        const int32_t f = A.col[j], c = f / SP_ROWS;
-        const int32_t p = off[tk * tiles + c] + j - start[tk * (tiles + 1) + c];
-        const int32_t b = first[c] + p / SP_BATCH - w0, k = p % SP_BATCH;
-        if (b < 0 || b >= wn) continue;
-        uint16_t *rec = win + b * 128 + (k >> 3) * 32;      // 16 lanes of two halves each
-        const int x = (k & 7) >> 1, half = k & 1;
-        rec[(4 * x + 0) * 2 + half] = (uint16_t)Elem<T>::raw(((const T *)A.val)[A.src ? A.src[j] : j]);
-        rec[(4 * x + 1) * 2 + half] = (uint16_t)(1u << tk);
-        rec[(4 * (k & 3) + 3) * 2 + ((k >> 2) & 1)] =
-            (uint16_t)sp_half_place((uint32_t)(f - c * SP_ROWS), (stage0 + c) & buffers);
+    for (int32_t w0 = 0; w0 < nb; w0 += REC_WINDOW) {
+      const int32_t wn = nb - w0 < REC_WINDOW ? nb - w0 : REC_WINDOW;
+      for (int32_t b = 0; b < wn; ++b) win[b * SP_REC_WORDS + lane] = 0u;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      uint32_t next = first;
+      for (int32_t i0 = 0; i0 < n; i0 += 64) {
+        int tk;
+        int32_t j;
+        const bool on = i0 + lane < n;
+        entry(on ? i0 + lane : n - 1, tk, j);
+        const uint32_t f = (uint32_t)A.col[j], cls = f & 7u;
+        const uint64_t v = __ballot(on), b0 = __ballot(cls & 1u), b1 = __ballot(cls & 2u), b2 = __ballot(cls & 4u);
+        const uint64_t same = same_class(v, b0, b1, b2, cls);
+        const uint32_t p = __shfl(next, (int)cls) + __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+        next += (uint32_t)__popcll(same_class(v, b0, b1, b2, (uint32_t)lane));
+        const uint32_t slot = __umulhi(p, magic), h = p - slot * (uint32_t)halves;
+        const int32_t b = (int32_t)(h >> 2) - w0;
+        if (!on || b < 0 || b >= wn) continue;
+        // half read h % 4 of batch h / 4: h & 1 the half of the wavefront, h & 2 the second four entries of its lane quartets
+        uint16_t *rec = (uint16_t *)(win + b * SP_REC_WORDS) + (h & 1u) * 64;
+        auto place = [&](uint32_t sl, uint16_t at) {
+          rec[(sl >> 2) * 32 + (4 * (sl & 3u) + 3) * 2 + ((h >> 1) & 1u)] = at;
+        };
+        const uint32_t k = (slot & 3u) + ((h & 2u) << 1), x = (slot >> 2) * 32 + 8 * (k >> 1) + (k & 1u);
+        rec[x] = (uint16_t)Elem<T>::raw(((const T *)A.val)[A.src ? A.src[j] : j]);
+        rec[x + 2] = (uint16_t)(1u << tk);
+        const uint16_t at = (uint16_t)sp_half_place(f - (uint32_t)c * SP_ROWS, (stage0 + c) & buffers);
+        place(slot, at);
+        if (slot == 0)                                     // the places of this half read that stay empty
+          for (uint32_t sl = __umulhi((uint32_t)n - 1u - p, magic) + 1u; sl < 8u; ++sl) place(sl, at);
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int32_t b = 0; b < wn; ++b) A.recs[(uint64_t)(base + dest[c] + (uint32_t)(w0 + b)) * SP_REC_WORDS + lane] = win[b * SP_REC_WORDS + lane];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __syncthreads();
-    for (int32_t b = tid >> 6; b < wn; b += REC_THREADS / 64) {
-      A.recs[(uint64_t)where[b] * 64 + lane] = reinterpret_cast<const uint32_t *>(win)[b * 64 + lane];
-    }
-    __syncthreads();
   }
 }
 
@@ -247,12 +283,12 @@ __device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_o
 // cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so that one of
 // them brings it from HBM and the others find it in the L2.
 //
-// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.35 ms (98.6 GB of gathered rows, 29
-// TB/s) and 0.26 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.8 and 0.55
-// against 34.2 ms (profiles/forward_c1_kernel_trace.txt, forward_c2_kernel_trace.txt).  Bound by LDS, which is busy in 72 % of
-// the cycles: 21 ns per batch and CU are 2.4 ms, of which 19 % for the entries that fill batches up
-// (profiles/decode_tiles_c1_lds_counters.txt); in the rest wavefronts wait for the slowest one of a stage and records queue
-// behind tile lines that come from HBM (7.9 GB a launch, 2.9 of them weights).
+// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.17 ms (98.6 GB of gathered rows, 31
+// TB/s) and 0.20 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.6 and 0.37
+// against 34.2 ms (profiles/forward_c1_kernel_trace.txt, forward_c2_kernel_trace.txt).  Bound by the chain of a batch's steps,
+// four wavefronts per SIMD: without any one of them - the reads, the products, the operand of values, the records - the launch takes
+// 8 - 12 % less (22 ns per batch and CU; a fifth of the batches' places are filling).  Tiles that come from HBM instead of
+// the L2 cost 0.3 ms of it (2.2 of the 15.6).
 // Measured and dropped: a wavefront of its own for the fills (fifteen share 64 groups badly: 3.98 ms); fewer lines on
 // their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought into the L2 early
 // (3.46 ms: the early loads block the records just as well).
@@ -697,11 +733,8 @@ static void sp_place_workspace(RecArgs &ra, const SpLayout &l, char *ws) {
 
 template <typename T> static int launch_records(RecArgs ra, hipStream_t stream) {
   const int tiles = ra.p.tiles;
-  // a group's batches are put together at once where they are as many as usual
-  ra.window = tiles <= 16 ? 32 : 128;
   const size_t count_lds = sizeof(int32_t) * (size_t)SP_GROUP * (tiles + 1);
-  const size_t fill_lds = sizeof(int32_t) * (size_t)(SP_GROUP * (tiles + 1) + SP_GROUP * tiles + 2 * tiles + 1 + ra.window) +
-                          (size_t)ra.window * SP_REC_WORDS * 4 + 8;
+  const size_t fill_lds = count_lds + sizeof(uint32_t) * ((size_t)tiles + (size_t)REC_THREADS / 64 * REC_WINDOW * SP_REC_WORDS);
   if (hipFuncSetAttribute((const void *)k_rec_fill<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_lds) != hipSuccess)
     return CLT_ERR_LAUNCH;
   const dim3 grid((unsigned)ra.p.groups, (unsigned)ra.L);

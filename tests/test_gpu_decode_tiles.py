@@ -95,6 +95,30 @@ def test_decode_tiles_against_dense_products(L, T, F, d, per_token, dtype, tying
             assert (got[t].double() - ref).abs().le(bound).all(), (t, (got[t].double() - ref).abs().max())
 
 
+@pytest.mark.parametrize("pattern", ["one class", "every column", "two entries", "33 entries", "one row of a group"])
+def test_decode_tiles_wherever_entries_are_dealt_to(pattern):
+    """Tiles whose entries fall into one class of columns (all half reads of a batch meet it), fill more batches than a
+    wavefront puts together at a time, or leave most places of a batch empty."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 1, 40, 1100, 64
+    g = torch.Generator().manual_seed(11)
+    act = torch.randn(L, T, F, generator=g).bfloat16()
+    cols, rows = torch.arange(F), torch.arange(T).unsqueeze(1)
+    keep = {"one class": (cols % 8 == 3) & (rows >= 0), "every column": (cols >= 0) & (rows >= 0),
+            "two entries": (cols % 512 == 17) & (rows % 16 < 2), "33 entries": (cols % 512 < 11) & (rows % 16 < 3),
+            "one row of a group": (cols % 3 == 0) & (rows % 16 == 5)}[pattern]
+    act[0][~keep] = 0
+    nz = act.reshape(T, F) != 0
+    row_ptr = torch.zeros(T + 1, dtype=torch.int32)
+    row_ptr[1:] = torch.cumsum(nz.sum(1), 0)
+    col, val = nz.nonzero()[:, 1].int(), act.reshape(T, F)[nz]
+    w = (torch.rand(1, F, d, generator=g) - 0.5).bfloat16()
+    got = _run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, 1, 1, True, col.numel(), False)
+    ref, mag = act[0].double() @ w[0].double(), act[0].double().abs() @ w[0].double().abs()
+    # exact products; each addition is off by at most 2^-23 of what has been summed
+    assert (got[0].double() - ref).abs().le((nz.sum(1, keepdim=True).double() + 2) * 2.0 ** -23 * mag).all()
+
+
 def test_decode_tiles_of_empty_lists():
     """No stream has a record: every wavefront meets the one behind the last stream."""
     dev = torch.device("cuda:0")
