@@ -69,12 +69,13 @@ template <typename T> struct RankZ {
 template <typename T, bool GLOBAL> struct RankOf;
 template <typename T> struct RankOf<T, false> {
   typedef RankRaw type;
-  __device__ static RankRaw make(const float *, const float *, int64_t, int64_t) { return RankRaw(); }
+  __device__ static RankRaw make(const float *, const float *, int64_t) { return RankRaw(); }
 };
 template <typename T> struct RankOf<T, true> {
   typedef RankZ<T> type;
-  __device__ static RankZ<T> make(const float *mean, const float *denom, int64_t l, int64_t F) {
-    RankZ<T> r; r.mean = mean + l * F; r.denom = denom + l * F; return r;
+  // `at`: where the row's statistics begin in [L][F]
+  __device__ static RankZ<T> make(const float *mean, const float *denom, int64_t at) {
+    RankZ<T> r; r.mean = mean + at; r.denom = denom + at; return r;
   }
 };
 
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256) void k_sample_keys(
     if (GLOBAL) { int64_t rowlen = L * F; t = idx / rowlen; int64_t rem = idx - t * rowlen; l = rem / F; f = rem - l * F; }
     else { l = p; t = idx / F; f = idx - t * F; }
     float x = Elem<T>::to_f32(pre[l * lstride + t * F + f]);
-    typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+    typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l * F);
     sample[(int64_t)p * sample_n + si] = rank_key_of<T>(rk(x, f));
   }
 }
@@ -336,6 +337,18 @@ template <> __device__ __forceinline__ float vec_elem<f16_t>(const uint4 &w, int
   return f16_bits_to_f32((j & 1) ? (u >> 16) : (u & 0xFFFFu));
 }
 
+// 16-bit floats as signed integers in the order of the values: the negative ones' magnitude bits are inverted.  -0.0 becomes -1,
+// NaNs lie beyond the infinities on the side of their sign.
+__device__ __forceinline__ int32_t ordered16(uint32_t raw) {
+  const int32_t v = (int32_t)(int16_t)(uint16_t)raw;
+  return v ^ ((v >> 15) & 0x7FFF);
+}
+typedef short sel_i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ sel_i16x2 ordered16x2(uint32_t raw) {
+  const sel_i16x2 v = __builtin_bit_cast(sel_i16x2, raw);
+  return v ^ ((v >> (short)15) & (short)0x7FFF);
+}
+
 // Global ranking: for every (layer, feature) the lowest value x whose z-score reaches the cut
 // key (binary search over the ordered keys of the element type; the z-score with its two
 // roundings is monotone in x).  NaN when only a NaN reaches the cut.
@@ -353,11 +366,36 @@ __global__ __launch_bounds__(256) void k_col_cut(const float *mean, const float 
     const float xv = __uint_as_float(key_value_bits<T>(mid));
     if (rank_key_of<T>(rk(xv, i)) >= cut_key) hi = mid; else lo = mid + 1u;
   }
-  const uint32_t bits = key_value_bits<T>(lo);
-  xcut[i] = Elem<T>::from_f32(__uint_as_float(bits));   // exact: the value is one of T
+  const T bound = Elem<T>::from_f32(__uint_as_float(key_value_bits<T>(lo)));   // exact: the value is one of T
+  if constexpr (sizeof(T) == 2) {
+    // as an integer in the order of the values, less one (see the pass); zero as -0.0, which both zeros reach, and a NaN as
+    // the first one
+    int32_t b = ordered16((uint32_t)Elem<T>::raw(bound));
+    if (b == 0) b = -1;
+    const int32_t first_nan = (int32_t)Elem<T>::INF16 + 1;
+    b = (b > first_nan ? first_nan : b) - 1;
+    xcut[i] = Elem<T>::from_raw((uint32_t)(b < -32768 ? -32768 : b) & 0xFFFFu);
+  } else {
+    xcut[i] = bound;
+  }
 }
 
-// The streaming pass: one wavefront per row.  A step covers PASS_NV vectors of 64 lanes x 16
+// raw bits of 16-bit element j of a vector
+__device__ __forceinline__ uint32_t w4_elem(const uint4 &w, int j) {
+  const uint32_t u = (j >> 1) == 0 ? w.x : (j >> 1) == 1 ? w.y : (j >> 1) == 2 ? w.z : w.w;
+  return (j & 1) ? u >> 16 : u & 0xFFFFu;
+}
+
+// Few, long rows would leave most of the chip without work, so a row is cut into `split` (a power of two) rows of F columns each:
+// the matrix [T][split * F] read as [T * split][F], in which every element keeps its flat index and so its place among
+// equals.  Row t of the cut matrix holds columns (t % split) * F .. of its token; where a column's statistics and
+// number begin:
+__device__ __forceinline__ int64_t row_columns(int64_t l, int64_t t, int64_t F, int split) {
+  return (l * split + (t & (split - 1))) * F;
+}
+
+// The streaming pass: one wavefront per row, bound by instruction issue (T = 3000, L = 12, F = 24576, bf16, ranked together:
+// 597 -> 470 us with compares of two values at a time and pool space of the wavefronts' own).  A step covers PASS_NV vectors of 64 lanes x 16
 // bytes.  Lanes keep a bit per element that reaches the cut; when any lane has one, the raw
 // vectors are staged in LDS (column order), two packed prefix scans give every candidate its
 // place in column order, each lane writes the columns of its set bits, and then the lanes
@@ -366,7 +404,7 @@ template <typename T, int V, bool GLOBAL>
 __global__ __launch_bounds__(256) void k_select_pass(
     const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t lstride, const float *mean,
     const float *denom, const SelState *st, uint32_t *hist, uint32_t *pool_count, uint2 *pool,
-    unsigned long long pool_cap, uint32_t *row_first, int phase, const T *xcut) {
+    unsigned long long pool_cap, uint32_t *row_first, int phase, const T *xcut, int split, uint32_t slot_size) {
   constexpr int KB = Elem<T>::KEYBITS;
   static_assert(PASS_NV == 4, "the packed prefix below holds four 16-bit fields");
   constexpr int STEP = PASS_NV * 64 * V;  // elements per step
@@ -386,18 +424,26 @@ __global__ __launch_bounds__(256) void k_select_pass(
   uint2 *wbuf = wbuf_all[wv];
   T *stage = stage_all[wv];
   uint2 *mypool = pool + (unsigned long long)p * pool_cap;
-  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+  // this wavefront's own part of the pool, and where the part that is handed out by a counter begins
+  const uint32_t waves = gridDim.x * (uint32_t)nwv;
+  uint32_t own = ((GLOBAL ? (uint32_t)l * waves : 0u) + blockIdx.x * (uint32_t)nwv + (uint32_t)wv) * slot_size;
+  const uint32_t own_end = own + slot_size, shared_at = (GLOBAL ? gridDim.y * waves : waves) * slot_size;
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
+    const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
     const int64_t r = (int64_t)l * Tn + t;
     const T *row = pre + l * lstride + t * F;
+    const T *xcut_row = xcut ? xcut + row_columns(l, t, F, split) : nullptr;
     uint32_t n_buf = 0, first = ROW_NONE, prev = ROW_NONE;
     bool dense = false;
     auto flush = [&]() {
       if (n_buf == 0) return;
       if (!dense) {
-        uint32_t off = 0;
-        if (lane == 0) off = atomicAdd(&pool_count[p], n_buf + 1u);
-        off = __builtin_amdgcn_readfirstlane(off);
+        uint32_t off = own;
+        if (own_end - own > n_buf) own += n_buf + 1u;
+        else {
+          if (lane == 0) off = atomicAdd(&pool_count[p], n_buf + 1u);
+          off = __builtin_amdgcn_readfirstlane(off) + shared_at;
+        }
         if ((unsigned long long)off + n_buf + 1ull > pool_cap) dense = true;
         else {
           if (lane == 0) {
@@ -427,9 +473,35 @@ __global__ __launch_bounds__(256) void k_select_pass(
         if (V > 1) w[q] = *reinterpret_cast<const uint4 *>(row + cl);
         else w[q] = make_uint4(sizeof(T) == 2 ? ((uint32_t)Elem<T>::raw(row[cl]) << 16) : (uint32_t)Elem<T>::raw(row[cl]), 0, 0, 0);
         xc[q] = make_uint4(0, 0, 0, 0);
-        if (V > 1 && by_column) xc[q] = *reinterpret_cast<const uint4 *>(xcut + (int64_t)l * F + cl);
+        if (V > 1 && by_column) xc[q] = *reinterpret_cast<const uint4 *>(xcut_row + cl);
       }
       uint32_t m = 0;  // bit q*V + j: element j of vector q reaches the cut
+      // 16-bit values against their columns' bounds, two per instruction: x reaches b exactly if (b - 1) - x is negative (saturated),
+      // both as ordered integers.  NaNs of the type's upper end compare as what they are; one of the lower end, which the
+      // ranking puts on top as well, sends the step to the compares element by element.
+      bool compared = false;
+      if constexpr (sizeof(T) == 2 && V > 1) {
+        if (by_column) {
+          sel_i16x2 low = {0, 0};
+#pragma unroll
+          for (int q = 0; q < PASS_NV; ++q) {
+            const uint32_t w4[4] = {w[q].x, w[q].y, w[q].z, w[q].w}, b4[4] = {xc[q].x, xc[q].y, xc[q].z, xc[q].w};
+            uint32_t a = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const sel_i16x2 x = ordered16x2(w4[k]);
+              const sel_i16x2 d = __builtin_elementwise_sub_sat(__builtin_bit_cast(sel_i16x2, b4[k]), x);
+              a |= __builtin_bit_cast(uint32_t, d >> (short)15) & ((1u << (2 * k)) | (0x20000u << (2 * k)));
+              low = __builtin_elementwise_min(low, x);
+            }
+            if (on[q]) m |= ((a | (a >> 16)) & 0xFFu) << (q * V);
+          }
+          const short minus_inf = (short)~Elem<T>::INF16;
+          compared = ballot64(low.x < minus_inf || low.y < minus_inf) == 0;
+          if (!compared) m = 0;
+        }
+      }
+      if (!compared)
 #pragma unroll
       for (int q = 0; q < PASS_NV; ++q) {
         const int64_t col = c0 + (int64_t)q * 64 * V + (int64_t)lane * V;
@@ -438,7 +510,9 @@ __global__ __launch_bounds__(256) void k_select_pass(
         for (int j = 0; j < V; ++j) {
           const float xv = V > 1 ? vec_elem<T>(w[q], j) : Elem<T>::to_f32(Elem<T>::from_raw(sizeof(T) == 2 ? (w[q].x >> 16) : w[q].x));
           bool c;
-          if (by_column) c = xv >= vec_elem<T>(xc[q], j) || xv != xv;
+          if (by_column && sizeof(T) == 2)
+            c = ordered16(w4_elem(w[q], j)) > (int32_t)(int16_t)(uint16_t)w4_elem(xc[q], j) || xv != xv;
+          else if (by_column) c = xv >= vec_elem<T>(xc[q], j) || xv != xv;
           else {
             const float rv = rk(xv, col + j);
             c = cut_nan ? (rv != rv) : !(rv < cutf);
@@ -657,7 +731,7 @@ template <typename T, bool GLOBAL>
 __global__ __launch_bounds__(256) void k_select_level(
     const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t lstride, const float *mean,
     const float *denom, const SelState *st, uint32_t *hist, const uint32_t *row_first,
-    const uint2 *pool, unsigned long long pool_cap, int level) {
+    const uint2 *pool, unsigned long long pool_cap, int level, int split) {
   __shared__ uint32_t lh[NBINS];
   const int l = blockIdx.y, p = GLOBAL ? 0 : l;
   const SelState s = st[p];
@@ -665,8 +739,8 @@ __global__ __launch_bounds__(256) void k_select_level(
   for (int i = threadIdx.x; i < NBINS; i += blockDim.x) lh[i] = 0;
   __syncthreads();
   const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
+    const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
     visit_candidates<T, GLOBAL>(pre, Tn, F, lstride, l, t, rk, s.cut_key, row_first, pool + (unsigned long long)p * pool_cap,
       [&](bool act, uint32_t, uint32_t, uint32_t key) {
         if (act) {
@@ -687,13 +761,13 @@ template <typename T, bool GLOBAL>
 __global__ __launch_bounds__(256) void k_select_count(
     const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t lstride, const float *mean,
     const float *denom, const SelState *st, const uint32_t *row_first, const uint2 *pool,
-    unsigned long long pool_cap, uint32_t *row_gt, uint32_t *row_eq) {
+    unsigned long long pool_cap, uint32_t *row_gt, uint32_t *row_eq, int split) {
   const int l = blockIdx.y, p = GLOBAL ? 0 : l;
   const SelState s = st[p];
   if (s.path != PATH_ROWS) return;
   const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6, lane = lane_id();
-  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
+    const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
     uint32_t ngt = 0, neq = 0;
     visit_candidates<T, GLOBAL>(pre, Tn, F, lstride, l, t, rk, s.cut_key, row_first, pool + (unsigned long long)p * pool_cap,
       [&](bool act, uint32_t, uint32_t, uint32_t key) {
@@ -730,7 +804,7 @@ constexpr int SCAN_ITEMS = 4;
 template <bool GLOBAL>
 __global__ __launch_bounds__(SCAN_THREADS) void k_select_allot(
     const SelState *st, int64_t Tn, int64_t L, const uint32_t *row_gt, const uint32_t *row_eq,
-    uint32_t *allot, uint32_t *keep, int32_t *row_ptr, unsigned long long K) {
+    uint32_t *allot, uint32_t *keep, int32_t *row_ptr, unsigned long long K, int split) {
   const int p = blockIdx.x, tid = threadIdx.x;
   const unsigned long long budget = st[p].tie_budget;
   const int64_t nrows = GLOBAL ? Tn * L : Tn;
@@ -741,7 +815,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_select_allot(
 #pragma unroll
     for (int j = 0; j < SCAN_ITEMS; ++j) {
       const int64_t i = i0 + (int64_t)tid * SCAN_ITEMS + j;
-      r[j] = i < nrows ? (GLOBAL ? ((i % L) * Tn + i / L) : ((int64_t)p * Tn + i)) : -1;
+      // global order: by token, then layer, then the parts of the layer's row
+      const int64_t h = i / split;
+      r[j] = i < nrows ? (GLOBAL ? ((h % L) * Tn + h / L * split + (i & (split - 1))) : ((int64_t)p * Tn + i)) : -1;
       eq[j] = r[j] >= 0 ? row_eq[r[j]] : 0;
       gt[j] = r[j] >= 0 ? row_gt[r[j]] : 0;
       eq_sum += eq[j];
@@ -800,16 +876,20 @@ template <typename T, bool GLOBAL>
 __global__ __launch_bounds__(256) void k_select_emit(
     const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t lstride, const float *mean,
     const float *denom, const SelState *st, const uint32_t *row_first, const uint2 *pool,
-    unsigned long long pool_cap, const uint32_t *allot, const int32_t *row_ptr, int32_t *col_out, T *val_out) {
+    unsigned long long pool_cap, const uint32_t *allot, const int32_t *row_ptr, int32_t *col_out, T *val_out, int split,
+    int32_t *row_ptr_out) {
   const int l = blockIdx.y, p = GLOBAL ? 0 : l;
   const SelState s = st[p];
   if (s.path != PATH_ROWS) return;
   const int wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+  if (row_ptr_out && blockIdx.x == 0 && l == (int)L - 1 && threadIdx.x == 0) row_ptr_out[L * Tn / split] = row_ptr[L * Tn];
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
+    const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
+    const uint32_t col0 = (uint32_t)((t & (split - 1)) * F);
     const int64_t r = (int64_t)l * Tn + t;
     const int64_t base = row_ptr[r];
     const uint32_t my_allot = allot[r];
+    if (row_ptr_out && col0 == 0 && lane_id() == 0) row_ptr_out[r / split] = (int32_t)base;    // the token's first survivor
     uint32_t kept = 0, ties = 0;
     visit_candidates<T, GLOBAL>(pre, Tn, F, lstride, l, t, rk, s.cut_key, row_first, pool + (unsigned long long)p * pool_cap,
       [&](bool act, uint32_t col, uint32_t raw, uint32_t key) {
@@ -819,7 +899,7 @@ __global__ __launch_bounds__(256) void k_select_emit(
         uint64_t bk = ballot64(keepit);
         if (keepit) {
           int64_t pos = base + kept + mbcnt64(bk);
-          col_out[pos] = (int32_t)col;
+          col_out[pos] = (int32_t)(col0 + col);
           val_out[pos] = Elem<T>::from_raw(raw);
         }
         kept += (uint32_t)__popcll(bk);
@@ -1327,7 +1407,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_token_threshold(
     for (int li = 0; li < nl; ++li) {
       const int64_t l = l0 + li;
       const T *row = pre + l * lstride + t * F;
-      typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+      typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l * F);
       for (int64_t f = tid; f < F; f += SCAN_THREADS) {
         const uint32_t key = rank_key_of<T>(rk(Elem<T>::to_f32(row[f]), f));
         if ((key & prefix_mask) == prefix) atomicAdd(&lh[(key >> sh) & dm], 1u);
@@ -1347,7 +1427,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_token_threshold(
   for (int li = 0; li < nl; ++li) {
     const int64_t l = l0 + li;
     const T *row = pre + l * lstride + t * F;
-    typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+    typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l * F);
     uint32_t g = 0, e = 0;
     for (int64_t f = tid; f < F; f += SCAN_THREADS) {
       const uint32_t key = rank_key_of<T>(rk(Elem<T>::to_f32(row[f]), f));
@@ -1380,7 +1460,7 @@ __global__ __launch_bounds__(256) void k_token_emit(
   constexpr int KB = Elem<T>::KEYBITS;
   const int l = blockIdx.y;
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
-  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l, F);
+  typename RankOf<T, GLOBAL>::type rk = RankOf<T, GLOBAL>::make(mean, denom, l * F);
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
     const int64_t r = (int64_t)l * Tn + t;
     const uint32_t thr = thr_key[GLOBAL ? t : r];
@@ -1462,16 +1542,32 @@ static int run_tokentopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
 
 // ---- host side ------------------------------------------------------------------------
 struct SelLayout {
-  size_t off_state, off_hist, off_poolcnt, off_sample, off_first, off_gt, off_eq, off_allot, off_keep, off_xcut, off_pool, total;
+  size_t off_state, off_hist, off_poolcnt, off_sample, off_first, off_gt, off_eq, off_allot, off_keep, off_rows, off_xcut, off_pool, total;
   unsigned long long pool_cap;  // entries per problem
+  uint32_t slot_size;           // of them, entries that belong to each wavefront of the pass
   int nprob, sample_n;          // problems; keys of the sample gathered from the matrix, per problem
 };
 
-static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode) {
+// Into how many parts the rows are cut (row_columns): 8192 wavefronts fill the chip twice, a part of 1024 columns is half a step
+// of the pass.  77 tokens of L = 12, F = 24576, bf16, in 8 parts: pass 71 -> 21 us, count 28 -> 9, emit 21 -> 8; 8192 rows and
+// more gain nothing that the one workgroup of k_select_allot, which walks all rows, does not lose.
+static int row_split(int64_t T, int64_t F, int64_t L) {
+  int split = 1;
+  while (L * T * split < 8192 && F % (split * 16) == 0 && F / (split * 2) >= 1024) split *= 2;
+  return split;
+}
+
+// Workgroups of the pass along the (cut) rows of a layer: what the chip holds at once, four per compute unit, or eight rows each.
+static int pass_blocks(int64_t rows, int64_t L) {
+  const int64_t most = 1024 / L > 0 ? 1024 / L : 1, want = clt_ceil_div(rows, 8);
+  return (int)(want < most ? want : most);
+}
+
+static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode, int split) {
   SelLayout lo;
   lo.nprob = mode == CLT_TOPK_GLOBAL ? 1 : (int)L;
-  const size_t R = (size_t)(L * T);
-  const unsigned long long rows_p = mode == CLT_TOPK_GLOBAL ? (unsigned long long)R : (unsigned long long)T;
+  const size_t R = (size_t)(L * T * split);
+  const unsigned long long rows_p = mode == CLT_TOPK_GLOBAL ? (unsigned long long)R : (unsigned long long)(T * split);
   const unsigned long long N = (unsigned long long)T * F * (mode == CLT_TOPK_GLOBAL ? L : 1);
   unsigned long long K = (unsigned long long)k * T;
   if (K > N) K = N;
@@ -1479,6 +1575,12 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   unsigned long long cap = 4ull * K + 2ull * rows_p + 4096ull;
   const unsigned long long hard = N + 2ull * rows_p + 4096ull;
   if (cap > hard) cap = hard;
+  // In front of those, a part for each wavefront of the pass, which holds its candidates unless they are more than 2 K's
+  // share.  A counter per problem, asked for every row's place, was what bounded the pass: requests to one address are served
+  // one by one, 15 ns apart (36 000 rows ranked together: 590 us, whatever the rows held).
+  const unsigned long long waves = 4ull * (unsigned long long)pass_blocks(T * split, L) * (mode == CLT_TOPK_GLOBAL ? (unsigned long long)L : 1ull);
+  lo.slot_size = (uint32_t)((2ull * K + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull);
+  cap += waves * lo.slot_size;
   if (cap > 0xFFF00000ull) cap = 0xFFF00000ull;
   lo.pool_cap = cap;
   // A sample with e keys above the threshold gives a cut with up to (1.25 + 6 / sqrt(e) + 17 / e) K candidates:
@@ -1500,6 +1602,7 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   lo.off_eq = take(4 * R);
   lo.off_allot = take(4 * R);
   lo.off_keep = take(4 * R);
+  lo.off_rows = take(split > 1 ? 4 * (R + 1) : 0);                              // row pointers of the cut rows
   lo.off_xcut = take(mode == CLT_TOPK_GLOBAL ? 4 * (size_t)F * (size_t)L : 0);   // per-column bounds, element type
   lo.off_pool = take(8 * (size_t)cap * (size_t)lo.nprob);
   lo.total = o;
@@ -1512,7 +1615,8 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
                          char *ws, hipStream_t stream) {
   constexpr int KB = Elem<T>::KEYBITS;
   const int mode = GLOBAL ? CLT_TOPK_GLOBAL : CLT_TOPK_PER_LAYER;
-  const SelLayout lo = sel_layout(Tn, F, L, k, mode);
+  const int split = row_split(Tn, F, L);
+  const SelLayout lo = sel_layout(Tn, F, L, k, mode, split);
   SelState *st = (SelState *)(ws + lo.off_state);
   uint32_t *hist = (uint32_t *)(ws + lo.off_hist);
   uint32_t *poolcnt = (uint32_t *)(ws + lo.off_poolcnt);
@@ -1533,18 +1637,19 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
     k_sample_cut<T, SAMPLE_PRE_N><<<nprob, SCAN_THREADS, 0, stream>>>(sample, lo.sample_n, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
   else
     k_sample_cut<T, 0><<<nprob, SCAN_THREADS, 0, stream>>>(sample, lo.sample_n, N, K, st, hist, poolcnt, nullptr, PATH_ROWS);
-  // two rows per wavefront: many more blocks than fit at once, so rows of very different
-  // candidate counts balance out over the CUs
-  int gx = (int)clt_ceil_div(Tn, 8);
-  if (gx > 65535 * 8) gx = 65535 * 8;
-  dim3 grid(gx, (unsigned)L);
   T *xcut = nullptr;
   if (GLOBAL && V > 1) {
     xcut = (T *)(ws + lo.off_xcut);
     k_col_cut<T><<<(unsigned)clt_ceil_div(L * F, 256), 256, 0, stream>>>(mean, denom, st, F, L, xcut);
   }
+  // from here on the rows are the cut ones
+  int32_t *const row_ptr_out = split > 1 ? row_ptr : nullptr;
+  if (split > 1) row_ptr = (int32_t *)(ws + lo.off_rows);
+  Tn *= split;
+  F /= split;
+  const dim3 grid((unsigned)pass_blocks(Tn, L), (unsigned)L);
   for (int phase = 0; phase < 2; ++phase) {
-    k_select_pass<T, V, GLOBAL><<<grid, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, poolcnt, pool, lo.pool_cap, first, phase, xcut);
+    k_select_pass<T, V, GLOBAL><<<grid, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, poolcnt, pool, lo.pool_cap, first, phase, xcut, split, lo.slot_size);
     k_select_scan<T><<<nprob, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, phase, 0);
   }
   int gx2 = (int)clt_ceil_div(Tn, 4);
@@ -1554,13 +1659,13 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
   dim3 grid2(gx2, (unsigned)L);
   const int nlev = KB == 32 ? 3 : 2;
   for (int level = 1; level < nlev; ++level) {
-    k_select_level<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, first, pool, lo.pool_cap, level);
+    k_select_level<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, first, pool, lo.pool_cap, level, split);
     k_select_scan<T><<<nprob, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 2, level);
   }
-  k_select_count<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, first, pool, lo.pool_cap, rgt, req);
-  k_select_allot<GLOBAL><<<nprob, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K);
+  k_select_count<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, first, pool, lo.pool_cap, rgt, req, split);
+  k_select_allot<GLOBAL><<<nprob, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K, split);
   if (GLOBAL) k_rowptr_scan<<<1, SCAN_THREADS, 0, stream>>>(keep, L * Tn, row_ptr);
-  k_select_emit<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, first, pool, lo.pool_cap, allot, row_ptr, col, val);
+  k_select_emit<T, GLOBAL><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, first, pool, lo.pool_cap, allot, row_ptr, col, val, split, row_ptr_out);
   return clt_check_launch();
 }
 
@@ -1620,7 +1725,7 @@ struct TileLayout {
 
 static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dtype) {
   TileLayout tl;
-  tl.sel = sel_layout(T, F, L, k, CLT_TOPK_PER_LAYER);
+  tl.sel = sel_layout(T, F, L, k, CLT_TOPK_PER_LAYER, 1);
   const int segw = dtype != CLT_F32 ? 128 : 64;
   tl.nseg = (int)(collect_grid_rows(F) / segw);   // whole feature tiles too (COLLECT_TILE_ROWS is the tile's side)
   const int64_t Tp = collect_grid_rows(T);   // the epilogue's books cover whole token tiles
@@ -1703,11 +1808,9 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
   const unsigned long long N = (unsigned long long)Tn * (unsigned long long)F;
   unsigned long long K = (unsigned long long)k * (unsigned long long)Tn;
   if (K > N) K = N;
-  int gx = (int)clt_ceil_div(Tn, 8);
-  if (gx > 65535 * 8) gx = 65535 * 8;
   // retry of the layers whose cut failed: streaming pass from the bottom key over `pre`
-  k_select_pass<T, VV, false><<<dim3(gx, (unsigned)L), 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist,
-                                                                        poolcnt, pool, lo.pool_cap, first, 1, nullptr);
+  k_select_pass<T, VV, false><<<dim3((unsigned)pass_blocks(Tn, L), (unsigned)L), 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist,
+                                                                        poolcnt, pool, lo.pool_cap, first, 1, nullptr, 1, lo.slot_size);
   k_select_scan<T><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 1, 0);
   int gx2 = (int)clt_ceil_div(Tn, 4);
   int maxgx2 = (int)clt_ceil_div(256 * 8, L);
@@ -1717,7 +1820,7 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
   const int nlev = KB == 32 ? 3 : 2;
   for (int level = 1; level < nlev; ++level) {
     k_pool_hist<T><<<dim3(256, (unsigned)L), 256, 0, stream>>>(st, tmeta, tl.ntile, tpool, tl.tpool_cap, hist, level);
-    k_select_level<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist, first, pool, lo.pool_cap, level);
+    k_select_level<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist, first, pool, lo.pool_cap, level, 1);
     k_select_scan<T><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 2, level);
   }
   dim3 grid3((unsigned)clt_ceil_div(Tn, 256), (unsigned)tl.nseg, (unsigned)L);
@@ -1726,11 +1829,11 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
   const int64_t Tp = collect_grid_rows(Tn);
   k_tile_count<T><<<grid3, 256, 0, stream>>>((int)Tn, (int)Tp, st, meta, tl.nseg, tpool, tl.tpool_cap, cgt, ceq);
   k_row_prefix<<<dim3((unsigned)clt_ceil_div(Tn, 64), (unsigned)L), 64, 0, stream>>>(Tn, Tp, st, tl.nseg, cgt, ceq, pgt, peq, rgt, req);
-  k_select_count<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, rgt, req);
-  k_select_allot<false><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K);
+  k_select_count<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, rgt, req, 1);
+  k_select_allot<false><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K, 1);
   k_tile_emit<T><<<grid3, 256, 0, stream>>>((int)Tn, (int)Tp, st, meta, tl.nseg, tpool, tl.tpool_cap, pgt, peq, allot, row_ptr, col, val);
   k_select_emit<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, allot,
-                                                     row_ptr, col, val);
+                                                     row_ptr, col, val, 1, nullptr);
   return clt_check_launch();
 }
 
@@ -1962,7 +2065,7 @@ extern "C" size_t clt_batchtopk_workspace_bytes(int64_t T, int64_t F, int64_t L,
   (void)dtype;
   if (T <= 0 || F <= 0 || L <= 0) return 256;
   if (k < 0) k = 0;
-  return sel_layout(T, F, L, k, mode).total;
+  return sel_layout(T, F, L, k, mode, row_split(T, F, L)).total;
 }
 
 extern "C" int clt_batchtopk_select(const void *pre, int64_t T, int64_t F, int64_t L, int64_t pre_layer_stride,
