@@ -71,6 +71,8 @@ _SIGNATURES = {
     "clt_decode_tiles_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64, _i64]),
     "clt_decode_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int, _i64,
                                 _vp, _sz, _vp]),
+    "clt_decode_thin_wanted": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _int, _int]),
+    "clt_decode_thin": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int, _vp]),
     "clt_decode_sparse_if_over": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int,
                                          _i64, _vp]),
     "clt_decode_route": (_int, [_i64, _i64, _i64, _i64, _int, _int, _sz]),

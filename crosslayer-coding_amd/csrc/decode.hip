@@ -6,6 +6,7 @@
 // decoder vector of every active feature (feature-major packing: one contiguous
 // d-element run, 16 bytes per lane per load) and accumulates in fp32 registers; the
 // output row is written once.
+#include <cmath>
 #include <type_traits>
 #include "clt_common.h"
 
@@ -703,6 +704,190 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(quarter_min
         }
       }
     }
+  }
+}
+
+// ---- thin lists --------------------------------------------------------------------------------------
+// Few survivors per (source, token) - all layers ranked together, a small k: a decoder row is then used by one or two tokens of
+// the batch, so keeping an eighth of a matrix in an L2 gains nothing, while the partial rows that the schedule by sources reads
+// and writes for every pair are most of its traffic.  Here a wavefront takes one (target, token) and a quarter of the
+// columns over all sources: the token's lists become one list, four quarter rows are fetched per load (as above), the sums
+// stay in registers and the output row is written once.  XCD x works on quarter x % 4 of one half of the tokens.
+// T = 3000, L = 12, F = 24576, d = 768, bf16, 200 survivors per token over all layers: 0.85 ms, 7.1 TB/s of rows out of the caches
+// and HBM (by sources 1.53); bounded by the rows in flight: 93 registers leave five wavefronts per SIMD with 16 quarter rows each.
+// Workgroups of 8 wavefronts held to 80 registers spill and take 1.1 ms.
+// ThinBatch: 4 UU rows of the (up to 64) survivors held one per lane.  In the last batch of a chunk the places past the
+// list's end stay zero, so that a row's infinity meets no weight but its own.
+template <typename T, int HQ, int HTAIL, int UU> struct ThinBatch {
+  uint4 wq[UU][HQ];
+  uint2 wt8[UU];
+  float v[UU];
+  __device__ __forceinline__ void load(const T *wpart, int64_t pitch, int32_t my_row, float my_val, int i0, int n, int ll, int grp) {
+    constexpr int V = WVec<T>::V;
+    const bool whole = i0 + QROWS * UU <= n;
+#pragma unroll
+    for (int u = 0; u < UU; ++u) {
+      const int idx = i0 + QROWS * u + grp;
+      const T *wrow = wpart + (int64_t)__shfl(my_row, idx) * pitch;
+      v[u] = __shfl(my_val, idx);
+      if (whole || idx < n) {
+#pragma unroll
+        for (int c = 0; c < HQ; ++c) wq[u][c] = *reinterpret_cast<const uint4 *>(wrow + c * QLANES * V + ll * V);
+        if (HTAIL) wt8[u] = *reinterpret_cast<const uint2 *>(wrow + HQ * QLANES * V + ll * (V / 2));
+      } else {
+        v[u] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < HQ; ++c) wq[u][c] = make_uint4(0, 0, 0, 0);
+        wt8[u] = make_uint2(0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void consume(float *acc) const {
+    constexpr int V = WVec<T>::V;
+    if constexpr (sizeof(T) == 2) {
+      static_assert(UU % 2 == 0, "rows are multiplied in pairs");
+#pragma unroll
+      for (int u = 0; u < UU; u += 2) {
+        const uint32_t vv = raw16_of<T>(v[u]) | (raw16_of<T>(v[u + 1]) << 16);
+#pragma unroll
+        for (int c = 0; c < HQ; ++c) WVec<T>::dot16(acc + c * V, wq[u][c], wq[u + 1][c], vv);
+        if (HTAIL) WVec<T>::dot8(acc + HQ * V, wt8[u], wt8[u + 1], vv);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < UU; ++u) {
+#pragma unroll
+        for (int c = 0; c < HQ; ++c) WVec<T>::fma16(acc + c * V, wq[u][c], v[u]);
+        if (HTAIL) WVec<T>::fma8(acc + HQ * V, wt8[u], v[u]);
+      }
+    }
+  }
+};
+
+// A token with a list of more than THIN_LONG (batch-wide top-k gives some tokens many times the average) is left to the end, when
+// the workgroup's wavefronts share its chunks of 64 and add their sums in LDS.
+constexpr int THIN_WAVES = 4, THIN_LONG = 256;
+template <typename T, int HQ, int HTAIL>
+__global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin(
+    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
+    const float *__restrict__ bias_sum, const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d,
+    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch) {
+  constexpr int V = WVec<T>::V, UU = 2, R = QROWS * UU;
+  constexpr int NACC = HQ * V + (HTAIL ? V / 2 : 0);      // columns per lane: d / 64
+  __shared__ int32_t totals[THIN_WAVES];
+  __shared__ float shares[THIN_WAVES][NACC][QLANES];
+  const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ll = lane & (QLANES - 1), grp = lane / QLANES;
+  const int cpart = (int)(blockIdx.x & 3), half = (int)((blockIdx.x >> 2) & 1);
+  const int64_t idx = blockIdx.x >> 3, in_half = (Tn + 1) / 2, per_t = (in_half + THIN_WAVES - 1) / THIN_WAVES;
+  const int64_t t = t_end - 1 - idx / per_t;               // longest first
+  const int64_t in0 = (idx % per_t) * THIN_WAVES;          // of the half: the first wavefront's token
+  const T *wpart = wp + (int64_t)cpart * (d / 4);
+
+  // where source `lane`'s list of a token begins, less what comes before it in the one list, and where it ends there
+  int32_t list_at, list_end, total;
+  auto find_list = [&](int64_t tok) {
+    list_at = list_end = 0;
+    if (lane <= t && ((src_mask >> lane) & 1ull)) {
+      list_at = row_ptr[lane * Tn + tok];
+      list_end = row_ptr[lane * Tn + tok + 1] - list_at;
+    }
+    list_at += list_end;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t up = __shfl_up(list_end, o);
+      if (lane >= o) list_end += up;
+    }
+    list_at -= list_end;
+    total = __builtin_amdgcn_readlane(list_end, 63);
+  };
+  struct Entry { int32_t row; T v; };
+  auto fetch = [&](int32_t i) {
+    Entry e{0, Elem<T>::from_raw(0u)};
+    int s = 0;
+    for (int u = 0; u < (int)t; ++u) s += i >= __builtin_amdgcn_readlane(list_end, u) ? 1 : 0;
+    const int32_t j = __shfl(list_at, s) + i;
+    if (i < total) {
+      e.row = (int32_t)decoder_slot(tying, s, t, L) * (int32_t)F + col[j];
+      e.v = val[j];
+    }
+    return e;
+  };
+  float acc[NACC];
+  // every `step`-th chunk of the token's list from chunk `from` on; the lane groups' sums end up as ((g0 + g1) + (g2 + g3))
+  auto gather = [&](int from, int step) {
+#pragma unroll
+    for (int j = 0; j < NACC; ++j) acc[j] = 0.0f;
+    Entry next = fetch(from * 64 + lane);
+    for (int32_t j0 = from * 64; j0 < total; j0 += step * 64) {
+      const int32_t my_row = next.row;
+      const float my_val = Elem<T>::to_f32(next.v);
+      const int n = total - j0 < 64 ? total - j0 : 64;
+      ThinBatch<T, HQ, HTAIL, UU> ra, rb;
+      ra.load(wpart, pitch, my_row, my_val, 0, n, ll, grp);
+      if (j0 + step * 64 < total) next = fetch(j0 + step * 64 + lane);
+      for (int i0 = 0; i0 < n; i0 += 2 * R) {
+        if (i0 + R < n) rb.load(wpart, pitch, my_row, my_val, i0 + R, n, ll, grp);
+        ra.consume(acc);
+        if (i0 + R < n) {
+          if (i0 + 2 * R < n) ra.load(wpart, pitch, my_row, my_val, i0 + 2 * R, n, ll, grp);
+          rb.consume(acc);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NACC; ++j) {
+      acc[j] += __shfl_xor(acc[j], 16);
+      acc[j] += __shfl_xor(acc[j], 32);
+    }
+  };
+  auto emit = [&](int64_t tok) {
+    if (grp != 0) return;
+    const int64_t col0 = (int64_t)cpart * (d / 4), at = (t * Tn + tok) * d;
+    auto emit4 = [&](int64_t o, const float *a) {
+      float4 y = make_float4(a[0], a[1], a[2], a[3]);
+      if (bias_sum) { const float4 b = *reinterpret_cast<const float4 *>(bias_sum + t * d + o); y.x += b.x; y.y += b.y; y.z += b.z; y.w += b.w; }
+      if (skip_add) { const float4 b = *reinterpret_cast<const float4 *>(skip_add + at + o); y.x += b.x; y.y += b.y; y.z += b.z; y.w += b.w; }
+      if (out_f32 || sizeof(T) == 4) *reinterpret_cast<float4 *>((float *)out + at + o) = y;
+      else *reinterpret_cast<uint2 *>((uint16_t *)out + at + o) = make_uint2(pack_pair<T>(y.x, y.y), pack_pair<T>(y.z, y.w));
+    };
+#pragma unroll
+    for (int c = 0; c < HQ; ++c)
+#pragma unroll
+      for (int j = 0; j < V; j += 4) emit4(col0 + c * QLANES * V + ll * V + j, acc + c * V + j);
+    if constexpr (HTAIL && V == 8) emit4(col0 + HQ * QLANES * V + ll * 4, acc + HQ * V);
+  };
+
+  // w < 0: each wavefront its own token; w >= 0: all of them wavefront w's, if that was left (one instance of the loop for both)
+  for (int w = -1; w < THIN_WAVES; ++w) {
+    if (w == 0) __syncthreads();
+    const int64_t in = in0 + (w < 0 ? wv : w), tok = half * in_half + in;
+    if (w < 0) {
+      const bool on = in < in_half && tok < Tn;
+      total = 0;
+      if (on) find_list(tok);
+      if (lane == 0) totals[wv] = total;
+      if (!on || total > THIN_LONG) continue;
+    } else {
+      if (totals[w] <= THIN_LONG) continue;                // the same for the whole workgroup
+      find_list(tok);
+    }
+    gather(w < 0 ? 0 : wv, w < 0 ? 1 : THIN_WAVES);
+    if (w >= 0) {
+      if (grp == 0) {
+#pragma unroll
+        for (int j = 0; j < NACC; ++j) shares[wv][j][ll] = acc[j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < NACC; ++j) {
+        acc[j] = 0.0f;
+#pragma unroll
+        for (int o = 0; o < THIN_WAVES; o += 2) acc[j] += shares[o][j][ll] + shares[o + 1][j][ll];
+      }
+      __syncthreads();
+    }
+    if (w < 0 || wv == w) emit(tok);
   }
 }
 
@@ -1578,6 +1763,88 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
 }
 
 }  // namespace
+
+template <typename T>
+static int launch_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *wp, const float *bias_sum,
+                              const float *skip_add, void *out, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
+                              int64_t t_end, uint64_t src_mask, int out_f32, hipStream_t stream) {
+  constexpr int V = WVec<T>::V;
+  const int64_t blocks = 8 * clt_ceil_div((Tn + 1) / 2, THIN_WAVES) * (t_end - t_begin);
+  if (blocks > 2147483647LL) return CLT_ERR_RANGE;
+  const int hq = (int)(d / 64) / V, htail = ((int)(d / 64) % V) != 0;
+#define CLT_THIN(HQN, HTN)                                                                                            \
+  k_decode_thin<T, HQN, HTN><<<(unsigned)blocks, THIN_WAVES * 64, 0, stream>>>(row_ptr, col, (const T *)val, (const T *)wp, bias_sum, \
+      skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)))
+  if constexpr (sizeof(T) == 2) {
+    if (hq == 1 && !htail) CLT_THIN(1, 0);
+    else if (hq == 1) CLT_THIN(1, 1);
+    else if (hq == 2) CLT_THIN(2, 0);
+    else CLT_THIN(4, 0);
+  } else {
+    if (hq == 2) CLT_THIN(2, 0);
+    else if (hq == 3) CLT_THIN(3, 0);
+    else CLT_THIN(4, 0);
+  }
+#undef CLT_THIN
+  return clt_check_launch();
+}
+
+// What k_decode_thin takes: row numbers over all decoders in 32 bits, rows in quarters that a lane group reads whole.
+static bool decode_thin_ok(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int tying, int dtype) {
+  if (!clt_model_dtype(dtype) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return false;
+  if (T <= 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || d <= 0 || d % 256 != 0) return false;
+  const int64_t n_dec = tying == CLT_TYING_NONE ? L * (L + 1) / 2 : L;
+  return quarter_shape_ok(d, clt_elem_bytes(dtype)) && n_dec * F <= 0x7FFFFFFFll && L * T < 0x7FFFFFFFll;
+}
+
+// What the gathers move: bytes of decoder rows, bytes of those that some token refers to, (source, target, token) triples.
+struct GatherWork { double bytes, distinct, triples; };
+static GatherWork gather_work(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const double row = (double)d * clt_elem_bytes(dtype), pairs = 0.5 * targets * (2 * L - targets + 1), list = (double)entries / L;
+  GatherWork g;
+  g.bytes = list * pairs * row;
+  g.distinct = (tying == CLT_TYING_NONE ? pairs : (double)L) * F * (1.0 - exp(-list / F)) * row;
+  g.triples = pairs * T;
+  return g;
+}
+
+// Against the schedules by sources (k_decode_quarter, k_decode_line), which move rows at 17 TB/s out of the L2s, bring each one there
+// from HBM and read and write the partial rows of every triple, and against the decodes from LDS tiles.  This kernel, from what it
+// measured (bf16 and float32; L 2 - 16, d 512 - 2048, F 1024 - 24576, T 32 - 8000, 1 - 200 survivors per source and token): 9.5
+// TB/s, as much time again for a row's first use, 0.25 ns per triple, and no less than a workgroup's chain over its lists, or over
+// one of some thousand entries, which is what a top-k over the batch gives a single token.  Within 15 %, but for rows used more than
+// 20 times, which it does faster.  us, schedule by sources / this: T = 3000, L = 12, F = 24576, d = 768, bf16, 200 survivors per
+// token over all layers 1530 / 854, 20 695 / 224; per layer 16: 1253 / 747; T = 1000, 50: 1100 / 790; T = 300, 200: 877 / 1078;
+// T = 77, 200: 340 / 356; float32, T = 600, 200: 2790 / 3910.
+extern "C" int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  if (entries < 0 || !decode_thin_ok(T, d, F, L, targets, tying, dtype)) return 0;
+  const GatherWork g = gather_work(T, d, F, L, targets, entries, tying, dtype);
+  const double flow = g.bytes / 9.5e6 + g.distinct / 10e6 + g.triples * 0.25e-3, longest = entries < 4000 ? (double)entries : 4000.0;
+  const double chain = 0.1 * (double)entries / T > 0.025 * longest ? 0.1 * (double)entries / T : 0.025 * longest;
+  const double thin = (flow > chain ? flow : chain) + 12;
+  return thin < 0.95 * (g.bytes / 17e6 + g.distinct / 6.3e6 + g.triples * (double)d * 16 / 3.2e6 + 5) &&
+         thin < clt_decode_tiles_us(T, d, F, L, targets, entries, tying, dtype) &&
+         thin < clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);
+}
+
+extern "C" int clt_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                               const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                               int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
+                               void *stream) {
+  if (!clt_model_dtype(dtype)) return CLT_ERR_DTYPE;
+  if (T < 0 || t_begin < 0 || t_end > L || t_begin > t_end) return CLT_ERR_ARG;
+  if (T == 0 || t_begin == t_end) return CLT_OK;
+  if (!decode_thin_ok(T, d, F, L, t_end - t_begin, tying, dtype)) return CLT_ERR_ARG;
+  if (!row_ptr || !col || !val || !w_packed || !out) return CLT_ERR_ARG;
+  if (!clt_aligned16(w_packed) || !clt_aligned16(out) || (bias_sum && !clt_aligned16(bias_sum)) || (skip_add && !clt_aligned16(skip_add)))
+    return CLT_ERR_ALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == CLT_BF16)
+    return launch_decode_thin<bf16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
+  if (dtype == CLT_F16)
+    return launch_decode_thin<f16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
+  return launch_decode_thin<float>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
+}
 
 extern "C" size_t clt_decode_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L) {
   (void)F;

@@ -368,18 +368,20 @@ static bool row_shape_ok(const RowLayout &l, int64_t row_bytes) {
 
 }  // namespace
 
+struct RowTimes { double rows, sparse; };   // us; the first large for what the tiles do not take
+
 // Both routes priced from what they measured (L 4 - 16, d 256 - 2048, F 2048 - 16384, T 64 - 3000, 20 - 200 survivors per token):
 // the gather moves its rows at 23 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage of the tiles takes
 // 1.4 us plus 5.7 ns per record, but no less than the 2.4 us in which 64 KB come into LDS, and the longest workgroup bounds a
 // launch of few.  us, gather / tiles: L = 12, d = 768, F = 6144, 1024 tokens: 667 / 941 with 20 per token, 1052 / 1045 with
 // 60, 2328 / 1798 with 200; L = 6, d = 1024, F = 16384, 3000 tokens x 200: 2599 / 2909; L = 16, d = 256, F = 2048, 1024 x 60:
 // 659 / 354.
-extern "C" int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
-                                      int dtype) {
-  if (dtype != CLT_F32 || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return 0;
-  if (T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return 0;
+static RowTimes row_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const RowTimes no = {1e30, 0};
+  if (dtype != CLT_F32 || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;
+  if (T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return no;
   const RowLayout l = row_layout(T, d, F, L, entries);
-  if (!row_shape_ok(l, clt_pitch(d, 4) * 4)) return 0;
+  if (!row_shape_ok(l, clt_pitch(d, 4) * 4)) return no;
   const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
   const double sparse_us = rows * d * 4 / 23e6 + pairs * T * d * 16 / 3.6e6;
   const double run = (double)entries / ((double)l.p.stages * T);
@@ -387,7 +389,17 @@ extern "C" int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L
   const double stage_us = 1.4 + recs * 0.0057;
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
   const double rows_us = (stages > longest ? stages : longest) * (stage_us > 2.4 ? stage_us : 2.4) + 20 + entries * 2e-5;
-  return rows_us < 0.95 * sparse_us;
+  return {rows_us, sparse_us};
+}
+
+extern "C" int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
+                                      int dtype) {
+  const RowTimes t = row_times(T, d, F, L, targets, entries, tying, dtype);
+  return t.rows < 0.95 * t.sparse;
+}
+
+double clt_decode_rows_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  return row_times(T, d, F, L, targets, entries, tying, dtype).rows;
 }
 
 extern "C" size_t clt_decode_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {

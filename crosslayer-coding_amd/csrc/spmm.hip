@@ -796,18 +796,20 @@ static int launch_grad(const int32_t *list_ptr, const int32_t *list_tok, const i
 
 }  // namespace
 
+struct TileTimes { double tiles, sparse; };   // us; the first large for what the tiles do not take
+
 // Both routes priced from what they measured (bf16; L 2 - 24, d 256 - 2048, F 4096 - 32768, T 256 - 8192, 17 - 216 survivors
 // per token): the gather moves its rows at 17 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage
 // of the tiles takes 1.0 us plus 20.5 ns per batch, but no less than the 2.24 us in which 64 KB come into LDS, and the
 // longest workgroup bounds a launch of few.  At the line the two differ by less than a fifth either way: e.g. L = 12,
 // d = 768, F = 24576: 200 survivors per token 6.25 / 3.31 ms at T = 4096, 2.03 / 1.57 at 1024, 1.23 / 1.25 at 512; 50 per
 // token 2.58 / 1.71 ms at 4096, 1.43 / 1.55 at 2048.
-extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
-                                       int dtype) {
-  if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return 0;
-  if (T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return 0;
+static TileTimes tile_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const TileTimes no = {1e30, 0};
+  if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;
+  if (T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return no;
   const SpLayout l = tile_layout(T, d, F, L, targets, entries);
-  if (!sp_shape_ok(l, clt_pitch(d, 2) * 2)) return 0;
+  if (!sp_shape_ok(l, clt_pitch(d, 2) * 2)) return no;
   // (source, target) pairs of the last `targets` layers, and the survivors they gather
   const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
   const double sparse_us = rows * d * 2 / 17e6 + pairs * T * d * 16 / 3.2e6;
@@ -815,7 +817,17 @@ extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t 
   const double stage_us = 1.0 + l.p.groups_per_part * (per_batch > 1 ? per_batch : 1) * 0.0205;
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
   const double tiles_us = (stages > longest ? stages : longest) * (stage_us > 2.24 ? stage_us : 2.24) + 20 + entries * 1.25e-5;
-  return tiles_us < 0.95 * sparse_us;
+  return {tiles_us, sparse_us};
+}
+
+extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
+                                       int dtype) {
+  const TileTimes t = tile_times(T, d, F, L, targets, entries, tying, dtype);
+  return t.tiles < 0.95 * t.sparse;
+}
+
+double clt_decode_tiles_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  return tile_times(T, d, F, L, targets, entries, tying, dtype).tiles;
 }
 
 extern "C" int64_t clt_decode_tiles_max_entries(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets) {

@@ -932,8 +932,9 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
     """Reconstructions [L, T, d] for targets [t_begin, t_end) (decoder.py:176-340).
 
     With a workspace and a batch large enough to fill the GPU a gather from LDS tiles (16 bits: ``clt_decode_tiles`` on the
-    matrix cores; fp32: ``clt_decode_rows``) or one of the XCD-sliced gathers from the L2s is used, whichever
-    ``clt_decode_tiles_wanted`` / ``clt_decode_rows_wanted`` prices lower."""
+    matrix cores; fp32: ``clt_decode_rows``) or one of the XCD-sliced gathers from the L2s is used, for few survivors per
+    source and token ``clt_decode_thin``, whichever ``clt_decode_thin_wanted`` / ``clt_decode_tiles_wanted`` /
+    ``clt_decode_rows_wanted`` price lowest."""
     nat.require_device(w_packed, "decode_sparse")
     L, T, F = surv.L, surv.T, surv.F
     t_end = L if t_end is None else t_end
@@ -956,6 +957,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
     need = lib.clt_decoder_slab_elems(d, F, L, nat.TYING[tying], nat.dtype_code(surv.dtype))
     if need < 0 or w_packed.numel() < need:
         raise nat.CLTNativeError(f"decode_sparse: packed decoders hold {w_packed.numel()} elements, the kernels index {need}")
+    sliced = ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(),
+                                                     d * w_packed.element_size())
     if (ws is not None and tying != "per_target" and feat_offset is None and feat_scale is None
             and _aligned16(w_packed, bias_sum, skip_add, out)):
         # the survivor total: exact, or (a threshold list, sized for any batch) the last one seen for this shape, or 1 %
@@ -965,6 +968,13 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
         if total is None:
             total = L * T * F // 100
         wide = surv.dtype == torch.float32
+        if sliced and total and lib.clt_decode_thin_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying],
+                                                           nat.dtype_code(surv.dtype)):
+            code = lib.clt_decode_thin(nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum),
+                                       nat.ptr(skip_add), nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin, t_end,
+                                       src_mask & ((1 << 64) - 1), nat.dtype_code(surv.dtype), 1 if out_f32 else 0, _stream(w_packed))
+            nat.check(code, "clt_decode_thin")
+            return out
         if total and not wide and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
             # room for twice that many, or what the records can count where that is less
             cap = total if exact else min(surv.capacity, 2 * total + 65536, lib.clt_decode_tiles_max_entries(T, d, F, L, t_end - t_begin))
@@ -985,8 +995,7 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
             nat.check(code, "clt_decode_rows")
             return out
     wbuf, wbytes = None, 0
-    if ws is not None and _wants_sliced_decode(T * (t_end - t_begin), w_packed.numel() * w_packed.element_size(),
-                                               d * w_packed.element_size()):
+    if sliced:
         wbytes = lib.clt_decode_workspace_bytes(T, d, F, L)
         wbuf = ws.get("decode", wbytes)
     code = lib.clt_decode_sparse(
