@@ -688,7 +688,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
         // candidate of its half row into the wavefront's list, at the candidate's ordered position; then
         // the lanes take one candidate each: 64 consecutive pool entries per store instruction, and the
         // number of rounds is the piece's count / 64 instead of the fullest row's count.
-        auto emit_piece = [&](const uint32_t (&Wh)[NWL], uint32_t first, uint32_t n, uint2 *dst) {
+        auto emit_piece = [&](const uint32_t (&Wh)[NWL], int h, uint32_t first, uint32_t n, uint2 *dst) {
           if (n <= (uint32_t)CAND_LIST) {
             uint16_t *lst = cand_list[wave];
             const uint32_t rowcode = ((uint32_t)l31 << 8) | (uint32_t)(hs * (SEGW / 2));
@@ -707,7 +707,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
               const int ml = (int)(code >> 8), c = (int)(code & 255u);
               const int sl = c / EPS, j = c % EPS;
               const T rawv = *reinterpret_cast<const T *>(park + ml * 256 + ((sl ^ (ml & 15)) * 16) + j * (int)sizeof(T));
-              dst[idx] = make_uint2((uint32_t)(ncol0 + c), Elem<T>::raw(rawv));
+              dst[idx] = make_uint2(collect_place(h * 32 + ml, (uint32_t)(ncol0 + c)), Elem<T>::raw(rawv));
             }
           } else {
             // more candidates than the list holds: every lane walks its own half row
@@ -720,7 +720,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
                 wd &= wd - 1u;
                 const int sl = c / EPS, j = c % EPS;
                 const T rawv = *reinterpret_cast<const T *>(myrow + ((sl ^ rsw) * 16) + j * (int)sizeof(T));
-                dst[pos++] = make_uint2((uint32_t)(ncol0 + c), Elem<T>::raw(rawv));
+                dst[pos++] = make_uint2(collect_place(h * 32 + l31, (uint32_t)(ncol0 + c)), Elem<T>::raw(rawv));
               }
             }
           }
@@ -767,7 +767,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
           tot[h] = __builtin_amdgcn_readlane(v, 31);
           const uint32_t before = h ? tot[0] : 0u;
           const uint32_t first = incl[h] - cnt[h] - (hs ? 0u : part[h]);
-          if (before + tot[h] <= ca.caps) emit_piece(W[h], first, tot[h], mypool + off + before);
+          if (before + tot[h] <= ca.caps) emit_piece(W[h], h, first, tot[h], mypool + off + before);
         }
         const uint32_t total = tot[0] + tot[1];
         bool ok = true;
@@ -783,20 +783,11 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
               park_rows(pass, h);
-              emit_piece(W[h], incl[h] - cnt[h] - (hs ? 0u : part[h]), tot[h], mypool + off + (h ? tot[0] : 0u));
+              emit_piece(W[h], h, incl[h] - cnt[h] - (hs ? 0u : part[h]), tot[h], mypool + off + (h ? tot[0] : 0u));
             }
           }
         }
         if (lane_e == 0) ca.tile_meta[(int64_t)layer * nseg * nrb + tile] = make_uint2(off, ok ? total : 0u);
-        uint2 *meta = ca.seg_meta + ((int64_t)layer * nseg + seg) * Mp + grow0;
-        if (hs == 0) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const uint32_t rowtot = cnt[h] + part[h];
-            const uint32_t rel = (h ? tot[0] : 0u) + incl[h] - rowtot;
-            meta[h * 32 + l31] = ok ? make_uint2(off + rel, rowtot) : make_uint2(0u, 0u);
-          }
-        }
       }
     }
     if (!has_next) break;
@@ -1100,7 +1091,7 @@ bool clt_encode_can_collect(const void *x, const void *w, const void *b, int64_t
                             int64_t xs, int64_t wstr, int64_t bs, int dtype) {
   const bool fast = dtype != CLT_F32 ? encode_fast_ok<bf16_t>(x, w, b, nullptr, T, d, F, xs, wstr, bs, 16)   // any 16-bit type
                                      : encode_fast_ok<float>(x, w, b, nullptr, T, d, F, xs, wstr, bs, 16);
-  return fast;
+  return fast && F <= (int64_t)COLLECT_COL + 1;
 }
 
 extern "C" int clt_encode_fast_path(const void *x, const void *w, const void *b, const void *pre, int64_t T, int64_t d,

@@ -1122,111 +1122,156 @@ __global__ __launch_bounds__(256) void k_pool_hist(const SelState *st, const uin
   }
 }
 
-// The three kernels below finish the selection on the encoder-collected candidates.  They all
-// map a wavefront to 64 consecutive token rows of one feature segment (lane = row): the rows'
-// bookkeeping entries are adjacent in seg_meta and their runs are adjacent in the tile extent,
-// so every access of a wavefront is (nearly) contiguous.
-//
-// k_tile_count: per (row, segment), how many entries beat the threshold key / equal it.
-// Grid: x = blocks of 256 rows, y = segment, z = layer.
-constexpr int TILE_NE = 4;   // entries of a run fetched in one batch
-template <typename T>
-__global__ __launch_bounds__(256) void k_tile_count(
-    int Tn, int Tp, const SelState *st, const uint2 *seg_meta, int nseg, const uint2 *pool, unsigned long long pool_cap,
-    uint8_t *cgt, uint8_t *ceq) {
-  constexpr int KB = Elem<T>::KEYBITS;
-  const int l = blockIdx.z, seg = blockIdx.y;
-  const SelState s = st[l];
-  if (s.path != PATH_TILES || s.status != ST_DONE) return;
-  const uint2 *mypool = pool + (unsigned long long)l * pool_cap;
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= Tn) return;
-  const int64_t at = ((int64_t)l * nseg + seg) * Tp + collect_grid_row(row, Tn, Tp);
-  const uint2 m = seg_meta[at];
-  uint32_t raw[TILE_NE];
+// The three kernels below finish the selection on the encoder-collected candidates.  A wavefront takes one block of 64 token
+// rows and TILE_PORTION consecutive segments, that is TILE_PORTION extents of the pool, lane = entry: the entries of all
+// of them are asked for at once, 64 consecutive ones per load, and say which row they belong to.  (With lane = row, each lane
+// walked runs of 1.3 entries through a book entry per run: as many bytes again, a chain of loads for the longest run of 64,
+// and seven cache lines per load.)  L = 12, T = 4096, F = 24576, k = 200, bf16, us: count / prefix / emit 133 / 29 / 256 with a
+// thread per run, 36 / 6 / 71 here; a threshold list of 24 layers, F = 32768: emit 382, count and emit here 61 + 172.
+constexpr int TILE_PORTION = 8, TILE_WAVES = 4;
+constexpr int TILE_NE = 2;   // loads of an extent in flight at once: 128 entries
+__host__ __device__ static inline int tile_portions(int nseg) { return (nseg + TILE_PORTION - 1) / TILE_PORTION; }
+
+// f(entry, live, n) for the entries of a portion in order of (segment, row, feature), 64 at a time, the first n lanes live.
+template <typename F> __device__ __forceinline__ void visit_portion(const uint2 *tile_meta, const uint2 *pool, int rowblk, int nrb, int seg0,
+                                                                    int nseg, F f) {
+  const int lane = lane_id();
+  const uint2 mine = lane < TILE_PORTION && seg0 + lane < nseg ? tile_meta[(int64_t)(seg0 + lane) * nrb + rowblk] : make_uint2(0u, 0u);
+  uint2 en[TILE_PORTION][TILE_NE];
 #pragma unroll
-  for (int e = 0; e < TILE_NE; ++e) raw[e] = (uint32_t)e < m.y ? mypool[m.x + e].y : 0u;
-  uint32_t ngt = 0, neq = 0;
+  for (int i = 0; i < TILE_PORTION; ++i) {
+    const uint32_t off = __builtin_amdgcn_readlane(mine.x, i), n = __builtin_amdgcn_readlane(mine.y, i);
 #pragma unroll
-  for (int e = 0; e < TILE_NE; ++e)
-    if ((uint32_t)e < m.y) {
-      const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(raw[e])));
-      ngt += key > s.thr_key ? 1u : 0u;
-      neq += key == s.thr_key ? 1u : 0u;
+    for (int e = 0; e < TILE_NE; ++e) {
+      const uint32_t at = e * 64 + lane;
+      en[i][e] = at < n ? pool[off + at] : make_uint2(0u, 0u);
     }
-  for (uint32_t e = TILE_NE; e < m.y; ++e) {
-    const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(mypool[m.x + e].y)));
-    ngt += key > s.thr_key ? 1u : 0u;
-    neq += key == s.thr_key ? 1u : 0u;
   }
-  cgt[at] = (uint8_t)ngt; ceq[at] = (uint8_t)neq;   // a run has at most 128 entries
+#pragma unroll
+  for (int i = 0; i < TILE_PORTION; ++i) {
+    const uint32_t off = __builtin_amdgcn_readlane(mine.x, i), n = __builtin_amdgcn_readlane(mine.y, i);
+#pragma unroll
+    for (int e = 0; e < TILE_NE; ++e)
+      if (e * 64u < n) f(en[i][e], e * 64u + lane < n);
+    for (uint32_t at = TILE_NE * 64 + lane; at - lane < n; at += 64) f(at < n ? pool[off + at] : make_uint2(0u, 0u), at < n);
+  }
 }
 
-// k_row_prefix: per row, exclusive prefix of those counts over the segments, and the row totals.
+// The token at row `grow` of the books' grid (see collect_grid_row), -1 in front of a shifted tile.
+__device__ __forceinline__ int collect_token(int grow, int Tn, int Tp) {
+  if (grow < Tp - COLLECT_TILE_ROWS) return grow;
+  return grow - (Tp - Tn) >= Tp - COLLECT_TILE_ROWS ? grow - (Tp - Tn) : -1;
+}
+
+// k_tile_count: per (row, portion), how many entries beat the threshold key (low half) / equal it (high half: a portion
+// has at most 1024 of a row).  Grid: x = blocks of 64 rows, y = blocks of TILE_WAVES portions, z = layer.
+template <typename T>
+__global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_count(int Tp, const SelState *st, const uint2 *tile_meta, int nseg,
+                                                                const uint2 *pool, unsigned long long pool_cap, uint32_t *counts) {
+  __shared__ uint32_t cnt[TILE_WAVES][COLLECT_ROWS];
+  const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
+  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  const SelState s = st[l];
+  if (s.path != PATH_TILES || s.status != ST_DONE || part >= nport) return;
+  cnt[wv][lane] = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+    [&](const uint2 &e, bool live) {
+      const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(e.y)));
+      if (live && key >= s.thr_key) atomicAdd(&cnt[wv][collect_row(e.x)], key == s.thr_key ? 1u << 16 : 1u);
+    });
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  counts[((int64_t)l * nport + part) * Tp + blockIdx.x * COLLECT_ROWS + lane] = cnt[wv][lane];
+}
+
+// k_row_prefix: per row, exclusive prefix of those counts over the portions, and the row totals.
 __global__ __launch_bounds__(256) void k_row_prefix(
-    int64_t Tn, int64_t Tp, const SelState *st, int nseg, const uint8_t *cgt, const uint8_t *ceq, uint32_t *pgt,
-    uint32_t *peq, uint32_t *row_gt, uint32_t *row_eq) {
+    int64_t Tn, int64_t Tp, const SelState *st, int nport, const uint32_t *counts, uint2 *before, uint32_t *row_gt, uint32_t *row_eq) {
   const int l = blockIdx.y;
   const SelState s = st[l];
   if (s.path != PATH_TILES || s.status != ST_DONE) return;
   const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= Tn) return;
   uint32_t g = 0, q = 0;
-  const int64_t base = (int64_t)l * nseg * Tp + collect_grid_row(row, Tn, Tp);
-  int seg = 0;
-  for (; seg + 8 <= nseg; seg += 8) {
-    uint32_t a[8], b[8];
+  const int64_t base = (int64_t)l * nport * Tp + collect_grid_row(row, Tn, Tp);
+  int part = 0;
+  for (; part + 8 <= nport; part += 8) {
+    uint32_t a[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { a[i] = cgt[base + (int64_t)(seg + i) * Tp]; b[i] = ceq[base + (int64_t)(seg + i) * Tp]; }
+    for (int i = 0; i < 8; ++i) a[i] = counts[base + (int64_t)(part + i) * Tp];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      pgt[base + (int64_t)(seg + i) * Tp] = g; peq[base + (int64_t)(seg + i) * Tp] = q;
-      g += a[i]; q += b[i];
+      before[base + (int64_t)(part + i) * Tp] = make_uint2(g, q);
+      g += a[i] & 0xFFFFu; q += a[i] >> 16;
     }
   }
-  for (; seg < nseg; ++seg) {
-    const uint32_t a = cgt[base + (int64_t)seg * Tp], b = ceq[base + (int64_t)seg * Tp];
-    pgt[base + (int64_t)seg * Tp] = g; peq[base + (int64_t)seg * Tp] = q;
-    g += a; q += b;
+  for (; part < nport; ++part) {
+    const uint32_t a = counts[base + (int64_t)part * Tp];
+    before[base + (int64_t)part * Tp] = make_uint2(g, q);
+    g += a & 0xFFFFu; q += a >> 16;
   }
   row_gt[(int64_t)l * Tn + row] = g; row_eq[(int64_t)l * Tn + row] = q;
 }
 
-// k_tile_emit: the ordered write.  An entry's place in its row = the row's start + the entries
-// kept in earlier segments (all that beat the key, and ties while the row's allotment lasts) +
-// the entries kept before it in its own run.
-template <typename T>
-__global__ __launch_bounds__(256) void k_tile_emit(
-    int Tn, int Tp, const SelState *st, const uint2 *seg_meta, int nseg, const uint2 *pool, unsigned long long pool_cap,
-    const uint32_t *pgt, const uint32_t *peq, const uint32_t *allot, const int32_t *row_ptr, int32_t *col_out,
-    T *val_out) {
-  constexpr int KB = Elem<T>::KEYBITS;
-  const int l = blockIdx.z, seg = blockIdx.y;
-  const SelState s = st[l];
-  if (s.path != PATH_TILES || s.status != ST_DONE) return;
-  const uint2 *mypool = pool + (unsigned long long)l * pool_cap;
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= Tn) return;
-  const int64_t at = ((int64_t)l * nseg + seg) * Tp + collect_grid_row(row, Tn, Tp);
-  const uint2 m = seg_meta[at];
-  if (m.y == 0) return;
-  const int64_t r = (int64_t)l * Tn + row;
-  uint2 en[TILE_NE];
-#pragma unroll
-  for (int e = 0; e < TILE_NE; ++e) en[e] = (uint32_t)e < m.y ? mypool[m.x + e] : make_uint2(0u, 0u);
-  const uint32_t al = allot[r];
-  uint32_t tie = peq[at];
-  int64_t pos = (int64_t)row_ptr[r] + pgt[at] + (tie < al ? tie : al);
-  auto put = [&](const uint2 &e2) {
-    const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(e2.y)));
-    bool keepit = key > s.thr_key;
-    if (key == s.thr_key) { keepit = tie < al; ++tie; }
-    if (keepit) { col_out[pos] = (int32_t)e2.x; val_out[pos] = Elem<T>::from_raw(e2.y); ++pos; }
-  };
-#pragma unroll
-  for (int e = 0; e < TILE_NE; ++e)
-    if ((uint32_t)e < m.y) put(en[e]);
-  for (uint32_t e = TILE_NE; e < m.y; ++e) put(mypool[m.x + e]);
+// k_tile_emit: the ordered write.  An entry's place in its row = the row's start + the entries kept in earlier portions (all
+// that beat the key, and ties while the row's allotment lasts) + those kept earlier in this one, which a counter per row
+// holds, + those kept before it among its row's lanes of the 64 at hand, from the lanes' votes.
+// ALL: a threshold list, every entry is kept (`before` then counts them in its first half).
+template <typename T, bool ALL>
+__global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_emit(
+    int Tn, int Tp, const SelState *st, const uint2 *tile_meta, int nseg, const uint2 *pool, unsigned long long pool_cap,
+    const uint2 *before, const uint32_t *allot, const int32_t *row_ptr, int32_t *col_out, T *val_out, const int32_t *skip) {
+  __shared__ uint32_t next_sh[TILE_WAVES][COLLECT_ROWS], tie_sh[ALL ? 1 : TILE_WAVES][COLLECT_ROWS], allot_sh[ALL ? 1 : TILE_WAVES][COLLECT_ROWS];
+  if (ALL && skip && *skip != 0) return;      // the list did not fit the caller's arrays: it was emptied
+  const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
+  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  uint32_t thr = 0;
+  if constexpr (!ALL) {
+    const SelState s = st[l];
+    if (s.path != PATH_TILES || s.status != ST_DONE) return;
+    thr = s.thr_key;
+  }
+  if (part >= nport) return;
+  uint32_t *next = next_sh[wv], *tie = tie_sh[ALL ? 0 : wv], *room = allot_sh[ALL ? 0 : wv];
+  {
+    const int grow = blockIdx.x * COLLECT_ROWS + lane, tok = collect_token(grow, Tn, Tp);
+    const uint2 pre = tok >= 0 ? before[((int64_t)l * nport + part) * Tp + grow] : make_uint2(0u, 0u);
+    const uint32_t at = tok >= 0 ? (uint32_t)row_ptr[(int64_t)l * Tn + tok] : 0u;
+    if constexpr (ALL) {
+      next[lane] = at + pre.x;
+    } else {
+      const uint32_t al = tok >= 0 ? allot[(int64_t)l * Tn + tok] : 0u;
+      next[lane] = at + pre.x + (pre.y < al ? pre.y : al);
+      tie[lane] = pre.y;
+      room[lane] = al;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+    [&](const uint2 &e, bool live) {
+      const int row = live ? collect_row(e.x) : -1, row_before = __shfl_up(row, 1), row_after = __shfl_down(row, 1);
+      // this row's lanes: from its first one (`first`: the lanes before that) on
+      const uint64_t heads = ballot64(lane == 0 || row != row_before);
+      const uint64_t first = (1ull << (63 - __clzll((long long)(heads & (~0ull >> (63 - lane)))))) - 1ull;
+      const bool last = live && (lane == 63 || row_after != row);
+      bool keep = live;
+      if constexpr (!ALL) {
+        const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(e.y)));
+        keep = live && key > thr;
+        const uint64_t ties = ballot64(live && key == thr);
+        if (ties != 0) {
+          const bool eq = live && key == thr;
+          const uint32_t rank = (live ? tie[row] : 0u) + mbcnt64(ties) - (uint32_t)__popcll(ties & first);
+          keep = keep || (eq && rank < room[row]);
+          if (last) tie[row] = rank + (eq ? 1u : 0u);
+        }
+      }
+      const uint64_t kept = ballot64(keep);
+      const uint32_t pos = (live ? next[row] : 0u) + mbcnt64(kept) - (uint32_t)__popcll(kept & first);
+      if (keep) { col_out[pos] = (int32_t)(e.x & COLLECT_COL); val_out[pos] = Elem<T>::from_raw(e.y); }
+      if (last) next[row] = pos + (keep ? 1u : 0u);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    });
 }
 
 // ---- post-hoc threshold estimation: per-feature minimum of the selected z-scores ---------------
@@ -1264,25 +1309,38 @@ __global__ void k_selected_min_accumulate(const uint32_t *keys, int64_t n, T *su
 }
 
 // ---- threshold activation on encoder-collected entries (every entry is a survivor) ----------
-// Per row: exclusive prefix of the run lengths over the segments, and the row total.
-__global__ __launch_bounds__(256) void k_row_prefix_meta(int64_t Tn, int64_t Tp, int nseg, const uint2 *seg_meta,
-                                                         uint32_t *pfx, uint32_t *row_cnt) {
+// Per (row, portion): the entries.  Grid as of k_tile_count.
+__global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_count_all(int Tp, const uint2 *tile_meta, int nseg, const uint2 *pool,
+                                                                    unsigned long long pool_cap, uint32_t *counts) {
+  __shared__ uint32_t cnt[TILE_WAVES][COLLECT_ROWS];
+  const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
+  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  if (part >= nport) return;
+  cnt[wv][lane] = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+    [&](const uint2 &e, bool live) { if (live) atomicAdd(&cnt[wv][collect_row(e.x)], 1u); });
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  counts[((int64_t)l * nport + part) * Tp + blockIdx.x * COLLECT_ROWS + lane] = cnt[wv][lane];
+}
+
+// Per row: exclusive prefix of those over the portions, and the row total.
+__global__ __launch_bounds__(256) void k_row_prefix_all(int64_t Tn, int64_t Tp, int nport, const uint32_t *counts, uint2 *before,
+                                                        uint32_t *row_cnt) {
   const int l = blockIdx.y;
   const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= Tn) return;
   uint32_t g = 0;
-  const int64_t base = (int64_t)l * nseg * Tp + collect_grid_row(row, Tn, Tp);
-  int seg = 0;
-  for (; seg + 8 <= nseg; seg += 8) {
+  const int64_t base = (int64_t)l * nport * Tp + collect_grid_row(row, Tn, Tp);
+  for (int part0 = 0; part0 < nport; part0 += 8) {
     uint32_t a[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) a[i] = seg_meta[base + (int64_t)(seg + i) * Tp].y;
+    for (int i = 0; i < 8; ++i) a[i] = part0 + i < nport ? counts[base + (int64_t)(part0 + i) * Tp] : 0u;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { pfx[base + (int64_t)(seg + i) * Tp] = g; g += a[i]; }
-  }
-  for (; seg < nseg; ++seg) {
-    const uint32_t a = seg_meta[base + (int64_t)seg * Tp].y;
-    pfx[base + (int64_t)seg * Tp] = g; g += a;
+    for (int i = 0; i < 8; ++i) {
+      if (part0 + i < nport) before[base + (int64_t)(part0 + i) * Tp] = make_uint2(g, 0u);
+      g += a[i];
+    }
   }
   row_cnt[(int64_t)l * Tn + row] = g;
 }
@@ -1293,32 +1351,6 @@ __global__ void k_thresh_finish(const SelState *st, int L, int32_t *row_ptr, int
   bool over = false;
   for (int l = 0; l < L; ++l) over = over || st[l].overflow != 0;
   if (over) row_ptr[R] = -1;
-}
-
-// Grid: x = blocks of 256 rows, y = segment, z = layer.
-template <typename T>
-__global__ __launch_bounds__(256) void k_tile_emit_all(
-    int Tn, int Tp, const uint2 *seg_meta, int nseg, const uint2 *pool, unsigned long long pool_cap, const uint32_t *pfx,
-    const int32_t *row_ptr, int32_t *col_out, T *val_out, const int32_t *skip) {
-  if (skip && *skip != 0) return;             // the list did not fit the caller's arrays: it was emptied
-  const int l = blockIdx.z, seg = blockIdx.y;
-  const uint2 *mypool = pool + (unsigned long long)l * pool_cap;
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= Tn) return;
-  const int64_t at = ((int64_t)l * nseg + seg) * Tp + collect_grid_row(row, Tn, Tp);
-  const uint2 m = seg_meta[at];
-  if (m.y == 0) return;
-  uint2 en[TILE_NE];
-#pragma unroll
-  for (int e = 0; e < TILE_NE; ++e) en[e] = (uint32_t)e < m.y ? mypool[m.x + e] : make_uint2(0u, 0u);
-  int64_t pos = (int64_t)row_ptr[(int64_t)l * Tn + row] + pfx[at];
-#pragma unroll
-  for (int e = 0; e < TILE_NE; ++e)
-    if ((uint32_t)e < m.y) { col_out[pos] = (int32_t)en[e].x; val_out[pos] = Elem<T>::from_raw(en[e].y); ++pos; }
-  for (uint32_t e = TILE_NE; e < m.y; ++e) {
-    const uint2 e2 = mypool[m.x + e];
-    col_out[pos] = (int32_t)e2.x; val_out[pos] = Elem<T>::from_raw(e2.y); ++pos;
-  }
 }
 
 // ---- threshold activations ----------------------------------------------------------
@@ -1717,7 +1749,7 @@ static int dispatch_threshold(bool emit, const void *pre, int64_t Tn, int64_t F,
 // ---- encoder-collected candidates: workspace and the two halves of the fused path ---------
 struct TileLayout {
   SelLayout sel;
-  size_t off_tmeta, off_meta, off_tpool, off_cgt, off_ceq, off_pgt, off_peq, off_tcount, total;
+  size_t off_tmeta, off_tpool, off_counts, off_before, off_tcount, total;
   unsigned long long tpool_cap;              // entries per layer
   uint32_t caps;                             // entries per fixed tile slot
   int nseg, ntile;
@@ -1744,13 +1776,10 @@ static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dt
   size_t o = tl.sel.total;
   auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
   tl.off_tmeta = take(8 * (size_t)tl.ntile * (size_t)L);
-  tl.off_meta = take(8 * (size_t)tl.nseg * (size_t)Tp * (size_t)L);
   tl.off_tpool = take(8 * (size_t)tl.tpool_cap * (size_t)L);
-  const size_t cells = (size_t)tl.nseg * (size_t)Tp * (size_t)L;   // (row, segment) pairs
-  tl.off_cgt = take(cells);
-  tl.off_ceq = take(cells);
-  tl.off_pgt = take(4 * cells);
-  tl.off_peq = take(4 * cells);
+  const size_t cells = (size_t)tile_portions(tl.nseg) * (size_t)Tp * (size_t)L;   // (row, portion) pairs
+  tl.off_counts = take(4 * cells);
+  tl.off_before = take(8 * cells);
   tl.off_tcount = take(4 * (size_t)L);
   tl.total = o;
   return tl;
@@ -1777,7 +1806,7 @@ static int run_encode_collect(const void *x, const void *w, const void *b, void 
   uint2 *tpool = (uint2 *)(ws + tl.off_tpool);
   CollectArgs ca;
   ca.st = st; ca.pool_count = (uint32_t *)(ws + tl.off_tcount); ca.pool = tpool; ca.pool_cap = tl.tpool_cap;
-  ca.tile_meta = (uint2 *)(ws + tl.off_tmeta); ca.seg_meta = (uint2 *)(ws + tl.off_meta); ca.caps = tl.caps;
+  ca.tile_meta = (uint2 *)(ws + tl.off_tmeta); ca.caps = tl.caps;
   ca.theta = nullptr; ca.theta_stride = 0;
   int rc = clt_launch_encode(x, w, b, nullptr, Tn, d, F, L, xs, wstr, bs, ps, dtype, 1, nullptr, &ca, stream);
   if (rc != CLT_OK) return rc;
@@ -1802,7 +1831,6 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
   uint32_t *rgt = (uint32_t *)(ws + lo.off_gt), *req = (uint32_t *)(ws + lo.off_eq);
   uint32_t *allot = (uint32_t *)(ws + lo.off_allot), *keep = (uint32_t *)(ws + lo.off_keep);
   uint2 *pool = (uint2 *)(ws + lo.off_pool);
-  const uint2 *meta = (const uint2 *)(ws + tl.off_meta);
   const uint2 *tmeta = (const uint2 *)(ws + tl.off_tmeta);
   const uint2 *tpool = (const uint2 *)(ws + tl.off_tpool);
   const unsigned long long N = (unsigned long long)Tn * (unsigned long long)F;
@@ -1823,15 +1851,16 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
     k_select_level<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist, first, pool, lo.pool_cap, level, 1);
     k_select_scan<T><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 2, level);
   }
-  dim3 grid3((unsigned)clt_ceil_div(Tn, 256), (unsigned)tl.nseg, (unsigned)L);
-  uint8_t *cgt = (uint8_t *)(ws + tl.off_cgt), *ceq = (uint8_t *)(ws + tl.off_ceq);
-  uint32_t *pgt = (uint32_t *)(ws + tl.off_pgt), *peq = (uint32_t *)(ws + tl.off_peq);
+  const int nport = tile_portions(tl.nseg);
   const int64_t Tp = collect_grid_rows(Tn);
-  k_tile_count<T><<<grid3, 256, 0, stream>>>((int)Tn, (int)Tp, st, meta, tl.nseg, tpool, tl.tpool_cap, cgt, ceq);
-  k_row_prefix<<<dim3((unsigned)clt_ceil_div(Tn, 64), (unsigned)L), 64, 0, stream>>>(Tn, Tp, st, tl.nseg, cgt, ceq, pgt, peq, rgt, req);
+  dim3 grid3((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(nport, TILE_WAVES), (unsigned)L);
+  uint32_t *counts = (uint32_t *)(ws + tl.off_counts);
+  uint2 *before = (uint2 *)(ws + tl.off_before);
+  k_tile_count<T><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, counts);
+  k_row_prefix<<<dim3((unsigned)clt_ceil_div(Tn, 64), (unsigned)L), 64, 0, stream>>>(Tn, Tp, st, nport, counts, before, rgt, req);
   k_select_count<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, rgt, req, 1);
   k_select_allot<false><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K, 1);
-  k_tile_emit<T><<<grid3, 256, 0, stream>>>((int)Tn, (int)Tp, st, meta, tl.nseg, tpool, tl.tpool_cap, pgt, peq, allot, row_ptr, col, val);
+  k_tile_emit<T, false><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tn, (int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, before, allot, row_ptr, col, val, nullptr);
   k_select_emit<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, allot,
                                                      row_ptr, col, val, 1, nullptr);
   return clt_check_launch();
@@ -1839,7 +1868,7 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
 
 // ---- JumpReLU on the encoder epilogue -----------------------------------------------------------
 struct ThreshLayout {
-  size_t off_state, off_tcount, off_tmeta, off_meta, off_tpool, off_pfx, off_rowcnt, total;
+  size_t off_state, off_tcount, off_tmeta, off_tpool, off_counts, off_before, off_rowcnt, total;
   unsigned long long tpool_cap;
   uint32_t caps;
   int nseg, ntile;
@@ -1865,9 +1894,10 @@ static ThreshLayout thresh_layout(int64_t T, int64_t F, int64_t L, int64_t densi
   tl.off_state = take(sizeof(SelState) * (size_t)L);
   tl.off_tcount = take(4 * (size_t)L);
   tl.off_tmeta = take(8 * (size_t)tl.ntile * (size_t)L);
-  tl.off_meta = take(8 * (size_t)tl.nseg * (size_t)Tp * (size_t)L);
   tl.off_tpool = take(8 * (size_t)tl.tpool_cap * (size_t)L);
-  tl.off_pfx = take(4 * (size_t)tl.nseg * (size_t)Tp * (size_t)L);
+  const size_t cells = (size_t)tile_portions(tl.nseg) * (size_t)Tp * (size_t)L;   // (row, portion) pairs
+  tl.off_counts = take(4 * cells);
+  tl.off_before = take(8 * cells);
   tl.off_rowcnt = take(4 * (size_t)T * (size_t)L);
   tl.total = o;
   return tl;
@@ -1914,14 +1944,18 @@ extern "C" int clt_encode_threshold_count(const void *x, const void *w, const vo
   k_fill_u32<<<8, 256, 0, s>>>((uint32_t *)(ws + tl.off_state), 0u, (int64_t)((tl.off_tmeta - tl.off_state) / 4));
   CollectArgs ca;
   ca.st = st; ca.pool_count = (uint32_t *)(ws + tl.off_tcount); ca.pool = (uint2 *)(ws + tl.off_tpool);
-  ca.pool_cap = tl.tpool_cap; ca.tile_meta = (uint2 *)(ws + tl.off_tmeta); ca.seg_meta = (uint2 *)(ws + tl.off_meta);
+  ca.pool_cap = tl.tpool_cap; ca.tile_meta = (uint2 *)(ws + tl.off_tmeta);
   ca.caps = tl.caps; ca.theta = theta; ca.theta_stride = theta_layer_stride;
   int rc = clt_launch_encode(x, w, b, nullptr, T, d, F, L, x_layer_stride, w_layer_stride, b_layer_stride, 0, dtype, 2,
                              nullptr, &ca, s);
   if (rc != CLT_OK) return rc;
   uint32_t *rowcnt = (uint32_t *)(ws + tl.off_rowcnt);
-  k_row_prefix_meta<<<dim3((unsigned)clt_ceil_div(T, 64), (unsigned)L), 64, 0, s>>>(T, collect_grid_rows(T), tl.nseg, ca.seg_meta,
-                                                                                    (uint32_t *)(ws + tl.off_pfx), rowcnt);
+  const int nport = tile_portions(tl.nseg);
+  const int64_t Tp = collect_grid_rows(T);
+  uint32_t *counts = (uint32_t *)(ws + tl.off_counts);
+  k_tile_count_all<<<dim3((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(nport, TILE_WAVES), (unsigned)L), TILE_WAVES * 64, 0, s>>>(
+      (int)Tp, ca.tile_meta, tl.nseg, ca.pool, tl.tpool_cap, counts);
+  k_row_prefix_all<<<dim3((unsigned)clt_ceil_div(T, 64), (unsigned)L), 64, 0, s>>>(T, Tp, nport, counts, (uint2 *)(ws + tl.off_before), rowcnt);
   k_rowptr_scan<<<1, SCAN_THREADS, 0, s>>>(rowcnt, L * T, row_ptr);
   k_thresh_finish<<<1, 64, 0, s>>>(st, (int)L, row_ptr, L * T);
   return clt_check_launch();
@@ -1994,16 +2028,16 @@ extern "C" int clt_encode_threshold_emit(int64_t T, int64_t F, int64_t L, int64_
   if (workspace_bytes < tl.total) return CLT_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   char *ws = (char *)workspace;
-  dim3 grid((unsigned)clt_ceil_div(T, 256), (unsigned)tl.nseg, (unsigned)L);
-  if (dtype == CLT_BF16)
-    k_tile_emit_all<bf16_t><<<grid, 256, 0, s>>>((int)T, (int)collect_grid_rows(T), (const uint2 *)(ws + tl.off_meta), tl.nseg, (const uint2 *)(ws + tl.off_tpool),
-                                                  tl.tpool_cap, (const uint32_t *)(ws + tl.off_pfx), row_ptr, col, (bf16_t *)val, skip);
-  else if (dtype == CLT_F16)
-    k_tile_emit_all<f16_t><<<grid, 256, 0, s>>>((int)T, (int)collect_grid_rows(T), (const uint2 *)(ws + tl.off_meta), tl.nseg, (const uint2 *)(ws + tl.off_tpool),
-                                                  tl.tpool_cap, (const uint32_t *)(ws + tl.off_pfx), row_ptr, col, (f16_t *)val, skip);
-  else
-    k_tile_emit_all<float><<<grid, 256, 0, s>>>((int)T, (int)collect_grid_rows(T), (const uint2 *)(ws + tl.off_meta), tl.nseg, (const uint2 *)(ws + tl.off_tpool),
-                                                 tl.tpool_cap, (const uint32_t *)(ws + tl.off_pfx), row_ptr, col, (float *)val, skip);
+  const int64_t Tp = collect_grid_rows(T);
+  dim3 grid((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(tile_portions(tl.nseg), TILE_WAVES), (unsigned)L);
+#define CLT_EMIT_ALL(TT)                                                                                                              \
+  k_tile_emit<TT, true><<<grid, TILE_WAVES * 64, 0, s>>>((int)T, (int)Tp, nullptr, (const uint2 *)(ws + tl.off_tmeta), tl.nseg,        \
+                                                         (const uint2 *)(ws + tl.off_tpool), tl.tpool_cap,                            \
+                                                         (const uint2 *)(ws + tl.off_before), nullptr, row_ptr, col, (TT *)val, skip)
+  if (dtype == CLT_BF16) CLT_EMIT_ALL(bf16_t);
+  else if (dtype == CLT_F16) CLT_EMIT_ALL(f16_t);
+  else CLT_EMIT_ALL(float);
+#undef CLT_EMIT_ALL
   return clt_check_launch();
 }
 

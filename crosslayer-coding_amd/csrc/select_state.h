@@ -48,15 +48,19 @@ __device__ __forceinline__ int64_t collect_grid_row(int64_t token, int64_t T, in
 // the fixed slot [i * caps, (i + 1) * caps) of the pool; only a tile with more than `caps`
 // candidates takes an extent behind the slots instead, handed out by an atomic counter (one
 // same-address atomic per tile from every CU at once would cost more than the whole epilogue).
-//   tile_meta[layer * ntile + i]                           = (offset of the extent, entries)
-//   seg_meta[(layer * nseg + segment) * Tp + grid row]     = (offset of the token's run, length)
+//   tile_meta[layer * ntile + i]    = (offset of the extent, entries)
+//   an entry                        = (feature | the token's place in the tile << 26, raw value bits)
+// (T F < 2^32 and at least COLLECT_TILE_ROWS tokens: a feature number has 24 bits at most.)
+constexpr uint32_t COLLECT_COL = (1u << 26) - 1u;
+__device__ __forceinline__ uint32_t collect_place(int row, uint32_t col) { return (uint32_t)row << 26 | col; }
+__device__ __forceinline__ int collect_row(uint32_t place) { return (int)(place >> 26); }
+
 struct CollectArgs {
   SelState *st;              // [L]
   uint32_t *pool_count;      // [L] entries handed out behind the fixed slots
-  uint2 *pool;               // [L][pool_cap] entries (feature, raw value bits)
+  uint2 *pool;               // [L][pool_cap] entries
   unsigned long long pool_cap;
   uint2 *tile_meta;          // [L][ntile]
-  uint2 *seg_meta;           // [L][nseg][Tp]
   uint32_t caps;             // entries per fixed slot
   const void *theta;         // COLLECT == 2: [L][F] thresholds in the model dtype
   int64_t theta_stride;
