@@ -41,6 +41,9 @@ class SurvivorList:
     status: Optional[torch.Tensor] = None
     # host-side estimate of the survivor total where one is known without a read-back (cost models only)
     nnz_hint: Optional[int] = None
+    # made by a selection over activations: its length says what a typical row holds.  A list of any other origin may
+    # hold all its entries in a few rows, and the schedule made for short rows (``clt_decode_thin``) is not priced by it
+    selected: bool = False
 
     @property
     def nnz(self) -> int:
@@ -61,7 +64,7 @@ class SurvivorList:
         if bad:
             raise nat.CLTNativeError("the batch has more active features than a survivor list can hold (2^31 - 1)")
         return SurvivorList(self.row_ptr, self.col[:total], self.val[:total], self.T, self.F, self.L, self.dtype,
-                            None, total)
+                            None, total, self.selected)
 
 
 def max_list_entries(L: int, T: int, F: int) -> int:
@@ -314,7 +317,7 @@ def batchtopk_select(pre: torch.Tensor, k: int, global_mode: bool, ws: Optional[
                                     nat.dtype_code(pre.dtype), nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val),
                                     nat.ptr(wbuf), wbuf.numel(), _stream(pre))
     nat.check(code, "clt_batchtopk_select")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype)
+    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, selected=True)
 
 
 def encode_collect_supported(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], k: int) -> bool:
@@ -362,7 +365,7 @@ def collect_select(handle) -> SurvivorList:
                                          nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val), nat.ptr(wbuf), wbuf.numel(),
                                          _stream(pre))
     nat.check(code, "clt_collect_select")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype)
+    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, selected=True)
 
 
 def tokentopk_select(pre: torch.Tensor, kk: int, global_mode: bool, ws: Optional[Workspace] = None,
@@ -387,7 +390,7 @@ def tokentopk_select(pre: torch.Tensor, kk: int, global_mode: bool, ws: Optional
                                     nat.dtype_code(pre.dtype), nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val),
                                     nat.ptr(wbuf), wbuf.numel(), _stream(pre))
     nat.check(code, "clt_tokentopk_select")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype)
+    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, selected=True)
 
 
 def _fit(row_ptr: torch.Tensor, capacity: int) -> torch.Tensor:
@@ -450,7 +453,7 @@ def threshold_select(pre: torch.Tensor, theta: Optional[torch.Tensor], pred: int
     code = lib.clt_threshold_emit(nat.ptr(pre), T, F, L, pre.stride(0), nat.ptr(theta), pred, code_dt,
                                   nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val), nat.ptr(status), _stream(pre))
     nat.check(code, "clt_threshold_emit")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, status, total if read_back else None)
+    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, status, total if read_back else None, selected=True)
 
 
 def encode_threshold(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], theta: torch.Tensor,
@@ -505,11 +508,11 @@ def encode_threshold(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor]
                                          nat.ptr(flags), nat.ptr(wbuf), wbuf.numel(), _stream(x))
     nat.check(code, "clt_encode_threshold_emit")
     if flags is None:
-        return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, x.dtype, None, total)
+        return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, x.dtype, None, total, selected=True)
     code = lib.clt_threshold_emit(nat.ptr(pre_scratch), T, F, L, pre_scratch.stride(0), nat.ptr(theta), nat.PRED_GE_THETA,
                                   dt, nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val), flags[1:].data_ptr(), _stream(x))
     nat.check(code, "clt_threshold_emit")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, x.dtype, flags[2:3])
+    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, x.dtype, flags[2:3], selected=True)
 
 
 # ---- evaluation reductions ------------------------------------------------------------------------------
@@ -933,7 +936,7 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
 
     With a workspace and a batch large enough to fill the GPU a gather from LDS tiles (16 bits: ``clt_decode_tiles`` on the
     matrix cores; fp32: ``clt_decode_rows``) or one of the XCD-sliced gathers from the L2s is used, for few survivors per
-    source and token ``clt_decode_thin``, whichever ``clt_decode_thin_wanted`` / ``clt_decode_tiles_wanted`` /
+    source and token of a selection ``clt_decode_thin``, whichever ``clt_decode_thin_wanted`` / ``clt_decode_tiles_wanted`` /
     ``clt_decode_rows_wanted`` price lowest."""
     nat.require_device(w_packed, "decode_sparse")
     L, T, F = surv.L, surv.T, surv.F
@@ -968,8 +971,8 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
         if total is None:
             total = L * T * F // 100
         wide = surv.dtype == torch.float32
-        if sliced and total and lib.clt_decode_thin_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying],
-                                                           nat.dtype_code(surv.dtype)):
+        if sliced and surv.selected and total and lib.clt_decode_thin_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying],
+                                                                             nat.dtype_code(surv.dtype)):
             code = lib.clt_decode_thin(nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum),
                                        nat.ptr(skip_add), nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin, t_end,
                                        src_mask & ((1 << 64) - 1), nat.dtype_code(surv.dtype), 1 if out_f32 else 0, _stream(w_packed))

@@ -134,6 +134,8 @@ def test_decode_thin_is_chosen_and_agrees_with_the_gather(monkeypatch, dtype):
     monkeypatch.setattr(lib, "clt_decode_thin", lambda *a: ran.append(1) or thin(*a))
     got = engine.decode_sparse(surv, w, "none", d, ws=ws, out_f32=True)
     assert ran == [1]
+    engine.decode_sparse(engine.SurvivorList(surv.row_ptr, surv.col, surv.val, T, F, L, dtype), w, "none", d, ws=ws)
+    assert ran == [1]                            # a list of unknown origin, whose length says nothing about a row
     monkeypatch.setattr(lib, "clt_decode_thin_wanted", lambda *a: 0)
     ref = engine.decode_sparse(surv, w, "none", d, ws=ws, out_f32=True)
     assert ran == [1] and float((got - ref).norm() / ref.norm()) < 1e-6     # fp32 sums in another order
