@@ -182,4 +182,6 @@ def require_device(t: torch.Tensor, what: str) -> None:
 
 
 def current_stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: building the Stream object around it costs more than a launch, and every launch asks
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

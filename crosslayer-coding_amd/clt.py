@@ -141,7 +141,7 @@ class CrossLayerTranscoder(BaseTranscoder):
         return torch.float32
 
     def _workspace(self) -> Workspace:
-        dev = self.encoder_module.encoders[0].weight.device
+        dev = self.encoder_module.first_weight().device
         if self._ws is None or self._ws.device != dev:
             self._ws = Workspace(dev)
         return self._ws
@@ -155,7 +155,7 @@ class CrossLayerTranscoder(BaseTranscoder):
 
     def _sync_device(self) -> None:
         """Follow the parameters after ``module.to(...)``."""
-        w = self.encoder_module.encoders[0].weight
+        w = self.encoder_module.first_weight()
         if w.device != self.device or w.dtype != self.dtype:
             self.device, self.dtype = w.device, w.dtype
             for m in (self.encoder_module, self.decoder_module, self.theta_manager):

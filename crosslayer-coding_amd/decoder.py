@@ -23,7 +23,7 @@ import torch.nn as nn
 from . import _native as nat
 from . import engine
 from .engine import SurvivorList
-from .parallel import RowParallelLinear, require_single_rank
+from .parallel import RowParallelLinear, own_parameter, require_single_rank
 
 logger = logging.getLogger(__name__)
 
@@ -163,15 +163,14 @@ class Decoder(nn.Module):
         """Decoder layers in slot order (untied: "0->0", "0->1", ..., as created)."""
         mods = self.decoders._modules      # straight to the registry: no parameter sync for internal walks
         cached = self.__dict__.get("_ordered_cache")
-        if cached is not None and cached[0] is mods and cached[1] == len(mods) and all(
-                a is b for a, b in zip(cached[3], mods.values())):
-            return cached[2]
+        if cached is not None and cached[0] is mods and cached[2] == list(mods.values()):     # (modules compare by identity)
+            return cached[1]
         if isinstance(self.decoders, nn.ModuleDict):
             L = self.config.num_layers
             out = [mods[f"{s}->{t}"] for s in range(L) for t in range(s, L)]
         else:
             out = list(mods.values())
-        self.__dict__["_ordered_cache"] = (mods, len(mods), out, list(mods.values()))
+        self.__dict__["_ordered_cache"] = (mods, out, list(mods.values()))
         return out
 
     # ---- parameters behind the working copy -------------------------------------------
@@ -211,9 +210,11 @@ class Decoder(nn.Module):
             return [(s, t) for s in range(L) for t in range(s, L)]
         return [(i, i) for i in range(L)]
 
-    def _pointer_table(self, name: str, tensors) -> torch.Tensor:
-        """Device int64 tensor with the addresses of ``tensors``, rebuilt only when one has moved."""
-        ptrs = tuple(t.data_ptr() for t in tensors)
+    def _pointer_table(self, name: str, tensors, ptrs: Optional[Tuple[int, ...]] = None) -> torch.Tensor:
+        """Device int64 tensor with the addresses of ``tensors`` (``ptrs``, where the caller has them), rebuilt only when
+        one has moved."""
+        if ptrs is None:
+            ptrs = tuple([t.data_ptr() for t in tensors])
         ent = self._tables.get(name)
         if ent is None or ent[0] != ptrs or ent[1].device != tensors[0].device:
             # through pinned memory and an asynchronous copy: building the table must not synchronise a forward
@@ -239,7 +240,8 @@ class Decoder(nn.Module):
         whose parameter changed are repacked - by the host where the parameter's version counter shows it, by the
         device itself where only the data does (``weight.data.fill_(...)``; ``watch_parameter_data``)."""
         decs = self._ordered()
-        w0 = decs[0].weight
+        ws = [own_parameter(dec, "weight") for dec in decs]
+        w0 = ws[0]
         F, d = self.config.num_features, self.config.d_model
         if (self._slab is None or self._slab.device != w0.device or self._slab.dtype != w0.dtype
                 or self._slab.shape[0] != len(decs)):
@@ -247,20 +249,19 @@ class Decoder(nn.Module):
             self._slab_keys = [None] * len(decs)
             self.device, self.dtype = w0.device, w0.dtype
             self._fp_state = None
-        for i, dec in enumerate(decs):
-            w = dec.weight
-            key = (w.data_ptr(), w._version)
-            if self._slab_keys[i] != key:
-                engine.pack_decoder(w.detach().contiguous(), self._slab[i])
-                self._slab_keys[i] = key
-                self._repacks = getattr(self, "_repacks", 0) + 1
-        if self.watch_parameter_data and not getattr(self, "_params_behind", False) \
-                and all(dec.weight.is_contiguous() for dec in decs):
+        keys = [(w.data_ptr(), w._version) for w in ws]
+        if self._slab_keys != keys:
+            for i, w in enumerate(ws):
+                if self._slab_keys[i] != keys[i]:
+                    engine.pack_decoder(w.detach().contiguous(), self._slab[i])
+                    self._slab_keys[i] = keys[i]
+                    self._repacks = getattr(self, "_repacks", 0) + 1
+        if self.watch_parameter_data and not getattr(self, "_params_behind", False) and all([w.is_contiguous() for w in ws]):
             if self._fp_state is None or self._fp_state.device != w0.device:
                 self._fp_state = torch.zeros(16 * len(decs), dtype=torch.int64, device=w0.device)
                 self._fp_changed = torch.zeros(len(decs), dtype=torch.int32, device=w0.device)
                 self._fp_fresh = False
-            table = self._pointer_table("w", [dec.weight for dec in decs])
+            table = self._pointer_table("w", ws, tuple([k[0] for k in keys]))
             if not self._fp_fresh:
                 # first use (or after invalidate_packed): the slab has just been made from these values: record them
                 engine.decoder_fingerprint(table, d, F, w0.dtype, self._fp_state, self._fp_changed, True)
@@ -292,8 +293,8 @@ class Decoder(nn.Module):
         it - one per contributing source (decoder.py:294-295 / parallel.py:380-381), or the
         target's own decoder for per_target tying (decoder.py:250-251)."""
         decs = self._ordered()
-        bs = [dec.bias_param for dec in decs]
-        if all(b is not None and b.is_contiguous() and b.is_cuda for b in bs):
+        bs = [own_parameter(dec, "bias_param") for dec in decs]
+        if all([b is not None and b.is_contiguous() and b.is_cuda for b in bs]):
             # computed anew on every call (one small launch): a write to a bias shows whichever way it was made
             return engine.bias_sum(self._pointer_table("b", bs), self.config.d_model, self.config.num_layers,
                                    self.config.decoder_tying, src_mask, bs[0].dtype)

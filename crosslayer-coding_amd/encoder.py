@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from . import engine
-from .parallel import ColumnParallelLinear, require_single_rank
+from .parallel import ColumnParallelLinear, own_parameter, require_single_rank
 
 logger = logging.getLogger(__name__)
 
@@ -39,6 +39,10 @@ class Encoder(nn.Module):
             for l in range(L))
 
     # ---- slab bookkeeping -------------------------------------------------------
+    def first_weight(self) -> torch.Tensor:
+        """The first layer's weight, which says where the model lives."""
+        return own_parameter(next(iter(self.encoders._modules.values())), "weight")
+
     def stacked(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """([L, F, d] weights, [L, F] biases) that alias the per-layer parameters.
 
@@ -46,12 +50,14 @@ class Encoder(nn.Module):
         longer aliases the slab, the slab is rebuilt from the parameters and they are
         pointed back at it.
         """
-        w0 = self.encoders[0].weight
+        w0 = self.first_weight()
         ok = (self._w_slab.device == w0.device and self._w_slab.dtype == w0.dtype)
         if ok:
-            for l, enc in enumerate(self.encoders):
-                if (enc.weight.data_ptr() != self._w_slab[l].data_ptr()
-                        or enc.bias_param.data_ptr() != self._b_slab[l].data_ptr()):
+            w_at, b_at, item = self._w_slab.data_ptr(), self._b_slab.data_ptr(), self._w_slab.element_size()
+            w_step, b_step = self._w_slab.stride(0) * item, self._b_slab.stride(0) * item
+            for l, enc in enumerate(self.encoders._modules.values()):
+                if (own_parameter(enc, "weight").data_ptr() != w_at + l * w_step
+                        or own_parameter(enc, "bias_param").data_ptr() != b_at + l * b_step):
                     ok = False
                     break
         if not ok:
@@ -147,7 +153,9 @@ class Encoder(nn.Module):
             x = inputs[l]
             if not (0 <= l < L) or x.dim() not in (2, 3) or x.shape[-1] != d:
                 return None
-            f = x.to(device=self.device, dtype=self.dtype).reshape(-1, d)
+            f = x if x.dtype == self.dtype and x.device == self.device else x.to(device=self.device, dtype=self.dtype)
+            if f.dim() != 2:
+                f = f.reshape(-1, d)
             if T is None:
                 T = f.shape[0]
             if f.shape[0] != T or T == 0:

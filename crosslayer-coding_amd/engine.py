@@ -317,7 +317,9 @@ def batchtopk_select(pre: torch.Tensor, k: int, global_mode: bool, ws: Optional[
                                     nat.dtype_code(pre.dtype), nat.ptr(row_ptr), nat.ptr(col), nat.ptr(val),
                                     nat.ptr(wbuf), wbuf.numel(), _stream(pre))
     nat.check(code, "clt_batchtopk_select")
-    return SurvivorList(row_ptr, col[:total], val[:total], T, F, L, pre.dtype, selected=True)
+    if total == 0:
+        col, val = col[:0], val[:0]
+    return SurvivorList(row_ptr, col, val, T, F, L, pre.dtype, selected=True)
 
 
 def encode_collect_supported(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], k: int) -> bool:

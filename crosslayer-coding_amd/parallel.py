@@ -96,6 +96,12 @@ class ColumnParallelLinear(_Linear):
         return y[0].view(*lead, self.full_out_features)
 
 
+def own_parameter(module: nn.Module, name: str) -> Optional[torch.Tensor]:
+    """``module.<name>`` without the walk of ``nn.Module.__getattr__`` where it is a registered parameter."""
+    p = module._parameters.get(name)
+    return p if p is not None else getattr(module, name)
+
+
 class RowParallelLinear(_Linear):
     """Decoder layer: y = a @ weight.T + bias_param with weight [d_model, F]
     (parallel.py:335-383).  ``a`` is compacted to its non-zeros and decoded sparsely."""
