@@ -1128,18 +1128,20 @@ __global__ __launch_bounds__(256) void k_pool_hist(const SelState *st, const uin
 // walked runs of 1.3 entries through a book entry per run: as many bytes again, a chain of loads for the longest run of 64,
 // and seven cache lines per load.)  L = 12, T = 4096, F = 24576, k = 200, bf16, us: count / prefix / emit 133 / 29 / 256 with a
 // thread per run, 36 / 6 / 71 here; a threshold list of 24 layers, F = 32768: emit 382, count and emit here 61 + 172.
-constexpr int TILE_PORTION = 8, TILE_WAVES = 4;
+// Few extents go two to a wavefront instead: the chain of a wavefront's steps is all there is then.  us of the three, eight / two
+// to a wavefront: 18 432 extents (L = 12, T = 1024, F = 6144, float32) 45 / 33, 36 864 44 / 39, 147 456 114 / 120.
+constexpr int TILE_WAVES = 4, TILE_PORTION = 8, TILE_PORTION_FEW = 2, TILE_FEW = 64 * 1024;
 constexpr int TILE_NE = 2;   // loads of an extent in flight at once: 128 entries
-__host__ __device__ static inline int tile_portions(int nseg) { return (nseg + TILE_PORTION - 1) / TILE_PORTION; }
+static int tile_portion(int64_t extents) { return extents < TILE_FEW ? TILE_PORTION_FEW : TILE_PORTION; }
 
 // f(entry, live, n) for the entries of a portion in order of (segment, row, feature), 64 at a time, the first n lanes live.
-template <typename F> __device__ __forceinline__ void visit_portion(const uint2 *tile_meta, const uint2 *pool, int rowblk, int nrb, int seg0,
+template <int P, typename F> __device__ __forceinline__ void visit_portion(const uint2 *tile_meta, const uint2 *pool, int rowblk, int nrb, int seg0,
                                                                     int nseg, F f) {
   const int lane = lane_id();
-  const uint2 mine = lane < TILE_PORTION && seg0 + lane < nseg ? tile_meta[(int64_t)(seg0 + lane) * nrb + rowblk] : make_uint2(0u, 0u);
-  uint2 en[TILE_PORTION][TILE_NE];
+  const uint2 mine = lane < P && seg0 + lane < nseg ? tile_meta[(int64_t)(seg0 + lane) * nrb + rowblk] : make_uint2(0u, 0u);
+  uint2 en[P][TILE_NE];
 #pragma unroll
-  for (int i = 0; i < TILE_PORTION; ++i) {
+  for (int i = 0; i < P; ++i) {
     const uint32_t off = __builtin_amdgcn_readlane(mine.x, i), n = __builtin_amdgcn_readlane(mine.y, i);
 #pragma unroll
     for (int e = 0; e < TILE_NE; ++e) {
@@ -1148,7 +1150,7 @@ template <typename F> __device__ __forceinline__ void visit_portion(const uint2 
     }
   }
 #pragma unroll
-  for (int i = 0; i < TILE_PORTION; ++i) {
+  for (int i = 0; i < P; ++i) {
     const uint32_t off = __builtin_amdgcn_readlane(mine.x, i), n = __builtin_amdgcn_readlane(mine.y, i);
 #pragma unroll
     for (int e = 0; e < TILE_NE; ++e)
@@ -1165,17 +1167,17 @@ __device__ __forceinline__ int collect_token(int grow, int Tn, int Tp) {
 
 // k_tile_count: per (row, portion), how many entries beat the threshold key (low half) / equal it (high half: a portion
 // has at most 1024 of a row).  Grid: x = blocks of 64 rows, y = blocks of TILE_WAVES portions, z = layer.
-template <typename T>
+template <typename T, int P>
 __global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_count(int Tp, const SelState *st, const uint2 *tile_meta, int nseg,
                                                                 const uint2 *pool, unsigned long long pool_cap, uint32_t *counts) {
   __shared__ uint32_t cnt[TILE_WAVES][COLLECT_ROWS];
   const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
-  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  const int nport = (nseg + P - 1) / P, nrb = Tp / COLLECT_ROWS;
   const SelState s = st[l];
   if (s.path != PATH_TILES || s.status != ST_DONE || part >= nport) return;
   cnt[wv][lane] = 0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+  visit_portion<P>(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * P, nseg,
     [&](const uint2 &e, bool live) {
       const uint32_t key = rank_key_of<T>(Elem<T>::to_f32(Elem<T>::from_raw(e.y)));
       if (live && key >= s.thr_key) atomicAdd(&cnt[wv][collect_row(e.x)], key == s.thr_key ? 1u << 16 : 1u);
@@ -1217,14 +1219,14 @@ __global__ __launch_bounds__(256) void k_row_prefix(
 // that beat the key, and ties while the row's allotment lasts) + those kept earlier in this one, which a counter per row
 // holds, + those kept before it among its row's lanes of the 64 at hand, from the lanes' votes.
 // ALL: a threshold list, every entry is kept (`before` then counts them in its first half).
-template <typename T, bool ALL>
+template <typename T, bool ALL, int P>
 __global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_emit(
     int Tn, int Tp, const SelState *st, const uint2 *tile_meta, int nseg, const uint2 *pool, unsigned long long pool_cap,
     const uint2 *before, const uint32_t *allot, const int32_t *row_ptr, int32_t *col_out, T *val_out, const int32_t *skip) {
   __shared__ uint32_t next_sh[TILE_WAVES][COLLECT_ROWS], tie_sh[ALL ? 1 : TILE_WAVES][COLLECT_ROWS], allot_sh[ALL ? 1 : TILE_WAVES][COLLECT_ROWS];
   if (ALL && skip && *skip != 0) return;      // the list did not fit the caller's arrays: it was emptied
   const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
-  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  const int nport = (nseg + P - 1) / P, nrb = Tp / COLLECT_ROWS;
   uint32_t thr = 0;
   if constexpr (!ALL) {
     const SelState s = st[l];
@@ -1247,7 +1249,7 @@ __global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_emit(
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+  visit_portion<P>(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * P, nseg,
     [&](const uint2 &e, bool live) {
       const int row = live ? collect_row(e.x) : -1, row_before = __shfl_up(row, 1), row_after = __shfl_down(row, 1);
       // this row's lanes: from its first one (`first`: the lanes before that) on
@@ -1310,15 +1312,16 @@ __global__ void k_selected_min_accumulate(const uint32_t *keys, int64_t n, T *su
 
 // ---- threshold activation on encoder-collected entries (every entry is a survivor) ----------
 // Per (row, portion): the entries.  Grid as of k_tile_count.
+template <int P>
 __global__ __launch_bounds__(TILE_WAVES * 64) void k_tile_count_all(int Tp, const uint2 *tile_meta, int nseg, const uint2 *pool,
                                                                     unsigned long long pool_cap, uint32_t *counts) {
   __shared__ uint32_t cnt[TILE_WAVES][COLLECT_ROWS];
   const int l = blockIdx.z, wv = threadIdx.x >> 6, lane = lane_id(), part = blockIdx.y * TILE_WAVES + wv;
-  const int nport = tile_portions(nseg), nrb = Tp / COLLECT_ROWS;
+  const int nport = (nseg + P - 1) / P, nrb = Tp / COLLECT_ROWS;
   if (part >= nport) return;
   cnt[wv][lane] = 0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  visit_portion(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * TILE_PORTION, nseg,
+  visit_portion<P>(tile_meta + (int64_t)l * nseg * nrb, pool + (unsigned long long)l * pool_cap, blockIdx.x, nrb, part * P, nseg,
     [&](const uint2 &e, bool live) { if (live) atomicAdd(&cnt[wv][collect_row(e.x)], 1u); });
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   counts[((int64_t)l * nport + part) * Tp + blockIdx.x * COLLECT_ROWS + lane] = cnt[wv][lane];
@@ -1752,7 +1755,7 @@ struct TileLayout {
   size_t off_tmeta, off_tpool, off_counts, off_before, off_tcount, total;
   unsigned long long tpool_cap;              // entries per layer
   uint32_t caps;                             // entries per fixed tile slot
-  int nseg, ntile;
+  int nseg, ntile, portion, nport;           // segments, extents; segments of a portion, portions of a row
 };
 
 static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dtype) {
@@ -1762,6 +1765,8 @@ static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dt
   tl.nseg = (int)(collect_grid_rows(F) / segw);   // whole feature tiles too (COLLECT_TILE_ROWS is the tile's side)
   const int64_t Tp = collect_grid_rows(T);   // the epilogue's books cover whole token tiles
   tl.ntile = tl.nseg * (int)(Tp / COLLECT_ROWS);
+  tl.portion = tile_portion(tl.ntile * L);
+  tl.nport = (int)clt_ceil_div(tl.nseg, tl.portion);
   // about 1.5x K candidates are expected, i.e. 1.5 * k / F of a tile's 64 * segw elements; a
   // slot holds three times that (at least 64, at most the whole tile)
   unsigned long long caps = (unsigned long long)(3.0 * 1.5 * (double)k / (double)F * (double)COLLECT_ROWS * segw) + 64ull;
@@ -1777,7 +1782,7 @@ static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dt
   auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
   tl.off_tmeta = take(8 * (size_t)tl.ntile * (size_t)L);
   tl.off_tpool = take(8 * (size_t)tl.tpool_cap * (size_t)L);
-  const size_t cells = (size_t)tile_portions(tl.nseg) * (size_t)Tp * (size_t)L;   // (row, portion) pairs
+  const size_t cells = (size_t)tl.nport * (size_t)Tp * (size_t)L;   // (row, portion) pairs
   tl.off_counts = take(4 * cells);
   tl.off_before = take(8 * cells);
   tl.off_tcount = take(4 * (size_t)L);
@@ -1851,16 +1856,18 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
     k_select_level<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist, first, pool, lo.pool_cap, level, 1);
     k_select_scan<T><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 2, level);
   }
-  const int nport = tile_portions(tl.nseg);
   const int64_t Tp = collect_grid_rows(Tn);
-  dim3 grid3((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(nport, TILE_WAVES), (unsigned)L);
+  dim3 grid3((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(tl.nport, TILE_WAVES), (unsigned)L);
+  const bool few = tl.portion == TILE_PORTION_FEW;
   uint32_t *counts = (uint32_t *)(ws + tl.off_counts);
   uint2 *before = (uint2 *)(ws + tl.off_before);
-  k_tile_count<T><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, counts);
-  k_row_prefix<<<dim3((unsigned)clt_ceil_div(Tn, 64), (unsigned)L), 64, 0, stream>>>(Tn, Tp, st, nport, counts, before, rgt, req);
+  if (few) k_tile_count<T, TILE_PORTION_FEW><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, counts);
+  else k_tile_count<T, TILE_PORTION><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, counts);
+  k_row_prefix<<<dim3((unsigned)clt_ceil_div(Tn, 64), (unsigned)L), 64, 0, stream>>>(Tn, Tp, st, tl.nport, counts, before, rgt, req);
   k_select_count<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, rgt, req, 1);
   k_select_allot<false><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, Tn, L, rgt, req, allot, keep, row_ptr, K, 1);
-  k_tile_emit<T, false><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tn, (int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, before, allot, row_ptr, col, val, nullptr);
+  if (few) k_tile_emit<T, false, TILE_PORTION_FEW><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tn, (int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, before, allot, row_ptr, col, val, nullptr);
+  else k_tile_emit<T, false, TILE_PORTION><<<grid3, TILE_WAVES * 64, 0, stream>>>((int)Tn, (int)Tp, st, tmeta, tl.nseg, tpool, tl.tpool_cap, before, allot, row_ptr, col, val, nullptr);
   k_select_emit<T, false><<<grid2, 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, first, pool, lo.pool_cap, allot,
                                                      row_ptr, col, val, 1, nullptr);
   return clt_check_launch();
@@ -1871,7 +1878,7 @@ struct ThreshLayout {
   size_t off_state, off_tcount, off_tmeta, off_tpool, off_counts, off_before, off_rowcnt, total;
   unsigned long long tpool_cap;
   uint32_t caps;
-  int nseg, ntile;
+  int nseg, ntile, portion, nport;           // as in TileLayout
 };
 
 static ThreshLayout thresh_layout(int64_t T, int64_t F, int64_t L, int64_t density_ppm, int dtype) {
@@ -1880,6 +1887,8 @@ static ThreshLayout thresh_layout(int64_t T, int64_t F, int64_t L, int64_t densi
   tl.nseg = (int)(collect_grid_rows(F) / segw);   // whole feature tiles too (COLLECT_TILE_ROWS is the tile's side)
   const int64_t Tp = collect_grid_rows(T);   // the epilogue's books cover whole token tiles
   tl.ntile = tl.nseg * (int)(Tp / COLLECT_ROWS);
+  tl.portion = tile_portion(tl.ntile * L);
+  tl.nport = (int)clt_ceil_div(tl.nseg, tl.portion);
   const double dens = (double)(density_ppm < 1 ? 1 : density_ppm) * 1e-6;
   // a fixed slot holds three times the expected entries of a tile (at least 64, at most the tile)
   unsigned long long caps = (unsigned long long)(3.0 * dens * (double)COLLECT_ROWS * segw) + 64ull;
@@ -1895,7 +1904,7 @@ static ThreshLayout thresh_layout(int64_t T, int64_t F, int64_t L, int64_t densi
   tl.off_tcount = take(4 * (size_t)L);
   tl.off_tmeta = take(8 * (size_t)tl.ntile * (size_t)L);
   tl.off_tpool = take(8 * (size_t)tl.tpool_cap * (size_t)L);
-  const size_t cells = (size_t)tile_portions(tl.nseg) * (size_t)Tp * (size_t)L;   // (row, portion) pairs
+  const size_t cells = (size_t)tl.nport * (size_t)Tp * (size_t)L;   // (row, portion) pairs
   tl.off_counts = take(4 * cells);
   tl.off_before = take(8 * cells);
   tl.off_rowcnt = take(4 * (size_t)T * (size_t)L);
@@ -1950,12 +1959,12 @@ extern "C" int clt_encode_threshold_count(const void *x, const void *w, const vo
                              nullptr, &ca, s);
   if (rc != CLT_OK) return rc;
   uint32_t *rowcnt = (uint32_t *)(ws + tl.off_rowcnt);
-  const int nport = tile_portions(tl.nseg);
   const int64_t Tp = collect_grid_rows(T);
   uint32_t *counts = (uint32_t *)(ws + tl.off_counts);
-  k_tile_count_all<<<dim3((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(nport, TILE_WAVES), (unsigned)L), TILE_WAVES * 64, 0, s>>>(
-      (int)Tp, ca.tile_meta, tl.nseg, ca.pool, tl.tpool_cap, counts);
-  k_row_prefix_all<<<dim3((unsigned)clt_ceil_div(T, 64), (unsigned)L), 64, 0, s>>>(T, Tp, nport, counts, (uint2 *)(ws + tl.off_before), rowcnt);
+  const dim3 grid((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(tl.nport, TILE_WAVES), (unsigned)L);
+  if (tl.portion == TILE_PORTION_FEW) k_tile_count_all<TILE_PORTION_FEW><<<grid, TILE_WAVES * 64, 0, s>>>((int)Tp, ca.tile_meta, tl.nseg, ca.pool, tl.tpool_cap, counts);
+  else k_tile_count_all<TILE_PORTION><<<grid, TILE_WAVES * 64, 0, s>>>((int)Tp, ca.tile_meta, tl.nseg, ca.pool, tl.tpool_cap, counts);
+  k_row_prefix_all<<<dim3((unsigned)clt_ceil_div(T, 64), (unsigned)L), 64, 0, s>>>(T, Tp, tl.nport, counts, (uint2 *)(ws + tl.off_before), rowcnt);
   k_rowptr_scan<<<1, SCAN_THREADS, 0, s>>>(rowcnt, L * T, row_ptr);
   k_thresh_finish<<<1, 64, 0, s>>>(st, (int)L, row_ptr, L * T);
   return clt_check_launch();
@@ -2029,15 +2038,17 @@ extern "C" int clt_encode_threshold_emit(int64_t T, int64_t F, int64_t L, int64_
   hipStream_t s = (hipStream_t)stream;
   char *ws = (char *)workspace;
   const int64_t Tp = collect_grid_rows(T);
-  dim3 grid((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(tile_portions(tl.nseg), TILE_WAVES), (unsigned)L);
-#define CLT_EMIT_ALL(TT)                                                                                                              \
-  k_tile_emit<TT, true><<<grid, TILE_WAVES * 64, 0, s>>>((int)T, (int)Tp, nullptr, (const uint2 *)(ws + tl.off_tmeta), tl.nseg,        \
+  dim3 grid((unsigned)(Tp / COLLECT_ROWS), (unsigned)clt_ceil_div(tl.nport, TILE_WAVES), (unsigned)L);
+#define CLT_EMIT_ALL_P(TT, PP)                                                                                                        \
+  k_tile_emit<TT, true, PP><<<grid, TILE_WAVES * 64, 0, s>>>((int)T, (int)Tp, nullptr, (const uint2 *)(ws + tl.off_tmeta), tl.nseg,        \
                                                          (const uint2 *)(ws + tl.off_tpool), tl.tpool_cap,                            \
                                                          (const uint2 *)(ws + tl.off_before), nullptr, row_ptr, col, (TT *)val, skip)
+#define CLT_EMIT_ALL(TT) do { if (tl.portion == TILE_PORTION_FEW) CLT_EMIT_ALL_P(TT, TILE_PORTION_FEW); else CLT_EMIT_ALL_P(TT, TILE_PORTION); } while (0)
   if (dtype == CLT_BF16) CLT_EMIT_ALL(bf16_t);
   else if (dtype == CLT_F16) CLT_EMIT_ALL(f16_t);
   else CLT_EMIT_ALL(float);
 #undef CLT_EMIT_ALL
+#undef CLT_EMIT_ALL_P
   return clt_check_launch();
 }
 

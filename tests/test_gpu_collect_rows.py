@@ -1,5 +1,5 @@
 """The ordered write of the candidates that the encoder's epilogue collects (k_tile_count, k_tile_emit) against the selection on
-stored pre-activations: 64 entries at a time, 128 in flight per extent, 8 segments per wavefront.  Rows that hold whole segments
+stored pre-activations: 64 entries at a time, 128 in flight per extent, 2 or 8 segments per wavefront.  Rows that hold whole segments
 (a run longer than a wavefront, rows cut by the 64s), rows with none, batches and features that are no whole number of
 tiles, and ties that a row's allotment cuts, all in small whole numbers, so that both sides have the same pre-activations."""
 import pytest
@@ -34,6 +34,7 @@ SHAPES = [
     (2, 300, 64, 2304, 40, True),
     (1, 511, 128, 520, 130, True),              # a quarter of the features kept
     (3, 640, 64, 4096, 3, True),
+    (8, 1030, 64, 53000, 4, True),              # extents enough for eight of them to a wavefront (two in the others)
 ]
 
 
