@@ -1614,7 +1614,9 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   // share.  A counter per problem, asked for every row's place, was what bounded the pass: requests to one address are served
   // one by one, 15 ns apart (36 000 rows ranked together: 590 us, whatever the rows held).
   const unsigned long long waves = 4ull * (unsigned long long)pass_blocks(T * split, L) * (mode == CLT_TOPK_GLOBAL ? (unsigned long long)L : 1ull);
-  lo.slot_size = (uint32_t)((2ull * K + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull);
+  // (All parts together stay below 2^30 entries: the kernel's places are 32-bit numbers, and K may reach 2^32.)
+  const unsigned long long share = (2ull * K + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull;
+  lo.slot_size = (uint32_t)(share < (1ull << 30) / waves ? share : (1ull << 30) / waves);
   cap += waves * lo.slot_size;
   if (cap > 0xFFF00000ull) cap = 0xFFF00000ull;
   lo.pool_cap = cap;
