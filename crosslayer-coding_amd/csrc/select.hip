@@ -426,8 +426,8 @@ __global__ __launch_bounds__(256) void k_select_pass(
   uint2 *mypool = pool + (unsigned long long)p * pool_cap;
   // this wavefront's own part of the pool, and where the part that is handed out by a counter begins
   const uint32_t waves = gridDim.x * (uint32_t)nwv;
-  uint32_t own = ((GLOBAL ? (uint32_t)l * waves : 0u) + blockIdx.x * (uint32_t)nwv + (uint32_t)wv) * slot_size;
-  const uint32_t own_end = own + slot_size, shared_at = (GLOBAL ? gridDim.y * waves : waves) * slot_size;
+  const uint32_t own = ((GLOBAL ? (uint32_t)l * waves : 0u) + blockIdx.x * (uint32_t)nwv + (uint32_t)wv) * slot_size;
+  PoolPart part = {own, own + slot_size, (GLOBAL ? gridDim.y * waves : waves) * slot_size, pool_cap, false};
   for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
     const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
     const int64_t r = (int64_t)l * Tn + t;
@@ -438,13 +438,12 @@ __global__ __launch_bounds__(256) void k_select_pass(
     auto flush = [&]() {
       if (n_buf == 0) return;
       if (!dense) {
-        uint32_t off = own;
-        if (own_end - own > n_buf) own += n_buf + 1u;
-        else {
-          if (lane == 0) off = atomicAdd(&pool_count[p], n_buf + 1u);
-          off = __builtin_amdgcn_readfirstlane(off) + shared_at;
-        }
-        if ((unsigned long long)off + n_buf + 1ull > pool_cap) dense = true;
+        const uint32_t off = part.take(n_buf + 1u, [&](uint32_t n) {
+          uint32_t was = 0;
+          if (lane == 0) was = atomicAdd(&pool_count[p], n);
+          return (uint32_t)__builtin_amdgcn_readfirstlane(was);
+        });
+        if (off == POOL_FULL) dense = true;
         else {
           if (lane == 0) {
             mypool[off] = make_uint2(ROW_NONE, n_buf);           // extent header: (next, count)
@@ -1614,11 +1613,11 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   // share.  A counter per problem, asked for every row's place, was what bounded the pass: requests to one address are served
   // one by one, 15 ns apart (36 000 rows ranked together: 590 us, whatever the rows held).
   const unsigned long long waves = 4ull * (unsigned long long)pass_blocks(T * split, L) * (mode == CLT_TOPK_GLOBAL ? (unsigned long long)L : 1ull);
-  // (All parts together stay below 2^30 entries: the kernel's places are 32-bit numbers, and K may reach 2^32.)
+  // (All parts together stay below 2^30 entries: places are 32-bit numbers, and K may reach 2^32.)
   const unsigned long long share = (2ull * K + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull;
   lo.slot_size = (uint32_t)(share < (1ull << 30) / waves ? share : (1ull << 30) / waves);
   cap += waves * lo.slot_size;
-  if (cap > 0xFFF00000ull) cap = 0xFFF00000ull;
+  if (cap > POOL_MOST) cap = POOL_MOST;
   lo.pool_cap = cap;
   // A sample with e keys above the threshold gives a cut with up to (1.25 + 6 / sqrt(e) + 17 / e) K candidates:
   // 2.8 K at SAMPLE_HITS.  K elements are one in 1500 when 12 layers of 24576 features are ranked together and 200

@@ -25,6 +25,27 @@ struct SelState {
   uint32_t overflow;  // the encoder epilogue ran out of pool space (set with atomicOr)
 };
 
+// Places of the streaming pass's candidate pool as one wavefront takes them: from its own part while that lasts, then from the end
+// that a counter per problem hands out.  Places are 32-bit numbers, the sum that makes one is not; and who has been told
+// that the pool is full asks no more - it stays full -, so that the counter ends at most one request per wavefront
+// beyond the pool's POOL_MOST entries and does not come round to its beginning.
+constexpr unsigned long long POOL_MOST = 0xF0000000ull;
+constexpr uint32_t POOL_FULL = 0xFFFFFFFFu;
+struct PoolPart {
+  uint32_t own, own_end;          // what is left of the own part
+  unsigned long long shared_at;   // where the shared end begins
+  unsigned long long cap;
+  bool full;
+  // `n` places in a row, or POOL_FULL; `ask(n)` adds n to the counter and returns what it was
+  template <typename Ask> __host__ __device__ uint32_t take(uint32_t n, Ask ask) {
+    if (own_end - own >= n) { own += n; return own - n; }
+    if (full) return POOL_FULL;
+    const unsigned long long at = shared_at + ask(n);
+    full = at + n > cap;
+    return full ? POOL_FULL : (uint32_t)at;
+  }
+};
+
 // tokens of one wave tile of the collecting encoder epilogue
 constexpr int COLLECT_ROWS = 64;
 // tokens of one workgroup tile of the encoder kernel
