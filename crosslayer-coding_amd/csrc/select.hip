@@ -428,7 +428,14 @@ __global__ __launch_bounds__(256) void k_select_pass(
   const uint32_t waves = gridDim.x * (uint32_t)nwv;
   const uint32_t own = ((GLOBAL ? (uint32_t)l * waves : 0u) + blockIdx.x * (uint32_t)nwv + (uint32_t)wv) * slot_size;
   PoolPart part = {own, own + slot_size, (GLOBAL ? gridDim.y * waves : waves) * slot_size, pool_cap, false};
-  for (int64_t t = (int64_t)blockIdx.x * nwv + wv; t < Tn; t += (int64_t)gridDim.x * nwv) {
+  // The wavefronts change places from one round over the rows to the next: tokens with many times the usual candidates may
+  // stand at any distance from each other, such as the number of wavefronts.  (Every 340th of 3000 tokens eight times as
+  // large, L = 12, F = 24576, bf16, ranked together / per layer: 1636 / 1056 us without, 996 / 712 with.)
+  for (int64_t round = 0; round * waves < Tn; ++round) {
+    uint32_t place = blockIdx.x * (uint32_t)nwv + (uint32_t)wv + __umulhi((uint32_t)round * 0x9E3779B9u, waves);
+    if (place >= waves) place -= waves;
+    const int64_t t = round * waves + place;
+    if (t >= Tn) continue;
     const auto rk = RankOf<T, GLOBAL>::make(mean, denom, row_columns(l, t, F, split));
     const int64_t r = (int64_t)l * Tn + t;
     const T *row = pre + l * lstride + t * F;
