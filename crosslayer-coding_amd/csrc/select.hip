@@ -1604,6 +1604,14 @@ static int pass_blocks(int64_t rows, int64_t L) {
   return (int)(want < most ? want : most);
 }
 
+// The same of a pass that runs again for the layers whose cut failed: usually one, which then has the chip to itself; the
+// workgroups of the others end at once.  (One of 12 layers, F = 24576, 3000 tokens, bf16: the whole selection 1824 us, 2493
+// with pass_blocks; where the encoder collects 2567, 3413.)
+static int retry_blocks(int64_t rows) {
+  const int64_t want = clt_ceil_div(rows, 8);
+  return (int)(want < 1024 ? want : 1024);
+}
+
 static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode, int split) {
   SelLayout lo;
   lo.nprob = mode == CLT_TOPK_GLOBAL ? 1 : (int)L;
@@ -1690,9 +1698,11 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
   if (split > 1) row_ptr = (int32_t *)(ws + lo.off_rows);
   Tn *= split;
   F /= split;
-  const dim3 grid((unsigned)pass_blocks(Tn, L), (unsigned)L);
   for (int phase = 0; phase < 2; ++phase) {
-    k_select_pass<T, V, GLOBAL><<<grid, 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, poolcnt, pool, lo.pool_cap, first, phase, xcut, split, lo.slot_size);
+    // all layers take part in a pass over the global ranking; the wavefronts of another grid share the same parts of the pool
+    const int usual = pass_blocks(Tn, L), blocks = phase == 0 || GLOBAL ? usual : retry_blocks(Tn);
+    const uint32_t slot = (uint32_t)((unsigned long long)lo.slot_size * (unsigned)usual / (unsigned)blocks);
+    k_select_pass<T, V, GLOBAL><<<dim3((unsigned)blocks, (unsigned)L), 256, 0, stream>>>(pre, Tn, F, L, lstride, mean, denom, st, hist, poolcnt, pool, lo.pool_cap, first, phase, xcut, split, slot);
     k_select_scan<T><<<nprob, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, phase, 0);
   }
   int gx2 = (int)clt_ceil_div(Tn, 4);
@@ -1850,7 +1860,7 @@ static int run_collect_select(const T *pre, int64_t Tn, int64_t F, int64_t L, in
   unsigned long long K = (unsigned long long)k * (unsigned long long)Tn;
   if (K > N) K = N;
   // retry of the layers whose cut failed: streaming pass from the bottom key over `pre`
-  k_select_pass<T, VV, false><<<dim3((unsigned)pass_blocks(Tn, L), (unsigned)L), 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist,
+  k_select_pass<T, VV, false><<<dim3((unsigned)retry_blocks(Tn), (unsigned)L), 256, 0, stream>>>(pre, Tn, F, L, lstride, nullptr, nullptr, st, hist,
                                                                         poolcnt, pool, lo.pool_cap, first, 1, nullptr, 1, lo.slot_size);
   k_select_scan<T><<<(unsigned)L, SCAN_THREADS, 0, stream>>>(st, hist, poolcnt, 1, 0);
   int gx2 = (int)clt_ceil_div(Tn, 4);
