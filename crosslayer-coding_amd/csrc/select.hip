@@ -24,6 +24,7 @@
 // again with the lowest cut, so the result is exact for any input; only the speed depends
 // on the sample being representative.
 #include "select_state.h"
+#include <cmath>
 #include <mutex>
 
 namespace {
@@ -1612,7 +1613,8 @@ static int retry_blocks(int64_t rows) {
   return (int)(want < 1024 ? want : 1024);
 }
 
-static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode, int split) {
+// `parts`: whether the wavefronts of the pass get parts of the pool of their own.
+static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode, int split, bool parts) {
   SelLayout lo;
   lo.nprob = mode == CLT_TOPK_GLOBAL ? 1 : (int)L;
   const size_t R = (size_t)(L * T * split);
@@ -1620,20 +1622,6 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   const unsigned long long N = (unsigned long long)T * F * (mode == CLT_TOPK_GLOBAL ? L : 1);
   unsigned long long K = (unsigned long long)k * T;
   if (K > N) K = N;
-  // about 2x K candidates are expected; every extent also stores one header entry
-  unsigned long long cap = 4ull * K + 2ull * rows_p + 4096ull;
-  const unsigned long long hard = N + 2ull * rows_p + 4096ull;
-  if (cap > hard) cap = hard;
-  // In front of those, a part for each wavefront of the pass, which holds its candidates unless they are more than 2 K's
-  // share.  A counter per problem, asked for every row's place, was what bounded the pass: requests to one address are served
-  // one by one, 15 ns apart (36 000 rows ranked together: 590 us, whatever the rows held).
-  const unsigned long long waves = 4ull * (unsigned long long)pass_blocks(T * split, L) * (mode == CLT_TOPK_GLOBAL ? (unsigned long long)L : 1ull);
-  // (All parts together stay below 2^30 entries: places are 32-bit numbers, and K may reach 2^32.)
-  const unsigned long long share = (2ull * K + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull;
-  lo.slot_size = (uint32_t)(share < (1ull << 30) / waves ? share : (1ull << 30) / waves);
-  cap += waves * lo.slot_size;
-  if (cap > POOL_MOST) cap = POOL_MOST;
-  lo.pool_cap = cap;
   // A sample with e keys above the threshold gives a cut with up to (1.25 + 6 / sqrt(e) + 17 / e) K candidates:
   // 2.8 K at SAMPLE_HITS.  K elements are one in 1500 when 12 layers of 24576 features are ranked together and 200
   // kept per token: the smallest sample then has 11 hits and a cut with 4.6 K, which is more than the pool holds -
@@ -1642,6 +1630,30 @@ static SelLayout sel_layout(int64_t T, int64_t F, int64_t L, int64_t k, int mode
   double ns = K ? SAMPLE_HITS * (double)N / (double)K : 0.0;
   lo.sample_n = SAMPLE_MIN;
   while (lo.sample_n < SAMPLE_MAX && (double)lo.sample_n < ns) lo.sample_n *= 4;
+  // room for 4 K; every extent also stores one header entry
+  const unsigned long long headers = 2ull * rows_p + 4096ull;
+  unsigned long long cap = (4ull * K < N ? 4ull * K : N) + headers;
+  // The beginning of it belongs to the wavefronts of the pass, a part each, which holds its candidates unless they are more than
+  // 2 K's share.  A counter per problem, asked for every row's place, was what bounded the pass: requests to one address
+  // are served one by one, 15 ns apart (36 000 rows ranked together: 590 us, whatever the rows held).  Behind the parts
+  // there is room for all candidates again, in case they are a few wavefronts'; that makes the pool larger than 4 K only
+  // where fewer than 100 of the sample are above the threshold, and never much larger than all elements.  (T = 8192, F = 8192,
+  // L = 16, k = 2000: 8.4 GB, as without parts; with the parts in front of 4 K it took 12.6.)
+  lo.slot_size = 0;
+  if (parts) {
+    const unsigned long long waves = 4ull * (unsigned long long)pass_blocks(T * split, L) * (mode == CLT_TOPK_GLOBAL ? (unsigned long long)L : 1ull);
+    // (All parts together stay below 2^30 entries: places are 32-bit numbers, and K may reach 2^32.)
+    const unsigned long long share = ((2ull * K < N / 2 ? 2ull * K : N / 2) + waves - 1) / waves + 2ull * ((rows_p + waves - 1) / waves) + 64ull;
+    lo.slot_size = (uint32_t)(share < (1ull << 30) / waves ? share : (1ull << 30) / waves);
+    const double e = (double)lo.sample_n * (double)K / (double)N, c = e > 0.0 ? 1.25 + 6.0 / sqrt(e) + 17.0 / e : 4.0;
+    const double most = (c < 4.0 ? c : 4.0) * (double)K;
+    const unsigned long long need = waves * lo.slot_size + (most < (double)N ? (unsigned long long)most : N) + headers;
+    const unsigned long long all = N + headers + waves * (unsigned long long)(WBUF + 64);   // and what a part has left over
+    const unsigned long long room = need < all ? need : all;
+    if (room > cap) cap = room;
+  }
+  if (cap > POOL_MOST) cap = POOL_MOST;
+  lo.pool_cap = cap;
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t at = o; o += (bytes + 255) & ~(size_t)255; return at; };
   lo.off_state = take(sizeof(SelState) * (size_t)lo.nprob);
@@ -1667,7 +1679,7 @@ static int run_batchtopk(const T *pre, int64_t Tn, int64_t F, int64_t L, int64_t
   constexpr int KB = Elem<T>::KEYBITS;
   const int mode = GLOBAL ? CLT_TOPK_GLOBAL : CLT_TOPK_PER_LAYER;
   const int split = row_split(Tn, F, L);
-  const SelLayout lo = sel_layout(Tn, F, L, k, mode, split);
+  const SelLayout lo = sel_layout(Tn, F, L, k, mode, split, true);
   SelState *st = (SelState *)(ws + lo.off_state);
   uint32_t *hist = (uint32_t *)(ws + lo.off_hist);
   uint32_t *poolcnt = (uint32_t *)(ws + lo.off_poolcnt);
@@ -1778,7 +1790,7 @@ struct TileLayout {
 
 static TileLayout tile_layout(int64_t T, int64_t F, int64_t L, int64_t k, int dtype) {
   TileLayout tl;
-  tl.sel = sel_layout(T, F, L, k, CLT_TOPK_PER_LAYER, 1);
+  tl.sel = sel_layout(T, F, L, k, CLT_TOPK_PER_LAYER, 1, false);   // its pool is for retries alone
   const int segw = dtype != CLT_F32 ? 128 : 64;
   tl.nseg = (int)(collect_grid_rows(F) / segw);   // whole feature tiles too (COLLECT_TILE_ROWS is the tile's side)
   const int64_t Tp = collect_grid_rows(T);   // the epilogue's books cover whole token tiles
@@ -2128,7 +2140,7 @@ extern "C" size_t clt_batchtopk_workspace_bytes(int64_t T, int64_t F, int64_t L,
   (void)dtype;
   if (T <= 0 || F <= 0 || L <= 0) return 256;
   if (k < 0) k = 0;
-  return sel_layout(T, F, L, k, mode, row_split(T, F, L)).total;
+  return sel_layout(T, F, L, k, mode, row_split(T, F, L), true).total;
 }
 
 extern "C" int clt_batchtopk_select(const void *pre, int64_t T, int64_t F, int64_t L, int64_t pre_layer_stride,

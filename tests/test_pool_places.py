@@ -1,11 +1,13 @@
-"""Places in the candidate pool of the selection's streaming pass, where they come near 2^32: the arithmetic of the kernel
-(select_state.h) in a host program."""
+"""The candidate pool of the selection's streaming pass: places where they come near 2^32, by the arithmetic of the kernel
+(select_state.h) in a host program, and the pool's size."""
 import os
 import shutil
 import subprocess
 
 import pytest
+import torch
 
+from crosslayer_coding_amd import _native as nat
 from crosslayer_coding_amd import build as clt_build
 
 PROGRAM = r"""
@@ -50,3 +52,20 @@ def test_places_near_the_end_of_32_bits(tmp_path):
     assert proc.returncode == 0, proc.stdout[-2000:]
     run = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, timeout=60)
     assert run.returncode == 0, run.stdout
+
+
+@pytest.mark.parametrize("L,T,F,k", [(16, 8192, 8192, 2000), (12, 4096, 24576, 200), (24, 4096, 32768, 256), (16, 2048, 8192, 3000),
+                                     (16, 2048, 8192, 8000)])
+def test_the_pool_holds_four_times_what_is_kept_or_all_elements(L, T, F, k):
+    """The largest part of a selection's workspace: 8 bytes for each of 4 K candidates of a layer, or for all its elements, and one
+    header per extent; 2^25 bytes hold the rest (sample, statistics of rows, ends of the wavefronts' parts)."""
+    lib = nat.load()
+    K, N, rest = k * T, T * F, 20 * L * T + 2 ** 25
+    room = L * 8 * (min(4 * K, N) + 2 * T + 4096)
+    assert room <= lib.clt_batchtopk_workspace_bytes(T, F, L, k, nat.TOPK_PER_LAYER, nat.dtype_code(torch.bfloat16)) <= room + rest
+    # where the encoder collects the candidates this pool is for repeated passes, its own one beside it has fixed slots for
+    # 4.5 times the share of a tile, 64 each, and 2 K behind them
+    tiles = (T + 255) // 256 * 4 * ((F + 255) // 256 * 2)
+    slot = min(int(4.5 * k / F * 64 * 128) + 64, 64 * 128)
+    own = L * 8 * (tiles * slot + min(2 * K + 4096, N)) + L * (8 * tiles + 12 * T * (F // 256 + 2))
+    assert lib.clt_encode_collect_workspace_bytes(T, 768, F, L, k, nat.dtype_code(torch.bfloat16)) <= room + own + rest
