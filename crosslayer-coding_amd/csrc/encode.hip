@@ -102,10 +102,10 @@ __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)p;
 }
 __device__ __forceinline__ void fill16(const void *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"((const char *)base + off), "s"(lds_at) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"((const char *)base + off), "{m0}"(lds_at) : "memory");
 }
 __device__ __forceinline__ void fill4(const void *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"((const char *)base + off), "s"(lds_at) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"((const char *)base + off), "{m0}"(lds_at) : "memory");
 }
 
 typedef __attribute__((ext_vector_type(2))) float f32x2_t;
@@ -841,7 +841,7 @@ constexpr int SK_STAGES = 3;
 
 // As fill16, from a scalar base.
 __device__ __forceinline__ void sk_fill16(const void *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds_at) : "memory");
 }
 
 template <typename T, int NF, int MT>

@@ -58,10 +58,10 @@ __device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stre
 // Direct-to-LDS loads, 16 or 4 bytes per lane (lane i lands at lds_at + 16 i / 4 i).  As asm statements, so that the
 // compiler does not wait for them in front of every LDS read; whoever reads the data waits by hand.
 __device__ __forceinline__ void sp_fill16(const char *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds_at) : "memory");
 }
 __device__ __forceinline__ void sp_fill4(const uint32_t *base, uint32_t off, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_at) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds_at) : "memory");
 }
 
 template <typename T> struct SpMma;

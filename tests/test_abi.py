@@ -86,3 +86,20 @@ def test_encoder_kernels_spill_nothing(tmp_path):
     kernels = {k: v for k, v in scratch.items() if "k_encode_mfma" in k}
     assert len(kernels) >= 18, sorted(kernels)      # 3 element types x 3 epilogues x even / odd stage counts, + segmented
     assert all(v == 0 for v in kernels.values()), {k: v for k, v in kernels.items() if v}
+
+
+def test_statements_declare_the_register_they_need():
+    """m0 holds the LDS address of a direct load.  A statement that set it by itself would change it behind the compiler's back; it
+    is an operand, which the compiler sets and knows of."""
+    from crosslayer_coding_amd import build as clt_build
+
+    seen = 0
+    for name in sorted(os.listdir(clt_build.CSRC)):
+        text = open(os.path.join(clt_build.CSRC, name)).read()
+        for m in re.finditer(r"asm\s+volatile\((.*?)\);", text, re.S):
+            code, _, rest = m.group(1).partition(":")
+            assert not re.search(r"\bm0\b", code), (name, code)
+            if "load_lds" in code:
+                assert '"{m0}"' in rest, (name, m.group(0))
+                seen += 1
+    assert seen > 0
