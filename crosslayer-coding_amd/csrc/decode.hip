@@ -764,9 +764,140 @@ template <typename T, int HQ, int HTAIL, int UU> struct ThinBatch {
   }
 };
 
+// The lists of a token over sources 0 .. t as one, a source per lane: where source `lane`'s list begins, less what comes before it
+// in the one list, and where it ends there.
+struct ThinList {
+  int32_t at, end, total;
+  __device__ __forceinline__ ThinList(const int32_t *row_ptr, int64_t Tn, int64_t tok, int64_t t, uint64_t src_mask, int lane) {
+    at = end = 0;
+    if (lane <= t && ((src_mask >> lane) & 1ull)) {
+      at = row_ptr[lane * Tn + tok];
+      end = row_ptr[lane * Tn + tok + 1] - at;
+    }
+    at += end;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int32_t up = __shfl_up(end, o);
+      if (lane >= o) end += up;
+    }
+    at -= end;
+    total = __builtin_amdgcn_readlane(end, 63);
+  }
+  // the i-th entry's decoder row and value; beyond the end row 0 and a zero
+  template <typename T>
+  __device__ __forceinline__ void fetch(int32_t i, const int32_t *col, const T *val, int64_t t, int64_t F, int64_t L, int tying,
+                                        int32_t &row, T &v) const {
+    row = 0; v = Elem<T>::from_raw(0u);
+    int s = 0;
+    for (int u = 0; u < (int)t; ++u) s += i >= __builtin_amdgcn_readlane(end, u) ? 1 : 0;
+    const int32_t j = __shfl(at, s) + i;
+    if (i < total) {
+      row = (int32_t)decoder_slot(tying, s, t, L) * (int32_t)F + col[j];
+      v = val[j];
+    }
+  }
+};
+
 // A token with a list of more than THIN_LONG (batch-wide top-k gives some tokens many times the average) is left to the end, when
-// the workgroup's wavefronts share its chunks of 64 and add their sums in LDS.
-constexpr int THIN_WAVES = 4, THIN_LONG = 256;
+// the workgroup's wavefronts share its chunks of 64 and add their sums in LDS: 25 ns per entry.  One with more than THIN_MOST
+// (an outlying token may hold a tenth of all survivors) would keep four workgroups busy long after the others: it goes to
+// k_decode_thin_longest.
+constexpr int THIN_WAVES = 4, THIN_LONG = 256, THIN_MOST = 8192, THIN_PARTS = 16;
+
+// The longest lists: a workgroup for every target, 128-byte line of the rows and sixteenth of the tokens, in which it looks for
+// such lists and sums its columns of them.  A compute unit has some 64 lines on their way, and here an entry is one line, on
+// d / 64 (16 bits) as many units: 8 ns per entry.  Usually it finds none: 7 us.
+// us of the decode, L = 6, T = 1500, F = 16384, d = 1024, bf16, 200 per token over all layers, tokens with 0 / 1 x 20 000 / 1 x
+// 98 304 / 4 x 50 000 of the 300 000 entries: 260 / 470 / 886 / 478; left to the tokens' own workgroups 256 / 525 / 1909 / 1007;
+// the schedule by sources 334 / 412 / 824 / 589.  (In the first workgroups of k_decode_thin's launch it would end with the others, but their
+// code together spills: 830 against 795 us for the 3000 tokens above.)
+template <typename T>
+__global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin_longest(
+    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
+    const float *__restrict__ bias_sum, const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d,
+    int64_t F, int64_t L, int tying, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch, int units) {
+  constexpr int V = WVec<T>::V, COLS = 8 * V, NU = 4;     // 8 lanes per line, 8 rows per load
+  __shared__ int32_t found[THIN_WAVES * 64], n_found[THIN_WAVES];
+  __shared__ float shares[THIN_WAVES][COLS];
+  const int tid = threadIdx.x, lane = lane_id(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ll = lane & 7, grp = lane >> 3;
+  // (the workgroups of one part of the tokens follow each other, over all XCDs)
+  const int per_part = gridDim.x / THIN_PARTS, part = blockIdx.x / per_part, of_part = blockIdx.x - part * per_part, unit = of_part % units;
+  const int64_t t = t_end - 1 - of_part / units, begin = Tn * part / THIN_PARTS, end = Tn * (part + 1) / THIN_PARTS;
+  const T *wpart = wp + (int64_t)unit * COLS + ll * V;
+  for (int64_t tok0 = begin; tok0 < end; tok0 += THIN_WAVES * 64) {
+    const int64_t mine = tok0 + tid;
+    int32_t n = 0;
+    if (mine < end) {
+      const int32_t *p = row_ptr + mine;
+#pragma unroll 4
+      for (int s = 0; s <= (int)t; ++s, p += Tn) n += (src_mask >> s) & 1ull ? p[1] - p[0] : 0;
+    }
+    const uint64_t votes = __ballot(n > THIN_MOST);
+    if (lane == 0) n_found[wv] = __popcll(votes);
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < THIN_WAVES; ++w) {
+      before += w < wv ? n_found[w] : 0;
+      all += n_found[w];
+    }
+    if (n > THIN_MOST) found[before + __builtin_amdgcn_mbcnt_hi((uint32_t)(votes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)votes, 0u))] = tid;
+    __syncthreads();
+    for (int k = 0; k < all; ++k) {
+      const int64_t tok = tok0 + found[k];
+      const ThinList list(row_ptr, Tn, tok, t, src_mask, lane);
+      float acc[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) acc[j] = 0.0f;
+      int32_t row, next_row;
+      T v, next_v;
+      list.fetch(wv * 64 + lane, col, val, t, F, L, tying, row, v);
+      for (int32_t j0 = wv * 64; j0 < list.total; j0 += THIN_WAVES * 64) {
+#pragma unroll 1
+        for (int h = 0; h < 8; h += NU) {
+          uint4 w[NU];
+          float a[NU];
+#pragma unroll
+          for (int u = 0; u < NU; ++u) {                   // past the end: zeros times zeros
+            const int idx = 8 * (h + u) + grp;
+            a[u] = __shfl(Elem<T>::to_f32(v), idx);
+            const int64_t at = (int64_t)__shfl(row, idx) * pitch;
+            w[u] = make_uint4(0, 0, 0, 0);
+            if (j0 + idx < list.total) w[u] = *reinterpret_cast<const uint4 *>(wpart + at);
+          }
+          if (h == 0) list.fetch(j0 + THIN_WAVES * 64 + lane, col, val, t, F, L, tying, next_row, next_v);
+#pragma unroll
+          for (int u = 0; u < NU; u += 2) {
+            if constexpr (sizeof(T) == 2) WVec<T>::dot16(acc, w[u], w[u + 1], raw16_of<T>(a[u]) | (raw16_of<T>(a[u + 1]) << 16));
+            else {
+              WVec<T>::fma16(acc, w[u], a[u]);
+              WVec<T>::fma16(acc, w[u + 1], a[u + 1]);
+            }
+          }
+        }
+        row = next_row; v = next_v;
+      }
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        acc[j] += __shfl_xor(acc[j], 8);
+        acc[j] += __shfl_xor(acc[j], 16);
+        acc[j] += __shfl_xor(acc[j], 32);
+        if (grp == 0) shares[wv][ll * V + j] = acc[j];
+      }
+      __syncthreads();
+      if (tid < COLS) {
+        float y = (shares[0][tid] + shares[1][tid]) + (shares[2][tid] + shares[3][tid]);
+        const int64_t c = (int64_t)unit * COLS + tid, at = (t * Tn + tok) * d + c;
+        if (bias_sum) y += bias_sum[t * d + c];
+        if (skip_add) y += skip_add[at];
+        if (out_f32 || sizeof(T) == 4) ((float *)out)[at] = y;
+        else ((T *)out)[at] = Elem<T>::from_f32(y);
+      }
+      __syncthreads();
+    }
+  }
+}
+
 template <typename T, int HQ, int HTAIL>
 __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin(
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
@@ -784,48 +915,21 @@ __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin(
   const int64_t in0 = (idx % per_t) * THIN_WAVES;          // of the half: the first wavefront's token
   const T *wpart = wp + (int64_t)cpart * (d / 4);
 
-  // where source `lane`'s list of a token begins, less what comes before it in the one list, and where it ends there
-  int32_t list_at, list_end, total;
-  auto find_list = [&](int64_t tok) {
-    list_at = list_end = 0;
-    if (lane <= t && ((src_mask >> lane) & 1ull)) {
-      list_at = row_ptr[lane * Tn + tok];
-      list_end = row_ptr[lane * Tn + tok + 1] - list_at;
-    }
-    list_at += list_end;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int32_t up = __shfl_up(list_end, o);
-      if (lane >= o) list_end += up;
-    }
-    list_at -= list_end;
-    total = __builtin_amdgcn_readlane(list_end, 63);
-  };
   struct Entry { int32_t row; T v; };
-  auto fetch = [&](int32_t i) {
-    Entry e{0, Elem<T>::from_raw(0u)};
-    int s = 0;
-    for (int u = 0; u < (int)t; ++u) s += i >= __builtin_amdgcn_readlane(list_end, u) ? 1 : 0;
-    const int32_t j = __shfl(list_at, s) + i;
-    if (i < total) {
-      e.row = (int32_t)decoder_slot(tying, s, t, L) * (int32_t)F + col[j];
-      e.v = val[j];
-    }
-    return e;
-  };
   float acc[NACC];
   // every `step`-th chunk of the token's list from chunk `from` on; the lane groups' sums end up as ((g0 + g1) + (g2 + g3))
-  auto gather = [&](int from, int step) {
+  auto gather = [&](const ThinList &list, int from, int step) {
 #pragma unroll
     for (int j = 0; j < NACC; ++j) acc[j] = 0.0f;
-    Entry next = fetch(from * 64 + lane);
-    for (int32_t j0 = from * 64; j0 < total; j0 += step * 64) {
+    Entry next;
+    list.fetch(from * 64 + lane, col, val, t, F, L, tying, next.row, next.v);
+    for (int32_t j0 = from * 64; j0 < list.total; j0 += step * 64) {
       const int32_t my_row = next.row;
       const float my_val = Elem<T>::to_f32(next.v);
-      const int n = total - j0 < 64 ? total - j0 : 64;
+      const int n = list.total - j0 < 64 ? list.total - j0 : 64;
       ThinBatch<T, HQ, HTAIL, UU> ra, rb;
       ra.load(wpart, pitch, my_row, my_val, 0, n, ll, grp);
-      if (j0 + step * 64 < total) next = fetch(j0 + step * 64 + lane);
+      if (j0 + step * 64 < list.total) list.fetch(j0 + step * 64 + lane, col, val, t, F, L, tying, next.row, next.v);
       for (int i0 = 0; i0 < n; i0 += 2 * R) {
         if (i0 + R < n) rb.load(wpart, pitch, my_row, my_val, i0 + R, n, ll, grp);
         ra.consume(acc);
@@ -862,17 +966,14 @@ __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin(
   for (int w = -1; w < THIN_WAVES; ++w) {
     if (w == 0) __syncthreads();
     const int64_t in = in0 + (w < 0 ? wv : w), tok = half * in_half + in;
+    const bool on = in < in_half && tok < Tn;
+    if (w >= 0 && (totals[w] <= THIN_LONG || totals[w] > THIN_MOST)) continue;     // the same for the whole workgroup
+    const ThinList list(row_ptr, Tn, on ? tok : 0, t, on ? src_mask : 0ull, lane);
     if (w < 0) {
-      const bool on = in < in_half && tok < Tn;
-      total = 0;
-      if (on) find_list(tok);
-      if (lane == 0) totals[wv] = total;
-      if (!on || total > THIN_LONG) continue;
-    } else {
-      if (totals[w] <= THIN_LONG) continue;                // the same for the whole workgroup
-      find_list(tok);
+      if (lane == 0) totals[wv] = list.total;
+      if (!on || list.total > THIN_LONG) continue;
     }
-    gather(w < 0 ? 0 : wv, w < 0 ? 1 : THIN_WAVES);
+    gather(list, w < 0 ? 0 : wv, w < 0 ? 1 : THIN_WAVES);
     if (w >= 0) {
       if (grp == 0) {
 #pragma unroll
@@ -1786,6 +1887,9 @@ static int launch_decode_thin(const int32_t *row_ptr, const int32_t *col, const 
     else CLT_THIN(4, 0);
   }
 #undef CLT_THIN
+  const int units = (int)(d / (8 * V));
+  k_decode_thin_longest<T><<<(unsigned)(THIN_PARTS * units * (t_end - t_begin)), THIN_WAVES * 64, 0, stream>>>(row_ptr, col, (const T *)val,
+      (const T *)wp, bias_sum, skip_add, out, Tn, d, F, L, tying, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)), units);
   return clt_check_launch();
 }
 
@@ -1812,7 +1916,7 @@ static GatherWork gather_work(int64_t T, int64_t d, int64_t F, int64_t L, int64_
 // from HBM and read and write the partial rows of every triple, and against the decodes from LDS tiles.  This kernel, from what it
 // measured (bf16 and float32; L 2 - 16, d 512 - 2048, F 1024 - 24576, T 32 - 8000, 1 - 200 survivors per source and token): 9.5
 // TB/s, as much time again for a row's first use, 0.25 ns per triple, and no less than a workgroup's chain over its lists, or over
-// one of some thousand entries, which is what a top-k over the batch gives a single token.  Within 15 %, but for rows used more than
+// one of 4000 entries, as a top-k over the batch may give a single token (k_decode_thin_longest says what longer ones cost).  Within 15 %, but for rows used more than
 // 20 times, which it does faster.  us, schedule by sources / this: T = 3000, L = 12, F = 24576, d = 768, bf16, 200 survivors per
 // token over all layers 1530 / 854, 20 695 / 224; per layer 16: 1253 / 747; T = 1000, 50: 1100 / 790; T = 300, 200: 877 / 1078;
 // T = 77, 200: 340 / 356; float32, T = 600, 200: 2790 / 3910.
@@ -1821,7 +1925,7 @@ extern "C" int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L
   const GatherWork g = gather_work(T, d, F, L, targets, entries, tying, dtype);
   const double flow = g.bytes / 9.5e6 + g.distinct / 10e6 + g.triples * 0.25e-3, longest = entries < 4000 ? (double)entries : 4000.0;
   const double chain = 0.1 * (double)entries / T > 0.025 * longest ? 0.1 * (double)entries / T : 0.025 * longest;
-  const double thin = (flow > chain ? flow : chain) + 12;
+  const double thin = (flow > chain ? flow : chain) + 18;
   return thin < 0.95 * (g.bytes / 17e6 + g.distinct / 6.3e6 + g.triples * (double)d * 16 / 3.2e6 + 5) &&
          thin < clt_decode_tiles_us(T, d, F, L, targets, entries, tying, dtype) &&
          thin < clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);

@@ -139,3 +139,65 @@ def test_decode_thin_is_chosen_and_agrees_with_the_gather(monkeypatch, dtype):
     monkeypatch.setattr(lib, "clt_decode_thin_wanted", lambda *a: 0)
     ref = engine.decode_sparse(surv, w, "none", d, ws=ws, out_f32=True)
     assert ran == [1] and float((got - ref).norm() / ref.norm()) < 1e-6     # fp32 sums in another order
+
+
+@pytest.mark.parametrize("L,T,F,d,dtype,tying,out_f32,extra", [
+    (3, 40, 9000, 512, torch.bfloat16, "none", True, True),
+    (2, 17, 9000, 768, torch.bfloat16, "per_source", False, False),
+    (3, 33, 8300, 512, torch.float16, "none", True, False),
+    (2, 19, 8300, 768, torch.float32, "none", False, True),
+])
+def test_decode_thin_of_the_longest_lists(L, T, F, d, dtype, tying, out_f32, extra):
+    """Lists around 8192 entries, above which a kernel of its own sums them: one entry more and one less, those that cross the line
+    with a later source, two in one sixteenth of the batch, and the last token."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(T)
+    n = torch.randint(0, 4, (L, T), generator=g)
+    n[:, 1] = torch.tensor([8192] + [0] * (L - 1))
+    n[:, 2] = torch.tensor([8193] + [0] * (L - 1))
+    n[:, 3] = torch.tensor([8191] + [1] * (L - 1))         # 8192 at target 1, at target 2 one more
+    n[:, T // 2] = F
+    n[:, T - 1] = torch.tensor([0, 8200] + [5] * (L - 2))
+    keep, act, row_ptr = _lists(L, T, F, n, dtype, g)
+    n_dec = L if tying == "per_source" else L * (L + 1) // 2
+    w = engine.alloc_packed(n_dec, F, d, dtype, dev)
+    w[:, :, :d] = torch.randn(n_dec, F, d, generator=g).to(dev, dtype)
+    bias = torch.randn(L, d, generator=g) if extra else None
+    skip = torch.randn(L, T, d, generator=g) if extra else None
+    got, again = (_decode(keep, act, row_ptr, w, tying, d, bias, skip, out_f32=out_f32) for _ in range(2))
+    assert torch.equal(got, again)
+    wc, x = w[:, :, :d].double(), act.double().to(dev)
+    for t in range(L):
+        zero = torch.zeros(T, d, dtype=torch.float64, device=dev)
+        ref, mag, n_t = zero, zero, 0
+        if extra:                                           # two summands: they may cancel
+            ref = bias[t].double().to(dev) + skip[t].double().to(dev)
+            mag = bias[t].double().abs().to(dev) + skip[t].double().abs().to(dev)
+        for s in range(t + 1):
+            m = wc[_slot(tying, s, t, L)]
+            ref, mag, n_t = ref + x[s] @ m, mag + x[s].abs() @ m.abs(), n_t + keep[s].sum(1, keepdim=True).to(dev)
+        tol = (n_t + 8.0) * 2.0 ** -24 * mag                # as above
+        if not out_f32 and dtype == torch.bfloat16:
+            tol = tol + (ref.abs() + tol) * 2.0 ** -8
+        assert bool(((got[t].double().to(dev) - ref).abs() <= tol).all()), t
+
+
+def test_decode_thin_of_a_long_list_keeps_values_that_are_not_finite():
+    dev = torch.device("cuda:0")
+    L, T, F, d = 1, 18, 8300, 512
+    g = torch.Generator().manual_seed(2)
+    n = torch.full((L, T), 3)
+    n[0, 4], n[0, 5] = 8195, 8197                          # no whole number of eights, nor of 64s
+    keep, act, row_ptr = _lists(L, T, F, n, torch.bfloat16, g)
+    w = engine.alloc_packed(1, F, d, torch.bfloat16, dev)
+    w[:, :, :d] = torch.randn(1, F, d, generator=g).to(dev, torch.bfloat16)
+    bad = int((keep[0, 4] & ~keep[0, 5]).nonzero()[0])
+    w[0, bad, 5], w[0, 0, 7] = float("inf"), float("nan")   # row 0 is what the places past the end refer to
+    keep[0, :, 0] = False
+    act[0, :, 0] = 0
+    row_ptr[1:] = torch.cumsum(keep.view(T, F).sum(1), 0)
+    got = _decode(keep, act, row_ptr, w, "none", d, out_f32=True)
+    hit = keep[0, :, bad]
+    assert bool(hit[4]) and not bool(hit[5])
+    assert bool(torch.isinf(got[0, hit, 5]).all()) and bool(torch.isfinite(got[0, ~hit]).all())
+    assert bool(torch.isfinite(got[0][:, [i for i in range(d) if i != 5]]).all())
