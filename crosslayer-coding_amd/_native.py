@@ -73,6 +73,8 @@ _SIGNATURES = {
                                 _vp, _sz, _vp]),
     "clt_decode_thin_wanted": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _int, _int]),
     "clt_decode_thin": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int, _vp]),
+    "clt_decode_thin_up_to": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int, _i64,
+                                     _vp]),
     "clt_decode_sparse_if_over": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64, _i64, _u64, _int, _int,
                                          _i64, _vp]),
     "clt_decode_route": (_int, [_i64, _i64, _i64, _i64, _int, _int, _sz]),

@@ -815,8 +815,9 @@ template <typename T>
 __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin_longest(
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
     const float *__restrict__ bias_sum, const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d,
-    int64_t F, int64_t L, int tying, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch, int units) {
+    int64_t F, int64_t L, int tying, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch, int units, int64_t max_entries) {
   constexpr int V = WVec<T>::V, COLS = 8 * V, NU = 4;     // 8 lanes per line, 8 rows per load
+  if (max_entries >= 0 && row_ptr[L * Tn] > max_entries) return;
   __shared__ int32_t found[THIN_WAVES * 64], n_found[THIN_WAVES];
   __shared__ float shares[THIN_WAVES][COLS];
   const int tid = threadIdx.x, lane = lane_id(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -902,8 +903,9 @@ template <typename T, int HQ, int HTAIL>
 __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin(
     const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ wp,
     const float *__restrict__ bias_sum, const float *__restrict__ skip_add, void *__restrict__ out, int64_t Tn, int64_t d,
-    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch) {
+    int64_t F, int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int out_f32, int64_t pitch, int64_t max_entries) {
   constexpr int V = WVec<T>::V, UU = 2, R = QROWS * UU;
+  if (max_entries >= 0 && row_ptr[L * Tn] > max_entries) return;
   constexpr int NACC = HQ * V + (HTAIL ? V / 2 : 0);      // columns per lane: d / 64
   __shared__ int32_t totals[THIN_WAVES];
   __shared__ float shares[THIN_WAVES][NACC][QLANES];
@@ -1868,14 +1870,14 @@ static int launch_decode(const int32_t *row_ptr, const int32_t *col, const void 
 template <typename T>
 static int launch_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *wp, const float *bias_sum,
                               const float *skip_add, void *out, int64_t Tn, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
-                              int64_t t_end, uint64_t src_mask, int out_f32, hipStream_t stream) {
+                              int64_t t_end, uint64_t src_mask, int out_f32, int64_t max_entries, hipStream_t stream) {
   constexpr int V = WVec<T>::V;
   const int64_t blocks = 8 * clt_ceil_div((Tn + 1) / 2, THIN_WAVES) * (t_end - t_begin);
   if (blocks > 2147483647LL) return CLT_ERR_RANGE;
   const int hq = (int)(d / 64) / V, htail = ((int)(d / 64) % V) != 0;
 #define CLT_THIN(HQN, HTN)                                                                                            \
   k_decode_thin<T, HQN, HTN><<<(unsigned)blocks, THIN_WAVES * 64, 0, stream>>>(row_ptr, col, (const T *)val, (const T *)wp, bias_sum, \
-      skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)))
+      skip_add, out, Tn, d, F, L, tying, t_begin, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)), max_entries)
   if constexpr (sizeof(T) == 2) {
     if (hq == 1 && !htail) CLT_THIN(1, 0);
     else if (hq == 1) CLT_THIN(1, 1);
@@ -1889,7 +1891,7 @@ static int launch_decode_thin(const int32_t *row_ptr, const int32_t *col, const 
 #undef CLT_THIN
   const int units = (int)(d / (8 * V));
   k_decode_thin_longest<T><<<(unsigned)(THIN_PARTS * units * (t_end - t_begin)), THIN_WAVES * 64, 0, stream>>>(row_ptr, col, (const T *)val,
-      (const T *)wp, bias_sum, skip_add, out, Tn, d, F, L, tying, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)), units);
+      (const T *)wp, bias_sum, skip_add, out, Tn, d, F, L, tying, t_end, src_mask, out_f32, clt_pitch(d, (int)sizeof(T)), units, max_entries);
   return clt_check_launch();
 }
 
@@ -1931,10 +1933,10 @@ extern "C" int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L
          thin < clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);
 }
 
-extern "C" int clt_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
-                               const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
-                               int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
-                               void *stream) {
+// max_entries < 0: whatever the lists hold
+static int decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed, const float *bias_sum,
+                       const float *skip_add, void *out, int64_t T, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
+                       int64_t t_end, uint64_t src_mask, int dtype, int out_f32, int64_t max_entries, void *stream) {
   if (!clt_model_dtype(dtype)) return CLT_ERR_DTYPE;
   if (T < 0 || t_begin < 0 || t_end > L || t_begin > t_end) return CLT_ERR_ARG;
   if (T == 0 || t_begin == t_end) return CLT_OK;
@@ -1944,10 +1946,25 @@ extern "C" int clt_decode_thin(const int32_t *row_ptr, const int32_t *col, const
     return CLT_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == CLT_BF16)
-    return launch_decode_thin<bf16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
+    return launch_decode_thin<bf16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, max_entries, s);
   if (dtype == CLT_F16)
-    return launch_decode_thin<f16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
-  return launch_decode_thin<float>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, s);
+    return launch_decode_thin<f16_t>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, max_entries, s);
+  return launch_decode_thin<float>(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, out_f32, max_entries, s);
+}
+
+extern "C" int clt_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                               const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                               int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
+                               void *stream) {
+  return decode_thin(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, dtype, out_f32, -1, stream);
+}
+
+extern "C" int clt_decode_thin_up_to(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed,
+                                     const float *bias_sum, const float *skip_add, void *out, int64_t T, int64_t d, int64_t F,
+                                     int64_t L, int tying, int64_t t_begin, int64_t t_end, uint64_t src_mask, int dtype, int out_f32,
+                                     int64_t max_entries, void *stream) {
+  if (max_entries < 0) return CLT_ERR_ARG;
+  return decode_thin(row_ptr, col, val, w_packed, bias_sum, skip_add, out, T, d, F, L, tying, t_begin, t_end, src_mask, dtype, out_f32, max_entries, stream);
 }
 
 extern "C" size_t clt_decode_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L) {

@@ -973,12 +973,17 @@ def decode_sparse(surv: SurvivorList, w_packed: torch.Tensor, tying: str, d: int
         if total is None:
             total = L * T * F // 100
         wide = surv.dtype == torch.float32
-        if sliced and surv.selected and total and lib.clt_decode_thin_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying],
-                                                                             nat.dtype_code(surv.dtype)):
-            code = lib.clt_decode_thin(nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum),
-                                       nat.ptr(skip_add), nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin, t_end,
-                                       src_mask & ((1 << 64) - 1), nat.dtype_code(surv.dtype), 1 if out_f32 else 0, _stream(w_packed))
-            nat.check(code, "clt_decode_thin")
+        if (sliced and surv.selected and total and (exact or not wide)
+                and lib.clt_decode_thin_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype))):
+            args = (nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w_packed), nat.ptr(bias_sum), nat.ptr(skip_add),
+                    nat.ptr(out), T, d, F, L, nat.TYING[tying], t_begin, t_end, src_mask & ((1 << 64) - 1),
+                    nat.dtype_code(surv.dtype), 1 if out_f32 else 0)
+            if exact:
+                nat.check(lib.clt_decode_thin(*args, _stream(w_packed)), "clt_decode_thin")
+            else:              # as with the tiles below: a batch that outgrew the estimate by a quarter is the gather's
+                cap = total + total // 4 + 4096
+                nat.check(lib.clt_decode_thin_up_to(*args, cap, _stream(w_packed)), "clt_decode_thin_up_to")
+                nat.check(lib.clt_decode_sparse_if_over(*args, cap, _stream(w_packed)), "clt_decode_sparse_if_over")
             return out
         if total and not wide and lib.clt_decode_tiles_wanted(T, d, F, L, t_end - t_begin, total, nat.TYING[tying], nat.dtype_code(surv.dtype)):
             # room for twice that many, or what the records can count where that is less

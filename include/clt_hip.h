@@ -417,15 +417,20 @@ int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, const void *va
 
 /*
  * The same sums (untied and per-source decoders, no feature offset / scale, d a multiple of 256) for lists with few survivors per
- * (source, token): one launch over all sources, no workspace.
+ * (source, token): all sources at once, no workspace.
  *   clt_decode_thin_wanted: whether it is faster than clt_decode_sparse with a workspace for `entries` survivors over L
  *   layers and `targets` target layers (0 also for what it does not take).
+ *   clt_decode_thin_up_to: for lists whose length the caller only estimates: does nothing where they hold more than `max_entries`,
+ *   as decided on the device; clt_decode_sparse_if_over with the same number does those.
  * Deterministic, equal to clt_decode_sparse up to fp32 summation order.
  */
 int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
 int clt_decode_thin(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed, const float *bias_sum,
                     const float *skip_add, void *out, int64_t T, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
                     int64_t t_end, uint64_t src_mask, int dtype, int out_f32, void *stream);
+int clt_decode_thin_up_to(const int32_t *row_ptr, const int32_t *col, const void *val, const void *w_packed, const float *bias_sum,
+                          const float *skip_add, void *out, int64_t T, int64_t d, int64_t F, int64_t L, int tying, int64_t t_begin,
+                          int64_t t_end, uint64_t src_mask, int dtype, int out_f32, int64_t max_entries, void *stream);
 
 /*
  * The same sums (untied and per-source decoders, no feature offset / scale, fp32, d a multiple of 32) with the decoder rows

@@ -95,3 +95,41 @@ def test_a_buffer_that_a_captured_graph_writes_outlives_its_successor(monkeypatc
         assert sum(r() is not None for r in alive) == held
     ws.release()
     assert all(r() is None for r in alive)
+
+
+class _ThinRecorder(_Recorder):
+    def clt_decode_thin_wanted(self, *args):
+        return 1
+
+    def clt_decode_thin(self, *args):
+        self.calls.append(("thin", args))
+        return 0
+
+    def clt_decode_thin_up_to(self, *args):
+        self.calls.append(("thin_up_to", args))
+        return 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("hint", [None, 180000])
+@pytest.mark.parametrize("exact", [True, False])
+def test_an_estimated_total_is_checked_on_the_device(recorder, monkeypatch, dtype, hint, exact):
+    """The gather for thin lists takes a list whose length is known; one whose length is estimated only where another
+    decode stands by for what the estimate left out."""
+    rec = _ThinRecorder(recorder._lib)
+    monkeypatch.setattr(nat, "load", lambda *a, **k: rec)
+    L, T, d, F, meta = 12, 3000, 768, 24576, torch.device("meta")
+    cap = 600000 if exact else engine.max_list_entries(L, T, F)
+    surv = engine.SurvivorList(torch.empty(L * T + 1, dtype=torch.int32, device=meta), torch.empty(cap, dtype=torch.int32, device=meta),
+                               torch.empty(cap, dtype=dtype, device=meta), T, F, L, dtype,
+                               None if exact else torch.empty(1, dtype=torch.int32, device=meta), hint, True)
+    w = torch.empty((L * (L + 1) // 2, F, engine.decoder_pitch(d, dtype)), dtype=dtype, device=meta)
+    engine.decode_sparse(surv, w, "none", d, ws=engine.Workspace(meta))
+    names = [name for name, _ in rec.calls]
+    if exact:
+        assert names == ["thin"]
+    elif dtype == torch.float32:
+        assert names == ["gather"]
+    else:
+        assert names == ["thin_up_to", "if_over"]
+        assert rec.calls[0][1][17] == rec.calls[1][1][17] >= (hint or L * T * F // 100)

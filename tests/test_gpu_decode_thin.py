@@ -201,3 +201,22 @@ def test_decode_thin_of_a_long_list_keeps_values_that_are_not_finite():
     assert bool(hit[4]) and not bool(hit[5])
     assert bool(torch.isinf(got[0, hit, 5]).all()) and bool(torch.isfinite(got[0, ~hit]).all())
     assert bool(torch.isfinite(got[0][:, [i for i in range(d) if i != 5]]).all())
+
+
+@pytest.mark.parametrize("hint", [20000, 400000])
+def test_a_threshold_list_that_outgrew_its_hint_is_decoded(monkeypatch, hint):
+    """The hint chooses the gather for thin lists; whether the list is one is decided on the device."""
+    dev, lib = torch.device("cuda:0"), nat.load()
+    L, T, F, d = 6, 1500, 4096, 768
+    g = torch.Generator().manual_seed(4)
+    pre = torch.randn(L, T, F, generator=g).to(dev, torch.bfloat16)
+    exact = engine.batchtopk_select(pre, 250, True)         # 375 000 entries
+    surv = engine.SurvivorList(exact.row_ptr, exact.col, exact.val, T, F, L, torch.bfloat16,
+                               torch.zeros(1, dtype=torch.int32, device=dev), hint, True)
+    w = engine.alloc_packed(L * (L + 1) // 2, F, d, torch.bfloat16, dev)
+    w[:, :, :d] = torch.randn(L * (L + 1) // 2, F, d, generator=g).to(dev, torch.bfloat16)
+    monkeypatch.setattr(lib, "clt_decode_thin_wanted", lambda *a: 1)
+    got = engine.decode_sparse(surv, w, "none", d, ws=engine.Workspace(dev), out_f32=True)
+    monkeypatch.setattr(lib, "clt_decode_thin_wanted", lambda *a: 0)
+    ref = engine.decode_sparse(exact, w, "none", d, ws=engine.Workspace(dev), out_f32=True)
+    assert float((got - ref).norm() / ref.norm()) < 1e-6    # fp32 sums in another order
