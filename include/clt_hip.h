@@ -416,8 +416,8 @@ int clt_decode_sparse(const int32_t *row_ptr, const int32_t *col, const void *va
                       void *stream);
 
 /*
- * The same sums (untied and per-source decoders, no feature offset / scale, d a multiple of 256) for lists with few survivors per
- * (source, token): all sources at once, no workspace.
+ * The same sums (untied and per-source decoders, no feature offset / scale; d 512, 768, 1024 or in 16 bits 2048, at most 2^31 - 1
+ * decoder rows) for lists with few survivors per (source, token): all sources at once, no workspace.
  *   clt_decode_thin_wanted: whether it is faster than clt_decode_sparse with a workspace for `entries` survivors over L
  *   layers and `targets` target layers (0 also for what it does not take).
  *   clt_decode_thin_up_to: for lists whose length the caller only estimates: does nothing where they hold more than `max_entries`,

@@ -133,3 +133,16 @@ def test_an_estimated_total_is_checked_on_the_device(recorder, monkeypatch, dtyp
     else:
         assert names == ["thin_up_to", "if_over"]
         assert rec.calls[0][1][17] == rec.calls[1][1][17] >= (hint or L * T * F // 100)
+
+
+@pytest.mark.parametrize("dtype,widths", [(torch.bfloat16, (512, 768, 1024, 2048)), (torch.float16, (512, 768, 1024, 2048)),
+                                          (torch.float32, (512, 768, 1024))])
+def test_widths_of_the_gather_for_thin_lists(dtype, widths):
+    """Others are refused by the decode and never wanted by its rule."""
+    lib, code = nat.load(), nat.dtype_code(dtype)
+    for d in (64, 128, 256, 512, 640, 768, 1000, 1024, 1280, 1536, 1792, 2048, 2304, 4096):
+        assert lib.clt_decode_thin_wanted(3000, d, 24576, 12, 12, 100000, 0, code) == (1 if d in widths else 0), d
+        # (widths that are taken get as far as the check of the addresses: CLT_ERR_ALIGN)
+        got = lib.clt_decode_thin(4096, 4096, 4096, 4100, None, None, 4096, 3000, d, 24576, 12, 0, 0, 12, 1, code, 0, None)
+        assert (got == -5) == (d in widths) and got < 0, (d, got)
+        assert lib.clt_decode_thin_up_to(4096, 4096, 4096, 4100, None, None, 4096, 3000, d, 24576, 12, 0, 0, 12, 1, code, 0, 5, None) == got
