@@ -134,8 +134,10 @@ __device__ __forceinline__ uint64_t same_class(uint64_t valid, uint64_t b0, uint
 // entries.  A place that stays empty refers to the half read's first row, which costs no bank of its own.
 // (L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, bf16: this kernel 213 -> 158 us against entries in the
 // order of the lists, row by row through a window of 128 batches, k_decode_tiles 3.33 -> 3.17 ms; L = 24, d = 1024, F = 32768:
-// 433 -> 266 us, 15.77 -> 15.59 ms.  Bound by the chain of a tile's steps in each wavefront.)
-constexpr int REC_WINDOW = 8;                              // batches a wavefront puts together at a time
+// 433 -> 266 us, 15.77 -> 15.59 ms.  Bound by the chain of a tile's steps in each wavefront.  Tiles with thousands of entries, L
+// = 2, 4096 tokens: 176 us where 16 tokens fire all of 512 neighbouring features, 440 in the gradients of 16 that always fire; with
+// all entries once per window 1614 and 4236.)
+constexpr int REC_WINDOW = 8;                              // batches a wavefront puts together in LDS
 template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(RecArgs A) {
   extern __shared__ int32_t fill_lds[];
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63, wave = tid >> 6;
@@ -204,10 +206,8 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
       }
       first -= mine;
     }
-    for (int32_t w0 = 0; w0 < nb; w0 += REC_WINDOW) {
-      const int32_t wn = nb - w0 < REC_WINDOW ? nb - w0 : REC_WINDOW;
-      for (int32_t b = 0; b < wn; ++b) win[b * SP_REC_WORDS + lane] = 0u;
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // all entries once more: those of batches w0 .. w0 + wn - 1 to their places in `batches`
+    auto fill = [&](uint32_t *batches, int32_t w0, int32_t wn) {
       uint32_t next = first;
       for (int32_t i0 = 0; i0 < n; i0 += 64) {
         int tk;
@@ -223,7 +223,7 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
         const int32_t b = (int32_t)(h >> 2) - w0;
         if (!on || b < 0 || b >= wn) continue;
         // half read h % 4 of batch h / 4: h & 1 the half of the wavefront, h & 2 the second four entries of its lane quartets
-        uint16_t *rec = (uint16_t *)(win + b * SP_REC_WORDS) + (h & 1u) * 64;
+        uint16_t *rec = (uint16_t *)(batches + b * SP_REC_WORDS) + (h & 1u) * 64;
         auto place = [&](uint32_t sl, uint16_t at) {
           rec[(sl >> 2) * 32 + (4 * (sl & 3u) + 3) * 2 + ((h >> 1) & 1u)] = at;
         };
@@ -235,9 +235,21 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
         if (slot == 0)                                     // the places of this half read that stay empty
           for (uint32_t sl = __umulhi((uint32_t)n - 1u - p, magic) + 1u; sl < 8u; ++sl) place(sl, at);
       }
+    };
+    uint32_t *const out = A.recs + (uint64_t)(base + dest[c]) * SP_REC_WORDS;
+    if (nb <= REC_WINDOW) {
+      for (int32_t b = 0; b < nb; ++b) win[b * SP_REC_WORDS + lane] = 0u;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      for (int32_t b = 0; b < wn; ++b) A.recs[(uint64_t)(base + dest[c] + (uint32_t)(w0 + b)) * SP_REC_WORDS + lane] = win[b * SP_REC_WORDS + lane];
+      fill(win, 0, nb);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int32_t b = 0; b < nb; ++b) out[b * SP_REC_WORDS + lane] = win[b * SP_REC_WORDS + lane];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+      // more than the window holds - up to 256, where 16 features fire on most tokens: put together where they are to lie, two
+      // bytes at a time, rather than all entries once per window
+      for (int32_t b = 0; b < nb; ++b) out[b * SP_REC_WORDS + lane] = 0u;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the zeros have arrived
+      fill(out, 0, nb);
     }
   }
 }

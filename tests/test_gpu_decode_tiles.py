@@ -310,3 +310,27 @@ def test_the_model_takes_the_tiles_when_they_are_priced_lower():
     assert want(64, 200) == 0 and want(4096, 2) == 0
     assert want(4096, 200, dtype=torch.float32) == 0 and want(4096, 200, tying="per_target") == 0
     assert cca is not None
+
+
+@pytest.mark.parametrize("entries", [256, 257, 288, 511, 2049, 8192])
+def test_decode_tiles_of_tiles_with_many_entries(entries):
+    """A tile of 16 tokens x 512 features with as many entries as are put together in LDS, one more, whole batches, all."""
+    dev = torch.device("cuda:0")
+    L, T, F, d = 1, 33, 1024, 64
+    g = torch.Generator().manual_seed(entries)
+    act = torch.randn(L, T, F, generator=g).bfloat16()
+    act[act == 0] = 1.0
+    keep = torch.rand(T, F, generator=g) < 0.02
+    tile = torch.zeros(16 * 512, dtype=torch.bool)
+    tile[torch.randperm(16 * 512, generator=g)[:entries]] = True
+    keep[16:32, 512:] = tile.view(16, 512)
+    act[0][~keep] = 0
+    row_ptr = torch.zeros(T + 1, dtype=torch.int32)
+    row_ptr[1:] = torch.cumsum(keep.sum(1), 0)
+    col, val = keep.nonzero()[:, 1].int(), act[0][keep]
+    w = (torch.rand(1, F, d, generator=g) - 0.5).bfloat16()
+    got = [_run(dev, act, row_ptr, col, val, w, "none", d, None, None, 0, 1, 1, True, col.numel(), False) for _ in range(2)]
+    assert torch.equal(got[0], got[1])
+    ref, mag = act[0].double() @ w[0].double(), act[0].double().abs() @ w[0].double().abs()
+    # exact products; each addition is off by at most 2^-23 of what has been summed
+    assert (got[0][0].double() - ref).abs().le((keep.sum(1, keepdim=True).double() + 2) * 2.0 ** -23 * mag).all()
