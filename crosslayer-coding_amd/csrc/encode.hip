@@ -17,7 +17,7 @@
 //   epilogue    rounding, then the tile goes through LDS so that the stores are 16 bytes per lane
 //               and 256 contiguous bytes per token
 //   bf16        v_mfma_f32_16x16x32_bf16, fp32 accumulate, one rounding (v_cvt_pk_bf16_f32)
-//   fp32        v_mfma_f32_32x32x2_f32
+//   fp32        v_mfma_f32_16x16x4_f32
 #include <type_traits>
 #include "select_state.h"
 
@@ -67,31 +67,26 @@ template <> __device__ __forceinline__ float slot_elem<float>(const uint4 &w, in
   return __uint_as_float(j == 0 ? w.x : j == 1 ? w.y : j == 2 ? w.z : w.w);
 }
 
-// What the 256 x 256 tiles are made of: products of SIDE x SIDE, `part` of PARTS of a pair of fragments.
-// 16 bits: 16 x 16, 64 bytes of K per row.  Under full load the part is held by its power limit, and this shape moves its
-// accumulators half as often per product: a loop of nothing but matrix instructions on random bf16 operands runs at 2065
-// TFLOP/s with it and at 1795 with 32 x 32 x 16.  float32: 32 x 32, one instruction per element of the fragments (16 x
-// 16 x 4 takes as long, L 3, T 1024, d 768, F 6144 386 against 385 us, and sums over K in another order).
-template <typename T> struct TileMma;
-template <> struct TileMma<bf16_t> {
-  static constexpr int SIDE = 16, PARTS = 1;
-  typedef f32x4_t acc_t;
-  __device__ static __forceinline__ void run(acc_t &acc, const uint4 &a, const uint4 &b, int) {
+// The same on 16 x 16 tiles, 64 bytes of K per row: what the 256 x 256 tiles are made of.  Under full load the part is held by
+// its power limit, and this shape moves its accumulators half as often per product: a loop of nothing but matrix
+// instructions on random bf16 operands runs at 2065 TFLOP/s with it and at 1795 with 32 x 32 x 16.
+template <typename T> struct Mma16;
+template <> struct Mma16<bf16_t> {
+  static constexpr int PARTS = 1;
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int) {
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
   }
 };
-template <> struct TileMma<f16_t> {
-  static constexpr int SIDE = 16, PARTS = 1;
-  typedef f32x4_t acc_t;
-  __device__ static __forceinline__ void run(acc_t &acc, const uint4 &a, const uint4 &b, int) {
+template <> struct Mma16<f16_t> {
+  static constexpr int PARTS = 1;
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int) {
     acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), acc, 0, 0, 0);
   }
 };
-template <> struct TileMma<float> {
-  static constexpr int SIDE = 32, PARTS = 4;
-  typedef f32x16_t acc_t;
-  __device__ static __forceinline__ void run(acc_t &acc, const uint4 &a, const uint4 &b, int part) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(slot_elem<float>(a, part), slot_elem<float>(b, part), acc, 0, 0, 0);
+template <> struct Mma16<float> {
+  static constexpr int PARTS = 4;        // one instruction per element of the fragments
+  __device__ static __forceinline__ void run(f32x4_t &acc, const uint4 &a, const uint4 &b, int part) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(slot_elem<float>(a, part), slot_elem<float>(b, part), acc, 0, 0, 0);
   }
 };
 
@@ -210,8 +205,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   // (one stage to arrive) and a wait for the epilogue's stores at the turn, ms, bf16:
   //   L 12, T 4096, d 768, F 24576   1.84 -> 1.66 (1117 TFLOP/s)      L 4, T 8192, d 2048, F 16384   1.82 -> 1.65 (1330)
   //   T 8192, d 16384, F 2048        0.453 -> 0.388 (1420)            T = d = F = 8192               0.852 -> 0.768 (1430)
-  // The vendor library takes 0.377 and 0.67 ms for the d 16384 and the 8192 product.  float32 (L 3, T 1024, d 768, F 6144):
-  // 0.388 and 0.385 ms.  Measured and dropped: the two wavefronts of a SIMD taking turns at multiplying and reading (1.95
+  // The vendor library takes 0.377 and 0.67 ms for the d 16384 and the 8192 product.  float32 (L 12, T 1024, d 768, F 6144):
+  // 0.915 ms both.  Measured and dropped: the two wavefronts of a SIMD taking turns at multiplying and reading (1.95
   // ms at the first shape: with 64 KB per stage also coming into LDS, the reads of a turn outlast the other's products).
   __shared__ __attribute__((aligned(16))) unsigned char stage0[STAGE];
   __shared__ __attribute__((aligned(16))) unsigned char stage1[STAGE];
@@ -321,25 +316,21 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
                 lds_address(stage) + (BM + (wave >> 2) * 128 + (i - 4) * 32 + (wave & 3) * 8) * ROWB);
   };
 
-  // ---- fragment reader: row ln of each group of SIDE rows; chunk (ks*NQ + lq) at its swizzled position
-  typedef TileMma<T> MM;
-  constexpr int SIDE = MM::SIDE, NQ = 64 / SIDE;        // lanes that share a row, each with 16 bytes of it
-  constexpr int XG = 64 / SIDE, WG = 32 / SIDE, KS = 8 / NQ;   // groups of tokens; of features in a quarter; k-steps of a stage
-  const int ln = lane & (SIDE - 1), lq = lane / SIDE;
-  const int xrow = (wm * 64 + ln) * ROWB;               // + i * SIDE * ROWB
-  const int wrow = BM * ROWB + (wn * 128 + ln) * ROWB;  // + j * SIDE * ROWB
-  int koff[KS];
+  // ---- fragment reader: row l15 of each 16-row group; chunk (ks*4 + lq) at its swizzled position
+  const int l15 = lane & 15, lq = lane >> 4;
+  const int xrow = (wm * 64 + l15) * ROWB;              // + i * 16 * ROWB
+  const int wrow = BM * ROWB + (wn * 128 + l15) * ROWB; // + j * 16 * ROWB
+  int koff[2];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) koff[ks] = ((ks * NQ + lq) ^ ((ln >> 1) & 7)) << 4;
+  for (int ks = 0; ks < 2; ++ks) koff[ks] = ((ks * 4 + lq) ^ ((l15 >> 1) & 7)) << 4;
 
   // The accumulators start from the bias (the matrix core adds its products onto them in fp32), so
-  // the epilogue has no bias loads or adds: accumulator (j, rg*4+q) of a lane belongs to feature
-  // j*SIDE + rg*8 + lq*4 + q of the wave tile, whatever the token group i.  Each wavefront brings
+  // the epilogue has no bias loads or adds: accumulator (j, q) of a lane belongs to feature
+  // j*16 + (lane>>4)*4 + q of the wave tile, whatever the token group i.  Each wavefront brings
   // the bias of its 128 features into LDS with one direct load ahead of the tile's stages - no register
   // holds it while the previous tile's epilogue runs - and reads it from there when the first stage has
   // landed.
-  constexpr int NRG = SIDE * SIDE / 256;                  // quads of an accumulator: 1 or 4
-  typename MM::acc_t acc[XG][4 * WG];
+  f32x4_t acc[4][8];
   constexpr int BIAS_LANES = 128 * (int)sizeof(T) / 16;   // lanes of the one 16-byte-per-lane load
   auto load_bias = [&](const TileAt &t, int slot) {
     if (bias && lane < BIAS_LANES) fill16(bias + (int64_t)t.layer * bs + t.n0 + wn * 128, lane * 16, lds_address(bias_lds[wave]));
@@ -354,29 +345,29 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   };
   if (!bias && lane < BIAS_LANES)   // no bias: the slot holds zeros for good
     *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned char *>(bias_lds[wave]) + lane * 16) = make_uint4(0u, 0u, 0u, 0u);
-  // The bias is read with hand-written LDS loads and a hand-placed wait.
-  const uint32_t bias_at = lds_address(bias_lds[wave]) + (uint32_t)lq * 4u * (uint32_t)sizeof(T);
+  // The bias is read with hand-written LDS loads and a hand-placed wait: the compiler, which cannot tell how
+  // many of the outstanding direct loads are older than the one into the bias slot, would otherwise wait for
+  // all of them (the stage just asked for included) before the first read.
+  const uint32_t bias_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)
+                               reinterpret_cast<unsigned char *>(bias_lds[wave]) + (uint32_t)(lane >> 4) * 4u * (uint32_t)sizeof(T);
   auto init_acc = [&]() {
     typedef typename std::conditional<sizeof(T) == 4, uint4, uint2>::type braw_t;
-    braw_t raw[4 * WG * NRG];
-    // raw[j * NRG + rg] = the 4 values at feature j * SIDE + rg * 8 + lq * 4.  Eight reads and their wait are one statement, so
-    // no register is looked at before its value has arrived.
+    braw_t raw[8];
+    // raw[j] = the 4 values at feature j * 16 of this lane's quarter.  All eight reads and their
+    // wait are one statement, so no register is looked at before its value has arrived.
     if constexpr (sizeof(T) == 4) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
         asm volatile(
                      "ds_read_b128 %0, %8\n\t"
-                     "ds_read_b128 %1, %8 offset:32\n\t"
-                     "ds_read_b128 %2, %8 offset:64\n\t"
-                     "ds_read_b128 %3, %8 offset:96\n\t"
-                     "ds_read_b128 %4, %8 offset:128\n\t"
-                     "ds_read_b128 %5, %8 offset:160\n\t"
-                     "ds_read_b128 %6, %8 offset:192\n\t"
-                     "ds_read_b128 %7, %8 offset:224\n\t"
+                     "ds_read_b128 %1, %8 offset:64\n\t"
+                     "ds_read_b128 %2, %8 offset:128\n\t"
+                     "ds_read_b128 %3, %8 offset:192\n\t"
+                     "ds_read_b128 %4, %8 offset:256\n\t"
+                     "ds_read_b128 %5, %8 offset:320\n\t"
+                     "ds_read_b128 %6, %8 offset:384\n\t"
+                     "ds_read_b128 %7, %8 offset:448\n\t"
                      "s_waitcnt lgkmcnt(0)"
-                     : "=&v"(raw[8 * h]), "=&v"(raw[8 * h + 1]), "=&v"(raw[8 * h + 2]), "=&v"(raw[8 * h + 3]), "=&v"(raw[8 * h + 4]),
-                       "=&v"(raw[8 * h + 5]), "=&v"(raw[8 * h + 6]), "=&v"(raw[8 * h + 7])
-                     : "v"(bias_at + 256u * h));
+                     : "=&v"(raw[0]), "=&v"(raw[1]), "=&v"(raw[2]), "=&v"(raw[3]), "=&v"(raw[4]), "=&v"(raw[5]), "=&v"(raw[6]), "=&v"(raw[7])
+                     : "v"(bias_at));
     } else {
         asm volatile(
                      "ds_read_b64 %0, %8\n\t"
@@ -393,7 +384,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 4 * WG * NRG; ++j) {
+    for (int j = 0; j < 8; ++j) {
       float bv[4];
       if constexpr (sizeof(T) == 4) {
         bv[0] = __uint_as_float(raw[j].x); bv[1] = __uint_as_float(raw[j].y); bv[2] = __uint_as_float(raw[j].z); bv[3] = __uint_as_float(raw[j].w);
@@ -402,13 +393,11 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
         unpack_pair<T>(raw[j].y, bv[2], bv[3]);
       }
 #pragma unroll
-      for (int i = 0; i < XG; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[i][j / NRG][j % NRG * 4 + q] = bv[q];
+      for (int i = 0; i < 4; ++i) acc[i][j] = f32x4_t{bv[0], bv[1], bv[2], bv[3]};
     }
   };
 
-  // Software pipeline over the K stages.  A stage is four quarters: quarter q multiplies all of the
+  // Software pipeline over the K stages.  A stage is four quarters of 16 matrix operations: quarter q multiplies all of the
   // wavefront's tokens with 32 of its features (rows 32 q of the W half tile), over the stage's whole K.  The x fragments
   // stay in registers for the stage, each being replaced by the next stage's behind its last use; the W fragments of the next
   // quarter are read under this one's products.
@@ -416,14 +405,10 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   // read by everybody, so six of the loads of the stage after next can be asked for, at the second the rest; and of the
   // stage's own loads, what the next two quarters read has landed: all of it but the last eight loads, so that a load has
   // a stage and a half to arrive.
-  // float32, whose products take eight times as long, has the second barrier alone and asks for all loads there: they have most of
-  // a stage to arrive, and every barrier costs the two wavefronts of a SIMD a 64-cycle product (T 1000, L 2, d 1024, F
-  // 4096: 267 us with two, 254 with one).
-  constexpr bool TWO = sizeof(T) == 2;
-  uint4 fx[XG][KS], fw[2][WG][KS];       // [token group][k-step], [buffer][feature group][k-step]
-  auto read_x = [&](const unsigned char *st, int i, int ks) { fx[i][ks] = *reinterpret_cast<const uint4 *>(st + xrow + i * SIDE * ROWB + koff[ks]); };
+  uint4 fx[4][2], fw[2][2][2];           // [token group][k-step], [buffer][feature group][k-step]
+  auto read_x = [&](const unsigned char *st, int i, int ks) { fx[i][ks] = *reinterpret_cast<const uint4 *>(st + xrow + i * 16 * ROWB + koff[ks]); };
   auto read_w = [&](const unsigned char *st, int q, int j, int ks) {
-    fw[q & 1][j][ks] = *reinterpret_cast<const uint4 *>(st + wrow + (q * WG + j) * SIDE * ROWB + koff[ks]);
+    fw[q & 1][j][ks] = *reinterpret_cast<const uint4 *>(st + wrow + (q * 2 + j) * 16 * ROWB + koff[ks]);
   };
   auto meet = [&]() {
     asm volatile("" ::: "memory");
@@ -439,35 +424,34 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   auto body = [&](unsigned char *st, unsigned char *next, bool last, bool fresh, auto first, auto rest, uint32_t m) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      if ((TWO && q == 1) || q == 3) {
+      if (q == 1 || q == 3) {
         if (q == 3 && last) __builtin_amdgcn_s_waitcnt(0xC07F);    // lgkmcnt(0)
         else if (q == 1 && fresh) __builtin_amdgcn_s_waitcnt(0xC07F);
-        else __builtin_amdgcn_s_waitcnt(TWO ? 0x0078 : 0x0070);   // vmcnt(8) / vmcnt(0), lgkmcnt(0)
+        else __builtin_amdgcn_s_waitcnt(0x0078);                  // vmcnt(8) lgkmcnt(0)
         meet();
       }
 #pragma unroll
       for (int g = 0; g < 8; ++g) {
-        const int ks = g / XG, i = g % XG;
+        const int ks = g >> 2, i = g & 3;
 #pragma unroll
-        for (int part = 0; part < MM::PARTS; ++part)
+        for (int part = 0; part < Mma16<T>::PARTS; ++part)
 #pragma unroll
-          for (int j = 0; j < WG; ++j) {
+          for (int j = 0; j < 2; ++j) {
             uint4 xv = fx[i][ks], wv = fw[q & 1][j][ks];
             if constexpr (ODD) {
               xv.x &= m; xv.y &= m; xv.z &= m; xv.w &= m;
               wv.x &= m; wv.y &= m; wv.z &= m; wv.w &= m;
             }
-            MM::run(acc[i][q * WG + j], wv, xv, part);
+            Mma16<T>::run(acc[i][q * 2 + j], wv, xv, part);
           }
-        if (q < 3 && g < 4) read_w(st, q + 1, g % WG, g / WG);
+        if (q < 3 && g < 4) read_w(st, q + 1, g & 1, g >> 1);
         if (q == 3 && !last) {
-          if (g < 4) read_w(next, 0, g % WG, g / WG);
+          if (g < 4) read_w(next, 0, g & 1, g >> 1);
           read_x(next, i, ks);
         }
         if (q == 0 && g == 1) rest(1);
-        if (TWO && (q == 1 || q == 2) && g < 6 && (g & 1) == 0) first((q - 1) * 3 + g / 2);
-        if (!TWO && q == 3 && g < 6) first(g);
-        if (q == 3 && g == (TWO ? 1 : 6)) rest(0);
+        if ((q == 1 || q == 2) && g < 6 && (g & 1) == 0) first((q - 1) * 3 + g / 2);
+        if (q == 3 && g == 1) rest(0);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -501,13 +485,13 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     init_acc();
 #pragma unroll
-    for (int j = 0; j < WG; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) read_w(stage0, 0, j, ks);
+      for (int ks = 0; ks < 2; ++ks) read_w(stage0, 0, j, ks);
 #pragma unroll
-    for (int i = 0; i < XG; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) read_x(stage0, i, ks);
+      for (int ks = 0; ks < 2; ++ks) read_x(stage0, i, ks);
     int kt = 0;                           // nk is even
     for (; kt < nk - 2; kt += 2) {
       const int k1 = stage_k0(cur, kt + 1), k2 = stage_k0(cur, kt + 2), k3 = stage_k0(cur, kt + 3);
@@ -516,15 +500,13 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
       body(stage1, stage0, false, false, [&](int i) { issue(stage1, xt, wt, k3, i); },
            [&](int i) { if (i == 0) issue(stage1, xt, wt, k3, 6); else issue(stage0, xt, wt, k2, 7); }, ~0u);
     }
-    // the last two stages: the first buffer takes the next tile's first stage (at the end, one that nobody reads, or none for
-    // float32, which has asked for it too late to have it by the epilogue); nothing may be on its way into the second
-    // one, which is parked in
+    // the last two stages: the first buffer takes the next tile's first stage (at the end, one that nobody reads);
+    // nothing may be on its way into the second one, which is parked in
     const int k1 = stage_k0(cur, kt + 1), k0 = stage_k0(nxt_tile, 0);
-    auto issue_next = [&](int i) { if (TWO || has_next) issue(stage0, xn, wn_, k0, i); };
-    body(stage0, stage1, false, kt == 0, [&](int i) { issue_next(i); },
-         [&](int i) { if (i == 0) issue_next(6); else if (kt > 0) issue(stage1, xt, wt, k1, 7); }, ~0u);
+    body(stage0, stage1, false, kt == 0, [&](int i) { issue(stage0, xn, wn_, k0, i); },
+         [&](int i) { if (i == 0) issue(stage0, xn, wn_, k0, 6); else if (kt > 0) issue(stage1, xt, wt, k1, 7); }, ~0u);
     body(stage1, stage0, true, false, [&](int i) { if (i == 0) load_bias(nxt_tile, slot ^ 1); },
-         [&](int i) { if (i == 1) issue_next(7); }, odd ? 0u : ~0u);
+         [&](int i) { if (i == 1) issue(stage0, xn, wn_, k0, 7); }, odd ? 0u : ~0u);
     // past the barrier of the last stage no wavefront reads either buffer any more
 
     // ---- epilogue.  The accumulator layout gives a lane 4 consecutive features of one token,
@@ -538,23 +520,21 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
     // invariants they would be computed once ahead of the tile loop and live across the K loop.
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    const int l31 = lane_e & 31, lh = lane_e >> 5, lne = lane_e & (SIDE - 1), lqe = lane_e / SIDE;
+    const int l31 = lane_e & 31, lh = lane_e >> 5, l15e = lane_e & 15, lqe = lane_e >> 4;
     unsigned char *park = stage1 + wave * (STAGE / 8);
     constexpr int NPASS = sizeof(T) == 2 ? 1 : 2;           // feature halves per pass
-    constexpr int JP = 4 * WG / NPASS;                       // groups of SIDE features per pass
+    constexpr int JP = 8 / NPASS;                            // 16-feature groups per pass
     // the 32 tokens h of feature pass `pass` -> rows of 256 bytes (128 bf16 / 64 fp32), 16-byte slots XOR-swizzled with
     // the row
     auto park_rows = [&](int pass, int h) {
 #pragma unroll
-      for (int jr = 0; jr < JP * NRG; ++jr) {
-        const int j = pass * JP + jr / NRG, rg = jr % NRG;
-        const int nl = jr / NRG * SIDE + rg * 8 + lqe * 4;   // feature inside this pass
+      for (int jj = 0; jj < JP; ++jj) {
+        const int j = pass * JP + jj;
+        const int nl = jj * 16 + lqe * 4;                    // feature inside this pass
 #pragma unroll
-        for (int ii = 0; ii < WG; ++ii) {
-          const int ml = ii * SIDE + lne;                    // row inside the parked piece
-          float y[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) y[q] = acc[h * WG + ii][j][rg * 4 + q];
+        for (int ii = 0; ii < 2; ++ii) {
+          const int ml = ii * 16 + l15e;                     // row inside the parked piece
+          const f32x4_t y = acc[h * 2 + ii][j];
           if (sizeof(T) == 4) {
             const int slot = (nl >> 2) ^ (ml & 15);
             *reinterpret_cast<float4 *>(park + ml * 256 + slot * 16) = make_float4(y[0], y[1], y[2], y[3]);
