@@ -806,7 +806,7 @@ constexpr int THIN_WAVES = 4, THIN_LONG = 256, THIN_MOST = 8192, THIN_PARTS = 16
 
 // The longest lists: a workgroup for every target, 128-byte line of the rows and sixteenth of the tokens, in which it looks for
 // such lists and sums its columns of them.  A compute unit has some 64 lines on their way, and here an entry is one line, on
-// d / 64 (16 bits) as many units: 8 ns per entry.  Usually it finds none: 7 us.
+// d / 64 (16 bits) as many units: 8 ns per entry.  Usually it finds none: 4 to 8 us.
 // us of the decode, L = 6, T = 1500, F = 16384, d = 1024, bf16, 200 per token over all layers, tokens with 0 / 1 x 20 000 / 1 x
 // 98 304 / 4 x 50 000 of the 300 000 entries: 260 / 470 / 886 / 478; left to the tokens' own workgroups 256 / 525 / 1909 / 1007;
 // the schedule by sources 334 / 412 / 824 / 589.  (In the first workgroups of k_decode_thin's launch it would end with the others, but their
@@ -830,9 +830,17 @@ __global__ __launch_bounds__(THIN_WAVES * 64) void k_decode_thin_longest(
     const int64_t mine = tok0 + tid;
     int32_t n = 0;
     if (mine < end) {
-      const int32_t *p = row_ptr + mine;
-#pragma unroll 4
-      for (int s = 0; s <= (int)t; ++s, p += Tn) n += (src_mask >> s) & 1ull ? p[1] - p[0] : 0;
+      for (int s0 = 0; s0 <= (int)t; s0 += 8) {            // eight sources asked for at once
+        int32_t a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int32_t *p = row_ptr + (s0 + u <= (int)t ? s0 + u : 0) * Tn + mine;
+          a[u] = p[0]; b[u] = p[1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (s0 + u <= (int)t && ((src_mask >> (s0 + u)) & 1ull)) n += b[u] - a[u];
+      }
     }
     const uint64_t votes = __ballot(n > THIN_MOST);
     if (lane == 0) n_found[wv] = __popcll(votes);
