@@ -14,8 +14,10 @@ per-stage figures, and a CPU baseline (the reference's dense algorithm, restated
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -56,21 +58,34 @@ def algorithmic_work(wl, nnz_rows_pairs: int, nnz_total: int):
 def profiled_traffic(workload: str):
     """({kernel name: (dispatches, HBM bytes per launch)}, forwards profiled) from the counter summary kept
     under profiles/ for this workload: FETCH_SIZE and WRITE_SIZE of `rocprofv3 --pmc`, each scaled by what
-    the same counter reads for the known-size copy of ``--copy-probe``.  ({}, 0) when there is no such file:
-    the traffic figures are then left out rather than guessed."""
+    the same counter reads for the known-size copy of ``--copy-probe``.  ({}, 0) when there is no such file or it is of
+    other kernels than these: the traffic figures are then left out rather than guessed."""
     path = os.path.join(ROOT, "profiles", f"forward_{workload}_hbm_traffic.txt")
-    table, forwards = {}, 0
+    table, forwards, digest = {}, 0, None
     try:
         for line in open(path):
             if line.startswith("forwards profiled:"):
                 forwards = int(line.split(":")[1])
+            elif line.startswith("kernel sources:"):
+                digest = line.split(":")[1].strip()
             elif line.startswith("k_"):
                 f = line.split()
                 name = " ".join(f[:-6])
                 table[name] = (int(f[-6]), float(f[-1]) * 1e6)
     except (OSError, ValueError, IndexError):
         return {}, 0
-    return table, forwards
+    return (table, forwards) if digest == kernel_sources_digest() else ({}, 0)
+
+
+def kernel_sources_digest() -> str:
+    """What tells the kernels of two builds apart: a digest of their sources without comments and white space."""
+    h = hashlib.sha1()
+    csrc = os.path.join(ROOT, "crosslayer-coding_amd", "csrc")
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".hip", ".h")):
+            text = re.sub(r"//[^\n]*|/\*.*?\*/", "", open(os.path.join(csrc, name)).read(), flags=re.S)
+            h.update((name + "".join(text.split())).encode())
+    return h.hexdigest()[:16]
 
 
 def gather_yardstick(lib, dev, table_bytes: int, row_bytes: int, steps: int = 5, reps: int = 4):
