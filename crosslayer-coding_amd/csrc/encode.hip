@@ -69,7 +69,7 @@ template <> __device__ __forceinline__ float slot_elem<float>(const uint4 &w, in
 
 // The same on 16 x 16 tiles, 64 bytes of K per row: what the 256 x 256 tiles are made of.  Under full load the part is held by
 // its power limit, and this shape moves its accumulators half as often per product: a loop of nothing but matrix
-// instructions on random bf16 operands runs at 2065 TFLOP/s with it and at 1795 with 32 x 32 x 16.
+// instructions on random bf16 operands runs at 2030 TFLOP/s with it and at 1806 with 32 x 32 x 16 (profiles/matrix_rates.txt).
 template <typename T> struct Mma16;
 template <> struct Mma16<bf16_t> {
   static constexpr int PARTS = 1;
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   //   L 12, T 4096, d 768, F 24576   1.84 -> 1.66 (1117 TFLOP/s)      L 4, T 8192, d 2048, F 16384   1.82 -> 1.65 (1330)
   //   T 8192, d 16384, F 2048        0.453 -> 0.388 (1420)            T = d = F = 8192               0.852 -> 0.768 (1430)
   // The vendor library takes 0.377 and 0.67 ms for the d 16384 and the 8192 product.  float32 (L 12, T 1024, d 768, F 6144):
-  // 0.915 ms both.  Measured and dropped: the two wavefronts of a SIMD taking turns at multiplying and reading (1.95
+  // 0.915 ms both (and with 32 x 32 x 2 products in this pipeline, one barrier a stage: which sums over K in another order).  Measured and dropped: the two wavefronts of a SIMD taking turns at multiplying and reading (1.95
   // ms at the first shape: with 64 KB per stage also coming into LDS, the reads of a turn outlast the other's products).
   __shared__ __attribute__((aligned(16))) unsigned char stage0[STAGE];
   __shared__ __attribute__((aligned(16))) unsigned char stage1[STAGE];
@@ -345,9 +345,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
   };
   if (!bias && lane < BIAS_LANES)   // no bias: the slot holds zeros for good
     *reinterpret_cast<uint4 *>(reinterpret_cast<unsigned char *>(bias_lds[wave]) + lane * 16) = make_uint4(0u, 0u, 0u, 0u);
-  // The bias is read with hand-written LDS loads and a hand-placed wait: the compiler, which cannot tell how
-  // many of the outstanding direct loads are older than the one into the bias slot, would otherwise wait for
-  // all of them (the stage just asked for included) before the first read.
+  // The bias is read with hand-written LDS loads and a hand-placed wait.
   const uint32_t bias_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)
                                reinterpret_cast<unsigned char *>(bias_lds[wave]) + (uint32_t)(lane >> 4) * 4u * (uint32_t)sizeof(T);
   auto init_acc = [&]() {
@@ -555,7 +553,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
         park_rows(pass, h);
-        if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores: see below
+        if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores
         // the wavefront reads its own piece back: lane -> (row = it*4 + lane/16, slot = lane%16)
 #pragma unroll 4
         for (int it = 0; it < 8; ++it) {
@@ -582,9 +580,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int ncol0 = n0 + wn * 128 + pass * SEGW;       // first feature of the segment
         uint32_t cut_bits = 0;
         if constexpr (COLLECT == 1) {
-          // The cut came in with the bias, ahead of the tile's stages, and has long landed.  Read by hand, with
-          // its own wait inside the statement: the compiler, which cannot tell the direct-to-LDS loads in flight
-          // (the next tile's first stage) from the one into this slot, would wait for all of them first.
+          // The cut came in with the bias, during the tile before, and has long landed.  Read by hand, with its own wait
+          // inside the statement: the compiler knows of no load that writes this slot.
           uint32_t cut_key_v;
           const uint32_t cut_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)cut_lds[slot][wave];
           asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(cut_key_v) : "v"(cut_at) : "memory");
@@ -741,7 +738,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           park_rows(pass, h);
-          if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores: see below
+          if (pass == 0 && h == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), ahead of the stores
           scan_piece(W[h]);
           // the first `shift` tokens of a shifted tile belong to its neighbour, which reports them, and so do the
           // features in front of on0 (bit b of word i of a lane = feature hs * SEGW / 2 + 32 i + b of the segment)

@@ -8,7 +8,7 @@ enum : uint32_t { ST_RUN = 0, ST_RETRY = 1, ST_DONE = 2 };
 // where the candidates of a problem live
 enum : uint32_t {
   PATH_ROWS = 0,   // per-row chains of extents written by the streaming pass
-  PATH_TILES = 1,  // per-(row, feature segment) runs written by the encoder epilogue
+  PATH_TILES = 1,  // an extent for every (64 rows, feature segment), written by the encoder epilogue
 };
 
 struct SelState {
@@ -71,7 +71,7 @@ __device__ __forceinline__ int64_t collect_grid_row(int64_t token, int64_t T, in
 // same-address atomic per tile from every CU at once would cost more than the whole epilogue).
 //   tile_meta[layer * ntile + i]    = (offset of the extent, entries)
 //   an entry                        = (feature | the token's place in the tile << 26, raw value bits)
-// (T F < 2^32 and at least COLLECT_TILE_ROWS tokens: a feature number has 24 bits at most.)
+// A feature number has the lower 26 bits: clt_encode_can_collect takes no more features.
 constexpr uint32_t COLLECT_COL = (1u << 26) - 1u;
 __device__ __forceinline__ uint32_t collect_place(int row, uint32_t col) { return (uint32_t)row << 26 | col; }
 __device__ __forceinline__ int collect_row(uint32_t place) { return (int)(place >> 26); }

@@ -7,8 +7,8 @@
 // The gathered operand comes out of LDS through the transposing read, which takes an address per lane.
 //
 // Why: a gather through the vector memory path is bound by the L1's outstanding lines (15 TB/s at best on this part);
-// LDS hands out randomly chosen 32-byte pieces at 59 TB/s (2.21 ns per 512-byte transposing read and CU with random
-// rows, 1.62 ns without any bank conflict; profiles/lds_read_probe.txt).  Fifteen sixteenths of the matrix instruction's products are with zeros,
+// LDS hands out 32-byte pieces at 60 TB/s if they are chosen at random and at 124 if no two of a half wavefront's meet in a bank
+// (2.19 and 1.06 ns per 512-byte transposing read and CU; profiles/lds_read_probe.txt).  Fifteen sixteenths of the matrix instruction's products are with zeros,
 // which still leaves as many useful ones per cycle as the vector unit's dot products deliver, without their
 // unpacking; and lists of unequal length cost nothing, because a batch is filled from any of 16 output rows.
 #pragma once
@@ -30,7 +30,7 @@ constexpr int SP_BATCH = 32;         // entries of a batch
 //   y = 3   half of where their tile rows begin in LDS: entry 8 q + x low, entry 8 q + 4 + x high
 // - every lane finds what it needs in its own row of 16 lanes, one DPP operand away, so that a record costs one dword of
 // LDS traffic per lane beside the eight transposing reads (broadcasting it with two 16-byte reads instead: five vector
-// instructions fewer, but 24 ns of LDS time per batch and CU instead of 19, and LDS is what bounds the product).
+// instructions fewer, but a quarter more LDS time per batch).
 constexpr int SP_REC_WORDS = 64;
 
 // A tile lies in LDS as two halves of 32 columns, 64 bytes per row; the two 32-byte pieces of a row are exchanged in

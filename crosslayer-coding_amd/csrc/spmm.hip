@@ -295,12 +295,13 @@ __device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_o
 // cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so that one of
 // them brings it from HBM and the others find it in the L2.
 //
-// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.17 ms (98.6 GB of gathered rows, 31
-// TB/s) and 0.20 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.6 and 0.37
+// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.03 ms (98.6 GB of gathered rows, 33
+// TB/s) and 0.19 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.5 and 0.39
 // against 34.2 ms (profiles/forward_c1_kernel_trace.txt, forward_c2_kernel_trace.txt).  Bound by the chain of a batch's steps,
-// four wavefronts per SIMD: without any one of them - the reads, the products, the operand of values, the records - the launch takes
-// 8 - 12 % less (22 ns per batch and CU; a fifth of the batches' places are filling).  Tiles that come from HBM instead of
-// the L2 cost 0.3 ms of it (2.2 of the 15.6).
+// four wavefronts per SIMD: LDS is busy in 46 % of the cycles, the matrix cores in 29 % (decode_tiles_c1_lds_counters.txt), and
+// without any one step - the reads, the products, the operand of values, the records - the launch takes 8 - 12 % less (26 ns
+// per batch and CU; a fifth of the batches' places are filling).  Tiles that come from HBM instead of the L2 cost 0.3
+// ms of it (2.2 of the 15.5).
 // Measured and dropped: a wavefront of its own for the fills (fifteen share 64 groups badly: 3.98 ms); fewer lines on
 // their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought into the L2 early
 // (3.46 ms: the early loads block the records just as well).
@@ -813,9 +814,9 @@ struct TileTimes { double tiles, sparse; };   // us; the first large for what th
 // Both routes priced from what they measured (bf16; L 2 - 24, d 256 - 2048, F 4096 - 32768, T 256 - 8192, 17 - 216 survivors
 // per token): the gather moves its rows at 17 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage
 // of the tiles takes 1.0 us plus 20.5 ns per batch, but no less than the 2.24 us in which 64 KB come into LDS, and the
-// longest workgroup bounds a launch of few.  At the line the two differ by less than a fifth either way: e.g. L = 12,
-// d = 768, F = 24576: 200 survivors per token 6.25 / 3.31 ms at T = 4096, 2.03 / 1.57 at 1024, 1.23 / 1.25 at 512; 50 per
-// token 2.58 / 1.71 ms at 4096, 1.43 / 1.55 at 2048.
+// longest workgroup bounds a launch of few.  At the line the two differ by less than a fifth either way (also where the other
+// one is the gather for thin lists): e.g. L = 12, d = 768, F = 24576: 200 survivors per token 5.85 / 3.24 ms at T = 4096,
+// 1.92 / 1.61 at 1024, 1.13 / 1.28 at 512; 50 per token 2.53 / 1.71 ms at 4096, 1.43 / 1.57 at 2048.
 static TileTimes tile_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
   const TileTimes no = {1e30, 0};
   if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;

@@ -42,7 +42,9 @@ class SurvivorList:
     # host-side estimate of the survivor total where one is known without a read-back (cost models only)
     nnz_hint: Optional[int] = None
     # made by a selection over activations: its length says what a typical row holds.  A list of any other origin may
-    # hold all its entries in a few rows, and the schedule made for short rows (``clt_decode_thin``) is not priced by it
+    # hold all its entries in a few rows, and the schedule made for short rows (``clt_decode_thin``) is not priced by it.
+    # Nor may one with empty layers be (``_expand_layers``): its sources have longer rows than the average over all says
+    # (12 layers, 3000 tokens, 200 per token in the first three: 1.17 ms against 0.95 of the gather by sources)
     selected: bool = False
 
     @property
