@@ -314,7 +314,9 @@ def run_gpu(args):
     # fused path: they are compared in the encoder epilogue)
     sel_kernels = ("k_tile_emit", "k_tile_count", "k_pool_hist", "k_row_prefix", "k_select_allot", "k_select_scan",
                    "k_select_pass", "k_select_emit", "k_select_count", "k_select_level", "k_rowptr_scan")
-    sel_real = sum(n * b for k, (n, b) in table.items() if k.split("<")[0] in sel_kernels) / forwards if forwards else None
+    # (the first of a forward's candidate histograms is made in the encoder's stage)
+    sel_real = sum((n - forwards if k.startswith("k_pool_hist") else n) * b for k, (n, b) in table.items()
+                   if k.split("<")[0] in sel_kernels) / forwards if forwards else None
     result = {
         "metric": "CLT forward tokens/sec at GPT-2-small x32 BatchTopK k=200; % of roofline per stage",
         "value": T * args.steps / wall,
