@@ -42,12 +42,11 @@ struct RecArgs {
   int64_t Rn, L, max_entries;
   uint64_t layer_mask;
   SpPlan p;
-  int alternate;           // 1: stages of all layers follow each other, in two buffers in turn; 0: one buffer
   int32_t *start;          // [L * groups][SP_GROUP][tiles + 1] list position where a row's entries of a tile begin
   uint16_t *batches;       // [L * tiles][groups] batches of (layer, tile, group)
-  uint16_t *counts;        // [streams][stages][DT_GPW] the same by stream
+  uint2 *counts;           // [streams][stages] the same by stream (sp_stage_counts)
   uint32_t *offset;        // [streams][stages] batches of the stream before the stage
-  uint32_t *total;         // [streams] batches of the stream
+  uint32_t *total;         // [streams] batches of the stream, in whole quads
   uint32_t *recs;
   uint32_t *bad;           // number of groups whose sums are not finite, and which
 };
@@ -108,12 +107,11 @@ __global__ __launch_bounds__(64) void k_rec_streams(RecArgs A) {
     }
     if (st < A.p.stages) {
       A.offset[(int64_t)stream * A.p.stages + st] = run + incl - sum;
-      *reinterpret_cast<uint2 *>(A.counts + ((int64_t)stream * A.p.stages + st) * DT_GPW) =
-          make_uint2(n[0] | (n[1] << 16), n[2] | (n[3] << 16));
+      A.counts[(int64_t)stream * A.p.stages + st] = sp_stage_counts(n[0], n[1], n[2], n[3]);
     }
     run += __shfl(incl, 63);
   }
-  if (lane == 0) A.total[stream] = run;
+  if (lane == 0) A.total[stream] = (run + SP_QUAD - 1) / SP_QUAD * SP_QUAD;
   if (stream == 0 && lane == 0) *A.bad = 0u;
 }
 
@@ -142,9 +140,6 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
   extern __shared__ int32_t fill_lds[];
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63, wave = tid >> 6;
   if (A.row_ptr[A.L * A.Rn] > A.max_entries) return;
-  // A wavefront at the end of its stream takes the record that follows for addresses, of LDS reads that nobody multiplies: the
-  // next stream's first one, or this one behind the last stream, which refers to the first row of the first buffer.
-  if (g == 0 && s == 0 && tid < 64) A.recs[(uint64_t)stream_first(A.total, A.p.streams, lane) * SP_REC_WORDS + lane] = 0u;
   if (!((A.layer_mask >> s) & 1ull)) return;
   int32_t *start = fill_lds;                               // [SP_GROUP][tiles + 1]
   uint32_t *dest = (uint32_t *)(start + SP_GROUP * (tiles + 1));       // [tiles] the tile's first batch among all of the stream
@@ -153,12 +148,11 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
   for (int i = tid; i < SP_GROUP * (tiles + 1); i += REC_THREADS) start[i] = src[i];
   const int part = g / A.p.groups_per_part, r = g - part * A.p.groups_per_part;
   const int stream = part * A.p.waves + r % A.p.waves, gi = r / A.p.waves;
-  const uint32_t stage0 = A.alternate ? (uint32_t)(__popcll(A.layer_mask & ((1ull << s) - 1ull)) * tiles) : 0u;
-  const uint32_t buffers = A.alternate ? 1u : 0u;
   for (int c = tid; c < tiles; c += REC_THREADS) {
     const int64_t at = (int64_t)stream * A.p.stages + (int64_t)s * tiles + c;
     uint32_t d = A.offset[at];
-    for (int j = 0; j < gi; ++j) d += A.counts[at * DT_GPW + j];
+    const uint32_t before = A.counts[at].x;                // (of groups before one that has batches, all are counted)
+    for (int j = 0; j < gi; ++j) d += (before >> (10 * j)) & 1023u;
     dest[c] = d;
   }
   const uint32_t base = stream_first(A.total, stream, lane);
@@ -206,8 +200,8 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
       }
       first -= mine;
     }
-    // all entries once more: those of batches w0 .. w0 + wn - 1 to their places in `batches`
-    auto fill = [&](uint32_t *batches, int32_t w0, int32_t wn) {
+    // all entries once more, to their places in the records: half_of(batch of the tile, half word of the batch)
+    auto fill = [&](auto half_of) {
       uint32_t next = first;
       for (int32_t i0 = 0; i0 < n; i0 += 64) {
         int tk;
@@ -220,36 +214,36 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
         const uint32_t p = __shfl(next, (int)cls) + __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
         next += (uint32_t)__popcll(same_class(v, b0, b1, b2, (uint32_t)lane));
         const uint32_t slot = __umulhi(p, magic), h = p - slot * (uint32_t)halves;
-        const int32_t b = (int32_t)(h >> 2) - w0;
-        if (!on || b < 0 || b >= wn) continue;
+        const int32_t b = (int32_t)(h >> 2);
+        if (!on) continue;
         // half read h % 4 of batch h / 4: h & 1 the half of the wavefront, h & 2 the second four entries of its lane quartets
-        uint16_t *rec = (uint16_t *)(batches + b * SP_REC_WORDS) + (h & 1u) * 64;
+        const uint32_t side = (h & 1u) * 64;
         auto place = [&](uint32_t sl, uint16_t at) {
-          rec[(sl >> 2) * 32 + (4 * (sl & 3u) + 3) * 2 + ((h >> 1) & 1u)] = at;
+          *half_of(b, side + (sl >> 2) * 32 + (4 * (sl & 3u) + 3) * 2 + ((h >> 1) & 1u)) = at;
         };
-        const uint32_t k = (slot & 3u) + ((h & 2u) << 1), x = (slot >> 2) * 32 + 8 * (k >> 1) + (k & 1u);
-        rec[x] = (uint16_t)Elem<T>::raw(((const T *)A.val)[A.src ? A.src[j] : j]);
-        rec[x + 2] = (uint16_t)(1u << tk);
-        const uint16_t at = (uint16_t)sp_half_place(f - (uint32_t)c * SP_ROWS, (stage0 + c) & buffers);
+        const uint32_t k = (slot & 3u) + ((h & 2u) << 1), x = side + (slot >> 2) * 32 + 8 * (k >> 1) + (k & 1u);
+        *half_of(b, x) = (uint16_t)Elem<T>::raw(((const T *)A.val)[A.src ? A.src[j] : j]);
+        *half_of(b, x + 2) = (uint16_t)(1u << tk);
+        const uint16_t at = (uint16_t)sp_place(f - (uint32_t)c * SP_ROWS);
         place(slot, at);
         if (slot == 0)                                     // the places of this half read that stay empty
           for (uint32_t sl = __umulhi((uint32_t)n - 1u - p, magic) + 1u; sl < 8u; ++sl) place(sl, at);
       }
     };
-    uint32_t *const out = A.recs + (uint64_t)(base + dest[c]) * SP_REC_WORDS;
+    const uint64_t b0 = (uint64_t)base + dest[c];
     if (nb <= REC_WINDOW) {
       for (int32_t b = 0; b < nb; ++b) win[b * SP_REC_WORDS + lane] = 0u;
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      fill(win, 0, nb);
+      fill([&](int32_t b, uint32_t i) { return (uint16_t *)win + b * (2 * SP_REC_WORDS) + i; });
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      for (int32_t b = 0; b < nb; ++b) out[b * SP_REC_WORDS + lane] = win[b * SP_REC_WORDS + lane];
+      for (int32_t b = 0; b < nb; ++b) A.recs[sp_rec_word(b0 + b, lane)] = win[b * SP_REC_WORDS + lane];
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     } else {
       // more than the window holds - up to 256, where 16 features fire on most tokens: put together where they are to lie, two
       // bytes at a time, rather than all entries once per window
-      for (int32_t b = 0; b < nb; ++b) out[b * SP_REC_WORDS + lane] = 0u;
+      for (int32_t b = 0; b < nb; ++b) A.recs[sp_rec_word(b0 + b, lane)] = 0u;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the zeros have arrived
-      fill(out, 0, nb);
+      fill([&](int32_t b, uint32_t i) { return (uint16_t *)(A.recs + sp_rec_word(b0 + b, i >> 1)) + (i & 1u); });
     }
   }
 }
@@ -257,7 +251,7 @@ template <typename T> __global__ __launch_bounds__(REC_THREADS) void k_rec_fill(
 // ---- decode -----------------------------------------------------------------------------------------
 struct TileArgs {
   SpPlan p;
-  const uint16_t *counts;
+  const uint2 *counts;
   const uint32_t *total;
   const uint32_t *recs;
   const void *wp;
@@ -273,9 +267,8 @@ struct TileArgs {
 };
 
 constexpr int DT_FILLS = SP_ROWS / 8 / DT_WAVES;           // direct-to-LDS loads of a tile per wavefront
-constexpr int DT_RING = 8;                                 // records a wavefront keeps in LDS or on their way
-constexpr int DT_LDS = 2 * SP_TILE_BYTES + DT_WAVES * DT_RING * 256;
-static_assert(DT_FILLS == 4 && DT_RING == 8, "the wait counts below are written out");
+constexpr int DT_LDS = 2 * SP_TILE_BYTES + DT_WAVES * SP_RING_BYTES;
+static_assert(DT_FILLS == 4, "the wait counts here and in SP_RING_READ are written out");
 
 // Whether a wavefront's sums of a group (16 rows from row0 on, of n rows) are all finite; if not, the group goes on the list.
 __device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_on, uint32_t *bad, uint32_t item) {
@@ -290,21 +283,21 @@ __device__ __forceinline__ bool sums_finite(const f32x4v_t (&acc)[4], bool row_o
 }
 
 // Two tiles of 512 features x 64 columns in LDS, one being multiplied while the other comes in.  Each wavefront owns four
-// groups of 16 tokens and consumes its stream of batches through a ring of eight records in LDS: the vector memory path
-// returns in order, so a record waits behind whatever tile lines were asked for before it, and eight batches (~2 us)
-// cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one XCD, so that one of
-// them brings it from HBM and the others find it in the L2.
+// groups of 16 tokens and consumes its stream of batches through a ring of two quads of records in LDS: the vector memory path
+// returns in order, so a record waits behind whatever tile lines were asked for before it, and the seven batches between a
+// quad's request and its use cover that.  Workgroups that share a decoder tile (the parts of the tokens) follow each other on one
+// XCD, so that one of them brings it from HBM and the others find it in the L2.
 //
-// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 3.03 ms (98.6 GB of gathered rows, 33
-// TB/s) and 0.19 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 15.5 and 0.39
-// against 34.2 ms (profiles/forward_c1_kernel_trace.txt, forward_c2_kernel_trace.txt).  Bound by the chain of a batch's steps,
-// four wavefronts per SIMD: LDS is busy in 46 % of the cycles, the matrix cores in 29 % (decode_tiles_c1_lds_counters.txt), and
-// without any one step - the reads, the products, the operand of values, the records - the launch takes 8 - 12 % less (26 ns
-// per batch and CU; a fifth of the batches' places are filling).  Tiles that come from HBM instead of the L2 cost 0.3
-// ms of it (2.2 of the 15.5).
-// Measured and dropped: a wavefront of its own for the fills (fifteen share 64 groups badly: 3.98 ms); fewer lines on
-// their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought into the L2 early
-// (3.46 ms: the early loads block the records just as well).
+// L = 12, d = 768, F = 24576, 4096 tokens, 200 survivors per token, untied, bf16: 2.82 ms (98.6 GB of gathered rows, 35
+// TB/s) and 0.19 ms for the records, against 6.45 ms of the gather from the L2s; L = 24, d = 1024, F = 32768: 14.4 and 0.39
+// against 34.2 ms.  A record at a time and one batch in the making took 3.10 and 15.5 ms.  It is 5.6 M cycles of a clock that the
+// power limit holds at 1.97 GHz (6.3 M at 2.09 before); in those vector instructions issue 53 % of the time, LDS is active 45 %,
+// the matrix cores 33 %, and the wavefronts wait 43 % of theirs, most of it at the barrier for the one with the heaviest
+// tokens (decode_tiles_c1_lds_counters.txt; with equal lists 2.65 ms).  Without batches the tiles alone take 1.65 ms to come in.
+// Measured and dropped: reads and products of a step interleaved, or the values' operand first (within 1 %: no single step binds);
+// heavy wavefronts at a higher wave priority (the same); a wavefront of its own for the fills (fifteen share 64 groups badly:
+// 3.98 ms); fewer lines on their way (4.5 ms: the fills are latency-bound); every parts-th line of the tile after next brought
+// into the L2 early (3.46 ms: the early loads block the records just as well).
 template <typename T>
 __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
   extern __shared__ __attribute__((aligned(128))) char tile_lds[];
@@ -323,110 +316,65 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
   // lane / 4 per lane; which 16 bytes a lane brings is what exchanges the pieces.  (Both halves of a line are asked for
   // one after the other: the second hits the L1.)
   const uint32_t pitch_b = (uint32_t)(A.pitch * (int64_t)sizeof(T));
-  const uint32_t col_b = (((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4);
-  const int row_a = wave * 32 + (lane >> 2);
-  const uint32_t off_a = (uint32_t)row_a * pitch_b + col_b;
-  auto fill = [&](const char *src, int rows, uint32_t lds_at) {
-    if (rows >= SP_ROWS) {
-#pragma unroll
-      for (int i = 0; i < DT_FILLS; ++i)
-        sp_fill16(src + (i & 1) * 64, off_a + (uint32_t)(i >> 1) * 16 * pitch_b, lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
-    } else {                                               // past the matrix: nobody refers to these rows
-#pragma unroll
-      for (int i = 0; i < DT_FILLS; ++i) {
-        const int r = row_a + (i >> 1) * 16;
-        sp_fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
-               lds_at + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
-      }
-    }
-  };
+  // Rows past the matrix, which nobody refers to, are read as its last one.
+  // Rows past the matrix, which nobody refers to, are read as its last one.
+  const uint32_t off_a = (uint32_t)(wave * 32 + (lane >> 2)) * pitch_b + ((((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4));
+  const uint32_t off_b = off_a + 16 * pitch_b;
+  auto last_row = [&](int rows) { return (uint32_t)((rows < SP_ROWS ? rows : SP_ROWS) - 1) * pitch_b + 48u; };
 
   auto tile_at = [&](int s) {
     return (const char *)A.wp + sp_slot(A.tying, s, t, A.L) * A.F * (int64_t)pitch_b + (int64_t)cp * 128;
   };
 
-  f32x4v_t acc[DT_GPW][4];
-#pragma unroll
-  for (int gi = 0; gi < DT_GPW; ++gi)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[gi][n] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
-
+  SpSums acc;
+  acc.clear();
   if (n_stages > 0) {
-    const uint32_t row_bit = 0x00010001u << (lane & 15);
-    const uint32_t ring = lds0 + 2 * SP_TILE_BYTES + (uint32_t)wave * (DT_RING * 256);
-    const uint32_t *recs = A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(stream_first(A.total, stream, lane)) * SP_REC_WORDS;
-    uint32_t rec_off = (uint32_t)lane * 4;                 // of the next record to ask for, this lane's word
-    uint32_t slot = 0;                                     // of the batch that is consumed next, in bytes
-    auto ask = [&](uint32_t at) {                          // the next record of the stream into the ring
-      sp_fill4(recs, rec_off, ring + at);
-      rec_off += SP_REC_WORDS * 4;
-    };
-    uint32_t word;                                         // of the record after the batch at hand
-    const uint32_t ring_lane = ring + (uint32_t)lane * 4;
-    auto look = [&](uint32_t at) { word = *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)(ring_lane + at); };
+    SpStream batches;
+    batches.begin(A.recs, __builtin_amdgcn_readfirstlane(stream_first(A.total, stream, lane)), lds0 + 2 * SP_TILE_BYTES + (uint32_t)wave * SP_RING_BYTES, lds0, lane);
     // the next tile to bring in: where it begins and how many rows of the matrix are left from there on
     uint64_t m = mask;
     int s = __ffsll((unsigned long long)m) - 1, c = 0, rows = (int)A.F;
     const char *tile = tile_at(s);
     const uint32_t tile_step = SP_ROWS * pitch_b, lds_share = lds0 + (uint32_t)wave * 2048;
-    fill(tile, rows, lds_share);
+    {
+      const uint32_t last = last_row(rows);
 #pragma unroll
-    for (int i = 0; i < DT_RING; ++i) ask((uint32_t)i * 256);
-    const auto counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages;
-    uint2 cnt = make_uint2(counts[s * A.p.tiles].x, counts[s * A.p.tiles].y);
+      for (int i = 0; i < DT_FILLS; ++i) {
+        const uint32_t off = i >> 1 ? off_b : off_a;
+        sp_fill16(tile + (i & 1) * 64, off < last ? off : last, lds_share + (uint32_t)((i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+      }
+    }
+    const auto stream_counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages;
+    auto counts = stream_counts + s * A.p.tiles;
+    uint2 cnt = make_uint2(counts->x, counts->y);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    look(0);
-    const uint32_t col = lds0 + (uint32_t)(lane & 3) * 8;
-    SpBatch<T> bt;
-    // The next batch's record becomes addresses and values, its slot in the ring the place of the one eight batches on.
-    // `since`: records asked for since the last tile's lines.
-    auto prepare = [&](int since) {
-      bt.address(word, col);
-      bt.read();                                           // (in vain if its tile is still on its way: read again then)
-      bt.pick(word, row_bit);
-      asm volatile("" ::"v"(bt.picked), "v"(bt.a0), "v"(bt.a1));        // the slot has been read
-      ask(slot);
-      slot = (slot + 256) & (DT_RING * 256 - 1);
-      // the record after it: seven were asked for since, and perhaps the four loads of a tile
-      asm volatile("s_cmp_lt_i32 %0, 8\n\ts_cbranch_scc1 .Lnot_late%=\n\ts_waitcnt vmcnt(7)\n.Lnot_late%=:\n\ts_waitcnt vmcnt(11)" ::"s"(since)
-                   : "scc", "memory");
-      look(slot);
-    };
-    prepare(DT_RING);
+    batches.begun();
+    asm volatile("" ::"v"(batches.words));
     for (int st = 0; st < n_stages; ++st) {
-      const bool more = st + 1 < n_stages;
-      if (more) {
+      uint32_t to = SP_NO_TILE;                            // where this wavefront's share of the next tile goes, if there is one
+      if (st + 1 < n_stages) {
         tile += tile_step;
         rows -= SP_ROWS;
+        ++counts;
         if (++c == A.p.tiles) {
           c = 0;
           m &= m - 1;
           s = __ffsll((unsigned long long)m) - 1;
           tile = tile_at(s);
           rows = (int)A.F;
+          counts = stream_counts + s * A.p.tiles;
         }
+        to = (lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES);
       }
-      const int at = s * A.p.tiles + c;
-      const uint2 cnt_next = make_uint2(counts[at].x, counts[at].y);
-      asm volatile("" ::: "memory");
+      const uint32_t last = last_row(rows);
+      const uint2 cnt_next = make_uint2(counts->x, counts->y);
+      const uint32_t off0 = off_a < last ? off_a : last, off1 = off_b < last ? off_b : last;
+      asm volatile("" ::"v"(off0), "v"(off1) : "memory");
       __builtin_amdgcn_s_barrier();                        // tile st is complete, and nobody reads the other one any more
       asm volatile("" ::: "memory");
-      bt.read();
-      if (more) fill(tile, rows, lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES);
-      int since = more ? 0 : DT_RING;                      // records asked for after these lines
-#pragma unroll
-      for (int gi = 0; gi < DT_GPW; ++gi) {
-        const int n = (int)((gi & 2 ? cnt.y : cnt.x) >> (gi & 1 ? 16 : 0)) & 0xFFFF;
-        for (int i = n; i > 0; --i) {
-          bt.finish(acc[gi]);
-          prepare(++since);
-        }
-      }
+      batches.stage<T>(acc, cnt, SpFill{tile, off0, off1, to});
+      batches.col += st & 1 ? -SP_TILE_BYTES : SP_TILE_BYTES;
       cnt = cnt_next;
-      // the tile's lines are waited for, not the records asked for behind them
-      if (since >= DT_RING) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-      else if (since >= DT_RING / 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may be on its way into LDS when the workgroup ends
   }
@@ -436,11 +384,13 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
     const int g = A.p.group(stream, gi);
     const int64_t tok = (int64_t)g * SP_GROUP + (lane & 15);
     if (g < 0) continue;
-    if (!sums_finite(acc[gi], tok < A.Tn, A.bad, (uint32_t)(((t - A.t_begin) * A.p.groups + g) * A.col_parts + cp)) || tok >= A.Tn) continue;
+    f32x4v_t sum[4];
+    acc.get(gi, sum);
+    if (!sums_finite(sum, tok < A.Tn, A.bad, (uint32_t)(((t - A.t_begin) * A.p.groups + g) * A.col_parts + cp)) || tok >= A.Tn) continue;
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       const int64_t o = (int64_t)cp * SP_COLS + n * 16 + (lane >> 4) * 4;
-      f32x4v_t a = acc[gi][n];
+      f32x4v_t a = sum[n];
       const int64_t at = ((int64_t)t * A.Tn + tok) * A.d + o;
       if (A.bias_sum) a += *reinterpret_cast<const f32x4v_t *>(A.bias_sum + (int64_t)t * A.d + o);
       if (A.skip_add) a += *reinterpret_cast<const f32x4v_t *>(A.skip_add + at);
@@ -485,13 +435,13 @@ template <typename T> __global__ __launch_bounds__(256) void k_decode_repair(Til
 // place of tokens - 16 features per group, tiles of 512 tokens x 64 columns of g[t].
 constexpr int GT_WAVES = 8;
 constexpr int GT_FILLS = SP_ROWS / 8 / GT_WAVES;
-constexpr int GT_LDS = SP_TILE_BYTES + GT_WAVES * DT_RING * 256;
+constexpr int GT_LDS = SP_TILE_BYTES + GT_WAVES * SP_RING_BYTES;
 constexpr int GT_PITCH = SP_COLS + 4;      // fp32 row pitch of a group's gradient on its way through LDS
 static_assert(GT_LDS * 2 <= 160 * 1024 && SP_GROUP * GT_PITCH * 4 * GT_WAVES <= SP_TILE_BYTES, "two workgroups per CU");
 
 struct GradArgs {
   SpPlan p;
-  const uint16_t *counts;
+  const uint2 *counts;
   const uint32_t *offset, *total, *recs;
   const void *g;             // [L][T][d]
   void *w;                   // packed decoders, or null: the gradient goes to `out`
@@ -527,51 +477,28 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
   const int stream = part * GT_WAVES + wave;
 
   const uint32_t pitch_b = (uint32_t)(A.d * (int64_t)sizeof(T));
-  const uint32_t col_b = (((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4);
-  const int row_a = wave * 64 + (lane >> 2);
-  auto fill = [&](const char *src, int rows) {
+  const uint32_t off_a = (uint32_t)(wave * 64 + (lane >> 2)) * pitch_b + ((((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4));
+  auto fill = [&](const char *src, int rows) {             // as in k_decode_tiles
+    const uint32_t last = (uint32_t)((rows < SP_ROWS ? rows : SP_ROWS) - 1) * pitch_b + 48u;
 #pragma unroll
     for (int i = 0; i < GT_FILLS; ++i) {
-      const int r = row_a + (i >> 1) * 16;
-      sp_fill16(src + (i & 1) * 64, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b,
-             lds0 + (uint32_t)(wave * 4096 + (i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
+      const uint32_t off = off_a + (uint32_t)(i >> 1) * 16 * pitch_b;
+      sp_fill16(src + (i & 1) * 64, off < last ? off : last, lds0 + (uint32_t)(wave * 4096 + (i >> 1) * 1024 + (i & 1) * SP_HALF_BYTES));
     }
   };
 
-  f32x4v_t acc[DT_GPW][4];
-#pragma unroll
-  for (int gi = 0; gi < DT_GPW; ++gi)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[gi][n] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
+  SpSums acc;
+  acc.clear();
   {
-    const uint32_t row_bit = 0x00010001u << (lane & 15);
-    const uint32_t ring = lds0 + SP_TILE_BYTES + (uint32_t)wave * (DT_RING * 256);
     const int stage0 = s * A.p.tiles;
-    const uint32_t *recs = A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(
-        stream_first(A.total, stream, lane) + A.offset[(int64_t)stream * A.p.stages + stage0]) * SP_REC_WORDS;
-    uint32_t rec_off = (uint32_t)lane * 4, at = 0, word;
-    const uint32_t ring_lane = ring + (uint32_t)lane * 4, col = lds0 + (uint32_t)(lane & 3) * 8;
+    SpStream batches;
+    batches.begin(A.recs, __builtin_amdgcn_readfirstlane(stream_first(A.total, stream, lane) + A.offset[(int64_t)stream * A.p.stages + stage0]),
+                  lds0 + SP_TILE_BYTES + (uint32_t)wave * SP_RING_BYTES, lds0, lane);
     const auto counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages + stage0;
     const char *tile = (const char *)A.g + (int64_t)t * A.Tn * (int64_t)pitch_b + (int64_t)cp * 128;
     fill(tile, (int)A.Tn);
-#pragma unroll
-    for (int i = 0; i < DT_RING; ++i) { sp_fill4(recs, rec_off, ring + (uint32_t)i * 256); rec_off += SP_REC_WORDS * 4; }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    auto look = [&]() { word = *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)(ring_lane + at); };
-    look();
-    SpBatch<T> bt;
-    auto prepare = [&]() {                                 // as in k_decode_tiles; no tile line is ever behind a record
-      bt.address(word, col);
-      bt.read();
-      bt.pick(word, row_bit);
-      asm volatile("" ::"v"(bt.picked), "v"(bt.a0), "v"(bt.a1));
-      sp_fill4(recs, rec_off, ring + at);
-      rec_off += SP_REC_WORDS * 4;
-      at = (at + 256) & (DT_RING * 256 - 1);
-      asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-      look();
-    };
-    prepare();
+    batches.begun();
     int rows = (int)A.Tn;
     for (int st = 0; st < A.p.tiles; ++st) {
       const uint2 cnt = make_uint2(counts[st].x, counts[st].y);
@@ -587,12 +514,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      bt.read();
-#pragma unroll
-      for (int gi = 0; gi < DT_GPW; ++gi) {
-        const int n = (int)((gi & 2 ? cnt.y : cnt.x) >> (gi & 1 ? 16 : 0)) & 0xFFFF;
-        for (int i = n; i > 0; --i) { bt.finish(acc[gi]); prepare(); }
-      }
+      batches.stage<T>(acc, cnt, SpNoFill{});              // (there is one buffer: no tile comes in meanwhile)
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();                          // the tile's LDS is free
@@ -604,7 +526,9 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
   for (int gi = 0; gi < DT_GPW; ++gi) {
     const int g = A.p.group(stream, gi);
     if (g < 0) break;
-    if (!sums_finite(acc[gi], (int64_t)g * SP_GROUP + (lane & 15) < A.F, A.bad, (uint32_t)((slot * A.p.groups + g) * A.col_parts + cp))) continue;
+    f32x4v_t sum[4];
+    acc.get(gi, sum);
+    if (!sums_finite(sum, (int64_t)g * SP_GROUP + (lane & 15) < A.F, A.bad, (uint32_t)((slot * A.p.groups + g) * A.col_parts + cp))) continue;
     // rows of 64 columns: lane 16 r + c takes columns 4 c .. 4 c + 3 of rows r, r + 4, r + 8, r + 12
     const int c4 = (lane & 15) * 4;
     const int64_t f0 = (int64_t)g * SP_GROUP + (lane >> 4);
@@ -624,7 +548,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n)
-      *reinterpret_cast<f32x4v_t *>(mine + (lane & 15) * GT_PITCH + n * 16 + (lane >> 4) * 4) = acc[gi][n];
+      *reinterpret_cast<f32x4v_t *>(mine + (lane & 15) * GT_PITCH + n * 16 + (lane >> 4) * 4) = sum[n];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -714,23 +638,25 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
   }
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
   p.streams = p.parts * waves;
-  // every (layer, tile, group) may leave its last batch part empty; a stream asks for a ring of batches and one more past its end
-  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + DT_RING + 1;
+  // every (layer, tile, group) may leave its last batch part empty, and every stream its last quad; a stream asks for up to three
+  // quads past its end
+  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + 9;
+  const int64_t rec_batches = l.n_batches + (int64_t)(SP_QUAD - 1) * p.streams + 4 * SP_QUAD;
   size_t at = 0;
   auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
   l.start = take(sizeof(int32_t) * (size_t)L * p.groups * SP_GROUP * (p.tiles + 1));
   l.batches = take(sizeof(uint16_t) * (size_t)p.stages * p.groups);
-  l.counts = take(sizeof(uint16_t) * (size_t)p.streams * p.stages * DT_GPW);
+  l.counts = take(sizeof(uint2) * (size_t)p.streams * p.stages);
   l.offset = take(sizeof(uint32_t) * (size_t)p.streams * p.stages);
   l.total = take(sizeof(uint32_t) * (size_t)p.streams);
-  l.recs = take((size_t)l.n_batches * SP_REC_WORDS * 4);
+  l.recs = take((size_t)rec_batches * SP_REC_WORDS * 4);
   l.n_groups = outputs * p.groups * l.col_parts;
   l.bad = take(sizeof(uint32_t) * (size_t)(l.n_groups + 1));
   l.bytes = at;
   return l;
 }
 
-// LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile; 16-bit batch counts
+// LDS for the run starts of every tile; 32-bit offsets of rows within a tile; 16-bit batch counts; batches whose records take 4 GB
 constexpr int64_t SP_MAX_BATCHES = 0x00FFFFFF;
 static bool sp_shape_ok(const SpLayout &l, int64_t row_bytes) {
   return l.p.tiles <= REC_MAX_TILES && l.n_batches <= SP_MAX_BATCHES && row_bytes * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
@@ -739,7 +665,7 @@ static bool sp_shape_ok(const SpLayout &l, int64_t row_bytes) {
 
 static void sp_place_workspace(RecArgs &ra, const SpLayout &l, char *ws) {
   ra.p = l.p;
-  ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint16_t *)(ws + l.counts);
+  ra.start = (int32_t *)(ws + l.start); ra.batches = (uint16_t *)(ws + l.batches); ra.counts = (uint2 *)(ws + l.counts);
   ra.offset = (uint32_t *)(ws + l.offset); ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint32_t *)(ws + l.recs);
   ra.bad = (uint32_t *)(ws + l.bad);
 }
@@ -784,7 +710,7 @@ static int launch_grad(const int32_t *list_ptr, const int32_t *list_tok, const i
   if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
   RecArgs ra;
   ra.row_ptr = list_ptr; ra.col = list_tok; ra.src = list_src; ra.val = val; ra.Rn = a.F; ra.L = a.L; ra.max_entries = a.max_entries;
-  ra.layer_mask = ~0ull; ra.alternate = 0;
+  ra.layer_mask = ~0ull;
   sp_place_workspace(ra, l, (char *)workspace);
   const int code = launch_records<bf16_t>(ra, stream);
   if (code != CLT_OK) return code;
@@ -873,7 +799,7 @@ extern "C" int clt_decode_tiles(const int32_t *row_ptr, const int32_t *col, cons
   if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
   RecArgs ra;
   ra.row_ptr = row_ptr; ra.col = col; ra.src = nullptr; ra.val = val; ra.Rn = T; ra.L = L; ra.max_entries = max_entries;
-  ra.layer_mask = src_mask; ra.alternate = 1;
+  ra.layer_mask = src_mask;
   sp_place_workspace(ra, l, (char *)workspace);
   TileArgs ta;
   ta.p = l.p; ta.counts = ra.counts; ta.total = ra.total; ta.recs = ra.recs;
