@@ -78,7 +78,7 @@ class _ReconstructionsWithGraph(torch.autograd.Function):
             if go is not None:
                 g[l] = go.reshape(T, d)
         g_model = g.to(model.dtype)
-        raw = model._raw_gradients_from(ctx.inputs, surv, g, g_model, g.sum(dim=1))
+        raw = model._raw_gradients_from(ctx.inputs, surv, g, g_model, g.sum(dim=1), as_parameters=True)
         named = model._named_gradients(raw)
         grads = []
         for name, p in zip(ctx.names, ctx.params):
@@ -295,10 +295,11 @@ class CrossLayerTranscoder(BaseTranscoder):
         return loss_l, self._raw_gradients_from(inputs, surv, g, g_model, bias_grad, decoder_step)
 
     def _raw_gradients_from(self, inputs: Dict[int, torch.Tensor], surv, g: torch.Tensor, g_model: torch.Tensor,
-                            bias_grad: torch.Tensor, decoder_step=None):
+                            bias_grad: torch.Tensor, decoder_step=None, as_parameters: bool = False):
         """The raw parameter gradients (see ``_loss_and_raw_gradients``) of any loss, given d loss / d reconstruction:
         ``g`` fp32 [L, T, d], ``g_model`` the same in the model dtype, ``bias_grad`` [L, d] its sums over tokens.
-        ``surv`` is the (trimmed) survivor list of the forward on ``inputs``."""
+        ``surv`` is the (trimmed) survivor list of the forward on ``inputs``.  ``as_parameters``: decoder gradients may come in their
+        parameters' layout and dtype instead, as ``dec_param`` [n_dec, d, F] (``dec_w`` is None then)."""
         cfg = self.config
         L, d, F = cfg.num_layers, cfg.d_model, cfg.num_features
         ws = self._workspace()
@@ -321,7 +322,11 @@ class CrossLayerTranscoder(BaseTranscoder):
                        else (None, None))
         # ``decoder_step`` (an optimiser whose ``fuses_decoder_step()`` holds): the decoder weights take their
         # step inside the weight-gradient kernel, after everything that reads the old decoders (below)
-        dw_dec = None if decoder_step is not None else engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
+        dw_dec = dw_param = None
+        if as_parameters and cfg.decoder_tying == "none" and off is None and sc is None:
+            dw_param = engine.decoder_parameter_grad(lists, surv, g_model, ws)
+        if decoder_step is None and dw_param is None:
+            dw_dec = engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
         _, x_slab, _, _ = self.encoder_module.prepare_slab(inputs)
         x_slab = x_slab.contiguous()
         dw_enc, db_enc = engine.encoder_weight_grad(lists, dval, x_slab, F)
@@ -345,8 +350,8 @@ class CrossLayerTranscoder(BaseTranscoder):
             dec_b = torch.flip(torch.cumsum(torch.flip(bias_grad, dims=[0]), dim=0), dims=[0])
         else:
             dec_b = bias_grad
-        return {"enc_w": dw_enc, "enc_b": db_enc, "dec_w": dw_dec, "dec_b": dec_b.contiguous(), "theta": theta_grad,
-                "skip": d_skip, "feat_offset": d_off, "feat_scale": d_sc}
+        return {"enc_w": dw_enc, "enc_b": db_enc, "dec_w": dw_dec, "dec_param": dw_param, "dec_b": dec_b.contiguous(),
+                "theta": theta_grad, "skip": d_skip, "feat_offset": d_off, "feat_scale": d_sc}
 
     def _log_threshold_gradient(self, x_slab: torch.Tensor, g_model: torch.Tensor, ws, surv=None, dval=None) -> torch.Tensor:
         """fp32 [L, F] gradient of ``log_threshold`` (JumpReLU.backward, activations.py:196-199, through
@@ -523,7 +528,8 @@ class CrossLayerTranscoder(BaseTranscoder):
         else:
             keys = [str(i) for i in range(L)]
         for slot, key in enumerate(keys):
-            grads[f"decoder_module.decoders.{key}.weight"] = raw["dec_w"][slot].t()   # [d, F] view
+            grads[f"decoder_module.decoders.{key}.weight"] = (raw["dec_w"][slot].t() if raw.get("dec_param") is None   # [d, F] view
+                                                              else raw["dec_param"][slot])
             grads[f"decoder_module.decoders.{key}.bias_param"] = raw["dec_b"][slot]
         if raw.get("theta") is not None:
             grads["theta_manager.log_threshold"] = raw["theta"]

@@ -678,6 +678,23 @@ def grad_tiles_supported(T: int, d: int, F: int, L: int, entries: int, dtype: to
     return dtype == torch.bfloat16 and bool(nat.load().clt_grad_tiles_supported(T, d, F, L, entries, nat.dtype_code(dtype)))
 
 
+def decoder_parameter_grad(lists, surv: SurvivorList, g: torch.Tensor, ws: Optional[Workspace] = None) -> Optional[torch.Tensor]:
+    """Gradients of untied decoders in their parameters' layout and dtype, [n_dec, d, F]: ``decoder_weight_grad``'s rounded once and
+    transposed, in one pass.  None where the matrix-core kernels do not take the shapes."""
+    ptr, tok, src = lists
+    L, T, F = surv.L, surv.T, surv.F
+    d, n = g.shape[2], surv.capacity
+    if g.dtype != surv.dtype or F % 8 or not _aligned16(g) or not g.is_contiguous() or not grad_tiles_supported(T, d, F, L, n, surv.dtype):
+        return None
+    out = torch.empty((L * (L + 1) // 2, d, F), dtype=surv.dtype, device=g.device)
+    lib = nat.load()
+    wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_tiles_workspace_bytes(T, d, F, L, n))
+    code = lib.clt_decoder_grad_param_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(out), T, d,
+                                            F, L, n, nat.dtype_code(surv.dtype), nat.ptr(wbuf), wbuf.numel(), _stream(g))
+    nat.check(code, "clt_decoder_grad_param_tiles")
+    return out
+
+
 def decoder_weight_grad(lists, surv: SurvivorList, g: torch.Tensor, tying: str,
                         feat_offset: Optional[torch.Tensor] = None, feat_scale: Optional[torch.Tensor] = None,
                         ws: Optional[Workspace] = None) -> torch.Tensor:

@@ -21,5 +21,5 @@ def test_tile_kernels_spill_nothing(tmp_path):
     assert proc.returncode == 0, proc.stdout[-2000:]
     text = open(out).read()
     scratch = re.findall(r"^(_Z\w*k_(?:decode|grad)_tiles\w*):.*?^; ScratchSize: (\d+)", text, re.S | re.M)
-    assert len(scratch) == 4, scratch               # two 16-bit types; with the step and without
+    assert len(scratch) == 5, scratch               # two 16-bit types; with the step, as rows and as parameters
     assert all(int(size) == 0 for _, size in scratch), scratch
