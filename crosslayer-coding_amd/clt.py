@@ -73,12 +73,21 @@ class _ReconstructionsWithGraph(torch.autograd.Function):
                                "backward: the gradient would be taken at other weights than the output was")
         surv = ctx.surv
         L, T, d = surv.L, surv.T, model.config.d_model
-        g = torch.zeros((L, T, d), dtype=torch.float32, device=surv.row_ptr.device)
-        for l, go in enumerate(grad_outs):
-            if go is not None:
-                g[l] = go.reshape(T, d)
-        g_model = g.to(model.dtype)
+        if all(go is not None and go.dtype == model.dtype for go in grad_outs):
+            g_model = torch.stack([go.reshape(T, d) for go in grad_outs])
+            g = g_model.float()
+        else:
+            g = torch.zeros((L, T, d), dtype=torch.float32, device=surv.row_ptr.device)
+            for l, go in enumerate(grad_outs):
+                if go is not None:
+                    g[l] = go.reshape(T, d)
+            g_model = g.to(model.dtype)
         raw = model._raw_gradients_from(ctx.inputs, surv, g, g_model, g.sum(dim=1), as_parameters=True)
+        # families of parameters in one cast each: the gradients are views of one tensor, as a float32 model's are
+        if all(p.dtype == model.dtype for n, p in zip(ctx.names, ctx.params) if not n.startswith("theta_manager.")):
+            for key in ("enc_w", "enc_b", "dec_b", "skip"):
+                if raw.get(key) is not None:
+                    raw[key] = raw[key].to(model.dtype)
         named = model._named_gradients(raw)
         grads = []
         for name, p in zip(ctx.names, ctx.params):
@@ -316,7 +325,8 @@ class CrossLayerTranscoder(BaseTranscoder):
             # optimiser applies it)
             return self._raw_gradients_dense(inputs, surv, g, g_model, bias_grad)
         off, sc = dec._affine()                     # per-target feature offset / scale of tied decoders, or None
-        dval = engine.decode_backward_values(surv, dec.packed(), g, cfg.decoder_tying, mask, ws, feat_scale=sc)
+        packed = dec.packed()
+        dval = engine.decode_backward_values(surv, packed, g, cfg.decoder_tying, mask, ws, feat_scale=sc)
         lists = engine.feature_lists(surv, ws)
         d_off, d_sc = (engine.feature_affine_grad(lists, surv, ws, off, sc, mask) if (off is not None or sc is not None)
                        else (None, None))
@@ -339,13 +349,13 @@ class CrossLayerTranscoder(BaseTranscoder):
                 engine.skip_weight_grad(g[t], x_slab[s_], d_skip[i])
         theta_grad = None
         if cfg.activation_fn == "jumprelu" and self.theta_manager.log_threshold is not None:
-            theta_grad = self._log_threshold_gradient(x_slab, g_model, ws, surv, dval if sc is not None else None)
+            theta_grad = self._log_threshold_gradient(x_slab, g_model, ws, packed, surv, dval if sc is not None else None)
         if decoder_step is not None:
             decoder_step.decoder_weight_step(lists, surv, g_model)
         # bias_grad[t] = column sums of d loss / d rec[t]; a decoder's bias takes the rows of the targets
         # it is added to: its own pair's target, all targets >= its source, or its target (once)
         if cfg.decoder_tying == "none":
-            dec_b = bias_grad[torch.tensor([t for s_ in range(L) for t in range(s_, L)], device=bias_grad.device)]
+            dec_b = torch.cat([bias_grad[s_:] for s_ in range(L)])       # (an index built on the host would be waited for)
         elif cfg.decoder_tying == "per_source":
             dec_b = torch.flip(torch.cumsum(torch.flip(bias_grad, dims=[0]), dim=0), dims=[0])
         else:
@@ -353,7 +363,8 @@ class CrossLayerTranscoder(BaseTranscoder):
         return {"enc_w": dw_enc, "enc_b": db_enc, "dec_w": dw_dec, "dec_param": dw_param, "dec_b": dec_b.contiguous(),
                 "theta": theta_grad, "skip": d_skip, "feat_offset": d_off, "feat_scale": d_sc}
 
-    def _log_threshold_gradient(self, x_slab: torch.Tensor, g_model: torch.Tensor, ws, surv=None, dval=None) -> torch.Tensor:
+    def _log_threshold_gradient(self, x_slab: torch.Tensor, g_model: torch.Tensor, ws, packed: torch.Tensor, surv=None,
+                                dval=None) -> torch.Tensor:
         """fp32 [L, F] gradient of ``log_threshold`` (JumpReLU.backward, activations.py:196-199, through
         theta = exp(log_threshold), theta.py:70-79).  The band |x - theta| <= bandwidth / 2 holds elements
         on both sides of the threshold, so this part is dense: per source layer, d loss / d activation
@@ -368,7 +379,6 @@ class CrossLayerTranscoder(BaseTranscoder):
         w, b = self.encoder_module.stacked()
         pre = engine.encode(x_slab.contiguous(), w, b, out=ws.typed("pre", tuple(x_slab.shape[:2]) + (F,), self.dtype))
         theta = self.theta_manager.thresholds(self.dtype)
-        packed = self.decoder_module.packed()
         out = torch.empty((L, F), dtype=torch.float32, device=pre.device)
         T = g_model.shape[1]
         g_model = g_model.contiguous()
@@ -484,7 +494,7 @@ class CrossLayerTranscoder(BaseTranscoder):
         if theta_out is not None:
             theta_grad = theta_out * torch.exp(self.theta_manager.log_threshold.detach().float())
         if tying == "none":
-            dec_b = bias_grad[torch.tensor([t for s_ in range(L) for t in range(s_, L)], device=bias_grad.device)]
+            dec_b = torch.cat([bias_grad[s_:] for s_ in range(L)])       # (an index built on the host would be waited for)
         elif tying == "per_source":
             dec_b = torch.flip(torch.cumsum(torch.flip(bias_grad, dims=[0]), dim=0), dims=[0])
         else:
@@ -720,10 +730,12 @@ class CrossLayerTranscoder(BaseTranscoder):
         else:
             # the total travels to pinned memory behind the kernels; a later forward looks at it
             surv.nnz_hint = self._thr_last_total
-            host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-            host.copy_(surv.row_ptr[-1:], non_blocking=True)
+            host = torch.empty(2, dtype=torch.int32, pin_memory=True)
+            host[:1].copy_(surv.row_ptr[-1:], non_blocking=True)
+            host[1:].copy_(surv.status.view(-1)[:1], non_blocking=True)
             ev = torch.cuda.Event()
             ev.record()
+            surv.totals = (host, ev)
             self._thr_pending.append((host, ev, key))
         return surv
 
@@ -738,7 +750,7 @@ class CrossLayerTranscoder(BaseTranscoder):
             counts[l * T:(l + 1) * T] = per_row[i * T:(i + 1) * T]
         row_ptr = torch.zeros(L * T + 1, dtype=torch.int32, device=counts.device)
         row_ptr[1:] = torch.cumsum(counts, 0).to(torch.int32)
-        return SurvivorList(row_ptr, surv.col, surv.val, T, surv.F, L, surv.dtype, surv.status, surv.nnz_hint)
+        return SurvivorList(row_ptr, surv.col, surv.val, T, surv.F, L, surv.dtype, surv.status, surv.nnz_hint, totals=surv.totals)
 
     # ---- get_feature_activations -------------------------------------------------------------
     def get_feature_activations(self, inputs: Dict[int, torch.Tensor]) -> Dict[int, torch.Tensor]:
