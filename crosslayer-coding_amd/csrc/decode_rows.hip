@@ -16,14 +16,20 @@ constexpr int DR_COLS = 32;                // columns of a tile: one 128-byte li
 constexpr int DR_TOK = SP_GROUP;           // tokens of a wavefront: four accumulators per lane each
 constexpr int DR_REC = 8;                  // entries of a record: a wavefront reads 8 rows x 16 bytes per lane
 constexpr int DR_WAVES = 16;
-constexpr int DR_RING = 8;                 // slots of four records that a wavefront keeps in LDS or on their way
+constexpr int DR_QUAD = 4;                 // records of a slot
+constexpr int DR_RING = 8;                 // slots that a wavefront keeps in LDS or on their way
 constexpr int DR_LDS = 2 * SP_TILE_BYTES + DR_WAVES * DR_RING * 256;
 constexpr int DR_THREADS = 256;
 constexpr int DR_MAX_TILES = 512;
 static_assert(DR_LDS <= 160 * 1024 && SP_ROWS / DR_REC <= 255, "record counts of a run are bytes");
 
 // An entry: where its tile row begins in LDS (tile buffer and row), and its value.  A run - one token's entries of one tile -
-// takes whole records; what is left of its last one repeats its last entry's place with value 0.
+// takes whole records; what is left of its last one repeats its last entry's place with value 0.  Four records of a stream lie
+// together, the four that an eighth of a wavefront needs next to each other: two 16-byte reads bring them in.  Streams begin at
+// whole quads.
+__device__ __forceinline__ uint64_t dr_entry(uint64_t record, uint32_t e) {
+  return record / DR_QUAD * (DR_QUAD * DR_REC) + e * DR_QUAD + record % DR_QUAD;
+}
 struct RowPlan { int tiles, groups, parts, groups_per_part, stages; };
 
 struct RunArgs {
@@ -35,7 +41,7 @@ struct RunArgs {
   int32_t *start;          // [L * groups][DR_TOK][tiles + 1] list position where a token's entries of a tile begin
   uint4 *counts;           // [groups][stages] records per token, a byte each
   uint32_t *offset;        // [groups][stages] records of the stage, then of the stream before it
-  uint32_t *total;         // [groups] records of the stream
+  uint32_t *total;         // [groups] records of the stream, in whole quads
   uint2 *recs;
 };
 
@@ -95,7 +101,7 @@ __global__ __launch_bounds__(64) void k_row_streams(RunArgs A) {
     if (st < A.p.stages) off[st] = run + incl - n;
     run += __shfl(incl, 63);
   }
-  if (lane == 0) A.total[blockIdx.x] = run;
+  if (lane == 0) A.total[blockIdx.x] = (run + DR_QUAD - 1) / DR_QUAD * DR_QUAD;
 }
 
 // One workgroup per (group, layer): every run into its records.
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
       dest[tk * tiles + c] = d;
       if (n % DR_REC != 0) {
         const uint32_t row = (uint32_t)(A.col[b + n - 1] - c * SP_ROWS);
-        for (int i = n; i % DR_REC != 0; ++i) A.recs[(uint64_t)d * DR_REC + i] = make_uint2((((stage0 + c) & 1u) << 16) | (row << 7), 0u);
+        for (int i = n; i % DR_REC != 0; ++i) A.recs[dr_entry((uint64_t)d + i / DR_REC, i % DR_REC)] = make_uint2((((stage0 + c) & 1u) << 16) | (row << 7), 0u);
       }
       d += (uint32_t)(n + DR_REC - 1) / DR_REC;
     }
@@ -129,7 +135,8 @@ __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
     const int32_t e = A.row_ptr[r0 + tk + 1];
     for (int32_t j = A.row_ptr[r0 + tk] + lane; j < e; j += 64) {
       const int32_t f = A.col[j], c = f / SP_ROWS;
-      A.recs[(uint64_t)dest[tk * tiles + c] * DR_REC + (j - start[tk * (tiles + 1) + c])] =
+      const uint32_t i = (uint32_t)(j - start[tk * (tiles + 1) + c]);
+      A.recs[dr_entry((uint64_t)dest[tk * tiles + c] + i / DR_REC, i % DR_REC)] =
           make_uint2((((stage0 + c) & 1u) << 16) | ((uint32_t)(f - c * SP_ROWS) << 7), __float_as_uint(A.val[j]));
     }
   }
@@ -148,6 +155,142 @@ struct RowArgs {
   uint64_t src_mask;
   int tying, t_begin, t_end, col_parts;
 };
+
+// ---- the records of one stage ---------------------------------------------------------------------------
+// What a wavefront does between two barriers: the records of its 16 tokens that refer to the tile in LDS.  A record is one 16-byte
+// read per lane (8 lanes a row, 8 rows) and four multiply-adds; the reads of the next two are under way while one is added.  In
+// assembly, like the stages of spmm.h and for its reasons: there is code for every token and place of a record in two quads.
+// Registers: v0 - v63 the sums (token k: v[4 k ..]), v64 - v79 four rows, v80 - v95 places and values of two quads of records, s[40:41]
+// the next quad to ask for.  Behind the stage's last record two more are read in vain (their tile may still be on its way, and
+// behind a stream's end they may be anything: a place is kept inside the tiles); the next stage begins by reading them again.
+// Nothing is on its way into a register when the block ends.
+typedef float dr_f32x32_t __attribute__((ext_vector_type(32)));
+typedef uint32_t dr_u32x16_t __attribute__((ext_vector_type(16)));
+
+#define DR_ROW(W, S) "v_and_or_b32 v96, " W ", %[inside], %[col]\n\tds_read_b128 v[" S "], v96\n\t"
+// At places 0 and 4 the next quad is read (seven were asked for since that one, and the four loads of a tile if that is less than
+// eight quads ago); two places later it has arrived, and its slot goes to the quad eight on.
+#define DR_RING_READ(T, P, LO, HI)                                                              \
+  "s_cmp_lt_i32 %[since], 8\n\t"                                                                \
+  "s_cbranch_scc1 .Ldr_v" #T "_" #P "_%=\n\t"                                                   \
+  "s_waitcnt vmcnt(7)\n"                                                                        \
+  ".Ldr_v" #T "_" #P "_%=:\n\t"                                                                 \
+  "s_waitcnt vmcnt(11)\n\t"                                                                     \
+  "v_add_u32 v97, %[slot], %[ring_lane]\n\t"                                                    \
+  "ds_read_b128 v[" LO "], v97\n\t"                                                             \
+  "ds_read_b128 v[" HI "], v97 offset:16\n\t"
+#define DR_RING_ASK                                                                             \
+  "s_add_i32 m0, %[ring], %[slot]\n\t"                                                          \
+  "s_add_i32 %[slot], %[slot], 0x100\n\t"                                                       \
+  "global_load_lds_dword %[rec_lane], s[40:41]\n\t"                                             \
+  "s_add_u32 s40, s40, 0x100\n\t"                                                               \
+  "s_addc_u32 s41, s41, 0\n\t"                                                                  \
+  "s_and_b32 %[slot], %[slot], 0x7ff\n\t"                                                       \
+  "s_add_i32 %[since], %[since], 1\n\t"
+#define DR_BOOKS_0(T) DR_RING_READ(T, 0, "88:91", "92:95")
+#define DR_BOOKS_1(T)
+#define DR_BOOKS_2(T) DR_RING_ASK
+#define DR_BOOKS_3(T)
+#define DR_BOOKS_4(T) DR_RING_READ(T, 4, "80:83", "84:87")
+#define DR_BOOKS_5(T)
+#define DR_BOOKS_6(T) DR_RING_ASK
+#define DR_BOOKS_7(T)
+// The record at place P of token T (sums A - D), and the one at place P + 2 with the word W, whose row goes to S; of the record's own
+// row R0 - R3 and value V; BEHIND: reads under way behind the row's.
+#define DR_CODE(T, A, B, C, D, P, N, W, S, V, R0, R1, R2, R3, BEHIND)                           \
+  ".Ldr_b" #T "_" #P "_%=:\n\t"                                                                 \
+  DR_BOOKS_##P(T) DR_ROW(W, S)                                                                  \
+  "s_waitcnt lgkmcnt(" BEHIND ")\n\t"                                                           \
+  "v_fmac_f32 " A ", " V ", " R0 "\n\t"                                                         \
+  "v_fmac_f32 " B ", " V ", " R1 "\n\t"                                                         \
+  "v_fmac_f32 " C ", " V ", " R2 "\n\t"                                                         \
+  "v_fmac_f32 " D ", " V ", " R3 "\n\t"                                                         \
+  "s_sub_u32 %[n], %[n], 1\n\t"                                                                 \
+  "s_cbranch_scc1 .Ldr_x" #T "_" #N "_%=\n"
+#define DR_TOKEN(T, A, B, C, D)                                                                 \
+  DR_CODE(T, A, B, C, D, 0, 1, "v84", "72:75", "v81", "v64", "v65", "v66", "v67", "4")          \
+  DR_CODE(T, A, B, C, D, 1, 2, "v86", "76:79", "v83", "v68", "v69", "v70", "v71", "2")          \
+  DR_CODE(T, A, B, C, D, 2, 3, "v88", "64:67", "v85", "v72", "v73", "v74", "v75", "2")          \
+  DR_CODE(T, A, B, C, D, 3, 4, "v90", "68:71", "v87", "v76", "v77", "v78", "v79", "2")          \
+  DR_CODE(T, A, B, C, D, 4, 5, "v92", "72:75", "v89", "v64", "v65", "v66", "v67", "4")          \
+  DR_CODE(T, A, B, C, D, 5, 6, "v94", "76:79", "v91", "v68", "v69", "v70", "v71", "2")          \
+  DR_CODE(T, A, B, C, D, 6, 7, "v80", "64:67", "v93", "v72", "v73", "v74", "v75", "2")          \
+  DR_CODE(T, A, B, C, D, 7, 0, "v82", "68:71", "v95", "v76", "v77", "v78", "v79", "2")          \
+  "s_branch .Ldr_b" #T "_0_%=\n"
+// behind token T, at place P: token N, whose number of records is COUNT (the subtraction borrows if there is none)
+#define DR_SWITCH(T, N, COUNT, P)                                                               \
+  ".Ldr_x" #T "_" #P "_%=:\n\t"                                                                 \
+  "s_bfe_u32 %[n], " COUNT "\n\t"                                                               \
+  "s_sub_u32 %[n], %[n], 1\n\t"                                                                 \
+  "s_cbranch_scc0 .Ldr_b" #N "_" #P "_%=\n\t"                                                   \
+  "s_branch .Ldr_x" #N "_" #P "_%=\n"
+#define DR_SWITCHES(T, N, COUNT)                                                                \
+  DR_SWITCH(T, N, COUNT, 0) DR_SWITCH(T, N, COUNT, 1) DR_SWITCH(T, N, COUNT, 2) DR_SWITCH(T, N, COUNT, 3) \
+  DR_SWITCH(T, N, COUNT, 4) DR_SWITCH(T, N, COUNT, 5) DR_SWITCH(T, N, COUNT, 6) DR_SWITCH(T, N, COUNT, 7)
+// four loads of the tile after this one, if there is one
+#define DR_FILL(L)                                                                              \
+  "s_mov_b32 %[since], 8\n\t"                                                                   \
+  "s_cmp_eq_i32 %[to], -1\n\t"                                                                  \
+  "s_cbranch_scc1 .Ldr_f" L "_%=\n\t"                                                           \
+  "s_mov_b32 m0, %[to]\n\t"                                                                     \
+  "s_mov_b32 %[since], 0\n\t"                                                                   \
+  "global_load_lds_dwordx4 %[off0], %[from]\n\t"                                                \
+  "s_add_i32 m0, %[to], 0x400\n\t"                                                              \
+  "s_nop 0\n\t"                                                                                 \
+  "global_load_lds_dwordx4 %[off1], %[from]\n\t"                                                \
+  "s_add_i32 m0, %[to], 0x800\n\t"                                                              \
+  "s_nop 0\n\t"                                                                                 \
+  "global_load_lds_dwordx4 %[off2], %[from]\n\t"                                                \
+  "s_add_i32 m0, %[to], 0xc00\n\t"                                                              \
+  "s_nop 0\n\t"                                                                                 \
+  "global_load_lds_dwordx4 %[off3], %[from]\n"                                                  \
+  ".Ldr_f" L "_%=:\n\t"
+// the stage's first two records, the first one at place P: their tile is there
+#define DR_ENTER(P, W0, S0, W1, S1)                                                             \
+  ".Ldr_e" #P "_%=:\n\t" DR_ROW(W0, S0) DR_ROW(W1, S1) DR_FILL(#P)                              \
+  "s_bfe_u32 %[n], %[c0], 0x80000\n\t"                                                          \
+  "s_sub_u32 %[n], %[n], 1\n\t"                                                                 \
+  "s_cbranch_scc0 .Ldr_b0_" #P "_%=\n\t"                                                        \
+  "s_branch .Ldr_x0_" #P "_%=\n"
+#define DR_LAST(P) ".Ldr_x15_" #P "_%=:\n"
+#define DR_STAGE                                                                                \
+  "s_or_b32 %[n], %[c0], %[c1]\n\ts_or_b32 %[n], %[n], %[c2]\n\ts_or_b32 %[n], %[n], %[c3]\n\t" \
+  "s_cmp_eq_u32 %[n], 0\n\ts_cbranch_scc1 .Ldr_none_%=\n\t"                                     \
+  "s_bitcmp1_b32 %[at], 2\n\ts_cbranch_scc1 .Ldr_eb_%=\n\t"                                     \
+  "s_bitcmp1_b32 %[at], 1\n\ts_cbranch_scc1 .Ldr_ea_%=\n\t"                                     \
+  "s_bitcmp1_b32 %[at], 0\n\ts_cbranch_scc1 .Ldr_e1_%=\n"                                       \
+  DR_ENTER(0, "v80", "64:67", "v82", "68:71") DR_ENTER(1, "v82", "68:71", "v84", "72:75")       \
+  ".Ldr_ea_%=:\n\ts_bitcmp1_b32 %[at], 0\n\ts_cbranch_scc1 .Ldr_e3_%=\n"                        \
+  DR_ENTER(2, "v84", "72:75", "v86", "76:79") DR_ENTER(3, "v86", "76:79", "v88", "64:67")       \
+  ".Ldr_eb_%=:\n\ts_bitcmp1_b32 %[at], 1\n\ts_cbranch_scc1 .Ldr_ec_%=\n\t"                      \
+  "s_bitcmp1_b32 %[at], 0\n\ts_cbranch_scc1 .Ldr_e5_%=\n"                                       \
+  DR_ENTER(4, "v88", "64:67", "v90", "68:71") DR_ENTER(5, "v90", "68:71", "v92", "72:75")       \
+  ".Ldr_ec_%=:\n\ts_bitcmp1_b32 %[at], 0\n\ts_cbranch_scc1 .Ldr_e7_%=\n"                        \
+  DR_ENTER(6, "v92", "72:75", "v94", "76:79") DR_ENTER(7, "v94", "76:79", "v80", "64:67")       \
+  DR_TOKEN(0, "v0", "v1", "v2", "v3") DR_SWITCHES(0, 1, "%[c0], 0x80008")                       \
+  DR_TOKEN(1, "v4", "v5", "v6", "v7") DR_SWITCHES(1, 2, "%[c0], 0x80010")                       \
+  DR_TOKEN(2, "v8", "v9", "v10", "v11") DR_SWITCHES(2, 3, "%[c0], 0x80018")                     \
+  DR_TOKEN(3, "v12", "v13", "v14", "v15") DR_SWITCHES(3, 4, "%[c1], 0x80000")                   \
+  DR_TOKEN(4, "v16", "v17", "v18", "v19") DR_SWITCHES(4, 5, "%[c1], 0x80008")                   \
+  DR_TOKEN(5, "v20", "v21", "v22", "v23") DR_SWITCHES(5, 6, "%[c1], 0x80010")                   \
+  DR_TOKEN(6, "v24", "v25", "v26", "v27") DR_SWITCHES(6, 7, "%[c1], 0x80018")                   \
+  DR_TOKEN(7, "v28", "v29", "v30", "v31") DR_SWITCHES(7, 8, "%[c2], 0x80000")                   \
+  DR_TOKEN(8, "v32", "v33", "v34", "v35") DR_SWITCHES(8, 9, "%[c2], 0x80008")                   \
+  DR_TOKEN(9, "v36", "v37", "v38", "v39") DR_SWITCHES(9, 10, "%[c2], 0x80010")                  \
+  DR_TOKEN(10, "v40", "v41", "v42", "v43") DR_SWITCHES(10, 11, "%[c2], 0x80018")                \
+  DR_TOKEN(11, "v44", "v45", "v46", "v47") DR_SWITCHES(11, 12, "%[c3], 0x80000")                \
+  DR_TOKEN(12, "v48", "v49", "v50", "v51") DR_SWITCHES(12, 13, "%[c3], 0x80008")                \
+  DR_TOKEN(13, "v52", "v53", "v54", "v55") DR_SWITCHES(13, 14, "%[c3], 0x80010")                \
+  DR_TOKEN(14, "v56", "v57", "v58", "v59") DR_SWITCHES(14, 15, "%[c3], 0x80018")                \
+  DR_TOKEN(15, "v60", "v61", "v62", "v63")                                                      \
+  ".Ldr_none_%=:\n\t" DR_FILL("n")                                                              \
+  DR_LAST(0) DR_LAST(1) DR_LAST(2) DR_LAST(3) DR_LAST(4) DR_LAST(5) DR_LAST(6) DR_LAST(7)       \
+  /* the tile's lines are waited for, not the quads asked for behind them; this wavefront's reads of the tile are over */ \
+  "s_cmp_ge_i32 %[since], 8\n\ts_cbranch_scc1 .Ldr_8_%=\n\t"                                    \
+  "s_cmp_ge_i32 %[since], 4\n\ts_cbranch_scc1 .Ldr_4_%=\n\t"                                    \
+  "s_waitcnt vmcnt(0)\n"                                                                        \
+  ".Ldr_4_%=:\n\ts_waitcnt vmcnt(4)\n"                                                          \
+  ".Ldr_8_%=:\n\ts_waitcnt vmcnt(8) lgkmcnt(0)"
 
 // Two tiles of 512 features x 32 columns in LDS, one being read while the other comes in.  A wavefront owns 16 tokens; a
 // record is one 16-byte read per lane (8 lanes a row, 8 rows) and four multiply-adds, its eight partial sums per column meet
@@ -171,70 +314,55 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
   const bool mine = wave < A.p.groups_per_part && g < A.p.groups;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)tile_lds;
 
-  // this wavefront's share of a tile: 32 rows, eight at a time, 16 bytes per lane
-  const uint32_t pitch_b = (uint32_t)(A.pitch * 4);
-  const int row_a = wave * 32 + (lane >> 3);
-  const uint32_t col_b = (uint32_t)(lane & 7) * 16;
-  auto fill = [&](const char *src, int rows, uint32_t lds_at) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = row_a + 8 * i;                         // past the matrix: nobody refers to these rows
-      sp_fill16(src, (uint32_t)(r < rows ? r : rows - 1) * pitch_b + col_b, lds_at + (uint32_t)i * 1024);
-    }
+  // this wavefront's share of a tile: 32 rows, eight at a time, 16 bytes per lane; rows past the matrix, which nobody refers to,
+  // are read as its last one
+  const uint32_t pitch_b = (uint32_t)(A.pitch * 4), col_b = (uint32_t)(lane & 7) * 16;
+  const uint32_t off_a = (uint32_t)(wave * 32 + (lane >> 3)) * pitch_b + col_b;
+  auto row_off = [&](int i, int rows) {
+    const uint32_t off = off_a + (uint32_t)i * 8 * pitch_b, last = (uint32_t)((rows < SP_ROWS ? rows : SP_ROWS) - 1) * pitch_b + 112u;
+    return off < last ? off : last;
   };
   auto tile_at = [&](int s) { return (const char *)A.wp + sp_slot(A.tying, s, t, A.L) * A.F * (int64_t)pitch_b + (int64_t)cp * 128; };
 
-  f32x4v_t acc[DR_TOK];
+  dr_f32x32_t lo, hi;                                      // tokens 0 - 7 and 8 - 15
 #pragma unroll
-  for (int i = 0; i < DR_TOK; ++i) acc[i] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
-
+  for (int i = 0; i < 32; ++i) { lo[i] = 0.f; hi[i] = 0.f; }
   if (n_stages > 0) {
     const uint32_t ring = lds0 + 2 * SP_TILE_BYTES + (uint32_t)wave * (DR_RING * 256);
-    const uint32_t *recs = (const uint32_t *)(A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(stream_first(A.total, mine ? g : 0, lane)) * DR_REC);
-    uint32_t rec_off = (uint32_t)lane * 4;                 // of the next slot to ask for, this lane's word
-    auto ask = [&](uint32_t at) {
-      sp_fill4(recs, rec_off, ring + at);
-      rec_off += 256;
+    const uint32_t rec_lane = (uint32_t)lane * 4, ring_lane = ring + (uint32_t)(lane >> 3) * 32, col_lane = lds0 + col_b;
+    const char *quad = (const char *)(A.recs + (uint64_t)__builtin_amdgcn_readfirstlane(stream_first(A.total, mine ? g : 0, lane)) * DR_REC);
+    auto ask = [&](uint32_t slot) {
+      sp_fill4((const uint32_t *)quad, rec_lane, ring + slot);
+      quad += 256;
     };
     uint64_t m = mask;
     int s = __ffsll((unsigned long long)m) - 1, c = 0, rows = (int)A.F;
     const char *tile = tile_at(s);
     const uint32_t lds_share = lds0 + (uint32_t)wave * 4096;
-    fill(tile, rows, lds_share);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sp_fill16(tile, row_off(i, rows), lds_share + (uint32_t)i * 1024);
 #pragma unroll
     for (int i = 0; i < DR_RING; ++i) ask((uint32_t)i * 256);
-    const auto counts = (const __attribute__((address_space(4))) uint4 *)(uintptr_t)A.counts + (int64_t)(mine ? g : 0) * A.p.stages;
+    const auto stream_counts = (const __attribute__((address_space(4))) uint4 *)(uintptr_t)A.counts + (int64_t)(mine ? g : 0) * A.p.stages;
     auto count_at = [&](int at) {
-      return mine ? make_uint4(counts[at].x, counts[at].y, counts[at].z, counts[at].w) : make_uint4(0u, 0u, 0u, 0u);
+      return mine ? make_uint4(stream_counts[at].x, stream_counts[at].y, stream_counts[at].z, stream_counts[at].w) : make_uint4(0u, 0u, 0u, 0u);
     };
     uint4 cnt = count_at(s * A.p.tiles);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-
-    uint32_t at = 0;                                       // of the next record to read, within the ring
-    int since = DR_RING;                                   // slots asked for since the last tile's lines
-    const uint32_t ring_lane = ring + (uint32_t)(lane >> 3) * 8, col_lane = lds0 + col_b;
-    auto next = [&](u32x2_t &r) {
-      r = *(__attribute__((address_space(3))) u32x2_t *)(uintptr_t)(ring_lane + at);
-      at = (at + 64) & (DR_RING * 256 - 1);
-      if ((at & 255) == 0) {
-        asm volatile("" ::"v"(r.x), "v"(r.y));             // the slot has been read
-        ask((at - 256) & (DR_RING * 256 - 1));
-        ++since;
-        // the slot after it: seven were asked for since, and perhaps the four loads of a tile
-        if (since < DR_RING) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-      }
-    };
-    // (what lies behind the stream's end may hold anything: the place is kept inside the tiles)
-    auto read = [&](const u32x2_t &r) {
-      return *(__attribute__((address_space(3))) f32x4v_t *)(uintptr_t)((r.x & 0x1FF80u) + col_lane);
-    };
-    u32x2_t r0, r1;                                        // the next two records
-    next(r0);
-    next(r1);
+    // the first quad's places and values: places 0 - 3 of eight; the next one's are read with the first record
+    dr_u32x16_t words;
+    {
+      const auto q = (const __attribute__((address_space(3))) u32x4_t *)(uintptr_t)ring_lane;
+      const u32x4_t a = q[0], b = q[1];
+      words = __builtin_shufflevector(__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7), __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7),
+                                      0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+      asm volatile("" ::"v"(words));                       // the slot has been read
+      ask(0);
+    }
+    uint32_t slot = 256, at = 0;                           // of the next quad to read; place of the next record
     for (int st = 0; st < n_stages; ++st) {
-      const bool more = st + 1 < n_stages;
-      if (more) {
+      uint32_t to = SP_NO_TILE;                            // where this wavefront's share of the next tile goes, if there is one
+      if (st + 1 < n_stages) {
         tile += SP_ROWS * pitch_b;
         rows -= SP_ROWS;
         if (++c == A.p.tiles) {
@@ -244,41 +372,32 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
           tile = tile_at(s);
           rows = (int)A.F;
         }
+        to = lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES;
       }
       const uint4 cnt_next = count_at(s * A.p.tiles + c);
-      asm volatile("" ::: "memory");
+      const uint32_t off0 = row_off(0, rows), off1 = row_off(1, rows), off2 = row_off(2, rows), off3 = row_off(3, rows);
+      asm volatile("" ::"v"(off0), "v"(off1), "v"(off2), "v"(off3) : "memory");
       __builtin_amdgcn_s_barrier();                        // tile st is complete, and nobody reads the other one any more
       asm volatile("" ::: "memory");
-      if (more) {
-        fill(tile, rows, lds_share ^ (uint32_t)((st & 1) ^ 1) * SP_TILE_BYTES);
-        since = 0;
-      } else since = DR_RING;
-      const uint32_t words[4] = {cnt.x, cnt.y, cnt.z, cnt.w};
-#pragma unroll
-      for (int tk = 0; tk < DR_TOK; ++tk) {
-        int n = (int)(words[tk >> 2] >> (8 * (tk & 3))) & 0xFF;
-        for (; n >= 2; n -= 2) {
-          const f32x4v_t w0 = read(r0), w1 = read(r1);
-          const float v0 = __uint_as_float(r0.y), v1 = __uint_as_float(r1.y);
-          next(r0);
-          next(r1);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[tk][q] = fmaf(v1, w1[q], fmaf(v0, w0[q], acc[tk][q]));
-        }
-        if (n > 0) {
-          const f32x4v_t w0 = read(r0);
-          const float v0 = __uint_as_float(r0.y);
-          r0 = r1;
-          next(r1);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[tk][q] = fmaf(v0, w0[q], acc[tk][q]);
-        }
-      }
+      uint32_t n, m0, since;
+      at = __builtin_amdgcn_readfirstlane(at);             // (uniform, which the compiler does not see everywhere)
+      slot = __builtin_amdgcn_readfirstlane(slot);
+      uint64_t next = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)(uintptr_t)quad >> 32)) << 32) |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint64_t)(uintptr_t)quad);
+      asm volatile(DR_STAGE
+                   : "+{v[0:31]}"(lo), "+{v[32:63]}"(hi), "+{v[80:95]}"(words), "+{s[40:41]}"(next), [slot] "+s"(slot), [since] "=&s"(since),
+                     [n] "=&s"(n), "=&{m0}"(m0)
+                   : [at] "s"(at), [c0] "s"(cnt.x), [c1] "s"(cnt.y), [c2] "s"(cnt.z), [c3] "s"(cnt.w), [ring] "s"(ring), [inside] "s"(0x1FF80u),
+                     [from] "s"(tile), [to] "s"(to), [off0] "v"(off0), [off1] "v"(off1), [off2] "v"(off2), [off3] "v"(off3), [col] "v"(col_lane),
+                     [ring_lane] "v"(ring_lane), [rec_lane] "v"(rec_lane)
+                   : "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v96", "v97",
+                     "scc", "memory");
+      quad = (const char *)(uintptr_t)next;
+      // the stage's records, a byte per token (at most 64 each)
+      const uint32_t even = (cnt.x & 0x00FF00FFu) + (cnt.y & 0x00FF00FFu) + (cnt.z & 0x00FF00FFu) + (cnt.w & 0x00FF00FFu);
+      const uint32_t odd = ((cnt.x >> 8) & 0x00FF00FFu) + ((cnt.y >> 8) & 0x00FF00FFu) + ((cnt.z >> 8) & 0x00FF00FFu) + ((cnt.w >> 8) & 0x00FF00FFu);
+      at += (even + odd) + ((even + odd) >> 16);           // (only its low three bits are looked at)
       cnt = cnt_next;
-      // the tile's lines are waited for, not the slots asked for behind them; this wavefront's reads of the tile are over
-      if (since >= DR_RING) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-      else if (since >= DR_RING / 2) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may be on its way into LDS when the workgroup ends
   }
@@ -304,7 +423,10 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
   uint32_t again = 0;                                      // tokens whose sums are not finite
 #pragma unroll
   for (int tk = 0; tk < DR_TOK; ++tk) {
-    const f32x4v_t a = meet(acc[tk]);
+    f32x4v_t sum;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] = tk < 8 ? lo[(tk & 7) * 4 + q] : hi[(tk & 7) * 4 + q];
+    const f32x4v_t a = meet(sum);
     const float z = fmaf(a[0], 0.0f, fmaf(a[1], 0.0f, fmaf(a[2], 0.0f, a[3] * 0.0f)));
     if (ballot64(z != z) != 0) again |= 1u << tk;
     else write(tk, a);
@@ -346,7 +468,8 @@ static RowLayout row_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t
   p.parts = (int)clt_ceil_div(p.groups, DR_WAVES);
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
   l.col_parts = (int)(d / DR_COLS);
-  // every run may leave its last record part empty, but no more runs than entries; a stream reads a ring past its end
+  // every run may leave its last record part empty, but no more runs than entries; every stream its last quad; and a stream reads
+  // a ring past its end
   const int64_t runs = (int64_t)p.stages * p.groups * DR_TOK;
   l.n_recs = entries / DR_REC + (runs < entries ? runs : entries) + (DR_RING + 2) * 4;
   size_t at = 0;
@@ -355,7 +478,7 @@ static RowLayout row_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t
   l.counts = take(sizeof(uint4) * (size_t)p.groups * p.stages);
   l.offset = take(sizeof(uint32_t) * (size_t)p.groups * p.stages);
   l.total = take(sizeof(uint32_t) * (size_t)p.groups);
-  l.recs = take((size_t)l.n_recs * DR_REC * sizeof(uint2));
+  l.recs = take((size_t)(l.n_recs + (int64_t)(DR_QUAD - 1) * p.groups) * DR_REC * sizeof(uint2));
   l.bytes = at;
   return l;
 }

@@ -506,11 +506,11 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
     const auto counts = (const __attribute__((address_space(4))) uint2 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages + stage0;
     const char *tile = (const char *)A.g + (int64_t)t * A.Tn * (int64_t)pitch_b + (int64_t)cp * 128;
     fill(tile, (int)A.Tn);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint2 cnt = make_uint2(counts->x, counts->y);
+    asm volatile("s_waitcnt vmcnt(0)" ::"s"(cnt.x), "s"(cnt.y) : "memory");
     batches.begun();
     int rows = (int)A.Tn;
     for (int st = 0; st < A.p.tiles; ++st) {
-      const uint2 cnt = make_uint2(counts[st].x, counts[st].y);
       if (st > 0) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();                      // nobody reads the last tile any more
@@ -518,9 +518,10 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
         tile += SP_ROWS * pitch_b;
         rows -= SP_ROWS;
         fill(tile, rows);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        cnt = make_uint2(counts[st].x, counts[st].y);      // (arrives before the tile does)
+        asm volatile("s_waitcnt vmcnt(0)" ::"s"(cnt.x), "s"(cnt.y) : "memory");
       }
-      asm volatile("" ::: "memory");
+      asm volatile("" ::"v"(batches.words) : "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       batches.stage<T>(acc, cnt, SpNoFill{});              // (there is one buffer: no tile comes in meanwhile)
