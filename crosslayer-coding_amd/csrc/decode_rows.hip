@@ -296,11 +296,12 @@ typedef uint32_t dr_u32x16_t __attribute__((ext_vector_type(16)));
 // record is one 16-byte read per lane (8 lanes a row, 8 rows) and four multiply-adds, its eight partial sums per column meet
 // at the end.  The records come through a ring as in k_decode_tiles.  Workgroups that share a tile follow each other on one XCD.
 //
-// L = 12, d = 768, F = 6144, 1024 tokens, 200 survivors per token, untied: 1.80 ms (49 GB of gathered rows, 27 TB/s) against
-// 2.33 ms of the gather from the L2s; 2.05 against 2.67 ms where tokens differ in their survivors (a stage waits for its
-// fullest wavefront).  Bound by what LDS returns: 5.7 ns per record and CU for 1 KB of rows and half as much of record.
-// Measured and dropped: the rows of the next record asked for ahead of the barrier (6.8 ns: register moves); four records in
-// one word per lane, handed out by DPP operands (7.6 ns: bound by instruction issue).
+// L = 12, d = 768, F = 6144, 1024 tokens, 200 survivors per token of which some have many more than others, untied: 1.44 ms (49 GB of
+// gathered rows, 34 TB/s) against 2.62 ms of the gather from the L2s; 1.97 ms in loops over a token's records with the books of the
+// ring in each step.  Bound by what LDS returns and by the number of a wavefront's instructions alike: 4.1 ns per record and CU for 1
+// KB of rows and half as much of records, 10 instructions.
+// Measured and dropped (in loops): the rows of the next record asked for ahead of the barrier (register moves); four records in one
+// word per lane, handed out by DPP operands (bound by instruction issue).
 __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
   extern __shared__ __attribute__((aligned(128))) char tile_lds[];
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -493,25 +494,27 @@ static bool row_shape_ok(const RowLayout &l, int64_t row_bytes) {
 
 struct RowTimes { double rows, sparse; };   // us; the first large for what the tiles do not take
 
-// Both routes priced from what they measured (L 4 - 16, d 256 - 2048, F 2048 - 16384, T 64 - 3000, 20 - 200 survivors per token):
-// the gather moves its rows at 23 TB/s and reads and writes two fp32 partial rows per (pair, token); a stage of the tiles takes
-// 1.4 us plus 5.7 ns per record, but no less than the 2.4 us in which 64 KB come into LDS, and the longest workgroup bounds a
-// launch of few.  us, gather / tiles: L = 12, d = 768, F = 6144, 1024 tokens: 667 / 941 with 20 per token, 1052 / 1045 with
-// 60, 2328 / 1798 with 200; L = 6, d = 1024, F = 16384, 3000 tokens x 200: 2599 / 2909; L = 16, d = 256, F = 2048, 1024 x 60:
-// 659 / 354.
+// Both routes priced from what they measured (28 shapes of L 2 - 16, d 256 - 2048, F 2048 - 16384, T 128 - 4096, 20 - 200 survivors per
+// token; the prices are off by 4 % (tiles) and 18 % (gather) in the mean, and the choice costs 2 % against the better of the two).  A
+// stage of the tiles takes 1.33 us plus 3.1 ns per record, but no less than the 1.9 us in which 64 KB come into LDS; workgroups of
+// unequal length end a third of the longest behind the mean, and the longest one bounds a launch of few.  us, tiles / gather: L = 12, d =
+// 768, F = 6144: 1469 / 2618 with 200 per token at T = 1024, 949 / 1198 with 60, 805 / 717 with 20; 647 / 1112 with 200 at 256; L =
+// 6, d = 1024, F = 16384: 2519 / 2796 at 3000 x 200, 2169 / 1704 at 3000 x 100; L = 16, d = 256, F = 2048, 1024 x 30: 234 / 565.
 static RowTimes row_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
   const RowTimes no = {1e30, 0};
   if (dtype != CLT_F32 || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;
   if (T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return no;
   const RowLayout l = row_layout(T, d, F, L, entries);
   if (!row_shape_ok(l, clt_pitch(d, 4) * 4)) return no;
-  const double pairs = 0.5 * targets * (2 * L - targets + 1), rows = (double)entries / L * pairs;
-  const double sparse_us = rows * d * 4 / 23e6 + pairs * T * d * 16 / 3.6e6;
+  const double pairs = 0.5 * targets * (2 * L - targets + 1);
   const double run = (double)entries / ((double)l.p.stages * T);
   const double recs = l.p.groups_per_part * DR_TOK * (run < run / DR_REC + 0.5 ? run : run / DR_REC + 0.5);
-  const double stage_us = 1.4 + recs * 0.0057;
+  const double stage_us = 1.33 + recs * 0.0031;
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
-  const double rows_us = (stages > longest ? stages : longest) * (stage_us > 2.4 ? stage_us : 2.4) + 20 + entries * 2e-5;
+  const double last = stages + 0.36 * longest > 1.26 * longest ? stages + 0.36 * longest : 1.26 * longest;
+  const double rows_us = last * (stage_us > 1.9 ? stage_us : 1.9) + 20 + entries * 2e-5;
+  const GatherPrice gather = {21.6e6, 6.5e6, 5.5e6, 5.9};
+  const double sparse_us = gather.us(T, d, F, L, targets, entries, tying, 4);
   return {rows_us, sparse_us};
 }
 
