@@ -267,7 +267,7 @@ class CrossLayerTranscoder(BaseTranscoder):
 
     def _loss_and_raw_gradients(self, inputs: Dict[int, torch.Tensor], targets: Dict[int, torch.Tensor],
                                 normalization_method: Optional[str] = None, mean_tg=None, std_tg=None,
-                                decoder_step=None):
+                                decoder_step=None, encoder_step=None):
         """(per-layer losses [L] fp32, raw gradients): ``enc_w`` [L, F, d], ``enc_b`` [L, F],
         ``dec_w`` [n_dec, F, d] (feature-major, decoders in slot order: "s->t" pairs, or one per source /
         per target for tied decoders), ``dec_b`` [n_dec, d] (bias gradient of each decoder); all fp32."""
@@ -301,10 +301,10 @@ class CrossLayerTranscoder(BaseTranscoder):
         tgt = torch.stack([targets[l].to(device=self.device, dtype=self.dtype).reshape(-1, d) for l in range(L)])
         mode, mean, std, scale = self._denorm_args(normalization_method, mean_tg, std_tg)
         loss_l, g, g_model, bias_grad = engine.mse_loss_grad(rec, tgt.contiguous(), ws, mode, mean, std, scale)
-        return loss_l, self._raw_gradients_from(inputs, surv, g, g_model, bias_grad, decoder_step)
+        return loss_l, self._raw_gradients_from(inputs, surv, g, g_model, bias_grad, decoder_step, encoder_step=encoder_step)
 
     def _raw_gradients_from(self, inputs: Dict[int, torch.Tensor], surv, g: torch.Tensor, g_model: torch.Tensor,
-                            bias_grad: torch.Tensor, decoder_step=None, as_parameters: bool = False):
+                            bias_grad: torch.Tensor, decoder_step=None, as_parameters: bool = False, encoder_step=None):
         """The raw parameter gradients (see ``_loss_and_raw_gradients``) of any loss, given d loss / d reconstruction:
         ``g`` fp32 [L, T, d], ``g_model`` the same in the model dtype, ``bias_grad`` [L, d] its sums over tokens.
         ``surv`` is the (trimmed) survivor list of the forward on ``inputs``.  ``as_parameters``: decoder gradients may come in their
@@ -339,7 +339,12 @@ class CrossLayerTranscoder(BaseTranscoder):
             dw_dec = engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
         _, x_slab, _, _ = self.encoder_module.prepare_slab(inputs)
         x_slab = x_slab.contiguous()
-        dw_enc, db_enc = engine.encoder_weight_grad(lists, dval, x_slab, F)
+        # ``encoder_step`` (an optimiser whose ``fuses_encoder_step(x)`` holds): likewise for the encoder weights, after everything
+        # that reads the old ones
+        encoder_step = encoder_step if encoder_step is not None and encoder_step.fuses_encoder_step(x_slab) else None
+        dw_enc = db_enc = None
+        if encoder_step is None:
+            dw_enc, db_enc = engine.encoder_weight_grad(lists, dval, x_slab, F)
         d_skip = None
         if dec.skip_weights is not None:
             # rec[t] += x[s] @ W_skip[s->t].T (untied, every pair) or x[t] @ W_skip[t].T (tied): dW = g[t].T @ x
@@ -350,6 +355,8 @@ class CrossLayerTranscoder(BaseTranscoder):
         theta_grad = None
         if cfg.activation_fn == "jumprelu" and self.theta_manager.log_threshold is not None:
             theta_grad = self._log_threshold_gradient(x_slab, g_model, ws, packed, surv, dval if sc is not None else None)
+        if encoder_step is not None:
+            db_enc = encoder_step.encoder_weight_step(lists, dval, x_slab)
         if decoder_step is not None:
             decoder_step.decoder_weight_step(lists, surv, g_model)
         # bias_grad[t] = column sums of d loss / d rec[t]; a decoder's bias takes the rows of the targets
@@ -560,7 +567,8 @@ class CrossLayerTranscoder(BaseTranscoder):
         De-normalisation arguments as in ``loss_and_gradients``."""
         self._no_half("training_step")
         fuse = optimizer if getattr(optimizer, "fuses_decoder_step", lambda: False)() else None
-        loss_l, raw = self._loss_and_raw_gradients(inputs, targets, normalization_method, mean_tg, std_tg, decoder_step=fuse)
+        loss_l, raw = self._loss_and_raw_gradients(inputs, targets, normalization_method, mean_tg, std_tg, decoder_step=fuse,
+                                                    encoder_step=optimizer if hasattr(optimizer, "fuses_encoder_step") else None)
         optimizer.step(raw)
         return loss_l.sum()
 

@@ -777,21 +777,22 @@ __global__ __launch_bounds__(FL_THREADS) void k_fl_fill(const int32_t *__restric
 // fits its L2, was measured and dropped: with four rows in flight per wavefront whole rows are 8 % faster.)
 constexpr int FO_NU = 8;
 // T8: as in k_bwd_values_sliced, the last piece of a lane is 8 bytes wide and every lane has one.
-// ADAM (untied decoders only): the row is not written; it is the gradient of an Adam step applied on the
-// spot to the moments [n_dec][F][d] and to the feature-major working copy [n_dec][F][pitch] of the decoder.
+// ADAM (untied decoders, encoders): the row is not written; it is the gradient of an Adam step applied on the
+// spot to the moments [n_dec][F][d] and to the feature-major working copy [n_dec][F][pitch] of the decoder, or to the moments and
+// weights [L][F][d] of the encoder.
 struct AdamInPlace {
   float *m, *v;      // moments, dense like the gradient would be
-  void *w_packed;    // the decoders' working copy
+  void *w_packed;    // the decoders' working copy, or the encoder weights
   int64_t pitch;
   AdamCoef c;
 };
+constexpr int FO_ADAM_PIECES = 4;          // of an encoder row that takes its Adam step in place: rows of 4 KB, whose moments fit the registers
 template <typename T, typename CoefT, int NCH, bool DECODER, bool T8 = false, bool ADAM = false>
 __global__ __launch_bounds__(BW_THREADS) void k_feature_outer(
     const int32_t *__restrict__ ptr, const int32_t *__restrict__ ltok, const int32_t *__restrict__ lsrc,
     const CoefT *__restrict__ coef, const T *__restrict__ src, float *__restrict__ out, float *__restrict__ rowsum,
     int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t target, int tying, const T *__restrict__ foff = nullptr,
     const T *__restrict__ fscale = nullptr, AdamInPlace ad = AdamInPlace()) {
-  static_assert(!ADAM || DECODER, "the in-place step is for decoder rows");
   constexpr int EV = Piece<T>::EV;
   const int lane = lane_id(), wv = threadIdx.x >> 6, nwv = blockDim.x >> 6;
   // One launch per layer of the gathered matrix, so that every wavefront of a launch gathers from the
@@ -824,12 +825,12 @@ __global__ __launch_bounds__(BW_THREADS) void k_feature_outer(
     typedef float bw_f4 __attribute__((ext_vector_type(4)));
     typedef uint32_t bw_u2 __attribute__((ext_vector_type(2)));
     typedef uint32_t bw_u4 __attribute__((ext_vector_type(4)));
-    constexpr int NG = ADAM ? NFULL * (EV / 4) + (T8 ? 1 : 0) : 1;
+    constexpr int NG = ADAM && DECODER ? NFULL * (EV / 4) + (T8 ? 1 : 0) : 1;
     bw_f4 am[NG], av[NG];
     typename std::conditional<sizeof(T) == 2, bw_u2, bw_u4>::type aw[NG];
     float *mrow = nullptr, *vrow = nullptr;
     T *wrow = nullptr;
-    if constexpr (ADAM) {
+    if constexpr (ADAM && DECODER) {
       const int64_t rowi = bw_decoder_slot(tying, s, t, L) * F + f;
       mrow = ad.m + rowi * d; vrow = ad.v + rowi * d;
       wrow = reinterpret_cast<T *>(ad.w_packed) + rowi * ad.pitch;
@@ -898,6 +899,72 @@ __global__ __launch_bounds__(BW_THREADS) void k_feature_outer(
     }
     }
     const int64_t q = s * F + f;
+    if constexpr (ADAM && !DECODER) {
+      // The row goes through LDS, so that the streams of the step are whole lines: four elements next to each other per lane and load,
+      // where the eight of a gathered piece would take half lines twice (that way, asked for before the gather or behind it: 2.0 - 2.5
+      // TB/s).  A layer, gradient and k_adam_vec -> this: T = 1500, d = 1024, F = 16384, 3 entries per feature 24 + 81 -> 62 us (5.4
+      // TB/s); T = 4096, d = 768, F = 24576, 33 entries 118 + 84 -> 180 us, bound by the lines an L1 has on their way, of
+      // which the gather takes 2 in 3; float32, T = 1024, d = 768, F = 6144 39 + 22 -> 59.
+      constexpr int NQ = T8 ? (NFULL * EV + HV) / 4 : NCH * EV / 4;
+      __shared__ __attribute__((aligned(16))) float rows[BW_THREADS / 64][NQ * 256];
+      float *const mine = rows[wv];
+      float *const m_at = ad.m + q * d, *const v_at = ad.v + q * d;
+      T *const w_at = reinterpret_cast<T *>(ad.w_packed) + q * d;
+      typedef typename std::conditional<sizeof(T) == 2, bw_u2, bw_u4>::type raw4;
+      bw_f4 mm[NQ], vv[NQ];
+      raw4 ww[NQ];
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int64_t at = i * 256 + lane * 4;
+        if (at < d) {
+          mm[i] = __builtin_nontemporal_load(reinterpret_cast<const bw_f4 *>(m_at + at));
+          vv[i] = __builtin_nontemporal_load(reinterpret_cast<const bw_f4 *>(v_at + at));
+          ww[i] = __builtin_nontemporal_load(reinterpret_cast<const raw4 *>(w_at + at));
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < NFULL; ++c)
+#pragma unroll
+        for (int k = 0; k < EV; k += 4)
+          *reinterpret_cast<float4 *>(mine + c * 64 * EV + lane * EV + k) = make_float4(acc[c][k], acc[c][k + 1], acc[c][k + 2], acc[c][k + 3]);
+      if constexpr (T8)
+        *reinterpret_cast<float4 *>(mine + tail_at) = make_float4(acc[NFULL][0], acc[NFULL][1], acc[NFULL][2], acc[NFULL][3]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) {
+        const int64_t at = i * 256 + lane * 4;
+        const float4 g4 = *reinterpret_cast<const float4 *>(mine + at);
+        const float gk[4] = {g4.x, g4.y, g4.z, g4.w};
+        float p[4];
+        if constexpr (sizeof(T) == 2) {
+          unpack_pair<T>(ww[i][0], p[0], p[1]);
+          unpack_pair<T>(ww[i][1], p[2], p[3]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) p[k] = __uint_as_float(ww[i][k]);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float m1 = mm[i][k], v1 = vv[i][k];
+          p[k] = adam_update(p[k], gk[k], m1, v1, ad.c);
+          mm[i][k] = m1;
+          vv[i][k] = v1;
+        }
+        if (at < d) {
+          __builtin_nontemporal_store(mm[i], reinterpret_cast<bw_f4 *>(m_at + at));
+          __builtin_nontemporal_store(vv[i], reinterpret_cast<bw_f4 *>(v_at + at));
+          if constexpr (sizeof(T) == 2) {
+            const bw_u2 o = {pack_pair<T>(p[0], p[1]), pack_pair<T>(p[2], p[3])};
+            *reinterpret_cast<bw_u2 *>(w_at + at) = o;
+          } else {
+            *reinterpret_cast<float4 *>(w_at + at) = make_float4(p[0], p[1], p[2], p[3]);
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read before the next row is written
+      if (rowsum && lane == 0) rowsum[q] = csum;
+      continue;
+    }
     if constexpr (ADAM) {
       // groups of four elements, as they were asked for ahead of the gather
       auto step4 = [&](int gi, int64_t at, const float *gk) {
@@ -1387,6 +1454,38 @@ extern "C" int clt_encoder_weight_grad(const int32_t *list_ptr, const int32_t *l
   else CLT_EW(float, 16);
 #undef CLT_EW_N
 #undef CLT_EW
+  return clt_check_launch();
+}
+
+extern "C" int clt_encoder_weight_grad_adam(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src,
+                                            const float *dval, const void *x, void *w_enc, float *m, float *v, float *db_enc,
+                                            int64_t T, int64_t d, int64_t F, int64_t L, double lr, double beta1, double beta2,
+                                            double eps, int64_t step, int dtype, void *stream) {
+  if (dtype != CLT_F32 && dtype != CLT_BF16) return CLT_ERR_DTYPE;
+  if (T <= 0 || F <= 0 || L <= 0 || L > 65535 || step < 1 || !(beta1 >= 0 && beta1 < 1) || !(beta2 >= 0 && beta2 < 1) || !list_ptr ||
+      !list_tok || !list_src || !dval || !x || !w_enc || !m || !v)
+    return CLT_ERR_ARG;
+  const int esz = dtype == CLT_BF16 ? 2 : 4, ev = 16 / esz;
+  const int nc4 = (int)clt_ceil_div(d / ev, 64);   // 16-byte pieces per lane
+  if (!bw_shape_ok(d, dtype) || nc4 > FO_ADAM_PIECES) return CLT_ERR_RANGE;
+  if (!clt_aligned16(x) || !clt_aligned16(w_enc) || !clt_aligned16(m) || !clt_aligned16(v)) return CLT_ERR_ALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  AdamInPlace ad;
+  ad.m = m; ad.v = v; ad.w_packed = w_enc; ad.pitch = d; ad.c = adam_coef(lr, beta1, beta2, eps, step);
+#define CLT_EWA(ST, N, T8)                                                                                                 \
+  for (int64_t l = 0; l < L; ++l)                                                                                          \
+  k_feature_outer<ST, float, N, false, T8, true><<<bw_resident_blocks(k_feature_outer<ST, float, N, false, T8, true>), BW_THREADS, 0, s>>>( \
+      list_ptr, list_tok, list_src, dval, (const ST *)x, nullptr, db_enc, T, d, F, L, l, CLT_TYING_NONE, nullptr, nullptr, ad)
+#define CLT_EWA_N(ST)                                                                                \
+  switch (nc4) {                                                                                     \
+    case 1: CLT_EWA(ST, 1, false); break; case 2: CLT_EWA(ST, 2, false); break;                      \
+    case 3: CLT_EWA(ST, 3, false); break; default: CLT_EWA(ST, 4, false); break;                     \
+  }
+  if (dtype == CLT_BF16 && d == 768) CLT_EWA(bf16_t, 2, true);
+  else if (dtype == CLT_BF16) { CLT_EWA_N(bf16_t) }
+  else { CLT_EWA_N(float) }
+#undef CLT_EWA_N
+#undef CLT_EWA
   return clt_check_launch();
 }
 

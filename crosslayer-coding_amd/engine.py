@@ -892,6 +892,28 @@ def encoder_weight_grad(lists, dval: torch.Tensor, x: torch.Tensor, F: int):
     return dw, db
 
 
+def encoder_step_fits(d: int, dtype: torch.dtype) -> bool:
+    """Whether ``encoder_weight_grad_adam`` takes encoder rows of ``d`` elements."""
+    return d % (8 if dtype == torch.bfloat16 else 4) == 0 and d * dtype.itemsize <= 4096 and dtype in (torch.bfloat16, torch.float32)
+
+
+def encoder_weight_grad_adam(lists, dval: torch.Tensor, x: torch.Tensor, w: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
+                             lr: float, betas, eps: float, step: int) -> torch.Tensor:
+    """``encoder_weight_grad`` with the Adam step ``step`` of the stacked weights ``w`` and their moments [L, F, d] taken on the
+    spot (bit-identical to the two calls); returns the bias gradients, fp32 [L, F]."""
+    ptr, tok, src = lists
+    L, T, d = x.shape
+    F = w.shape[1]
+    assert x.is_contiguous() and w.is_contiguous() and w.dtype == x.dtype and tuple(w.shape) == (L, F, d) and dval.dtype == torch.float32
+    assert m.shape == w.shape and v.shape == w.shape and m.dtype == v.dtype == torch.float32 and m.is_contiguous() and v.is_contiguous()
+    db = torch.empty((L, F), dtype=torch.float32, device=x.device)
+    code = nat.load().clt_encoder_weight_grad_adam(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(dval), nat.ptr(x), nat.ptr(w),
+                                                   nat.ptr(m), nat.ptr(v), nat.ptr(db), T, d, F, L, lr, betas[0], betas[1], eps, step,
+                                                   nat.dtype_code(x.dtype), _stream(x))
+    nat.check(code, "clt_encoder_weight_grad_adam")
+    return db
+
+
 def parameter_gradient(g: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """A raw fp32 gradient in the parameter's dtype and layout.  A transposed view (a decoder's [F, d] rows seen as [d, F]) is
     written out in one pass: autograd would otherwise keep its strides in the cast and copy it once more, element by element."""

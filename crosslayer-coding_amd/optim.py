@@ -24,7 +24,8 @@ class CLTAdam:
         self.lr, self.betas, self.eps = float(lr), (float(betas[0]), float(betas[1])), float(eps)
         self.step_count = 0
         self.fuse_decoder_step = True    # untied decoders: Adam inside the weight-gradient kernel (training_step)
-        # ... over column tiles, when the shape allows: float32 and widths that are not whole tiles of 64 take that kernel
+        self.fuse_encoder_step = True    # the same for the encoder weights, whatever the decoders' tying
+        # Decoder step over column tiles, when the shape allows: float32 and widths that are not whole tiles of 64 take that kernel
         # (moments and a weight copy tiled) or go row by row; for bf16 in whole tiles of 64 columns, which the matrix-core
         # kernel takes either way, only what the moments are laid out as
         self.tile_decoder_step = True
@@ -79,6 +80,22 @@ class CLTAdam:
         dec = self.model.decoder_module
         return (self.fuse_decoder_step and self.model.config.decoder_tying == "none"
                 and dec.feature_offset is None and dec.feature_scale is None)
+
+    def fuses_encoder_step(self, x: torch.Tensor) -> bool:
+        """Whether the encoder weights can take their Adam step inside the weight-gradient kernel, for the batch ``x`` [L, T, d]
+        (``fuse_encoder_step = False`` switches it off)."""
+        from . import engine
+        w, _ = self.model.encoder_module.stacked()
+        return (self.fuse_encoder_step and w.dtype == x.dtype and engine.encoder_step_fits(x.shape[2], x.dtype)
+                and engine._aligned16(x, w, *self.state["enc_w"]))
+
+    @torch.no_grad()
+    def encoder_weight_step(self, lists, dval: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+        """The encoder weights' part of the NEXT ``step`` (which must follow with ``raw["enc_w"] = None``); returns the bias
+        gradients.  Bit-identical to gradient-then-Adam."""
+        from . import engine
+        w, _ = self.model.encoder_module.stacked()
+        return engine.encoder_weight_grad_adam(lists, dval, x, w, *self.state["enc_w"], self.lr, self.betas, self.eps, self.step_count + 1)
 
     def _decoder_moments_to(self, layout: str, cols: int = 0) -> None:
         """Regroup both decoder moments: "rows" [n_dec, F, d] <-> "tiles" [n_dec, d // cols, F, cols].  Happens when the
@@ -172,11 +189,12 @@ class CLTAdam:
     @torch.no_grad()
     def step(self, raw) -> None:
         """``raw``: the gradient tensors of ``CrossLayerTranscoder._loss_and_raw_gradients``; ``dec_w`` is None
-        when ``decoder_weight_step`` has already applied it."""
+        when ``decoder_weight_step`` has already applied it, ``enc_w`` when ``encoder_weight_step`` has."""
         model = self.model
         self.step_count += 1
         w_slab, b_slab = model.encoder_module.stacked()
-        self._adam(w_slab, raw["enc_w"], *self.state["enc_w"])
+        if raw["enc_w"] is not None:
+            self._adam(w_slab, raw["enc_w"], *self.state["enc_w"])
         self._adam(b_slab, raw["enc_b"], *self.state["enc_b"])
         dec = model.decoder_module
         packed = dec.packed()

@@ -610,6 +610,9 @@ int clt_decoder_norms(const void *w_packed, void *norms, int64_t d, int64_t F,
  *   out [d][d] fp32, accumulate != 0 adds to out.
  * clt_encoder_weight_grad: dw_enc[s][f][:] = sum over the list of dval * x[s][token][:],
  *   db_enc[s][f] = sum of dval (fp32; x [L][T][d] in the model dtype).
+ * clt_encoder_weight_grad_adam: the same with the Adam step of the weights in the place of dw_enc (trainer.py:663-778): moments m, v
+ *   and weights w_enc [L][F][d] are updated in place, bit for bit as clt_adam_step does with that gradient; db_enc is written.
+ *   Rows of at most 4 KB.  Everything that reads the old encoder weights must have been launched before.
  * Limits: d % 8 == 0 (bf16) / d % 4 == 0 (fp32) and d <= 4096.
  */
 size_t clt_mse_workspace_bytes(int64_t T, int64_t d, int64_t L);
@@ -641,6 +644,10 @@ int clt_decoder_weight_grad(const int32_t *list_ptr, const int32_t *list_tok, co
 int clt_encoder_weight_grad(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src,
                             const float *dval, const void *x, float *dw_enc, float *db_enc,
                             int64_t T, int64_t d, int64_t F, int64_t L, int dtype, void *stream);
+int clt_encoder_weight_grad_adam(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src,
+                                 const float *dval, const void *x, void *w_enc, float *m, float *v, float *db_enc,
+                                 int64_t T, int64_t d, int64_t F, int64_t L, double lr, double beta1, double beta2,
+                                 double eps, int64_t step, int dtype, void *stream);
 
 /*
  * Adam update with fp32 moments and fp32 gradients on parameters in the model dtype
