@@ -100,6 +100,11 @@ _SIGNATURES = {
     "clt_decoder_fingerprint": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp, _int, _vp]),
     "clt_pack_decoders_if": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "clt_bias_sum": (_int, [_vp, _i64, _i64, _i64, _int, _u64, _int, _vp, _vp]),
+    "clt_grad_rows_supported": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
+    "clt_grad_rows_wanted": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
+    "clt_grad_rows_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
+    "clt_decoder_grad_adam_rows": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _f64, _f64, _f64,
+                                          _f64, _i64, _vp, _sz, _vp]),
     "clt_grad_tiles_supported": (_int, [_i64, _i64, _i64, _i64, _i64, _int]),
     "clt_grad_tiles_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "clt_decoder_grad_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),

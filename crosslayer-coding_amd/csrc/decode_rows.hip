@@ -6,6 +6,9 @@
 //                   k_decode_rows consumes them: by source, tile of SP_ROWS features, token
 //   k_decode_rows   one workgroup per (target, 32 columns, part of the tokens): every tile of every source's decoder passes
 //                   through LDS once, the sums stay in registers over all sources and features
+//   k_grad_rows     the transposed product of the backward pass: decoder weight gradients from the same lists by feature,
+//                   with the Adam step of the weights taken on the spot
+#include "adam.h"
 #include "spmm.h"
 
 namespace {
@@ -30,18 +33,24 @@ static_assert(DR_LDS <= 160 * 1024 && SP_ROWS / DR_REC <= 255, "record counts of
 __device__ __forceinline__ uint64_t dr_entry(uint64_t record, uint32_t e) {
   return record / DR_QUAD * (DR_QUAD * DR_REC) + e * DR_QUAD + record % DR_QUAD;
 }
-struct RowPlan { int tiles, groups, parts, groups_per_part, stages; };
+// A stream is a group's, over all layers - or, `by_layer`, a group's of one layer (number layer * groups + group).
+struct RowPlan {
+  int tiles, groups, parts, groups_per_part, stages, by_layer;        // stages: of a stream
+  __device__ __forceinline__ int stream(int g, int s) const { return by_layer ? s * groups + g : g; }
+  __device__ __forceinline__ int stage(int s, int c) const { return by_layer ? c : s * tiles + c; }
+};
 
 struct RunArgs {
   const int32_t *row_ptr, *col;
+  const int32_t *src;      // the entry's value is val[src[j]]; null: val[j]
   const float *val;
   int64_t Tn, L;
   uint64_t layer_mask;
   RowPlan p;
   int32_t *start;          // [L * groups][DR_TOK][tiles + 1] list position where a token's entries of a tile begin
-  uint4 *counts;           // [groups][stages] records per token, a byte each
-  uint32_t *offset;        // [groups][stages] records of the stage, then of the stream before it
-  uint32_t *total;         // [groups] records of the stream, in whole quads
+  uint4 *counts;           // [streams][stages] records per token, a byte each
+  uint32_t *offset;        // [streams][stages] records of the stage, then of the stream before it
+  uint32_t *total;         // [streams] records of the stream, in whole quads; by_layer: of the streams before it (k_row_firsts)
   uint2 *recs;
 };
 
@@ -78,7 +87,7 @@ __global__ __launch_bounds__(DR_THREADS) void k_row_runs(RunArgs A) {
       w[tk >> 2] |= n << (8 * (tk & 3));
       sum += n;
     }
-    const int64_t at = (int64_t)g * A.p.stages + (int64_t)s * tiles + c;
+    const int64_t at = (int64_t)A.p.stream(g, s) * A.p.stages + A.p.stage(s, c);
     A.counts[at] = make_uint4(w[0], w[1], w[2], w[3]);
     A.offset[at] = sum;
   }
@@ -104,6 +113,34 @@ __global__ __launch_bounds__(64) void k_row_streams(RunArgs A) {
   if (lane == 0) A.total[blockIdx.x] = (run + DR_QUAD - 1) / DR_QUAD * DR_QUAD;
 }
 
+// Many streams: their totals become first records, by one workgroup.
+constexpr int DR_FIRSTS = 1024;
+__global__ __launch_bounds__(DR_FIRSTS) void k_row_firsts(uint32_t *total, int streams) {
+  __shared__ uint32_t sums[DR_FIRSTS / 64];
+  const int lane = lane_id(), wave = threadIdx.x >> 6;
+  uint32_t before = 0;
+  for (int i0 = 0; i0 < streams; i0 += DR_FIRSTS) {
+    const int i = i0 + threadIdx.x;
+    const uint32_t n = i < streams ? total[i] : 0u;
+    uint32_t incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t up = __shfl_up(incl, o);
+      if (lane >= o) incl += up;
+    }
+    if (lane == 63) sums[wave] = incl;
+    __syncthreads();
+    uint32_t mine = before, all = 0;
+    for (int w = 0; w < DR_FIRSTS / 64; ++w) {
+      mine += w < wave ? sums[w] : 0u;
+      all += sums[w];
+    }
+    if (i < streams) total[i] = mine + incl - n;
+    before += all;
+    __syncthreads();
+  }
+}
+
 // One workgroup per (group, layer): every run into its records.
 __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
   extern __shared__ int32_t fill_lds[];
@@ -114,11 +151,12 @@ __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
   const int64_t tok0 = (int64_t)g * DR_TOK, r0 = (int64_t)s * A.Tn + tok0;
   const int32_t *src = A.start + ((int64_t)s * A.p.groups + g) * DR_TOK * (tiles + 1);
   for (int i = tid; i < DR_TOK * (tiles + 1); i += DR_THREADS) start[i] = src[i];
-  const uint32_t base = stream_first(A.total, g, lane);
+  const int stream = A.p.stream(g, s);
+  const uint32_t base = A.p.by_layer ? A.total[stream] : stream_first(A.total, g, lane);
   const uint32_t stage0 = (uint32_t)(__popcll(A.layer_mask & ((1ull << s) - 1ull)) * tiles);
   __syncthreads();
   for (int c = tid; c < tiles; c += DR_THREADS) {
-    uint32_t d = base + A.offset[(int64_t)g * A.p.stages + (int64_t)s * tiles + c];
+    uint32_t d = base + A.offset[(int64_t)stream * A.p.stages + A.p.stage(s, c)];
     for (int tk = 0; tk < DR_TOK; ++tk) {
       const int32_t b = start[tk * (tiles + 1) + c], n = start[tk * (tiles + 1) + c + 1] - b;
       dest[tk * tiles + c] = d;
@@ -137,7 +175,7 @@ __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
       const int32_t f = A.col[j], c = f / SP_ROWS;
       const uint32_t i = (uint32_t)(j - start[tk * (tiles + 1) + c]);
       A.recs[dr_entry((uint64_t)dest[tk * tiles + c] + i / DR_REC, i % DR_REC)] =
-          make_uint2((((stage0 + c) & 1u) << 16) | ((uint32_t)(f - c * SP_ROWS) << 7), __float_as_uint(A.val[j]));
+          make_uint2((((stage0 + c) & 1u) << 16) | ((uint32_t)(f - c * SP_ROWS) << 7), __float_as_uint(A.val[A.src ? A.src[j] : j]));
     }
   }
 }
@@ -292,6 +330,16 @@ typedef uint32_t dr_u32x16_t __attribute__((ext_vector_type(16)));
   ".Ldr_4_%=:\n\ts_waitcnt vmcnt(4)\n"                                                          \
   ".Ldr_8_%=:\n\ts_waitcnt vmcnt(8) lgkmcnt(0)"
 
+#define DR_STAGE_ASM(INSIDE, TILE, TO, OFF0, OFF1, OFF2, OFF3)                                                                       \
+  asm volatile(DR_STAGE                                                                                                            \
+               : "+{v[0:31]}"(lo), "+{v[32:63]}"(hi), "+{v[80:95]}"(words), "+{s[40:41]}"(next), [slot] "+s"(slot), [since] "=&s"(since), \
+                 [n] "=&s"(n), "=&{m0}"(m0)                                                                                        \
+               : [at] "s"(at), [c0] "s"(cnt.x), [c1] "s"(cnt.y), [c2] "s"(cnt.z), [c3] "s"(cnt.w), [ring] "s"(ring), [inside] "s"(INSIDE), \
+                 [from] "s"(TILE), [to] "s"(TO), [off0] "v"(OFF0), [off1] "v"(OFF1), [off2] "v"(OFF2), [off3] "v"(OFF3), [col] "v"(col_lane), \
+                 [ring_lane] "v"(ring_lane), [rec_lane] "v"(rec_lane)                                                              \
+               : "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v96", "v97", \
+                 "scc", "memory")
+
 // Two tiles of 512 features x 32 columns in LDS, one being read while the other comes in.  A wavefront owns 16 tokens; a
 // record is one 16-byte read per lane (8 lanes a row, 8 rows) and four multiply-adds, its eight partial sums per column meet
 // at the end.  The records come through a ring as in k_decode_tiles.  Workgroups that share a tile follow each other on one XCD.
@@ -385,14 +433,7 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
       slot = __builtin_amdgcn_readfirstlane(slot);
       uint64_t next = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)(uintptr_t)quad >> 32)) << 32) |
                       (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint64_t)(uintptr_t)quad);
-      asm volatile(DR_STAGE
-                   : "+{v[0:31]}"(lo), "+{v[32:63]}"(hi), "+{v[80:95]}"(words), "+{s[40:41]}"(next), [slot] "+s"(slot), [since] "=&s"(since),
-                     [n] "=&s"(n), "=&{m0}"(m0)
-                   : [at] "s"(at), [c0] "s"(cnt.x), [c1] "s"(cnt.y), [c2] "s"(cnt.z), [c3] "s"(cnt.w), [ring] "s"(ring), [inside] "s"(0x1FF80u),
-                     [from] "s"(tile), [to] "s"(to), [off0] "v"(off0), [off1] "v"(off1), [off2] "v"(off2), [off3] "v"(off3), [col] "v"(col_lane),
-                     [ring_lane] "v"(ring_lane), [rec_lane] "v"(rec_lane)
-                   : "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "v96", "v97",
-                     "scc", "memory");
+      DR_STAGE_ASM(0x1FF80u, tile, to, off0, off1, off2, off3);
       quad = (const char *)(uintptr_t)next;
       // the stage's records, a byte per token (at most 64 each)
       const uint32_t even = (cnt.x & 0x00FF00FFu) + (cnt.y & 0x00FF00FFu) + (cnt.z & 0x00FF00FFu) + (cnt.w & 0x00FF00FFu);
@@ -451,6 +492,183 @@ __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
   }
 }
 
+// ---- decoder weight gradient and Adam -------------------------------------------------------------------
+// dW[s->t][f][:] = sum over the tokens of feature f of value * g[t][token][:]: the same sums with features in the place of tokens
+// - 16 features per wavefront, tiles of 512 tokens x 32 columns of g[t].
+constexpr int GR_WAVES = 8;
+constexpr int GR_LDS = SP_TILE_BYTES + GR_WAVES * DR_RING * 256;
+static_assert(GR_LDS * 2 <= 160 * 1024, "two workgroups per CU");
+
+struct GradRowArgs {
+  RowPlan p;
+  const uint4 *counts;
+  const uint32_t *first;
+  const uint2 *recs;
+  const float *g;            // [L][T][d]
+  float *w, *m, *v;          // packed decoders, moments
+  const int32_t *list_ptr, *list_tok, *list_src;
+  const float *val;
+  int64_t Tn, d, F, L, pitch;
+  int64_t m_row, m_cols;     // moments: elements between rows and between column parts of eight
+  int col_parts, items;      // items of one (source, target) pair per XCD
+  AdamCoef adam;
+};
+
+// One workgroup per (source, target, 32 columns, 128 features).  Weights and moments stream through once (24 bytes per weight), in
+// lines of 128 bytes: two workgroups share a CU (one tile buffer each), and one's sums run under the other's streaming.
+//
+// L = 12, d = 768, F = 6144, 1024 tokens, 200 survivors per token: 2.55 ms (8.8 GB of weights and moments, 3.4 TB/s), against 3.39 ms of 32-byte
+// tiles and 0.57 ms for bringing those back into the slab; the training step 9.95 -> 8.76 ms.  Without entries 2.2 ms: what bounds it
+// is the chain of a workgroup, tile, sums, tile, sums, moments, of which a CU has two under way.
+__global__ __launch_bounds__(GR_WAVES * 64, 4) void k_grad_rows(GradRowArgs A) {
+  extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
+  const int slot_dec = seq / A.items, item = xcd * A.items + seq % A.items;
+  if (item >= A.p.parts * A.col_parts) return;
+  const int part = item / A.col_parts, cp = item % A.col_parts;
+  int s = 0, t = slot_dec;                                 // decoder "0->0", "0->1", ..: source s, target t
+  while (t >= (int)A.L - s) { t -= (int)A.L - s; ++s; }
+  t += s;
+  const int g = part * GR_WAVES + wave;
+  const bool mine = g < A.p.groups;
+  const int stream = s * A.p.groups + (mine ? g : 0);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)tile_lds;
+
+  // this wavefront's share of a tile: 64 rows, eight at a time, 16 bytes per lane; rows past the batch are read as its last one
+  const uint32_t pitch_b = (uint32_t)(A.d * 4), col_b = (uint32_t)(lane & 7) * 16;
+  const char *tile = (const char *)A.g + (int64_t)t * A.Tn * (int64_t)pitch_b + (int64_t)cp * 128;
+  auto fill = [&](int rows) {
+    const uint32_t last = (uint32_t)((rows < SP_ROWS ? rows : SP_ROWS) - 1);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t row = (uint32_t)(wave * 64 + i * 8 + (lane >> 3));
+      sp_fill16(tile, (row < last ? row : last) * pitch_b + col_b, lds0 + (uint32_t)(wave * 8192 + i * 1024));
+    }
+  };
+
+  dr_f32x32_t lo, hi;                                      // features 0 - 7 and 8 - 15
+#pragma unroll
+  for (int i = 0; i < 32; ++i) { lo[i] = 0.f; hi[i] = 0.f; }
+  {
+    const uint32_t ring = lds0 + SP_TILE_BYTES + (uint32_t)wave * (DR_RING * 256);
+    const uint32_t rec_lane = (uint32_t)lane * 4, ring_lane = ring + (uint32_t)(lane >> 3) * 32, col_lane = lds0 + col_b;
+    const char *quad = (const char *)(A.recs + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)A.first[stream]) * DR_REC);
+    auto ask = [&](uint32_t slot) {
+      sp_fill4((const uint32_t *)quad, rec_lane, ring + slot);
+      quad += 256;
+    };
+    int rows = (int)A.Tn;
+    fill(rows);
+#pragma unroll
+    for (int i = 0; i < DR_RING; ++i) ask((uint32_t)i * 256);
+    const auto stream_counts = (const __attribute__((address_space(4))) uint4 *)(uintptr_t)A.counts + (int64_t)stream * A.p.stages;
+    auto count_at = [&](int at) {
+      return mine ? make_uint4(stream_counts[at].x, stream_counts[at].y, stream_counts[at].z, stream_counts[at].w) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    uint4 cnt = count_at(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::"s"(cnt.x), "s"(cnt.y), "s"(cnt.z), "s"(cnt.w) : "memory");
+    dr_u32x16_t words;                                     // as in k_decode_rows
+    {
+      const auto q = (const __attribute__((address_space(3))) u32x4_t *)(uintptr_t)ring_lane;
+      const u32x4_t a = q[0], b = q[1];
+      words = __builtin_shufflevector(__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7), __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7),
+                                      0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+      asm volatile("" ::"v"(words));                       // the slot has been read
+      ask(0);
+    }
+    uint32_t slot = 256, at = 0;
+    for (int st = 0; st < A.p.tiles; ++st) {
+      if (st > 0) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();                      // nobody reads the last tile any more
+        asm volatile("" ::: "memory");
+        tile += SP_ROWS * (uint64_t)pitch_b;
+        rows -= SP_ROWS;
+        fill(rows);
+        cnt = count_at(st);                                // (arrives before the tile does)
+        asm volatile("s_waitcnt vmcnt(0)" ::"s"(cnt.x), "s"(cnt.y), "s"(cnt.z), "s"(cnt.w) : "memory");
+      }
+      asm volatile("" ::"v"(words) : "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      uint32_t n, m0, since;
+      at = __builtin_amdgcn_readfirstlane(at);
+      slot = __builtin_amdgcn_readfirstlane(slot);
+      uint64_t next = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)(uintptr_t)quad >> 32)) << 32) |
+                      (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint64_t)(uintptr_t)quad);
+      // (one buffer: no tile comes in meanwhile, and the records' buffer bit is left out)
+      DR_STAGE_ASM(0x0FF80u, tile, SP_NO_TILE, 0u, 0u, 0u, 0u);
+      quad = (const char *)(uintptr_t)next;
+      const uint32_t even = (cnt.x & 0x00FF00FFu) + (cnt.y & 0x00FF00FFu) + (cnt.z & 0x00FF00FFu) + (cnt.w & 0x00FF00FFu);
+      const uint32_t odd = ((cnt.x >> 8) & 0x00FF00FFu) + ((cnt.y >> 8) & 0x00FF00FFu) + ((cnt.z >> 8) & 0x00FF00FFu) + ((cnt.w >> 8) & 0x00FF00FFu);
+      at += (even + odd) + ((even + odd) >> 16);           // (only its low three bits are looked at)
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may be on its way into LDS when the workgroup ends
+  }
+  if (!mine) return;
+
+  // lane 8 j + i: of the features of one half, row j, columns 4 i .. 4 i + 3
+  const int64_t c = (int64_t)cp * DR_COLS + (lane & 7) * 4;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    const int64_t f = (int64_t)g * DR_TOK + half * 8 + (lane >> 3);
+    const bool on = f < A.F;
+    const int64_t at = ((int64_t)slot_dec * A.F) * A.d + c / 8 * A.m_cols + (on ? f : A.F - 1) * A.m_row + c % 8;
+    float *const w_at = A.w + ((int64_t)slot_dec * A.F + (on ? f : A.F - 1)) * A.pitch + c;
+    f32x4v_t mm = __builtin_nontemporal_load(reinterpret_cast<const f32x4v_t *>(A.m + at));
+    f32x4v_t vv = __builtin_nontemporal_load(reinterpret_cast<const f32x4v_t *>(A.v + at));
+    f32x4v_t ww = __builtin_nontemporal_load(reinterpret_cast<const f32x4v_t *>(w_at));
+    // the eight partial sums of eight rows: a lane gives away half of its rows at each step
+    float sum[8][4];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) sum[i >> 2][i & 3] = half ? hi[i] : lo[i];
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) {
+      const bool up = (lane >> 3) & o;
+#pragma unroll
+      for (int k = 0; k < o; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float keep = up ? sum[k + o][q] : sum[k][q], give = up ? sum[k][q] : sum[k + o][q];
+          sum[k][q] = keep + __shfl_xor(give, o * 8);
+        }
+    }
+    f32x4v_t gr{sum[0][0], sum[0][1], sum[0][2], sum[0][3]};
+    const float z = fmaf(gr[0], 0.0f, fmaf(gr[1], 0.0f, fmaf(gr[2], 0.0f, gr[3] * 0.0f)));
+    // Rows that are not finite once more without the places that fill records up: 0 * inf of such a place gives a NaN.
+    for (uint64_t again = ballot64(on && z != z); again != 0;) {
+      const int row = __ffsll((unsigned long long)again) - 1 >> 3;
+      again &= ~(0xFFull << (8 * row));
+      f32x4v_t a{0.f, 0.f, 0.f, 0.f};
+      const int32_t *lp = A.list_ptr + (int64_t)s * A.F + (int64_t)g * DR_TOK + half * 8 + row;
+      for (int32_t j = lp[0] + (lane >> 3); j < lp[1]; j += DR_REC) {
+        const f32x4v_t x = *reinterpret_cast<const f32x4v_t *>(A.g + ((int64_t)t * A.Tn + A.list_tok[j]) * A.d + c);
+        const float value = A.val[A.list_src[j]];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] = fmaf(value, x[q], a[q]);
+      }
+#pragma unroll
+      for (int o = 8; o < 64; o <<= 1)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[q] += __shfl_xor(a[q], o);
+      if ((lane >> 3) == row) gr = a;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float m1 = mm[q], v1 = vv[q];
+      ww[q] = adam_update(ww[q], gr[q], m1, v1, A.adam);
+      mm[q] = m1;
+      vv[q] = v1;
+    }
+    if (on) {
+      __builtin_nontemporal_store(mm, reinterpret_cast<f32x4v_t *>(A.m + at));
+      __builtin_nontemporal_store(vv, reinterpret_cast<f32x4v_t *>(A.v + at));
+      *reinterpret_cast<f32x4v_t *>(w_at) = ww;
+    }
+  }
+}
+
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct RowLayout {
@@ -466,6 +684,7 @@ static RowLayout row_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t
   p.tiles = (int)clt_ceil_div(F, SP_ROWS);
   p.groups = (int)clt_ceil_div(Tn, DR_TOK);
   p.stages = (int)(L * p.tiles);
+  p.by_layer = 0;
   p.parts = (int)clt_ceil_div(p.groups, DR_WAVES);
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
   l.col_parts = (int)(d / DR_COLS);
@@ -482,6 +701,33 @@ static RowLayout row_layout(int64_t Tn, int64_t d, int64_t F, int64_t L, int64_t
   l.recs = take((size_t)(l.n_recs + (int64_t)(DR_QUAD - 1) * p.groups) * DR_REC * sizeof(uint2));
   l.bytes = at;
   return l;
+}
+
+static RowLayout grad_row_layout(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  RowLayout l;
+  RowPlan &p = l.p;
+  p.tiles = (int)clt_ceil_div(T, SP_ROWS);
+  p.groups = (int)clt_ceil_div(F, DR_TOK);
+  p.stages = p.tiles;
+  p.by_layer = 1;
+  p.parts = (int)clt_ceil_div(p.groups, GR_WAVES);
+  p.groups_per_part = GR_WAVES;
+  l.col_parts = (int)(d / DR_COLS);
+  const int64_t streams = L * p.groups, runs = streams * p.tiles * DR_TOK;
+  l.n_recs = entries / DR_REC + (runs < entries ? runs : entries) + (DR_QUAD - 1) * streams + (DR_RING + 2) * 4;
+  size_t at = 0;
+  auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
+  l.start = take(sizeof(int32_t) * (size_t)streams * DR_TOK * (p.tiles + 1));
+  l.counts = take(sizeof(uint4) * (size_t)streams * p.tiles);
+  l.offset = take(sizeof(uint32_t) * (size_t)streams * p.tiles);
+  l.total = take(sizeof(uint32_t) * (size_t)streams);
+  l.recs = take((size_t)l.n_recs * DR_REC * sizeof(uint2));
+  l.bytes = at;
+  return l;
+}
+static bool grad_row_shape_ok(const RowLayout &l, int64_t d, int64_t L) {
+  return l.p.tiles <= DR_MAX_TILES && l.n_recs <= 0x03FFFFFFll && d * 4 * SP_ROWS <= 0x7FFFFFFFll && l.p.groups <= 0xFFFF &&
+         L * l.p.groups * l.p.tiles <= 0x07FFFFFFll && 8 * clt_ceil_div((int64_t)l.p.parts * l.col_parts, 8) * (L * (L + 1) / 2) <= 0x7FFFFFFFll;
 }
 
 // LDS for the run starts of every tile; 32-bit offsets of records and of rows within a tile
@@ -552,7 +798,7 @@ extern "C" int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const
   hipStream_t s = (hipStream_t)stream;
   char *ws = (char *)workspace;
   RunArgs ra;
-  ra.row_ptr = row_ptr; ra.col = col; ra.val = val; ra.Tn = T; ra.L = L; ra.layer_mask = src_mask; ra.p = l.p;
+  ra.row_ptr = row_ptr; ra.col = col; ra.src = nullptr; ra.val = val; ra.Tn = T; ra.L = L; ra.layer_mask = src_mask; ra.p = l.p;
   ra.start = (int32_t *)(ws + l.start); ra.counts = (uint4 *)(ws + l.counts); ra.offset = (uint32_t *)(ws + l.offset);
   ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint2 *)(ws + l.recs);
   RowArgs a;
@@ -574,5 +820,71 @@ extern "C" int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const
   k_row_streams<<<(unsigned)l.p.groups, 64, 0, s>>>(ra);
   k_row_fill<<<grid, DR_THREADS, fill_bytes, s>>>(ra);
   k_decode_rows<<<(unsigned)(pairs * l.p.parts), DR_WAVES * 64, DR_LDS, s>>>(a);
+  return clt_check_launch();
+}
+
+extern "C" int clt_grad_rows_supported(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype) {
+  if (dtype != CLT_F32 || T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || entries <= 0) return 0;
+  return grad_row_shape_ok(grad_row_layout(T, d, F, L, entries), d, L);
+}
+
+// Measured at 46 shapes (L 2 - 16, d 256 - 2048, F 256 - 32768, T 32 - 8192) against the other in-place steps of float32 decoders, by the
+// entries of a list.  A tile takes some 4 us whatever it holds, so few entries do not pay for many tiles: from 9 per tile on
+// (8 for up to two tiles) this is the fastest or second to rows by microseconds.  Lists of fewer than 8 go row by row: nothing is
+// regrouped, and few rows are gathered.  us, here / 32-byte tiles / rows: L = 12, d = 768, F = 6144, T = 1024: 2602 / 3926 / 4036 with 33
+// entries, 2285 / 2682 / 2553 with 13, 2216 / 2357 / 1891 with 5; T = 4096: 7853 / 13002 / 21267 with 133, 7209 / 3130 / 4359 with 20; L
+// = 8, d = 1024, F = 8192, T = 4096: 6042 / 7208 / 13117 with 90, 5877 / 4489 / 7872 with 50; L = 6, d = 1024, F = 16384, T = 1500: 3199 / 2217 /
+// 1657 with 3; L = 6, d = 512, F = 8192, T = 3000: 1104 / 605 / 549 with 7.  Launches that do not fill the chip once are left as they were.
+extern "C" int clt_grad_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype) {
+  if (!clt_grad_rows_supported(T, d, F, L, entries, dtype)) return 0;
+  const RowLayout l = grad_row_layout(T, d, F, L, entries);
+  if ((int64_t)l.p.parts * l.col_parts * (L * (L + 1) / 2) < 512) return 0;
+  const double per_list = (double)entries / ((double)L * F);
+  if (per_list < 8) return 2;
+  return l.p.tiles <= 2 || per_list >= 9.0 * l.p.tiles;
+}
+
+extern "C" size_t clt_grad_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {
+  if (T <= 0 || d < DR_COLS || F <= 0 || L <= 0 || entries <= 0) return 0;
+  return grad_row_layout(T, d, F, L, entries).bytes;
+}
+
+extern "C" int clt_decoder_grad_adam_rows(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const float *val,
+                                          const float *g, float *w_packed, float *m, float *v, int moments_by_tile, int64_t T, int64_t d,
+                                          int64_t F, int64_t L, int64_t entries, double lr, double beta1, double beta2, double eps,
+                                          int64_t step, void *workspace, size_t workspace_bytes, void *stream) {
+  if (!clt_grad_rows_supported(T, d, F, L, entries, CLT_F32)) return CLT_ERR_ARG;
+  if (step < 1 || !(beta1 >= 0 && beta1 < 1) || !(beta2 >= 0 && beta2 < 1)) return CLT_ERR_ARG;
+  if (!list_ptr || !list_tok || !list_src || !val || !g || !w_packed || !m || !v || !workspace) return CLT_ERR_ARG;
+  if (!clt_aligned16(g) || !clt_aligned16(w_packed) || !clt_aligned16(m) || !clt_aligned16(v) || !clt_aligned16(workspace)) return CLT_ERR_ALIGN;
+  const RowLayout l = grad_row_layout(T, d, F, L, entries);
+  if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
+  hipStream_t s = (hipStream_t)stream;
+  char *ws = (char *)workspace;
+  RunArgs ra;
+  ra.row_ptr = list_ptr; ra.col = list_tok; ra.src = list_src; ra.val = val; ra.Tn = F; ra.L = L; ra.layer_mask = ~0ull; ra.p = l.p;
+  ra.start = (int32_t *)(ws + l.start); ra.counts = (uint4 *)(ws + l.counts); ra.offset = (uint32_t *)(ws + l.offset);
+  ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint2 *)(ws + l.recs);
+  GradRowArgs a;
+  a.p = l.p; a.counts = ra.counts; a.first = ra.total; a.recs = ra.recs;
+  a.g = g; a.w = w_packed; a.m = m; a.v = v;
+  a.list_ptr = list_ptr; a.list_tok = list_tok; a.list_src = list_src; a.val = val;
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = clt_pitch(d, 4);
+  a.m_row = moments_by_tile ? 8 : d;
+  a.m_cols = moments_by_tile ? F * 8 : 8;
+  a.col_parts = l.col_parts;
+  a.items = (int)clt_ceil_div((int64_t)l.p.parts * l.col_parts, 8);
+  a.adam = adam_coef(lr, beta1, beta2, eps, step);
+  const int streams = (int)L * l.p.groups;
+  const size_t run_lds = sizeof(int32_t) * (size_t)DR_TOK * (l.p.tiles + 1), fill_bytes = run_lds + sizeof(uint32_t) * (size_t)DR_TOK * l.p.tiles;
+  if (hipFuncSetAttribute((const void *)k_grad_rows, hipFuncAttributeMaxDynamicSharedMemorySize, GR_LDS) != hipSuccess ||
+      hipFuncSetAttribute((const void *)k_row_fill, hipFuncAttributeMaxDynamicSharedMemorySize, (int)fill_bytes) != hipSuccess)
+    return CLT_ERR_LAUNCH;
+  const dim3 grid((unsigned)l.p.groups, (unsigned)L);
+  k_row_runs<<<grid, DR_THREADS, run_lds, s>>>(ra);
+  k_row_streams<<<(unsigned)streams, 64, 0, s>>>(ra);
+  k_row_firsts<<<1, DR_FIRSTS, 0, s>>>(ra.total, streams);
+  k_row_fill<<<grid, DR_THREADS, fill_bytes, s>>>(ra);
+  k_grad_rows<<<(unsigned)(8 * a.items * (L * (L + 1) / 2)), GR_WAVES * 64, GR_LDS, s>>>(a);
   return clt_check_launch();
 }

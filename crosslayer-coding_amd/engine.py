@@ -772,6 +772,33 @@ def decoder_grad_adam_tiles(lists, surv: SurvivorList, g: torch.Tensor, w_packed
     nat.check(code, "clt_decoder_grad_adam_tiles")
 
 
+def grad_rows_wanted(T: int, d: int, F: int, L: int, entries: int, dtype: torch.dtype) -> int:
+    """The fastest in-place step of float32 untied decoders by its shape: 1 ``decoder_grad_adam_rows``, 2 ``decoder_weight_grad_adam``,
+    0 neither."""
+    return int(nat.load().clt_grad_rows_wanted(T, d, F, L, entries, nat.dtype_code(dtype))) if dtype == torch.float32 else 0
+
+
+def decoder_grad_adam_rows(lists, surv: SurvivorList, g: torch.Tensor, w_packed: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
+                           lr: float, betas, eps: float, step: int, ws: Optional[Workspace] = None) -> None:
+    """``decoder_weight_grad_adam`` of float32 decoders from LDS tiles: moments as [n_dec, F, d] or as [n_dec, d // 8, F, 8]."""
+    assert g.dtype == surv.dtype == torch.float32 and g.is_contiguous() and w_packed.dtype == surv.dtype and w_packed.is_contiguous()
+    ptr, tok, src = lists
+    L, T, F = surv.L, surv.T, surv.F
+    d = g.shape[2]
+    n_dec = L * (L + 1) // 2
+    by_tile = m.dim() == 4
+    assert tuple(w_packed.shape) == (n_dec, F, decoder_pitch(d, surv.dtype))
+    assert tuple(m.shape) == ((n_dec, d // 8, F, 8) if by_tile else (n_dec, F, d)) and v.shape == m.shape
+    assert m.dtype == torch.float32 and v.dtype == torch.float32 and m.is_contiguous() and v.is_contiguous()
+    lib = nat.load()
+    n = surv.capacity
+    wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_rows_workspace_bytes(T, d, F, L, n))
+    code = lib.clt_decoder_grad_adam_rows(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(w_packed),
+                                          nat.ptr(m), nat.ptr(v), 1 if by_tile else 0, T, d, F, L, n, lr, betas[0], betas[1], eps, step,
+                                          nat.ptr(wbuf), wbuf.numel(), _stream(g))
+    nat.check(code, "clt_decoder_grad_adam_rows")
+
+
 def unpack_decoders(w_packed: torch.Tensor, w_refs_dev: torch.Tensor, w_refs_host, d: int, F: int) -> None:
     """Checkpoint-layout parameters [d, F] (their addresses in the device int64 tensor ``w_refs_dev`` and in the
     host ctypes array ``w_refs_host``) from the packed working copy [n_dec, F, pitch]."""

@@ -129,10 +129,11 @@ class CLTAdam:
         """The decoder weights' part of the NEXT ``step`` (which must follow with ``raw["dec_w"] = None``), taken
         straight from the survivor lists: gradient rows go from registers into the update of the moments and
         of the working copy of the weights; the checkpoint-layout parameters are then rewritten from that copy.
-        Three routes: bf16 on the matrix cores over tiles of 64 columns (``engine.grad_tiles_supported``; updates the
-        feature-major slab itself, whatever the moments' layout); float32, and widths that are not whole tiles, over
-        tiles of 32 bytes (tiled moments and a tiled weight copy) when ``engine.decoder_tile_width`` takes the shape; else
-        row by row on the feature-major slab.  The first and the last are bit-identical to gradient-then-Adam; the
+        Four routes: bf16 on the matrix cores over tiles of 64 columns (``engine.grad_tiles_supported``; updates the
+        feature-major slab itself, whatever the moments' layout); float32 from LDS tiles of the loss gradients where that is
+        fastest (``engine.grad_rows_wanted``; the slab itself too); float32, and widths that are not whole tiles, over tiles of
+        32 bytes (tiled moments and a tiled weight copy) when ``engine.decoder_tile_width`` takes the shape; else, and for
+        float32 lists of few entries, row by row on the feature-major slab.  The first and the last are bit-identical to gradient-then-Adam; the
         32-byte tiles sum the lists they cut between lanes in another fixed association (equal to fp32 rounding)."""
         from . import engine
         dec = self.model.decoder_module
@@ -153,6 +154,16 @@ class CLTAdam:
                                            self.step_count + 1, ws=self.model._workspace())
             self._after_slab_step(packed, w_dev, w_host, d, F)
             return
+        rows = engine.grad_rows_wanted(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype) if self.tile_decoder_step else 0
+        if rows == 1 and self._dec_cols in (0, 8) and engine._aligned16(g_model, packed, *self.state["dec_w"]):
+            # (moments either way here too; the slab changes under the tiled copy)
+            self._w_tiles_gen = None
+            engine.decoder_grad_adam_rows(lists, surv, g_model, packed, *self.state["dec_w"], self.lr, self.betas, self.eps,
+                                          self.step_count + 1, ws=self.model._workspace())
+            self._after_slab_step(packed, w_dev, w_host, d, F)
+            return
+        if rows == 2 and self._dec_layout == "rows":
+            cs = 0                        # short lists row by row, unless a batch before has left the moments in tiles
         if cs and all(w.data_ptr() % 16 == 0 for w in ws):
             self._decoder_moments_to("tiles", cs)
             dec._derived_copies = True      # the packed copy tells when the device may have repacked it

@@ -711,6 +711,19 @@ int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_t *list_tok
                                 const void *g_model, void *w_packed, float *m, float *v, int moments_by_tile, int64_t T,
                                 int64_t d, int64_t F, int64_t L, int64_t entries, double lr, double beta1, double beta2,
                                 double eps, int64_t step, int dtype, void *workspace, size_t workspace_bytes, void *stream);
+/*
+ * The same Adam step for float32, d a multiple of 32, from LDS tiles: w_packed (clt_decoder_pitch rows) and both moments [n_dec][F][d],
+ * or [n_dec][d / 8][F][8] (moments_by_tile), are updated in place; val and g fp32.  _wanted: 1 where it is the fastest by its shape, 2 where clt_decoder_weight_grad_adam is.
+ * Equal to clt_decoder_weight_grad_adam up to summation order, repeatable bit for bit.
+ */
+int clt_grad_rows_supported(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype);
+int clt_grad_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype);
+size_t clt_grad_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries);
+int clt_decoder_grad_adam_rows(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const float *val,
+                               const float *g, float *w_packed, float *m, float *v, int moments_by_tile,
+                               int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
+                               double lr, double beta1, double beta2, double eps, int64_t step,
+                               void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * The same step over COLUMN TILES (same reference lines; the gradient sums of lists that the kernel
