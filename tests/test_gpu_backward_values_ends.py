@@ -38,3 +38,30 @@ def test_value_gradients_at_the_ends_of_lists(d, dtype):
     size = torch.stack([gd[0].abs() @ rows[0].t().abs() + gd[1].abs() @ rows[1].t().abs(), gd[1].abs() @ rows[2].t().abs()])
     # a lane adds d / 64 products, six exchanges add the lanes, one addition the targets: so many roundings of 2^-24 per term
     assert bool(((got - dense[keep]).abs() <= size[keep] * (d / 64 + 8) * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("L,empty", [(1, ()), (2, (0,)), (5, (1, 2, 4)), (7, ()), (64, (0, 31, 32, 63)), (3, (0, 1))])
+def test_value_gradients_of_sources_without_survivors(L, empty):
+    dev = torch.device("cuda:0")
+    T, F, d = 9, 24, 64
+    g = torch.Generator().manual_seed(L)
+    keep = torch.rand(L, T, F, generator=g) < 0.2
+    for s in empty:
+        keep[s] = False
+    row_ptr = torch.zeros(L * T + 1, dtype=torch.int32)
+    row_ptr[1:] = torch.cumsum(keep.view(L * T, F).sum(1), 0)
+    col = keep.view(L * T, F).nonzero()[:, 1].int()
+    surv = engine.SurvivorList(row_ptr.to(dev), col.to(dev), torch.ones(col.numel(), device=dev), T, F, L, torch.float32)
+    w = torch.zeros(L * (L + 1) // 2, F, engine.decoder_pitch(d, torch.float32))
+    w[:, :, :d] = torch.randn(w.shape[0], F, d, generator=g)
+    grad = torch.randn(L, T, d, generator=g)
+    mask = (1 << L) - 1 if L < 5 else ((1 << L) - 1) & ~(1 << 3)         # (source 3 left out: its gradients are zeros)
+    got = engine.decode_backward_values(surv, w.to(dev), grad.to(dev), "none", mask).cpu().double()
+    rows, gd, dense, size = w[:, :, :d].double(), grad.double(), [], []
+    for s in range(L):
+        first = s * L - s * (s - 1) // 2
+        on = float((mask >> s) & 1)
+        dense.append(on * sum(gd[t] @ rows[first + t - s].t() for t in range(s, L)))
+        size.append(sum(gd[t].abs() @ rows[first + t - s].t().abs() for t in range(s, L)))
+    # d / 64 products per lane, six exchanges, one addition per target
+    assert bool(((got - torch.stack(dense)[keep]).abs() <= torch.stack(size)[keep] * (d / 64 + 6 + L) * 2.0 ** -24).all())
