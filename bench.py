@@ -713,10 +713,12 @@ def run_backward(args):
     hbm_bytes = pairs * F * d * ((16 + 4 * esz) if fused else 4) + L * wl.tokens * d * esz + surv.nnz * (8 + esz)
     tiled = fused and opt._dec_layout == "tiles"
     matrix = fused and engine.grad_tiles_supported(surv.T, d, F, surv.L, surv.capacity, surv.dtype)
-    if matrix:
+    lds_rows = (fused and not matrix and opt.tile_decoder_step
+                and engine.grad_rows_wanted(surv.T, d, F, surv.L, surv.capacity, surv.dtype) == 1)
+    if matrix or lds_rows:
         # through the HBM interface go both moments and the weights, read and written, the loss gradient and the lists
         hbm_bytes = pairs * F * d * (16 + 2 * esz) + L * wl.tokens * d * esz + surv.nnz * (8 + esz)
-        roofline = {"kernel": f"k_grad_tiles ({dw_name}, one launch per step, with the regrouping of the lists before it)",
+        roofline = {"kernel": f"{'k_grad_tiles' if matrix else 'k_grad_rows'} ({dw_name}, one launch per step, with the regrouping of the lists before it)",
                     "bound": "hbm", "achieved": hbm_bytes / dw_sec / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": hbm_bytes / dw_sec / 1e9 / HBM_PEAK_GBS, "traffic": None, "lds_gather_GBps": gathered / dw_sec / 1e9,
                     "note": "achieved = compulsory HBM bytes of the stage (moments, weights, loss gradient, lists) / the stage's time"}
@@ -752,7 +754,7 @@ def run_backward(args):
                             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": adam_bytes / adam_sec / 1e9 / HBM_PEAK_GBS}
     return {
         "stages_ms": stages, "roofline": roofline,
-        "decoder_step_route": (("matrix cores" if matrix else "column tiles" if tiled else "rows") if fused else "gradient then Adam") if opt is not None else None,
+        "decoder_step_route": (("matrix cores" if matrix else "LDS rows" if lds_rows else "column tiles" if tiled else "rows") if fused else "gradient then Adam") if opt is not None else None,
         "metric": ("CLT training step tokens/sec (forward, MSE loss, gradients, Adam lr 1e-4 with fp32 moments)"
                    if opt is not None else "CLT forward + MSE loss + gradients tokens/sec (no optimizer step)"),
         "value": wl.tokens * args.steps / wall, "unit": "tokens/s", "n_gpus": 1, "steps": args.steps,
