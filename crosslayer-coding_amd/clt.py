@@ -355,10 +355,6 @@ class CrossLayerTranscoder(BaseTranscoder):
         theta_grad = None
         if cfg.activation_fn == "jumprelu" and self.theta_manager.log_threshold is not None:
             theta_grad = self._log_threshold_gradient(x_slab, g_model, ws, packed, surv, dval if sc is not None else None)
-        if encoder_step is not None:
-            db_enc = encoder_step.encoder_weight_step(lists, dval, x_slab)
-        if decoder_step is not None:
-            decoder_step.decoder_weight_step(lists, surv, g_model)
         # bias_grad[t] = column sums of d loss / d rec[t]; a decoder's bias takes the rows of the targets
         # it is added to: its own pair's target, all targets >= its source, or its target (once)
         if cfg.decoder_tying == "none":
@@ -367,7 +363,16 @@ class CrossLayerTranscoder(BaseTranscoder):
             dec_b = torch.flip(torch.cumsum(torch.flip(bias_grad, dims=[0]), dim=0), dims=[0])
         else:
             dec_b = bias_grad
-        return {"enc_w": dw_enc, "enc_b": db_enc, "dec_w": dw_dec, "dec_param": dw_param, "dec_b": dec_b.contiguous(),
+        dec_b = dec_b.contiguous()
+        # The steps taken in place come last and ask for their memory before they write: a batch that does not fit raises
+        # with weights, moments and step count as they were, and can be taken again in halves.
+        if encoder_step is not None:
+            db_enc = torch.empty((L, F), dtype=torch.float32, device=g.device)
+        if decoder_step is not None:
+            decoder_step.decoder_weight_step(lists, surv, g_model)
+        if encoder_step is not None:
+            encoder_step.encoder_weight_step(lists, dval, x_slab, db_enc)
+        return {"enc_w": dw_enc, "enc_b": db_enc, "dec_w": dw_dec, "dec_param": dw_param, "dec_b": dec_b,
                 "theta": theta_grad, "skip": d_skip, "feat_offset": d_off, "feat_scale": d_sc}
 
     def _log_threshold_gradient(self, x_slab: torch.Tensor, g_model: torch.Tensor, ws, packed: torch.Tensor, surv=None,

@@ -925,15 +925,17 @@ def encoder_step_fits(d: int, dtype: torch.dtype) -> bool:
 
 
 def encoder_weight_grad_adam(lists, dval: torch.Tensor, x: torch.Tensor, w: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
-                             lr: float, betas, eps: float, step: int) -> torch.Tensor:
+                             lr: float, betas, eps: float, step: int, db: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``encoder_weight_grad`` with the Adam step ``step`` of the stacked weights ``w`` and their moments [L, F, d] taken on the
-    spot (bit-identical to the two calls); returns the bias gradients, fp32 [L, F]."""
+    spot (bit-identical to the two calls); returns the bias gradients, fp32 [L, F], in ``db`` where it is given."""
     ptr, tok, src = lists
     L, T, d = x.shape
     F = w.shape[1]
     assert x.is_contiguous() and w.is_contiguous() and w.dtype == x.dtype and tuple(w.shape) == (L, F, d) and dval.dtype == torch.float32
     assert m.shape == w.shape and v.shape == w.shape and m.dtype == v.dtype == torch.float32 and m.is_contiguous() and v.is_contiguous()
-    db = torch.empty((L, F), dtype=torch.float32, device=x.device)
+    if db is None:
+        db = torch.empty((L, F), dtype=torch.float32, device=x.device)
+    assert tuple(db.shape) == (L, F) and db.dtype == torch.float32 and db.is_contiguous()
     code = nat.load().clt_encoder_weight_grad_adam(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(dval), nat.ptr(x), nat.ptr(w),
                                                    nat.ptr(m), nat.ptr(v), nat.ptr(db), T, d, F, L, lr, betas[0], betas[1], eps, step,
                                                    nat.dtype_code(x.dtype), _stream(x))

@@ -90,12 +90,12 @@ class CLTAdam:
                 and engine._aligned16(x, w, *self.state["enc_w"]))
 
     @torch.no_grad()
-    def encoder_weight_step(self, lists, dval: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-        """The encoder weights' part of the NEXT ``step`` (which must follow with ``raw["enc_w"] = None``); returns the bias
-        gradients.  Bit-identical to gradient-then-Adam."""
+    def encoder_weight_step(self, lists, dval: torch.Tensor, x: torch.Tensor, db: torch.Tensor) -> None:
+        """The encoder weights' part of the NEXT ``step`` (which must follow with ``raw["enc_w"] = None``); ``db`` takes the bias
+        gradients, fp32 [L, F].  Bit-identical to gradient-then-Adam.  Asks for no memory: it may follow the decoder step."""
         from . import engine
         w, _ = self.model.encoder_module.stacked()
-        return engine.encoder_weight_grad_adam(lists, dval, x, w, *self.state["enc_w"], self.lr, self.betas, self.eps, self.step_count + 1)
+        engine.encoder_weight_grad_adam(lists, dval, x, w, *self.state["enc_w"], self.lr, self.betas, self.eps, self.step_count + 1, db)
 
     def _decoder_moments_to(self, layout: str, cols: int = 0) -> None:
         """Regroup both decoder moments: "rows" [n_dec, F, d] <-> "tiles" [n_dec, d // cols, F, cols].  Happens when the

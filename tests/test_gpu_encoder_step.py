@@ -39,3 +39,37 @@ def test_encoder_step_in_the_gradient_kernel(d, dtype):
 def test_wide_rows_keep_the_two_calls():
     assert not engine.encoder_step_fits(2056, torch.bfloat16) and not engine.encoder_step_fits(1028, torch.float32)
     assert not engine.encoder_step_fits(768, torch.float16)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_a_step_that_finds_no_memory_leaves_the_model_as_it_was(monkeypatch, dtype):
+    """The workspace of the decoder step is what a longer batch outgrows first: the call raises before anything has moved, and the
+    same call afterwards is the first step of a model that never raised."""
+    import crosslayer_coding_amd as cca
+    from crosslayer_coding_amd import synth
+    dev = torch.device("cuda:0")
+    wl = synth.Workload("retry", 3, 3, 128, 512, 300, dtype, k=12)
+    ends = []
+    for fails in (False, True):
+        model, x, _ = synth.build_model(wl, dev, 1)
+        y = synth.make_targets(wl, dev, 1)
+        opt, inputs, targets = cca.CLTAdam(model, lr=1e-2), {l: x[l] for l in range(3)}, {l: y[l] for l in range(3)}
+
+        def state():
+            return [t.clone() for t in (*model.encoder_module.stacked(), model.decoder_module.packed(), *opt.decoder_moments(),
+                                        *opt.state["enc_w"], *opt.state["enc_b"], *opt.state["dec_b"])]
+
+        if fails:
+            before, get = state(), engine.Workspace.get
+            with monkeypatch.context() as patch:
+                def no_room(self, name, nbytes):
+                    if name in ("grad_tiles", "decoder_tiles"):
+                        raise torch.OutOfMemoryError(name)
+                    return get(self, name, nbytes)
+                patch.setattr(engine.Workspace, "get", no_room)
+                with pytest.raises(torch.OutOfMemoryError):
+                    model.training_step(inputs, targets, opt)
+            assert opt.step_count == 0 and all(torch.equal(a, b) for a, b in zip(before, state()))
+        loss = model.training_step(inputs, targets, opt)
+        ends.append([loss] + state())
+    assert all(torch.equal(a, b) for a, b in zip(*ends))
