@@ -192,7 +192,8 @@ static inline int clt_check_launch() {
 static inline bool clt_aligned16(const void *p) { return (((uintptr_t)p) & 15u) == 0; }
 static inline int64_t clt_ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// the decodes from LDS tiles in microseconds (spmm.hip, decode_rows.hip), for the rule of the gather for thin lists; large if they
-// take no such call
+// The decodes in microseconds, for the rules that choose between them: the gather that stands behind all others (decode.hip), and those from
+// LDS tiles (spmm.hip, decode_rows.hip), large if they take no such call.
+double clt_decode_gather_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
 double clt_decode_tiles_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
 double clt_decode_rows_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);

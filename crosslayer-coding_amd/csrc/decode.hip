@@ -1933,12 +1933,42 @@ static GatherWork gather_work(int64_t T, int64_t d, int64_t F, int64_t L, int64_
   return g;
 }
 
+// What the prices of the decodes were measured at: 6006 shapes at random (L 2 - 16, d 256 - 2048, F 1024 - 32768, T 32 - 8192, 1 - 256
+// survivors per source and token, untied and tied per source), lists of equal length, lists with the heavy tokens of a top-k over the batch
+// and thresholds.  At 3753 other shapes the choice costs, against the best of the three, 1.2 % (float32) and 1.9 % (16 bits) for threshold
+// lists, 6.0 and 7.7 % for a top-k's; while each decode was priced from shapes of its own it cost 3.8, 3.3, 8.3 and 8.6 %.
+//
+// The schedules by sources: bytes per us of decoder rows out of the L2s, of fp32 partial rows written and read, of rows from HBM that some
+// token refers to, and us per source for its launches; off by 8 - 11 % in the mean.  With too little work for those (the lines of
+// engine._wants_sliced_decode) a wavefront walks a row's whole list: lists of equal length then take two thirds of the mean, heavy tokens
+// more, and the price is put a tenth below it.  In 16 bits, where a threshold list's total is the last batch's, the price by sources bounds
+// it there, so that small batches do not change route, and with it their rounding, from one call to the next.
+double clt_decode_gather_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const int esz = clt_elem_bytes(dtype);
+  const bool wide = dtype == CLT_F32;
+  const GatherWork g = gather_work(T, d, F, L, targets, entries, tying, dtype);
+  const int64_t n_dec = tying == CLT_TYING_NONE ? L * (L + 1) / 2 : L;
+  const double partial = g.triples * (double)d * 16;
+  if (T * targets < 8192 && n_dec * F * clt_pitch(d, esz) * esz < (128ll << 20) && d * esz < 5 * 1024) {
+    const double list = (double)entries / T;
+    if (wide) return 7.7 + g.bytes / 10.3e6 + g.distinct / 3.8e6 + list * 0.086;
+    const double walk = 11.2 + g.bytes / 11.5e6 + g.distinct / 5e6 + list * 0.111, sources = 0.3 * L + g.bytes / 18.1e6 + partial / 4.5e6 + g.distinct / 5.5e6;
+    return walk < sources ? walk : sources;
+  }
+  if (wide) {
+    const bool quarter = plan_route(d, F, tying, esz, true, true) == CLT_ROUTE_QUARTER;
+    return 11.5 + 0.4 * L + g.bytes / 23.5e6 + partial / (quarter ? 4e6 : 2.4e6) + g.distinct / 7.9e6;
+  }
+  return 14.5 + 0.3 * L + g.bytes / 20.4e6 + partial / 4e6 + g.distinct / 8.1e6;
+}
+
 // Against the schedules by sources (k_decode_quarter, k_decode_line), which move rows at 17 TB/s out of the L2s, bring each one there
 // from HBM and read and write the partial rows of every triple, and against the decodes from LDS tiles.  This kernel, from what it
 // measured (bf16 and float32; L 2 - 16, d 512 - 2048, F 1024 - 24576, T 32 - 8000, 1 - 200 survivors per source and token): 9.5
 // TB/s, as much time again for a row's first use, 0.25 ns per triple, and no less than a workgroup's chain over its lists, or over
 // one of 4000 entries, as a top-k over the batch may give a single token (k_decode_thin_longest says what longer ones cost).  Within 15 %, but for rows used more than
-// 20 times, which it does faster.  us, schedule by sources / this: T = 3000, L = 12, F = 24576, d = 768, bf16, 200 survivors per
+// 20 times, which it does faster; against the tiles a third more is let pass, because lists of equal length take that much less here than the mean (bf16,
+// T = 153, L = 12, d = 2048, F = 5224, 35 per token: 244 / 354 of the tiles; float32, 522, 9, 1024, 2960, 18: 167 / 278).  us, schedule by sources / this: T = 3000, L = 12, F = 24576, d = 768, bf16, 200 survivors per
 // token over all layers 1530 / 854, 20 695 / 224; per layer 16: 1253 / 747; T = 1000, 50: 1100 / 790; T = 300, 200: 877 / 1078;
 // T = 77, 200: 340 / 356; float32, T = 600, 200: 2790 / 3910.
 extern "C" int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
@@ -1948,8 +1978,8 @@ extern "C" int clt_decode_thin_wanted(int64_t T, int64_t d, int64_t F, int64_t L
   const double chain = 0.1 * (double)entries / T > 0.025 * longest ? 0.1 * (double)entries / T : 0.025 * longest;
   const double thin = (flow > chain ? flow : chain) + 18;
   return thin < 0.95 * (g.bytes / 17e6 + g.distinct / 6.3e6 + g.triples * (double)d * 16 / 3.2e6 + 5) &&
-         thin < clt_decode_tiles_us(T, d, F, L, targets, entries, tying, dtype) &&
-         thin < clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);
+         thin < 1.3 * clt_decode_tiles_us(T, d, F, L, targets, entries, tying, dtype) &&
+         thin < 1.3 * clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);
 }
 
 // max_entries < 0: whatever the lists hold

@@ -738,40 +738,29 @@ static bool row_shape_ok(const RowLayout &l, int64_t row_bytes) {
 
 }  // namespace
 
-struct RowTimes { double rows, sparse; };   // us; the first large for what the tiles do not take
-
-// Both routes priced from what they measured (28 shapes of L 2 - 16, d 256 - 2048, F 2048 - 16384, T 128 - 4096, 20 - 200 survivors per
-// token; the prices are off by 4 % (tiles) and 18 % (gather) in the mean, and the choice costs 2 % against the better of the two).  A
-// stage of the tiles takes 1.33 us plus 3.1 ns per record, but no less than the 1.9 us in which 64 KB come into LDS; workgroups of
-// unequal length end a third of the longest behind the mean, and the longest one bounds a launch of few.  us, tiles / gather: L = 12, d =
+// Priced from what it measured (2496 of the shapes of clt_decode_gather_us; off by 10 % in the mean): a stage of the tiles takes 1.2 us plus
+// 5 ns per record, but no less than 64 KB take to come into LDS, 2.0 us from HBM and 1.3 where the targets share a decoder; workgroups of
+// unequal length end a quarter of the longest behind the mean, and the longest one bounds a launch of few.  us, tiles / gather: L = 12, d =
 // 768, F = 6144: 1469 / 2618 with 200 per token at T = 1024, 949 / 1198 with 60, 805 / 717 with 20; 647 / 1112 with 200 at 256; L =
 // 6, d = 1024, F = 16384: 2519 / 2796 at 3000 x 200, 2169 / 1704 at 3000 x 100; L = 16, d = 256, F = 2048, 1024 x 30: 234 / 565.
-static RowTimes row_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
-  const RowTimes no = {1e30, 0};
+double clt_decode_rows_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const double no = 1e30;
   if (dtype != CLT_F32 || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;
   if (T <= 0 || d <= 0 || d % DR_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return no;
   const RowLayout l = row_layout(T, d, F, L, entries);
   if (!row_shape_ok(l, clt_pitch(d, 4) * 4)) return no;
-  const double pairs = 0.5 * targets * (2 * L - targets + 1);
-  const double run = (double)entries / ((double)l.p.stages * T);
-  const double recs = l.p.groups_per_part * DR_TOK * (run < run / DR_REC + 0.5 ? run : run / DR_REC + 0.5);
-  const double stage_us = 1.33 + recs * 0.0031;
+  const double pairs = 0.5 * targets * (2 * L - targets + 1), run = (double)entries / ((double)l.p.stages * T);
+  const double recs = l.p.groups_per_part * DR_TOK * (run < run / DR_REC + 0.29 ? run : run / DR_REC + 0.29);
+  const double stage = 1.16 + recs * 0.005, fill = tying == CLT_TYING_NONE ? 1.97 : 1.3;
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
-  const double last = stages + 0.36 * longest > 1.26 * longest ? stages + 0.36 * longest : 1.26 * longest;
-  const double rows_us = last * (stage_us > 1.9 ? stage_us : 1.9) + 20 + entries * 2e-5;
-  const GatherPrice gather = {21.6e6, 6.5e6, 5.5e6, 5.9};
-  const double sparse_us = gather.us(T, d, F, L, targets, entries, tying, 4);
-  return {rows_us, sparse_us};
+  const double last = stages + 0.28 * longest > longest ? stages + 0.28 * longest : longest;
+  return last * (stage > fill ? stage : fill) + 27 + entries * 1.5e-5;
 }
 
 extern "C" int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
                                       int dtype) {
-  const RowTimes t = row_times(T, d, F, L, targets, entries, tying, dtype);
-  return t.rows < 0.95 * t.sparse;
-}
-
-double clt_decode_rows_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
-  return row_times(T, d, F, L, targets, entries, tying, dtype).rows;
+  const double us = clt_decode_rows_us(T, d, F, L, targets, entries, tying, dtype);
+  return us < 1e30 && us < 0.95 * clt_decode_gather_us(T, d, F, L, targets, entries, tying, dtype);
 }
 
 extern "C" size_t clt_decode_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries) {

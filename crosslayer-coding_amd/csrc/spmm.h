@@ -12,7 +12,6 @@
 // which still leaves as many useful ones per cycle as the vector unit's dot products deliver, without their
 // unpacking; and lists of unequal length cost nothing, because a batch is filled from any of 16 output rows.
 #pragma once
-#include <math.h>
 #include <type_traits>
 #include "clt_common.h"
 
@@ -64,18 +63,6 @@ __device__ __forceinline__ uint32_t stream_first(const uint32_t *total, int stre
   for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
   return n;
 }
-
-// What the gather of decode.hip takes for the last `targets` layers, in us, from bytes per us that it was seen to reach: decoder rows
-// from the L2s, fp32 partial rows written and read, decoder rows that at least one survivor needs from HBM; and us per source for
-// its launches.
-struct GatherPrice {
-  double rows, partial, decoders, source;
-  double us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int elem) const {
-    const double pairs = 0.5 * targets * (2 * L - targets + 1), gathered = (double)entries / L * pairs * d * elem;
-    const double fires = (double)entries / ((double)L * T * F), used = 1 - pow(1 - (fires < 1 ? fires : 1), (double)T);
-    return gathered / rows + pairs * T * d * 16 / partial + (tying == CLT_TYING_PER_SOURCE ? (double)L : pairs) * F * d * elem * used / decoders + source * L;
-  }
-};
 
 // Direct-to-LDS loads, 16 or 4 bytes per lane (lane i lands at lds_at + 16 i / 4 i).  As asm statements, so that the
 // compiler does not wait for them in front of every LDS read; whoever reads the data waits by hand.

@@ -778,41 +778,29 @@ static int launch_grad(GradOut out, const int32_t *list_ptr, const int32_t *list
 
 }  // namespace
 
-struct TileTimes { double tiles, sparse; };   // us; the first large for what the tiles do not take
-
-// Both routes priced from what they measured (bf16; 29 shapes of L 2 - 16, d 256 - 2048, F 4096 - 24576, T 256 - 8192, 25 - 200
-// survivors per token; the prices are off by 10 % (tiles) and, from 8192 (token, target) rows on, by 12 % (gather) in the mean).  A stage
-// of the tiles takes 0.89 us plus 13.1 ns per batch, but no less than the 1.6 us in which 64 KB come into LDS; workgroups of unequal
-// length end a third of the longest behind the mean, and the longest one bounds a launch of few.  E.g. us, tiles / gather: L = 12, d = 768,
-// F = 24576: 2958 / 6769 with 200 per token at T = 4096, 1565 / 2782 at 1024, 1297 / 1440 at 512, 1360 / 846 at 256; 1700 / 2703
-// with 50 at 4096, 1545 / 1642 at 2048.  (Smaller problems, whose gather has no partial rows, stay with it, though the tiles may be up to
-// twice as fast there - L = 4, d = 512, F = 8192, 1024 tokens x 100: 137 / 238: whether they are turns on the density, which for a
-// threshold list is last batch's, and the route with it.)
-static TileTimes tile_times(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
-  const TileTimes no = {1e30, 0};
+// Priced from what it measured (16 bits; 3510 of the shapes of clt_decode_gather_us; off by 12 % in the mean): a stage of the tiles takes
+// 1.1 us plus 15 ns per batch, but no less than 64 KB take to come into LDS, 1.7 us from HBM and 0.5 where the targets share a decoder;
+// workgroups of unequal length end a quarter of the longest behind the mean, and the longest one bounds a launch of few.  E.g. us, tiles
+// / gather: L = 12, d = 768, F = 24576: 2958 / 6769 with 200 per token at T = 4096, 1565 / 2782 at 1024, 1297 / 1440 at 512, 1360 / 846 at
+// 256; 1700 / 2703 with 50 at 4096, 1545 / 1642 at 2048; L = 4, d = 512, F = 8192, 1024 x 100: 137 / 238.
+double clt_decode_tiles_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
+  const double no = 1e30;
   if ((dtype != CLT_BF16 && dtype != CLT_F16) || (tying != CLT_TYING_NONE && tying != CLT_TYING_PER_SOURCE)) return no;
   if (T <= 0 || d <= 0 || d % SP_COLS != 0 || F <= 0 || L <= 0 || L > 64 || targets <= 0 || targets > L || entries <= 0) return no;
   const SpLayout l = tile_layout(T, d, F, L, targets, entries);
   if (!sp_shape_ok(l, clt_pitch(d, 2) * 2)) return no;
   const double pairs = 0.5 * targets * (2 * L - targets + 1);
-  const double per_batch = (double)entries / ((double)l.p.stages * l.p.groups) / SP_BATCH + 0.5;
-  const double stage_us = 0.89 + l.p.groups_per_part * (per_batch > 1 ? per_batch : 1) * 0.0131;
+  const double per_batch = (double)entries / ((double)l.p.stages * l.p.groups) / SP_BATCH + 0.15;
+  const double stage = 1.09 + l.p.groups_per_part * (per_batch > 1 ? per_batch : 1) * 0.015, fill = tying == CLT_TYING_NONE ? 1.72 : 0.52;
   const double stages = pairs * l.p.tiles * l.col_parts * l.p.parts / 256, longest = (double)L * l.p.tiles;
-  const double last = stages + 0.36 * longest > 1.2 * longest ? stages + 0.36 * longest : 1.2 * longest;
-  const double tiles_us = last * (stage_us > 1.6 ? stage_us : 1.6) + 20 + entries * 1.25e-5;
-  const GatherPrice gather = {18.1e6, 4.5e6, 5.5e6, 0.3};
-  const double sparse_us = gather.us(T, d, F, L, targets, entries, tying, 2);
-  return {tiles_us, sparse_us};
+  const double last = stages + 0.23 * longest > 1.06 * longest ? stages + 0.23 * longest : 1.06 * longest;
+  return last * (stage > fill ? stage : fill) + 13 + entries * 1.3e-5;
 }
 
 extern "C" int clt_decode_tiles_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying,
                                        int dtype) {
-  const TileTimes t = tile_times(T, d, F, L, targets, entries, tying, dtype);
-  return t.tiles < 0.95 * t.sparse;
-}
-
-double clt_decode_tiles_us(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype) {
-  return tile_times(T, d, F, L, targets, entries, tying, dtype).tiles;
+  const double us = clt_decode_tiles_us(T, d, F, L, targets, entries, tying, dtype);
+  return us < 1e30 && us < 0.95 * clt_decode_gather_us(T, d, F, L, targets, entries, tying, dtype);
 }
 
 extern "C" int64_t clt_decode_tiles_max_entries(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets) {
