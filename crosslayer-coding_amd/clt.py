@@ -339,9 +339,9 @@ class CrossLayerTranscoder(BaseTranscoder):
             dw_dec = engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
         _, x_slab, _, _ = self.encoder_module.prepare_slab(inputs)
         x_slab = x_slab.contiguous()
-        # ``encoder_step`` (an optimiser whose ``fuses_encoder_step(x)`` holds): likewise for the encoder weights, after everything
-        # that reads the old ones
-        encoder_step = encoder_step if encoder_step is not None and encoder_step.fuses_encoder_step(x_slab) else None
+        # ``encoder_step`` (an optimiser whose ``fuses_encoder_step(x, survivors)`` holds): likewise for the encoder weights, after
+        # everything that reads the old ones
+        encoder_step = encoder_step if encoder_step is not None and encoder_step.fuses_encoder_step(x_slab, surv.capacity) else None
         dw_enc = db_enc = None
         if encoder_step is None:
             dw_enc, db_enc = engine.encoder_weight_grad(lists, dval, x_slab, F)

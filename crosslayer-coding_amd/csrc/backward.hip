@@ -798,7 +798,7 @@ struct AdamInPlace {
   int64_t pitch;
   AdamCoef c;
 };
-constexpr int FO_ADAM_PIECES = 4;          // of an encoder row that takes its Adam step in place: rows of 4 KB, whose moments fit the registers
+constexpr int FO_ADAM_PIECES = 4;          // of an encoder row that takes its Adam step in place: rows of 4 KB, with 208 registers at most; lists: engine.encoder_step_wanted
 template <typename T, typename CoefT, int NCH, bool DECODER, bool T8 = false, bool ADAM = false>
 __global__ __launch_bounds__(BW_THREADS) void k_feature_outer(
     const int32_t *__restrict__ ptr, const int32_t *__restrict__ ltok, const int32_t *__restrict__ lsrc,

@@ -924,6 +924,16 @@ def encoder_step_fits(d: int, dtype: torch.dtype) -> bool:
     return d % (8 if dtype == torch.bfloat16 else 4) == 0 and d * dtype.itemsize <= 4096 and dtype in (torch.bfloat16, torch.float32)
 
 
+def encoder_step_wanted(entries: int, F: int, L: int) -> bool:
+    """Whether ``encoder_weight_grad_adam`` is the faster of the two ways for ``entries`` survivors of all layers.  What it saves is the
+    gradient's way through memory, the same for every list; its own gather has fewer wavefronts in flight, which long lists pay for.
+    Measured with cold caches at 117 shapes (bf16 d 256 - 2048, float32 256 - 1024), time / that of the two calls by entries of a list: 0.73 -
+    0.83 at 3, 0.82 - 0.93 at 16, 0.80 - 1.00 at 33; at 66 0.91 - 1.05 of 8192 features and 0.90 - 1.02 of 24576; at 133 0.94 - 1.08 and
+    0.93 - 1.08; at 266 0.95 - 1.10."""
+    per_list = entries / (L * F)
+    return per_list <= 48 or (per_list <= 96 and F >= 16384)
+
+
 def encoder_weight_grad_adam(lists, dval: torch.Tensor, x: torch.Tensor, w: torch.Tensor, m: torch.Tensor, v: torch.Tensor,
                              lr: float, betas, eps: float, step: int, db: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``encoder_weight_grad`` with the Adam step ``step`` of the stacked weights ``w`` and their moments [L, F, d] taken on the

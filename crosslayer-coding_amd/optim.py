@@ -81,13 +81,13 @@ class CLTAdam:
         return (self.fuse_decoder_step and self.model.config.decoder_tying == "none"
                 and dec.feature_offset is None and dec.feature_scale is None)
 
-    def fuses_encoder_step(self, x: torch.Tensor) -> bool:
-        """Whether the encoder weights can take their Adam step inside the weight-gradient kernel, for the batch ``x`` [L, T, d]
-        (``fuse_encoder_step = False`` switches it off)."""
+    def fuses_encoder_step(self, x: torch.Tensor, entries: int = 0) -> bool:
+        """Whether the encoder weights take their Adam step inside the weight-gradient kernel, for the batch ``x`` [L, T, d] with
+        ``entries`` survivors (``fuse_encoder_step = False`` switches it off)."""
         from . import engine
         w, _ = self.model.encoder_module.stacked()
         return (self.fuse_encoder_step and w.dtype == x.dtype and engine.encoder_step_fits(x.shape[2], x.dtype)
-                and engine._aligned16(x, w, *self.state["enc_w"]))
+                and engine.encoder_step_wanted(entries, w.shape[1], w.shape[0]) and engine._aligned16(x, w, *self.state["enc_w"]))
 
     @torch.no_grad()
     def encoder_weight_step(self, lists, dval: torch.Tensor, x: torch.Tensor, db: torch.Tensor) -> None:

@@ -73,3 +73,22 @@ def test_a_step_that_finds_no_memory_leaves_the_model_as_it_was(monkeypatch, dty
         loss = model.training_step(inputs, targets, opt)
         ends.append([loss] + state())
     assert all(torch.equal(a, b) for a, b in zip(*ends))
+
+
+@pytest.mark.parametrize("T,taken", [(256, True), (700, False)])
+def test_a_training_step_takes_it_for_short_lists(monkeypatch, T, taken):
+    """24 of 128 features fire per token: lists of 48 and of 131 entries; the same bits either way."""
+    import crosslayer_coding_amd as cca
+    from crosslayer_coding_amd import synth
+    wl, ends, ran = synth.Workload("lists", 5, 2, 64, 128, T, "bfloat16", k=24), [], []
+    real = engine.encoder_weight_grad_adam
+    monkeypatch.setattr(engine, "encoder_weight_grad_adam", lambda *a: ran.append(1) or real(*a))
+    for fuse in (True, False):
+        model, x, _ = synth.build_model(wl, torch.device("cuda:0"), 1)
+        y = synth.make_targets(wl, torch.device("cuda:0"), 1)
+        opt = cca.CLTAdam(model, lr=1e-2)
+        opt.fuse_encoder_step = fuse
+        model.training_step({l: x[l] for l in range(2)}, {l: y[l] for l in range(2)}, opt)
+        ends.append([t.clone() for t in (*model.encoder_module.stacked(), *opt.state["enc_w"], *opt.state["enc_b"])])
+    assert ran == ([1] if taken else [])
+    assert all(torch.equal(a, b) for a, b in zip(*ends))
