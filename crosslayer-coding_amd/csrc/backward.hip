@@ -1493,7 +1493,12 @@ extern "C" int clt_encoder_weight_grad_adam(const int32_t *list_ptr, const int32
     case 1: CLT_EWA(ST, 1, false); break; case 2: CLT_EWA(ST, 2, false); break;                      \
     case 3: CLT_EWA(ST, 3, false); break; default: CLT_EWA(ST, 4, false); break;                     \
   }
-  if (dtype == CLT_BF16 && d == 768) CLT_EWA(bf16_t, 2, true);
+  // Rows of one or two and a half pieces: a half last piece for every lane rather than a whole one for half of them.  4 layers of 8192
+  // features, us, halves / whole pieces: d = 768, 33 entries 285 / 290, 133 774 / 871; d = 1280, 33 467 / 487, 133 1407 / 1501.  (Three and
+  // a half, d = 1792: 698 / 718 at 33, but 274 / 241 at 3.)
+  const bool halves = dtype == CLT_BF16 && d == (nc4 - 1) * 512 + 256;
+  if (halves && nc4 == 2) CLT_EWA(bf16_t, 2, true);
+  else if (halves && nc4 == 3) CLT_EWA(bf16_t, 3, true);
   else if (dtype == CLT_BF16) { CLT_EWA_N(bf16_t) }
   else { CLT_EWA_N(float) }
 #undef CLT_EWA_N

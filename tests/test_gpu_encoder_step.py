@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("d,dtype", [
-    (8, torch.bfloat16), (136, torch.bfloat16), (768, torch.bfloat16), (1024, torch.bfloat16), (1032, torch.bfloat16), (2048, torch.bfloat16),
+    (8, torch.bfloat16), (136, torch.bfloat16), (768, torch.bfloat16), (1024, torch.bfloat16), (1032, torch.bfloat16), (2048, torch.bfloat16), (256, torch.bfloat16), (1280, torch.bfloat16), (1792, torch.bfloat16),
     (4, torch.float32), (68, torch.float32), (512, torch.float32), (768, torch.float32), (1024, torch.float32),
 ])
 def test_encoder_step_in_the_gradient_kernel(d, dtype):
