@@ -109,6 +109,7 @@ _SIGNATURES = {
     "clt_grad_tiles_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64, _i64]),
     "clt_decoder_grad_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "clt_decoder_grad_param_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "clt_decoder_grad_params_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "clt_decoder_grad_adam_tiles": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64, _f64, _f64, _f64,
                                            _f64, _i64, _int, _vp, _sz, _vp]),
     "clt_decoder_tile_width": (_int, [_i64, _i64, _i64, _int]),

@@ -83,11 +83,13 @@ class _ReconstructionsWithGraph(torch.autograd.Function):
                     g[l] = go.reshape(T, d)
             g_model = g.to(model.dtype)
         raw = model._raw_gradients_from(ctx.inputs, surv, g, g_model, g.sum(dim=1), as_parameters=True)
-        # families of parameters in one cast each: the gradients are views of one tensor, as a float32 model's are
-        if all(p.dtype == model.dtype for n, p in zip(ctx.names, ctx.params) if not n.startswith("theta_manager.")):
+        # families of parameters in one cast each; every parameter's gradient has memory of its own, so that one that is kept or
+        # saved holds no other
+        if (model.dtype != torch.float32
+                and all(p.dtype == model.dtype for n, p in zip(ctx.names, ctx.params) if not n.startswith("theta_manager."))):
             for key in ("enc_w", "enc_b", "dec_b", "skip"):
                 if raw.get(key) is not None:
-                    raw[key] = raw[key].to(model.dtype)
+                    raw[key] = engine.parameter_gradients(raw[key], model.dtype)
         named = model._named_gradients(raw)
         grads = []
         for name, p in zip(ctx.names, ctx.params):
@@ -308,7 +310,7 @@ class CrossLayerTranscoder(BaseTranscoder):
         """The raw parameter gradients (see ``_loss_and_raw_gradients``) of any loss, given d loss / d reconstruction:
         ``g`` fp32 [L, T, d], ``g_model`` the same in the model dtype, ``bias_grad`` [L, d] its sums over tokens.
         ``surv`` is the (trimmed) survivor list of the forward on ``inputs``.  ``as_parameters``: decoder gradients may come in their
-        parameters' layout and dtype instead, as ``dec_param`` [n_dec, d, F] (``dec_w`` is None then)."""
+        parameters' layout and dtype instead, as ``dec_param``, n_dec tensors [d, F] (``dec_w`` is None then)."""
         cfg = self.config
         L, d, F = cfg.num_layers, cfg.d_model, cfg.num_features
         ws = self._workspace()
@@ -334,7 +336,7 @@ class CrossLayerTranscoder(BaseTranscoder):
         # step inside the weight-gradient kernel, after everything that reads the old decoders (below)
         dw_dec = dw_param = None
         if as_parameters and cfg.decoder_tying == "none" and off is None and sc is None:
-            dw_param = engine.decoder_parameter_grad(lists, surv, g_model, ws)
+            dw_param = engine.decoder_parameter_grad(lists, surv, g_model, ws, separate=True)
         if decoder_step is None and dw_param is None:
             dw_dec = engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying, off, sc, ws)
         _, x_slab, _, _ = self.encoder_module.prepare_slab(inputs)

@@ -446,7 +446,8 @@ struct GradArgs {
   const void *g;             // [L][T][d]
   void *w;                   // packed decoders (GT_ADAM)
   float *m, *v;              // moments
-  void *out;                 // the gradient otherwise: fp32 [n_dec][F][d] (GT_ROWS) or of T [n_dec][d][F] (GT_PARAM)
+  float *out;                // the gradient as fp32 [n_dec][F][d] (GT_ROWS)
+  void *const *params;       // [n_dec] where each decoder's gradient goes, [d][F] of T (GT_PARAM)
   int64_t Tn, d, F, L, pitch, max_entries;
   int64_t m_row, m_cols, m_dec;   // moments: elements between rows, between column parts of 64 and between decoders
   const int32_t *list_total, *list_ptr, *list_tok, *list_src;
@@ -549,7 +550,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
     __syncthreads();
     const int64_t f = (int64_t)part * A.p.groups_per_part * SP_GROUP + lane * 8;
     if (lane * 8 < A.p.groups_per_part * SP_GROUP && f < A.F) {      // (F is a multiple of eight)
-      T *const out = (T *)A.out + ((int64_t)slot * A.d + (int64_t)cp * SP_COLS) * A.F + f;
+      T *const out = (T *)A.params[slot] + (int64_t)cp * SP_COLS * A.F + f;
 #pragma unroll
       for (int c = wave; c < SP_COLS; c += GT_WAVES)
         *reinterpret_cast<uint4 *>(out + c * A.F) = *reinterpret_cast<const uint4 *>(cols + c * GT_PARAM_PITCH + lane * 8);
@@ -604,7 +605,7 @@ __global__ __launch_bounds__(GT_WAVES * 64, 4) void k_grad_tiles(GradArgs A) {
         __builtin_nontemporal_store(vv[i], reinterpret_cast<f32x4v_t *>(v_at + 4 * i * A.m_row));
         *reinterpret_cast<uint2 *>(w_at + 4 * i * A.pitch) = make_uint2(pack_pair<T>(p[0], p[1]), pack_pair<T>(p[2], p[3]));
       } else {
-        __builtin_nontemporal_store(gr, reinterpret_cast<f32x4v_t *>((float *)A.out + ((int64_t)slot * A.F + f0 + 4 * i) * A.d + (int64_t)cp * SP_COLS + c4));
+        __builtin_nontemporal_store(gr, reinterpret_cast<f32x4v_t *>(A.out + ((int64_t)slot * A.F + f0 + 4 * i) * A.d + (int64_t)cp * SP_COLS + c4));
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");    // read before the next group's sums are written
@@ -643,8 +644,8 @@ template <typename T, GradOut OUT> __global__ __launch_bounds__(256) void k_grad
       const int64_t c = (int64_t)cp * SP_COLS + c4;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        if constexpr (OUT == GT_ROWS) ((float *)A.out)[(slot * A.F + f) * A.d + c + q] = gr[q];
-        else ((T *)A.out)[(slot * A.d + c + q) * A.F + f] = Elem<T>::from_f32(gr[q]);
+        if constexpr (OUT == GT_ROWS) A.out[(slot * A.F + f) * A.d + c + q] = gr[q];
+        else ((T *)A.params[slot])[(c + q) * A.F + f] = Elem<T>::from_f32(gr[q]);
       }
     }
   }
@@ -657,7 +658,7 @@ struct SpLayout {
   SpPlan p;
   int col_parts;
   int64_t n_batches, n_groups;
-  size_t bad, start, batches, counts, offset, total, recs, bytes;
+  size_t bad, start, batches, counts, offset, total, recs, params, bytes;
 };
 
 // `rows` output rows and `cols` tile rows per layer; `per_part` workgroups for every part of the rows; `outputs` times that
@@ -691,6 +692,7 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
   l.recs = take((size_t)rec_batches * SP_REC_WORDS * 4);
   l.n_groups = outputs * p.groups * l.col_parts;
   l.bad = take(sizeof(uint32_t) * (size_t)(l.n_groups + 1));
+  l.params = take(sizeof(void *) * (size_t)outputs);
   l.bytes = at;
   return l;
 }
@@ -742,8 +744,16 @@ static SpLayout grad_layout(int64_t T, int64_t d, int64_t F, int64_t L, int64_t 
   return sp_layout(F, T, d, L, GT_WAVES, 1 << 20, L * (L + 1) / 2, entries);
 }
 
+// Addresses as kernel arguments, so that nothing on the host has to outlive the call.
+constexpr int ADDRESSES = 256;
+struct Addresses { void *at[ADDRESSES]; };
+__global__ __launch_bounds__(ADDRESSES) void k_set_addresses(Addresses a, int n, void **to) {
+  if ((int)threadIdx.x < n) to[threadIdx.x] = a.at[threadIdx.x];
+}
+
+// `params`: host array of n_dec addresses (GT_PARAM)
 static int launch_grad(GradOut out, const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val, GradArgs a,
-                       void *workspace, size_t workspace_bytes, hipStream_t stream) {
+                       void *const *params, void *workspace, size_t workspace_bytes, hipStream_t stream) {
   const SpLayout l = grad_layout(a.Tn, a.d, a.F, a.L, a.max_entries);
   if (!sp_shape_ok(l, a.d * 2)) return CLT_ERR_RANGE;
   if (workspace_bytes < l.bytes) return CLT_ERR_WORKSPACE;
@@ -770,6 +780,15 @@ static int launch_grad(GradOut out, const int32_t *list_ptr, const int32_t *list
     k_grad_tiles<bf16_t, GT_ROWS><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
     k_grad_repair<bf16_t, GT_ROWS><<<REPAIR_BLOCKS, 256, 0, stream>>>(a);
   } else {
+    void **const table = (void **)((char *)workspace + l.params);
+    const int n_dec = (int)(a.L * (a.L + 1) / 2);
+    for (int i0 = 0; i0 < n_dec; i0 += ADDRESSES) {
+      Addresses some;
+      const int n = n_dec - i0 < ADDRESSES ? n_dec - i0 : ADDRESSES;
+      for (int i = 0; i < ADDRESSES; ++i) some.at[i] = i < n ? params[i0 + i] : nullptr;
+      k_set_addresses<<<1, ADDRESSES, 0, stream>>>(some, n, table + i0);
+    }
+    a.params = table;
     k_grad_tiles<bf16_t, GT_PARAM><<<(unsigned)blocks, GT_WAVES * 64, GT_LDS, stream>>>(a);
     k_grad_repair<bf16_t, GT_PARAM><<<REPAIR_BLOCKS, 256, 0, stream>>>(a);
   }
@@ -858,31 +877,46 @@ extern "C" size_t clt_grad_tiles_workspace_bytes(int64_t T, int64_t d, int64_t F
 }
 
 static int grad_tiles(GradOut kind, const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
-                      const void *g_model, void *out, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype,
-                      void *workspace, size_t workspace_bytes, void *stream) {
+                      const void *g_model, float *out, void *const *params, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
+                      int dtype, void *workspace, size_t workspace_bytes, void *stream) {
   if (dtype != CLT_BF16) return CLT_ERR_DTYPE;
   if (!clt_grad_tiles_supported(T, d, F, L, entries, dtype)) return CLT_ERR_ARG;
-  if (!list_ptr || !list_tok || !list_src || !val || !g_model || !out || !workspace) return CLT_ERR_ARG;
+  if (!list_ptr || !list_tok || !list_src || !val || !g_model || !(kind == GT_ROWS ? (const void *)out : (const void *)params) || !workspace)
+    return CLT_ERR_ARG;
   if (!clt_aligned16(g_model) || !clt_aligned16(out) || !clt_aligned16(workspace)) return CLT_ERR_ALIGN;
+  for (int64_t i = 0; kind == GT_PARAM && i < L * (L + 1) / 2; ++i) {
+    if (!params[i]) return CLT_ERR_ARG;
+    if (!clt_aligned16(params[i])) return CLT_ERR_ALIGN;
+  }
   GradArgs a{};
   a.g = g_model; a.out = out;
   a.Tn = T; a.d = d; a.F = F; a.L = L; a.max_entries = entries;
-  return launch_grad(kind, list_ptr, list_tok, list_src, val, a, workspace, workspace_bytes, (hipStream_t)stream);
+  return launch_grad(kind, list_ptr, list_tok, list_src, val, a, params, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 extern "C" int clt_decoder_grad_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
                                       const void *g_model, float *out, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
                                       int dtype, void *workspace, size_t workspace_bytes, void *stream) {
-  return grad_tiles(GT_ROWS, list_ptr, list_tok, list_src, val, g_model, out, T, d, F, L, entries, dtype, workspace, workspace_bytes,
-                    stream);
+  return grad_tiles(GT_ROWS, list_ptr, list_tok, list_src, val, g_model, out, nullptr, T, d, F, L, entries, dtype, workspace,
+                    workspace_bytes, stream);
+}
+
+extern "C" int clt_decoder_grad_params_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
+                                             const void *g_model, void *const *outs, int64_t T, int64_t d, int64_t F, int64_t L,
+                                             int64_t entries, int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  if (F % 8 != 0) return CLT_ERR_ARG;
+  return grad_tiles(GT_PARAM, list_ptr, list_tok, list_src, val, g_model, nullptr, outs, T, d, F, L, entries, dtype, workspace,
+                    workspace_bytes, stream);
 }
 
 extern "C" int clt_decoder_grad_param_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
                                             const void *g_model, void *out, int64_t T, int64_t d, int64_t F, int64_t L,
                                             int64_t entries, int dtype, void *workspace, size_t workspace_bytes, void *stream) {
-  if (F % 8 != 0) return CLT_ERR_ARG;
-  return grad_tiles(GT_PARAM, list_ptr, list_tok, list_src, val, g_model, out, T, d, F, L, entries, dtype, workspace, workspace_bytes,
-                    stream);
+  if (!out || L <= 0 || L > 64) return CLT_ERR_ARG;
+  void *outs[64 * 65 / 2];
+  for (int64_t i = 0; i < L * (L + 1) / 2; ++i) outs[i] = (char *)out + i * d * F * 2;
+  return clt_decoder_grad_params_tiles(list_ptr, list_tok, list_src, val, g_model, outs, T, d, F, L, entries, dtype, workspace,
+                                       workspace_bytes, stream);
 }
 
 extern "C" int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
@@ -902,5 +936,5 @@ extern "C" int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_
   a.m_row = moments_by_tile ? SP_COLS : d;
   a.m_cols = moments_by_tile ? F * SP_COLS : SP_COLS;
   a.adam = adam_coef(lr, beta1, beta2, eps, step);
-  return launch_grad(GT_ADAM, list_ptr, list_tok, list_src, val, a, workspace, workspace_bytes, (hipStream_t)stream);
+  return launch_grad(GT_ADAM, list_ptr, list_tok, list_src, val, a, nullptr, workspace, workspace_bytes, (hipStream_t)stream);
 }

@@ -13,6 +13,7 @@ Layouts
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Dict, List, Optional
 
@@ -686,20 +687,26 @@ def grad_tiles_supported(T: int, d: int, F: int, L: int, entries: int, dtype: to
     return dtype == torch.bfloat16 and bool(nat.load().clt_grad_tiles_supported(T, d, F, L, entries, nat.dtype_code(dtype)))
 
 
-def decoder_parameter_grad(lists, surv: SurvivorList, g: torch.Tensor, ws: Optional[Workspace] = None) -> Optional[torch.Tensor]:
-    """Gradients of untied decoders in their parameters' layout and dtype, [n_dec, d, F]: ``decoder_weight_grad``'s rounded once and
-    transposed, in one pass.  None where the matrix-core kernels do not take the shapes."""
+def decoder_parameter_grad(lists, surv: SurvivorList, g: torch.Tensor, ws: Optional[Workspace] = None, separate: bool = False):
+    """Gradients of untied decoders in their parameters' layout and dtype, [n_dec, d, F] or, ``separate``, a list of n_dec tensors
+    [d, F] with memory of their own: ``decoder_weight_grad``'s rounded once and transposed, in one pass.  None where the matrix-core
+    kernels do not take the shapes."""
     ptr, tok, src = lists
     L, T, F = surv.L, surv.T, surv.F
-    d, n = g.shape[2], surv.capacity
+    d, n, n_dec = g.shape[2], surv.capacity, surv.L * (surv.L + 1) // 2
     if g.dtype != surv.dtype or F % 8 or not _aligned16(g) or not g.is_contiguous() or not grad_tiles_supported(T, d, F, L, n, surv.dtype):
         return None
-    out = torch.empty((L * (L + 1) // 2, d, F), dtype=surv.dtype, device=g.device)
+    if separate:
+        out = [torch.empty((d, F), dtype=surv.dtype, device=g.device) for _ in range(n_dec)]
+    else:
+        out = torch.empty((n_dec, d, F), dtype=surv.dtype, device=g.device)
+    addresses = (ctypes.c_void_p * n_dec)(*[t.data_ptr() for t in out])
     lib = nat.load()
     wbuf = (ws or Workspace(g.device)).get("grad_tiles", lib.clt_grad_tiles_workspace_bytes(T, d, F, L, n))
-    code = lib.clt_decoder_grad_param_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(out), T, d,
-                                            F, L, n, nat.dtype_code(surv.dtype), nat.ptr(wbuf), wbuf.numel(), _stream(g))
-    nat.check(code, "clt_decoder_grad_param_tiles")
+    code = lib.clt_decoder_grad_params_tiles(nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g),
+                                             ctypes.addressof(addresses), T, d, F, L, n, nat.dtype_code(surv.dtype), nat.ptr(wbuf),
+                                             wbuf.numel(), _stream(g))
+    nat.check(code, "clt_decoder_grad_params_tiles")
     return out
 
 
@@ -802,7 +809,6 @@ def decoder_grad_adam_rows(lists, surv: SurvivorList, g: torch.Tensor, w_packed:
 def unpack_decoders(w_packed: torch.Tensor, w_refs_dev: torch.Tensor, w_refs_host, d: int, F: int) -> None:
     """Checkpoint-layout parameters [d, F] (their addresses in the device int64 tensor ``w_refs_dev`` and in the
     host ctypes array ``w_refs_host``) from the packed working copy [n_dec, F, pitch]."""
-    import ctypes
     n_dec = w_packed.shape[0]
     assert w_refs_dev.dtype == torch.int64 and w_refs_dev.numel() == n_dec and w_packed.is_contiguous()
     code = nat.load().clt_unpack_decoders(nat.ptr(w_packed), nat.ptr(w_refs_dev), ctypes.addressof(w_refs_host), n_dec, d, F,
@@ -866,7 +872,6 @@ def untile_decoders(w_tiles: torch.Tensor, w_packed: torch.Tensor, w_refs_dev: O
                     w_refs_host=None) -> None:
     """The feature-major slab [n_dec, F, pitch] and (when their addresses are given, as for ``unpack_decoders``)
     the checkpoint-layout parameters [d, F], rewritten from the tiled weights."""
-    import ctypes
     n_dec, ns, F, cs = w_tiles.shape
     d = ns * cs
     assert w_tiles.is_contiguous() and w_packed.is_contiguous() and w_packed.dtype == w_tiles.dtype
@@ -966,6 +971,13 @@ def parameter_gradient(g: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
         nat.check(code, "clt_transpose_grad")
         return out
     return g.to(dtype)
+
+
+def parameter_gradients(stack: torch.Tensor, dtype: torch.dtype) -> List[torch.Tensor]:
+    """The raw gradients of a family of parameters, [n, ...], as n tensors of ``dtype`` with memory of their own, in few launches."""
+    out = [torch.empty(stack.shape[1:], dtype=dtype, device=stack.device) for _ in range(stack.shape[0])]
+    torch._foreach_copy_(out, list(stack.unbind(0)))
+    return out
 
 
 def scatter_survivor_values(surv: SurvivorList, src: torch.Tensor, layer: int, dense: torch.Tensor) -> None:

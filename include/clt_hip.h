@@ -695,6 +695,8 @@ int clt_unpack_decoders(const void *w_packed, void *const *w_refs_dev, void *con
  * decoder.py:253-338), entries = list_ptr[L*F].
  *   clt_decoder_grad_tiles       writes it, fp32 [n_dec][F][d]
  *   clt_decoder_grad_param_tiles writes it rounded once to bf16 in the parameters' layout [n_dec][d][F]; F a multiple of 8
+ *   clt_decoder_grad_params_tiles the same, each decoder's [d][F] to an address of its own (`outs`: host array of n_dec, read
+ *                                before the call returns; 16-byte aligned)
  *   clt_decoder_grad_adam_tiles  takes the Adam step instead: w_packed (clt_decoder_pitch rows) and both fp32 moments are
  *                                updated in place; moments [n_dec][F][d], or [n_dec][d / 64][F][64] (moments_by_tile)
  * Equal to clt_decoder_weight_grad / clt_decoder_weight_grad_adam up to fp32 summation order, repeatable bit for bit.
@@ -707,6 +709,9 @@ int clt_decoder_grad_tiles(const int32_t *list_ptr, const int32_t *list_tok, con
 int clt_decoder_grad_param_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
                                  const void *g_model, void *out, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
                                  int dtype, void *workspace, size_t workspace_bytes, void *stream);
+int clt_decoder_grad_params_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
+                                  const void *g_model, void *const *outs, int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries,
+                                  int dtype, void *workspace, size_t workspace_bytes, void *stream);
 int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_t *list_tok, const int32_t *list_src, const void *val,
                                 const void *g_model, void *w_packed, float *m, float *v, int moments_by_tile, int64_t T,
                                 int64_t d, int64_t F, int64_t L, int64_t entries, double lr, double beta1, double beta2,
