@@ -44,7 +44,7 @@ struct RunArgs {
   const int32_t *row_ptr, *col;
   const int32_t *src;      // the entry's value is val[src[j]]; null: val[j]
   const float *val;
-  int64_t Tn, L;
+  int64_t Tn, L, max_entries;      // what the records have room for: longer lists are left alone
   uint64_t layer_mask;
   RowPlan p;
   int32_t *start;          // [L * groups][DR_TOK][tiles + 1] list position where a token's entries of a tile begin
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(DR_FIRSTS) void k_row_firsts(uint32_t *total, int s
 __global__ __launch_bounds__(DR_THREADS) void k_row_fill(RunArgs A) {
   extern __shared__ int32_t fill_lds[];
   const int g = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, tiles = A.p.tiles, lane = tid & 63;
-  if (!((A.layer_mask >> s) & 1ull)) return;
+  if (A.row_ptr[A.L * A.Tn] > A.max_entries || !((A.layer_mask >> s) & 1ull)) return;
   int32_t *start = fill_lds;                               // [DR_TOK][tiles + 1]
   uint32_t *dest = (uint32_t *)(start + DR_TOK * (tiles + 1));      // [DR_TOK][tiles] first record of the run
   const int64_t tok0 = (int64_t)g * DR_TOK, r0 = (int64_t)s * A.Tn + tok0;
@@ -189,7 +189,7 @@ struct RowArgs {
   float *out;
   const int32_t *row_ptr, *col;
   const float *val;
-  int64_t Tn, d, F, L, pitch;
+  int64_t Tn, d, F, L, pitch, max_entries;
   uint64_t src_mask;
   int tying, t_begin, t_end, col_parts;
 };
@@ -352,6 +352,7 @@ typedef uint32_t dr_u32x16_t __attribute__((ext_vector_type(16)));
 // word per lane, handed out by DPP operands (bound by instruction issue).
 __global__ __launch_bounds__(DR_WAVES * 64) void k_decode_rows(RowArgs A) {
   extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  if (A.row_ptr[A.L * A.Tn] > A.max_entries) return;
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
   const int pair = (seq / A.p.parts) * 8 + xcd, part = seq % A.p.parts;
@@ -508,7 +509,7 @@ struct GradRowArgs {
   float *w, *m, *v;          // packed decoders, moments
   const int32_t *list_ptr, *list_tok, *list_src;
   const float *val;
-  int64_t Tn, d, F, L, pitch;
+  int64_t Tn, d, F, L, pitch, max_entries;
   int64_t m_row, m_cols;     // moments: elements between rows and between column parts of eight
   int col_parts, items;      // items of one (source, target) pair per XCD
   AdamCoef adam;
@@ -522,6 +523,7 @@ struct GradRowArgs {
 // is the chain of a workgroup, tile, sums, tile, sums, moments, of which a CU has two under way.
 __global__ __launch_bounds__(GR_WAVES * 64, 4) void k_grad_rows(GradRowArgs A) {
   extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  if (A.list_ptr[A.L * A.F] > A.max_entries) return;
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int xcd = blockIdx.x & 7, seq = blockIdx.x >> 3;
   const int slot_dec = seq / A.items, item = xcd * A.items + seq % A.items;
@@ -787,14 +789,14 @@ extern "C" int clt_decode_rows(const int32_t *row_ptr, const int32_t *col, const
   hipStream_t s = (hipStream_t)stream;
   char *ws = (char *)workspace;
   RunArgs ra;
-  ra.row_ptr = row_ptr; ra.col = col; ra.src = nullptr; ra.val = val; ra.Tn = T; ra.L = L; ra.layer_mask = src_mask; ra.p = l.p;
+  ra.row_ptr = row_ptr; ra.col = col; ra.src = nullptr; ra.val = val; ra.Tn = T; ra.L = L; ra.max_entries = entries; ra.layer_mask = src_mask; ra.p = l.p;
   ra.start = (int32_t *)(ws + l.start); ra.counts = (uint4 *)(ws + l.counts); ra.offset = (uint32_t *)(ws + l.offset);
   ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint2 *)(ws + l.recs);
   RowArgs a;
   a.p = l.p; a.counts = ra.counts; a.total = ra.total; a.recs = ra.recs;
   a.wp = w_packed; a.bias_sum = bias_sum; a.skip_add = skip_add; a.out = out;
   a.row_ptr = row_ptr; a.col = col; a.val = val;
-  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = pitch; a.src_mask = src_mask;
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = pitch; a.max_entries = entries; a.src_mask = src_mask;
   a.tying = tying; a.t_begin = (int)t_begin; a.t_end = (int)t_end; a.col_parts = l.col_parts;
   const int64_t pairs = clt_ceil_div((t_end - t_begin) * l.col_parts, 8) * 8;
   if (pairs * l.p.parts > 0x7FFFFFFFll) return CLT_ERR_RANGE;
@@ -851,14 +853,14 @@ extern "C" int clt_decoder_grad_adam_rows(const int32_t *list_ptr, const int32_t
   hipStream_t s = (hipStream_t)stream;
   char *ws = (char *)workspace;
   RunArgs ra;
-  ra.row_ptr = list_ptr; ra.col = list_tok; ra.src = list_src; ra.val = val; ra.Tn = F; ra.L = L; ra.layer_mask = ~0ull; ra.p = l.p;
+  ra.row_ptr = list_ptr; ra.col = list_tok; ra.src = list_src; ra.val = val; ra.Tn = F; ra.L = L; ra.max_entries = entries; ra.layer_mask = ~0ull; ra.p = l.p;
   ra.start = (int32_t *)(ws + l.start); ra.counts = (uint4 *)(ws + l.counts); ra.offset = (uint32_t *)(ws + l.offset);
   ra.total = (uint32_t *)(ws + l.total); ra.recs = (uint2 *)(ws + l.recs);
   GradRowArgs a;
   a.p = l.p; a.counts = ra.counts; a.first = ra.total; a.recs = ra.recs;
   a.g = g; a.w = w_packed; a.m = m; a.v = v;
   a.list_ptr = list_ptr; a.list_tok = list_tok; a.list_src = list_src; a.val = val;
-  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = clt_pitch(d, 4);
+  a.Tn = T; a.d = d; a.F = F; a.L = L; a.pitch = clt_pitch(d, 4); a.max_entries = entries;
   a.m_row = moments_by_tile ? 8 : d;
   a.m_cols = moments_by_tile ? F * 8 : 8;
   a.col_parts = l.col_parts;

@@ -438,7 +438,7 @@ int clt_decode_thin_up_to(const int32_t *row_ptr, const int32_t *col, const void
  * Deterministic, equal to clt_decode_sparse up to fp32 summation order.
  *   clt_decode_rows_wanted: whether it is the faster of the two for `entries` survivors over L layers and `targets` target
  *   layers (0 also for what it does not take).
- *   `entries` must be no less than the list's length: the workspace is sized for it.
+ *   `entries` must be no less than the list's length: the workspace is sized for it, and of a longer list no row is written.
  */
 int clt_decode_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t targets, int64_t entries, int tying, int dtype);
 size_t clt_decode_rows_workspace_bytes(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries);
@@ -719,7 +719,8 @@ int clt_decoder_grad_adam_tiles(const int32_t *list_ptr, const int32_t *list_tok
 /*
  * The same Adam step for float32, d a multiple of 32, from LDS tiles: w_packed (clt_decoder_pitch rows) and both moments [n_dec][F][d],
  * or [n_dec][d / 8][F][8] (moments_by_tile), are updated in place; val and g fp32.  _wanted: 1 where it is the fastest by its shape, 2 where clt_decoder_weight_grad_adam is.
- * Equal to clt_decoder_weight_grad_adam up to summation order, repeatable bit for bit.
+ * Equal to clt_decoder_weight_grad_adam up to summation order, repeatable bit for bit.  `entries` must be no less than list_ptr[L*F]: the
+ * workspace is sized for it, and with longer lists nothing is stepped.
  */
 int clt_grad_rows_supported(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype);
 int clt_grad_rows_wanted(int64_t T, int64_t d, int64_t F, int64_t L, int64_t entries, int dtype);

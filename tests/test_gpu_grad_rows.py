@@ -112,3 +112,33 @@ def test_training_takes_the_step_and_keeps_its_state_across_routes():
     for k, p in a[3].items():                              # parameters are what the packed copy holds
         if k.startswith("decoder_module.decoders.") and k.endswith(".weight"):
             assert float((p - b[3][k]).norm() / b[3][k].norm()) < 1e-4, k
+
+
+def _called_with(entries, surv, w, m, v, g, out):
+    """Both kernels with `entries` in the place of the list's length, on a workspace of that many in the middle of a larger one."""
+    from crosslayer_coding_amd import _native as nat
+    lib, (ptr, tok, src) = nat.load(), engine.feature_lists(surv)
+    L, T, F, d = surv.L, surv.T, surv.F, g.shape[2]
+    edges = []
+    for need, call in (
+            (lib.clt_grad_rows_workspace_bytes(T, d, F, L, entries), lambda ws, n: lib.clt_decoder_grad_adam_rows(
+                nat.ptr(ptr), nat.ptr(tok), nat.ptr(src), nat.ptr(surv.val), nat.ptr(g), nat.ptr(w), nat.ptr(m), nat.ptr(v), 0, T, d, F, L,
+                entries, 1e-2, 0.9, 0.999, 1e-8, 1, ws, n, nat.current_stream(g.device))),
+            (lib.clt_decode_rows_workspace_bytes(T, d, F, L, entries), lambda ws, n: lib.clt_decode_rows(
+                nat.ptr(surv.row_ptr), nat.ptr(surv.col), nat.ptr(surv.val), nat.ptr(w), None, None, nat.ptr(out), T, d, F, L, 0, 0, L,
+                (1 << L) - 1, entries, ws, n, nat.current_stream(g.device)))):
+        room = torch.full((need + (4 << 20),), 0x5A, dtype=torch.uint8, device=g.device)
+        assert call(room.data_ptr(), need) == 0
+        torch.cuda.synchronize()
+        edges.append(bool((room[need:] == 0x5A).all()))
+    return edges
+
+
+def test_lists_longer_than_the_workspace_holds_are_left_alone():
+    surv, _, w, m, v, g = _problem(2, 600, 300, 64, 0.05, 5)
+    out = torch.full((2, 600, 64), 7.0).cuda()
+    w1, m1, v1, out1 = w.clone(), m.clone(), v.clone(), out.clone()
+    assert _called_with(surv.capacity - 1, surv, w1, m1, v1, g.cuda(), out1) == [True, True]
+    assert torch.equal(w1, w) and torch.equal(m1, m) and torch.equal(v1, v) and torch.equal(out1, out)
+    assert _called_with(surv.capacity, surv, w1, m1, v1, g.cuda(), out1) == [True, True]
+    assert not torch.equal(w1, w) and not torch.equal(out1, out)
