@@ -205,6 +205,8 @@ struct RowArgs {
 typedef float dr_f32x32_t __attribute__((ext_vector_type(32)));
 typedef uint32_t dr_u32x16_t __attribute__((ext_vector_type(16)));
 
+// A row's place (bits 7 - 16) is put together with the lane's column by an exclusive choice of bits: the tiles begin at LDS address 0, where
+// dynamic LDS lies as long as the kernels and what is inlined into them have no static __shared__ of their own.
 #define DR_ROW(W, S) "v_and_or_b32 v96, " W ", %[inside], %[col]\n\tds_read_b128 v[" S "], v96\n\t"
 // At places 0 and 4 the next quad is read (seven were asked for since that one, and the four loads of a tile if that is less than
 // eight quads ago); two places later it has arrived, and its slot goes to the quad eight on.
