@@ -38,6 +38,9 @@ constexpr int SP_REC_WORDS = 64;
 constexpr int SP_QUAD = 4;                           // batches of a quad
 constexpr int SP_QUAD_BYTES = SP_QUAD * SP_REC_WORDS * 4;
 constexpr int SP_RING_BYTES = 2 * SP_QUAD_BYTES;     // quads that a wavefront keeps in LDS or on their way
+// Batches past the end of the last stream that are asked for: three quads are under way or read when the first batch is taken up, and one
+// more is asked for whenever a quad is through.
+constexpr int SP_PAST_END = 3 * SP_QUAD;
 // where word `w` of batch `b` (counted over all streams) lies
 __device__ __forceinline__ uint64_t sp_rec_word(uint64_t b, uint32_t w) {
   return (b / SP_QUAD) * (SP_QUAD * SP_REC_WORDS) + w * SP_QUAD + b % SP_QUAD;

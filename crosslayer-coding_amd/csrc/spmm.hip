@@ -317,7 +317,6 @@ __global__ __launch_bounds__(DT_WAVES * 64) void k_decode_tiles(TileArgs A) {
   // one after the other: the second hits the L1.)
   const uint32_t pitch_b = (uint32_t)(A.pitch * (int64_t)sizeof(T));
   // Rows past the matrix, which nobody refers to, are read as its last one.
-  // Rows past the matrix, which nobody refers to, are read as its last one.
   const uint32_t off_a = (uint32_t)(wave * 32 + (lane >> 2)) * pitch_b + ((((((uint32_t)lane & 3) >> 1) ^ sp_swap(lane >> 2)) << 5) | ((lane & 1) << 4));
   const uint32_t off_b = off_a + 16 * pitch_b;
   auto last_row = [&](int rows) { return (uint32_t)((rows < SP_ROWS ? rows : SP_ROWS) - 1) * pitch_b + 48u; };
@@ -678,10 +677,9 @@ static SpLayout sp_layout(int64_t rows, int64_t cols, int64_t d, int64_t L, int 
   }
   p.groups_per_part = (int)clt_ceil_div(p.groups, p.parts);
   p.streams = p.parts * waves;
-  // every (layer, tile, group) may leave its last batch part empty, and every stream its last quad; a stream asks for up to three
-  // quads past its end
-  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups + 9;
-  const int64_t rec_batches = l.n_batches + (int64_t)(SP_QUAD - 1) * p.streams + 4 * SP_QUAD;
+  // every (layer, tile, group) may leave its last batch part empty, and every stream its last quad
+  l.n_batches = max_entries / SP_BATCH + (int64_t)p.stages * p.groups;
+  const int64_t rec_batches = l.n_batches + (int64_t)(SP_QUAD - 1) * p.streams + SP_PAST_END;
   size_t at = 0;
   auto take = [&](size_t n) { const size_t here = at; at += align256(n); return here; };
   l.start = take(sizeof(int32_t) * (size_t)L * p.groups * SP_GROUP * (p.tiles + 1));
