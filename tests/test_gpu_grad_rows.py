@@ -142,3 +142,60 @@ def test_lists_longer_than_the_workspace_holds_are_left_alone():
     assert torch.equal(w1, w) and torch.equal(m1, m) and torch.equal(v1, v) and torch.equal(out1, out)
     assert _called_with(surv.capacity, surv, w1, m1, v1, g.cuda(), out1) == [True, True]
     assert not torch.equal(w1, w) and not torch.equal(out1, out)
+
+
+@pytest.mark.parametrize("L,T,F,d,density,by_tile", [(2, 511, 129, 64, 0.05, False), (2, 511, 129, 64, 0.05, True), (3, 700, 140, 96, 0.03, True)])
+def test_moments_of_earlier_steps(L, T, F, d, density, by_tile):
+    """A later step on moments that are not zero, in both their layouts, against the row kernel: m, v and w differ by what the rounding of
+    two gradients makes of them."""
+    surv, dense, w, _, _, g = _problem(L, T, F, d, density, T + F)
+    lists, gd = engine.feature_lists(surv), g.cuda()
+    gen = torch.Generator().manual_seed(7)
+    m, v = torch.randn(w.shape[0], F, d, generator=gen).cuda(), (torch.rand(w.shape[0], F, d, generator=gen) + 0.5).cuda()
+    tile = (lambda a: a.view(-1, F, d // 8, 8).permute(0, 2, 1, 3).contiguous()) if by_tile else (lambda a: a.clone())
+    back = (lambda a: a.permute(0, 2, 1, 3).reshape(-1, F, d)) if by_tile else (lambda a: a)
+    lr, step = 1e-2, 5
+    w1, m1, v1, w2, m2, v2 = w.clone(), tile(m), tile(v), w.clone(), m.clone(), v.clone()
+    engine.decoder_grad_adam_rows(lists, surv, gd, w1, m1, v1, lr, (0.9, 0.999), 1e-8, step)
+    engine.decoder_weight_grad_adam(lists, surv, gd, w2, m2, v2, lr, (0.9, 0.999), 1e-8, step)
+    m1, v1, w1, m2, v2, w2 = (t.cpu().double() for t in (back(m1), back(v1), w1[:, :, :d], m2, v2, w2[:, :, :d]))
+    pairs = [(s, t) for s in range(L) for t in range(s, L)]
+    size = torch.stack([dense[s].double().abs().t() @ g[t].double().abs() for s, t in pairs])
+    grad = torch.stack([dense[s].double().t() @ g[t].double() for s, t in pairs]).abs()
+    ulp = 2.0 ** -23
+    off = size * (T / 8 + 6 + T) * ulp / 2                 # of the two sums together
+    off_m, off_v = 0.1 * off + m2.abs() * 2 * ulp, 0.001 * (2 * grad * off + off * off) + v2 * 2 * ulp
+    assert bool(((m1 - m2).abs() <= off_m).all()) and bool(((v1 - v2).abs() <= off_v).all())
+    c1, c2 = 1 - 0.9 ** step, 1 - 0.999 ** step
+    root = (v2 / c2).sqrt()
+    off_w = lr * (off_m / c1 / root + m2.abs() / c1 / root ** 2 * (off_v / c2 / (2 * root))) + (lr * m2.abs() / c1 / root + w2.abs()) * 4 * ulp
+    assert bool(((w1 - w2).abs() <= off_w).all())
+    assert float((w2 - w.cpu().double()[:, :, :d]).abs().max()) > 1e-3
+
+
+def test_training_from_column_tiles_to_lds_tiles_and_back(monkeypatch):
+    """Batches of three tiles, two and three again: 32-byte column tiles, LDS tiles on moments that stay in column tiles, and column tiles on
+    a copy of the weights that the step before has put out of date; against the kernel row by row."""
+    import crosslayer_coding_amd as cca
+    from crosslayer_coding_amd import synth
+    took, runs = [], []
+    for name in ("decoder_weight_grad_adam_tiled", "decoder_grad_adam_rows", "decoder_weight_grad_adam"):
+        monkeypatch.setattr(engine, name, lambda *a, _f=getattr(engine, name), _n=name, **kw: took.append(_n) or _f(*a, **kw))
+    for tiles in (True, False):
+        model = None
+        for step, T in enumerate((1100, 683, 1100)):
+            wl = synth.Workload("there-and-back", step, 4, 512, 1024, T, "float32", k=16)
+            if model is None:
+                model, _, _ = synth.build_model(wl, torch.device("cuda:0"), 1)
+                opt = cca.CLTAdam(model, lr=1e-3)
+                opt.tile_decoder_step = tiles
+            gen = torch.Generator().manual_seed(step)
+            x = {l: torch.randn(T, 512, generator=gen).cuda() for l in range(4)}
+            y = {l: torch.randn(T, 512, generator=gen).cuda() for l in range(4)}
+            model.training_step(x, y, opt)
+            if tiles:
+                assert opt._dec_cols == 8 and took[-1] == ("decoder_grad_adam_rows" if T == 683 else "decoder_weight_grad_adam_tiled")
+        runs.append([t.clone() for t in opt.decoder_moments()] + [model.decoder_module.packed().clone()])
+    assert took[3:] == ["decoder_weight_grad_adam"] * 3
+    for a, b in zip(*runs):
+        assert float((a - b).norm() / b.norm()) < 1e-4     # a pre-activation at a cut may change sides once weights differ by a rounding
