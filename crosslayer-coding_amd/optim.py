@@ -36,6 +36,7 @@ class CLTAdam:
         self._dec_cols = 0               # CS of "tiles": 64 (matrix-core kernel) or 32 bytes of the model dtype
         self._w_tiles = None             # tiled copy of the decoder weights, valid while _w_tiles_gen matches the slab
         self._w_tiles_gen = None
+        self._batches_apart = 0          # in a row that went over the tiles though another route was faster for them
         cfg = model.config
         L, F, d = cfg.num_layers, cfg.num_features, cfg.d_model
         dev = model.device
@@ -116,6 +117,25 @@ class CLTAdam:
         self.state["dec_w"] = tuple(out)
         self._dec_layout, self._dec_cols = layout, cols
 
+    def _route_from_tiles(self, rows: int, cols: int, generation) -> int:
+        """``engine.grad_rows_wanted``'s answer ``rows`` for a batch that could take column tiles of ``cols``, or 0 where the step stays
+        with those: on the way back from LDS tiles the weights have to be tiled again, and from row by row the moments too.  One
+        batch among others stays, a run of them moves on.  us, of 368 M weights (12 x 768 x 6144): tiling them again 557, the moments there
+        and back 3216; a batch of the other routes saves up to 1324 and 466."""
+        at_tiles = cols > 0 and self._dec_cols == cols and (rows == 2 or self._w_tiles_gen == generation)
+        self._batches_apart = self._batches_apart + 1 if rows and at_tiles else 0
+        if not self._batches_apart:
+            return rows
+        if self._batches_apart < (2 if rows == 1 else 8):
+            return 0
+        if rows == 2:
+            self._w_tiles = self._w_tiles_gen = None        # (its memory is as much as one of the moments takes)
+            try:
+                self._decoder_moments_to("rows")
+            except torch.OutOfMemoryError:                  # no room for them side by side: as they were
+                self._batches_apart, rows = 0, 0
+        return rows
+
     def decoder_moments(self):
         """(m, v) of the decoder weights as [n_dec, F, d] whatever layout the optimiser keeps them in."""
         m, v = self.state["dec_w"]
@@ -155,6 +175,7 @@ class CLTAdam:
             self._after_slab_step(packed, w_dev, w_host, d, F)
             return
         rows = engine.grad_rows_wanted(surv.T, d, F, surv.L, surv.capacity, ws[0].dtype) if self.tile_decoder_step else 0
+        rows = self._route_from_tiles(rows, cs, dec.packed_generation())
         if rows == 1 and self._dec_cols in (0, 8) and engine._aligned16(g_model, packed, *self.state["dec_w"]):
             # (moments either way here too; the slab changes under the tiled copy)
             self._w_tiles_gen = None
@@ -163,7 +184,7 @@ class CLTAdam:
             self._after_slab_step(packed, w_dev, w_host, d, F)
             return
         if rows == 2 and self._dec_layout == "rows":
-            cs = 0                        # short lists row by row, unless a batch before has left the moments in tiles
+            cs = 0                        # short lists row by row
         if cs and all(w.data_ptr() % 16 == 0 for w in ws):
             self._decoder_moments_to("tiles", cs)
             dec._derived_copies = True      # the packed copy tells when the device may have repacked it
