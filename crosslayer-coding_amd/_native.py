@@ -59,6 +59,7 @@ _SIGNATURES = {
     "clt_encode_threshold_recover": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int,
                                             _vp, _i64, _vp, _vp, _sz, _vp]),
     "clt_transpose_grad": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
+    "clt_cast_many": (_int, [_vp, _vp, _vp, _i64, _int, _vp]),
     "clt_poison_if": (_int, [_vp, _i64, _vp, _vp]),
     "clt_pack_decoder": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp]),
     "clt_decode_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),

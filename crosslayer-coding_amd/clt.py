@@ -83,13 +83,12 @@ class _ReconstructionsWithGraph(torch.autograd.Function):
                     g[l] = go.reshape(T, d)
             g_model = g.to(model.dtype)
         raw = model._raw_gradients_from(ctx.inputs, surv, g, g_model, g.sum(dim=1), as_parameters=True)
-        # families of parameters in one cast each; every parameter's gradient has memory of its own, so that one that is kept or
+        # all families of parameters in one cast; every parameter's gradient has memory of its own, so that one that is kept or
         # saved holds no other
-        if (model.dtype != torch.float32
+        if (model.dtype == torch.bfloat16
                 and all(p.dtype == model.dtype for n, p in zip(ctx.names, ctx.params) if not n.startswith("theta_manager."))):
-            for key in ("enc_w", "enc_b", "dec_b", "skip"):
-                if raw.get(key) is not None:
-                    raw[key] = engine.parameter_gradients(raw[key], model.dtype)
+            keys = [key for key in ("enc_w", "enc_b", "dec_b", "skip") if raw.get(key) is not None]
+            raw.update(zip(keys, engine.parameter_gradients([raw[key].contiguous() for key in keys], model.dtype)))
         named = model._named_gradients(raw)
         grads = []
         for name, p in zip(ctx.names, ctx.params):

@@ -697,7 +697,7 @@ def decoder_parameter_grad(lists, surv: SurvivorList, g: torch.Tensor, ws: Optio
     if g.dtype != surv.dtype or F % 8 or not _aligned16(g) or not g.is_contiguous() or not grad_tiles_supported(T, d, F, L, n, surv.dtype):
         return None
     if separate:
-        out = [torch.empty((d, F), dtype=surv.dtype, device=g.device) for _ in range(n_dec)]
+        out = _apart(n_dec, (d, F), surv.dtype, g.device)
     else:
         out = torch.empty((n_dec, d, F), dtype=surv.dtype, device=g.device)
     addresses = (ctypes.c_void_p * n_dec)(*[t.data_ptr() for t in out])
@@ -973,15 +973,27 @@ def parameter_gradient(g: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return g.to(dtype)
 
 
-def parameter_gradients(stack: torch.Tensor, dtype: torch.dtype) -> List[torch.Tensor]:
-    """The raw gradients of a family of parameters, [n, ...], as n tensors of ``dtype`` with memory of their own, small ones in few
-    launches (us together / one cast each: 21 of 512 x 512 52 / 123), large ones, which memory bounds, one by one (12 of 6144 x 768 92 / 85,
-    6 of 16384 x 512 85 / 60)."""
-    parts = stack.unbind(0)
-    if stack.dtype != dtype and parts[0].numel() >= 1 << 22:
-        return [part.to(dtype) for part in parts]
-    out = [torch.empty_like(part, dtype=dtype) for part in parts]
-    torch._foreach_copy_(out, parts)
+def _apart(n: int, shape, dtype: torch.dtype, device) -> List[torch.Tensor]:
+    """n tensors with memory of their own."""
+    first = torch.empty(shape, dtype=dtype, device=device)
+    return [first] + [torch.empty_like(first) for _ in range(n - 1)]
+
+
+def parameter_gradients(families: List[torch.Tensor], dtype: torch.dtype) -> List[List[torch.Tensor]]:
+    """The raw fp32 gradients of families of parameters, [n, ...] each, as n tensors of ``dtype`` with memory of their own."""
+    assert all(g.dtype == torch.float32 and g.is_contiguous() for g in families)
+    out = [_apart(g.shape[0], g.shape[1:], dtype, g.device) for g in families]
+    source, target, size = [], [], []
+    for g, parts in zip(families, out):
+        base, n = g.data_ptr(), g.numel() // g.shape[0]
+        source += [base + 4 * n * i for i in range(len(parts))]
+        target += [part.data_ptr() for part in parts]
+        size += [n] * len(parts)
+    count = len(size)
+    source, target, size = (ctypes.c_void_p * count)(*source), (ctypes.c_void_p * count)(*target), (ctypes.c_int64 * count)(*size)
+    code = nat.load().clt_cast_many(ctypes.addressof(source), ctypes.addressof(target), ctypes.addressof(size), count,
+                                    nat.dtype_code(dtype), _stream(families[0]))
+    nat.check(code, "clt_cast_many")
     return out
 
 

@@ -294,6 +294,12 @@ int clt_poison_if(void *buf, int64_t bytes, const int32_t *flag, void *stream);
 int clt_transpose_grad(const float *g, void *out, int64_t F, int64_t d, int dtype, void *stream);
 
 /*
+ * to[i][0 .. n[i]) (bf16) = from[i][0 .. n[i]) (fp32), rounded to nearest even, for `count` tensors in few launches.  from, to and n are
+ * host arrays, read before the call returns; a tensor may begin at any address its type allows.  No counterpart in the reference.
+ */
+int clt_cast_many(const float *const *from, void *const *to, const int64_t *n, int64_t count, int dtype, void *stream);
+
+/*
  * clt_threshold_count for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
  * Same arguments and result as clt_threshold_count without the workspace: the per-row counters live
