@@ -694,7 +694,12 @@ def run_backward(args):
     else:
         dw_dec = timed(dw_name, lambda: engine.decoder_weight_grad(lists, surv, g_model, cfg.decoder_tying))
     _, x_slab, _, _ = model.encoder_module.prepare_slab(inputs)
-    dw_enc, db_enc = timed("encoder weight gradient", lambda: engine.encoder_weight_grad(lists, dval, x_slab.contiguous(), F))
+    x_slab = x_slab.contiguous()
+    if opt is not None and opt.fuses_encoder_step(x_slab, surv.capacity):
+        dw_enc, db_enc = None, torch.empty((L, F), dtype=torch.float32, device=dev)
+        timed("encoder weight gradient + its Adam step in place", lambda: opt.encoder_weight_step(lists, dval, x_slab, db_enc))
+    else:
+        dw_enc, db_enc = timed("encoder weight gradient", lambda: engine.encoder_weight_grad(lists, dval, x_slab, F))
     if opt is not None:
         dec_b = bias_grad[torch.tensor([t for s_ in range(L) for t in range(s_, L)], device=dev)].contiguous()
         timed("Adam (other parameters)" if fused else "Adam",
