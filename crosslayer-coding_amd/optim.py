@@ -84,10 +84,11 @@ class CLTAdam:
 
     def fuses_encoder_step(self, x: torch.Tensor, entries: int = 0) -> bool:
         """Whether the encoder weights take their Adam step inside the weight-gradient kernel, for the batch ``x`` [L, T, d] with
-        ``entries`` survivors (``fuse_encoder_step = False`` switches it off)."""
+        ``entries`` survivors (``fuse_encoder_step = False`` switches it off).  An optimiser with a ``step`` of its own sees all
+        gradients but the fused decoders'."""
         from . import engine
         w, _ = self.model.encoder_module.stacked()
-        return (self.fuse_encoder_step and w.dtype == x.dtype and engine.encoder_step_fits(x.shape[2], x.dtype)
+        return (self.fuse_encoder_step and getattr(self.step, "__func__", None) is CLTAdam.step and w.dtype == x.dtype and engine.encoder_step_fits(x.shape[2], x.dtype)
                 and engine.encoder_step_wanted(entries, w.shape[1], w.shape[0]) and engine._aligned16(x, w, *self.state["enc_w"]))
 
     @torch.no_grad()
